@@ -19,14 +19,19 @@
 //    point's position in its list. A point's later co-members in partition p
 //    are then the suffix of its cluster's list after its own position: no
 //    search and no pair materialisation.
-//  * Count/fill: one workgroup per row (rows handed out by atomic counters,
-//    one per XCD over its own stretch of the rows). Columns are covered in windows of 32768; each window has a
-//    dense array of u16 counters (two per u32 word, 64 KiB of LDS). Per window every partition's
-//    suffix cursor advances over the members inside the window (flattened
-//    over partitions so that lanes stream consecutive members), each member
-//    an LDS atomic increment. The window is then read in column order: pass 1
-//    counts non-zeros (row nnz, max count), pass 2 writes (col, value) after
-//    a block scan, so rows come out sorted without a per-row sort.
+//  * Count/fill: one workgroup per row (rows handed out by atomic counters).
+//    Columns are covered in windows of 16384; each window has a dense array
+//    of byte counters (16 KiB of LDS, seven workgroups per compute unit; u16
+//    beyond 255 partitions). Per window every partition's suffix cursor
+//    advances over the members inside the window (flattened over partitions
+//    so that lanes stream consecutive members), each member an LDS atomic
+//    increment. The window is then read in column order: pass 1 counts
+//    non-zeros (row nnz, max count), pass 2 writes (col, value) after a block
+//    scan, so rows come out sorted without a per-row sort. Bound: vector
+//    issue (0.6 instructions per unit and cycle, about 37 per 64 visits).
+//    Byte counters and windows emitted by set bit instead of by column took
+//    the whole build of 200,003 points x 64 partitions (4.6 G visits, 905 M
+//    entries) from 36.8 to 10.7 ms, and of 10,000 x 100 from 0.67 to 0.51.
 //  * Row offsets: exclusive scan of the per-row nnz into int64 (nnz > 2^31
 //    for the large ensembles).
 #include <cstring>
@@ -41,8 +46,11 @@ namespace {
 constexpr int kCB = 256;       // threads per row workgroup
 constexpr int kWin = 32768;    // columns per LDS window (two u16 counters per u32 word)
 constexpr int kMaxP = 1024;    // partitions staged in LDS
-constexpr int kMaxRanges = 8;  // row ranges (one per XCD)
-constexpr int kCtrs = kMaxRanges + 2;  // row counters, then the sampled nnz sum
+constexpr int kMaxRanges = 8;  // contiguous row ranges (one per XCD)
+constexpr int kStripes = 32;   // interleaved row ranges of a small matrix
+constexpr int kCtrPad = 16;    // row counters 128 bytes apart
+constexpr int kCtrSum = kStripes * kCtrPad;  // after the counters: the sampled nnz sum
+constexpr int kCtrs = kCtrSum + 2;
 
 // keys: global cluster id (unassigned points -> ktot, sorted last);
 // values: p * n + i
@@ -105,10 +113,16 @@ __global__ void k_win_table(const uint32_t* __restrict__ skey, const int32_t* __
   }
 }
 
-// 64-bit words of a window's run-start bitmap: the short-run path covers
-// fewer than 32 flattened members per partition (rounded up to an even
-// count: the counters after it stay 16-byte aligned).
-__host__ __device__ inline int co_bm_words(int P) { return ((P / 2 + 1) + 1) & ~1; }
+// 64-bit words of a window's run-start bitmap: the flattened path covers
+// windows of up to 128 members per partition on average (32 beyond 256
+// partitions, where the bitmap would crowd out the counters).
+__host__ __device__ inline int co_bm_words(int P) {
+  return P <= 256 ? 2 * P + 2 : ((P / 2 + 1) + 1) & ~1;
+}
+
+// Window counters are bytes while every count fits one: a pair meets at most
+// once per partition, so P <= 255; u16 beyond.
+inline bool co_bytes(int P) { return P <= 255; }
 
 struct CoPlan {
   const int32_t* labels;
@@ -121,13 +135,14 @@ struct CoPlan {
   const int32_t* wtab;    // window table (nullptr: search the window ends)
   int nw;                 // windows of the table: ceil(n / win)
   const int32_t* first;   // ranked fill: the partition processed first (device)
-  int ranges;             // row ranges with a counter each (1..kMaxRanges)
+  int ranges;             // row ranges with a counter each: contiguous ones
+                          // (1..kMaxRanges), or interleaved (-kStripes)
   int64_t row_stride;     // > 1: only rows 0, stride, 2*stride, ... (a sample)
 };
 
 // Outputs of the row kernel (pointers a pass does not use are null).
 struct CoOut {
-  unsigned long long* row_ctr;  // [kMaxRanges] row counters, zeroed
+  unsigned long long* row_ctr;  // row counters kCtrPad apart, zeroed
   int32_t* row_nnz;             // PASS 0 / 2: nnz of each row
   unsigned int* max_count;      // PASS 0 / 2: largest count
   unsigned long long* nnz_sum;  // PASS 0: sum of the visited rows' nnz
@@ -178,6 +193,63 @@ __global__ __launch_bounds__(256) void k_first_partition(const int32_t* __restri
   if (threadIdx.x == 0) first[0] = (int32_t)(s_best & 0xffffffffu);
 }
 
+// Window counters of type CT (u8 or u16): the words they take (a multiple of
+// four, read 16 bytes at a time) and how a lane reads them.
+__host__ __device__ inline int co_cnt_words(int win, int bytes) {
+  return ((win * bytes + 15) / 16) * 4;
+}
+template <typename CT>
+struct CoCnt {
+  static constexpr int kB = (int)sizeof(CT);
+  static constexpr int kPerWord = 4 / kB;   // columns per 32-bit word
+  static constexpr int kPerGroup = 16 / kB; // columns per 16-byte group
+  static constexpr int kPerLane = 2 * kPerGroup;  // columns a lane emits at a time
+  // emission steps of a full window (kWin columns over kCB lanes): unrolled
+  static constexpr int kIters = kWin / kPerLane / kCB;
+  // one count for window column jj
+  static __device__ __forceinline__ void add(uint32_t* cnt, int jj) {
+    if (kB == 1) atomicAdd(&cnt[jj >> 2], 1u << ((jj & 3) * 8));
+    else atomicAdd(&cnt[jj >> 1], 1u << ((jj & 1) * 16));
+  }
+  // bit c of the result: column c of the group has a non-zero counter. The
+  // high bit of each counter of ((x & lo) + lo) | x is set iff the counter
+  // is non-zero (lo: all bits but the high one); a byte dot product with
+  // the weights 1, 2, 4, 8 gathers a word's four flags (times 128).
+  static __device__ __forceinline__ uint32_t mask(const uint4& x) {
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+    if (kB == 1) {
+      uint32_t m = 0;
+#pragma unroll
+      for (int q = 3; q >= 0; --q) {
+        const uint32_t u =
+            (((w[q] & 0x7f7f7f7fu) + 0x7f7f7f7fu) | w[q]) & 0x80808080u;
+        m = (m << 4) + __builtin_amdgcn_udot4(u, 0x08040201u, 0u, false);
+      }
+      return m >> 7;
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int q = 3; q >= 0; --q) {
+      const uint32_t u = (((w[q] & 0x7fff7fffu) + 0x7fff7fffu) | w[q]) & 0x80008000u;
+      m = (m << 2) | (u >> 31 << 1) | ((u >> 15) & 1u);
+    }
+    return m;
+  }
+  static __device__ __forceinline__ uint32_t max_of(const uint4& x, uint32_t mx) {
+    const uint32_t w[4] = {x.x, x.y, x.z, x.w};
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (kB == 1) {
+        mx = max(mx, max(w[q] & 0xffu, w[q] >> 24));
+        mx = max(mx, max((w[q] >> 8) & 0xffu, (w[q] >> 16) & 0xffu));
+      } else {
+        mx = max(mx, max(w[q] & 0xffffu, w[q] >> 16));
+      }
+    }
+    return mx;
+  }
+};
+
 // One row: walk every partition's co-members > i (or all co-members != i for
 // full rows) window by window. PASS 0: per-row nnz and max count. PASS 1:
 // write (col, value) at indptr[i]. RANK (PASS 1 only): also write, per entry,
@@ -189,29 +261,31 @@ __global__ __launch_bounds__(256) void k_first_partition(const int32_t* __restri
 // segment table, and the row's nnz and the max count as in PASS 0; a
 // workgroup that finds the pool used up sets the overflow flag and stops.
 // U: member loads in flight per lane while visiting (4 or 8, a tuning knob).
-template <int PASS, bool RANK = false, int U = 4>
+template <int PASS, bool RANK, int U, typename CT>
 __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, int win,
                                                       CoOut out) {
+  using Cnt = CoCnt<CT>;
   unsigned long long* __restrict__ row_ctr = out.row_ctr;
   const int64_t* __restrict__ indptr = out.indptr;
   const int32_t w_offset = out.w_offset;
   int32_t* __restrict__ out_col = out.col;
   int32_t* __restrict__ out_val = out.val;
   int32_t* __restrict__ out_rank = out.rank;
-  // launch-time LDS: this window's run-start bitmap (co_bm_words(P)
-  // 64-bit words), the window counters (win / 2 words), with RANK the rank
-  // window (win words), then per partition the next member position, the
-  // cluster end, this window's member end and the flattened-range prefix
-  // (P + 1), the row's global cluster, this window's member position minus
-  // flattened index, each partition's rank; per run (non-empty partition
-  // range of this window) the position delta and the partition's rank; per
-  // bitmap word the run starts before it
+  // launch-time LDS: this window's run-start bitmap (co_bm_words(P) entries
+  // of 16 bytes: 64 bits, then the run starts marked in the words before),
+  // the window counters, with RANK the rank window (win words), then per
+  // partition the next member position, the cluster end, this window's
+  // member end and the flattened-range prefix (P + 1), the row's global
+  // cluster, this window's member position minus flattened index, each
+  // partition's rank; per run (non-empty partition range of this window) the
+  // position delta and the partition's rank
   extern __shared__ __align__(16) uint32_t s_dyn[];
-  uint64_t* s_bm = reinterpret_cast<uint64_t*>(s_dyn);
+  uint4* s_bm = reinterpret_cast<uint4*>(s_dyn);
   const int bmw = co_bm_words(pl.P);
-  uint32_t* s_cnt = s_dyn + 2 * bmw;
-  uint32_t* s_rank = s_cnt + win / 2;
-  int32_t* s_cur = reinterpret_cast<int32_t*>(s_cnt + win / 2 + (RANK ? win : 0));
+  const int cwords = co_cnt_words(win, Cnt::kB);
+  uint32_t* s_cnt = s_dyn + 4 * bmw;
+  uint32_t* s_rank = s_cnt + cwords;
+  int32_t* s_cur = reinterpret_cast<int32_t*>(s_cnt + cwords + (RANK ? win : 0));
   int32_t* s_end = s_cur + pl.P;
   int32_t* s_hi = s_end + pl.P;
   int32_t* s_pre = s_hi + pl.P;
@@ -220,17 +294,20 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
   int32_t* s_prank = s_d + pl.P;
   int32_t* s_dr = s_prank + pl.P;   // per run: member position - flattened index
   int32_t* s_rp = s_dr + pl.P;      // per run: rank of its partition
-  int32_t* s_wpre = s_rp + pl.P;    // per bitmap word: run starts in the words before
+  const uint4* s4 = reinterpret_cast<const uint4*>(s_cnt);
+  typedef CT __attribute__((may_alias)) CtAlias;
+  const CtAlias* s_ct = reinterpret_cast<const CtAlias*>(s_cnt);
   __shared__ uint32_t s_tmp[kCB / kWave + 1];
   __shared__ int64_t s_row;
   __shared__ unsigned long long s_chunk;
   __shared__ unsigned int s_max;
   const int t = threadIdx.x;
+  const int wv = __builtin_amdgcn_readfirstlane(t / kWave), ln = lane_id();
   const int64_t n = pl.n;
   const int P = pl.P;
   // the window is cleared once here; afterwards every window clears the
-  // words it used while reading them, so a clean window costs no pass
-  for (int v = t; v < win / 2; v += kCB) s_cnt[v] = 0;
+  // groups it used while reading them, so a clean window costs no pass
+  for (int v = t; v < cwords; v += kCB) s_cnt[v] = 0;
   if (RANK) {
     for (int v = t; v < win; v += kCB) s_rank[v] = ~0u;
     const int f = pl.first[0];
@@ -247,6 +324,12 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
   // through its own stretch of the order and its resident rows share their
   // clusters' member lists in that L2. A workgroup whose range is used up
   // moves on to the next ranges (thread 0 keeps the cursor).
+  // A small matrix (its member lists fit every L2) is bound by the counters
+  // instead: atomics on one address serialise at about 16 ns each, 160 us
+  // for 10,000 rows. There pl.ranges = -kStripes: row r belongs to range
+  // r mod kStripes, so the ranges cost alike, and a workgroup whose range is
+  // used up is done (10,000 rows x 100 partitions: the count pass 163 us
+  // with one counter).
   const int32_t* order = nullptr;
   {
     const int32_t a = pl.cstart[pl.k_off[0]], b = pl.cstart[pl.k_off[1]];
@@ -256,23 +339,29 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
   const int64_t stride = pl.row_stride > 1 ? pl.row_stride : 1;
   const int64_t nrows = (n + stride - 1) / stride;
   if (stride > 1) order = nullptr;
-  int xr = (int)(blockIdx.x % (unsigned)pl.ranges), tries = 0;
+  const int nctr = pl.ranges < 0 ? -pl.ranges : pl.ranges;
+  int xr = (int)(blockIdx.x % (unsigned)nctr), tries = 0;
   // PASS 2: the workgroup's pool chunk [chunk_pos, chunk_end) (uniform)
   int64_t chunk_pos = 0, chunk_end = 0;
-  uint32_t mx_row = 0;  // PASS 2: largest count this lane emitted
-  if (t == 0) s_max = 0;  // a workgroup may get no row
+  uint32_t mx_row = 0;  // largest count this lane met
+  if (t == 0) s_max = 0;
   for (;;) {
     if (t == 0) {
       int64_t r = nrows;
-      while (tries < pl.ranges) {
-        const int64_t lo = nrows * xr / pl.ranges, hi = nrows * (xr + 1) / pl.ranges;
-        const int64_t q = lo + (int64_t)atomicAdd(&row_ctr[xr], 1ull);
-        if (q < hi) {
-          r = q;
-          break;
+      if (pl.ranges < 0) {
+        r = xr + nctr * (int64_t)atomicAdd(&row_ctr[xr * kCtrPad], 1ull);
+        if (r > nrows) r = nrows;
+      } else {
+        while (tries < nctr) {
+          const int64_t lo = nrows * xr / nctr, hi = nrows * (xr + 1) / nctr;
+          const int64_t q = lo + (int64_t)atomicAdd(&row_ctr[xr * kCtrPad], 1ull);
+          if (q < hi) {
+            r = q;
+            break;
+          }
+          xr = xr + 1 == nctr ? 0 : xr + 1;
+          ++tries;
         }
-        xr = xr + 1 == pl.ranges ? 0 : xr + 1;
-        ++tries;
       }
       s_row = r;
     }
@@ -280,7 +369,6 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
     const int64_t r = s_row;
     if (r >= nrows) break;
     const int64_t i = order ? (int64_t)order[r] : r * stride;
-    if (t == 0) s_max = 0;
     for (int p = t; p < P; p += kCB) {
       int32_t q = pl.pos[(int64_t)p * n + i];
       if (q < 0) {  // unassigned in partition p
@@ -299,10 +387,11 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
     const int64_t w_first = full_rows ? 0 : (i + 1) / win;
     const int64_t seg0 = PASS == 2 ? seg_base(i, win, pl.nw, full_rows) : 0;
     uint32_t nnz_local = 0;
+    const int self = full_rows ? (int)i : -1;  // full rows skip the diagonal
     // windows aligned to multiples of win (columns <= i get no counts)
     for (int64_t c0 = full_rows ? 0 : ((i + 1) / win) * win; c0 < n; c0 += win) {
       const int64_t c1 = c0 + win < n ? c0 + win : n;
-      for (int v = t; v < bmw; v += kCB) s_bm[v] = 0ull;  // read back after the next barrier
+      for (int v = t; v < bmw; v += kCB) s_bm[v] = make_uint4(0u, 0u, 0u, 0u);
       // members of this window: [cur, hi) with member < c1 (lists ascending);
       // the last window takes every remaining member, no search. Otherwise
       // an exponential probe from cur (a window holds few members of each
@@ -335,17 +424,19 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
       }
       __syncthreads();
       // flattened ranges: prefix of (hi - cur) over partitions; the runs
-      // (non-empty ranges) in partition order, each start marked in the
-      // bitmap over the flattened indices (short windows), and per bitmap
-      // word the run starts before it. One wavefront: its LDS operations
-      // complete in order, so its bitmap reads see its own marks.
-      if (t < kWave) {
+      // (non-empty ranges) in partition order, each start but the first
+      // marked one index early in the bitmap over the flattened indices
+      // (short windows), and per bitmap word the marks before it: the marks
+      // below flattened index f are then the number of f's run. One
+      // wavefront: its LDS operations complete in order, so its bitmap reads
+      // see its own marks.
+      if (wv == 0) {
         int32_t carry = 0, rcarry = 0;
-        const uint64_t below = (1ull << t) - 1ull;
+        const uint64_t below = (1ull << ln) - 1ull;
         for (int p0 = 0; p0 < P; p0 += kWave) {
-          int p = p0 + t;
+          int p = p0 + ln;
           int32_t len = p < P ? s_hi[p] - s_cur[p] : 0;
-          int32_t inc = wave_incl_scan(len);
+          int32_t inc = (int32_t)wave_incl_scan_dpp((uint32_t)len);
           const uint64_t ne = __ballot(len > 0);
           if (p < P) {
             const int32_t pre = carry + inc - len;
@@ -355,164 +446,164 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
               const int r = rcarry + __popcll(ne & below);
               s_dr[r] = s_cur[p] - pre;
               if (RANK) s_rp[r] = s_prank[p];
-              if (pre < 64 * bmw) atomicOr(&s_bm[pre >> 6], 1ull << (pre & 63));
+              if (pre > 0 && pre <= 64 * bmw) {
+                const int b = pre - 1;
+                atomicOr(&s_dyn[(b >> 6) * 4 + ((b >> 5) & 1)], 1u << (b & 31));
+              }
             }
           }
-          carry += __shfl(inc, kWave - 1, kWave);
+          carry += __builtin_amdgcn_readlane(inc, kWave - 1);
           rcarry += __popcll(ne);
         }
-        if (t == 0) s_pre[P] = carry;
-        if (carry < 32 * P) {  // the bitmap covers the window: word prefix counts
+        if (ln == 0) s_pre[P] = carry;
+        if (carry <= 64 * bmw) {  // the bitmap covers the window: word prefix counts
           const int W = (carry + 63) >> 6;
           int32_t wc = 0;
           for (int w0 = 0; w0 < W; w0 += kWave) {
-            const int w = w0 + t;
-            const int32_t c = w < W ? (int32_t)__popcll(s_bm[w]) : 0;
-            const int32_t ci = wave_incl_scan(c);
-            if (w < W) s_wpre[w] = wc + ci - c;
-            wc += __shfl(ci, kWave - 1, kWave);
+            const int w = w0 + ln;
+            const int32_t c = w < W ? __popc(s_dyn[4 * w]) + __popc(s_dyn[4 * w + 1]) : 0;
+            const int32_t ci = (int32_t)wave_incl_scan_dpp((uint32_t)c);
+            if (w < W) s_dyn[4 * w + 2] = (uint32_t)(wc + ci - c);
+            wc += __builtin_amdgcn_readlane(ci, kWave - 1);
           }
         }
       }
       __syncthreads();
       const int32_t tot = s_pre[P];
-      // Flattened member index f -> partition p with s_pre[p] <= f <
-      // s_pre[p+1], member position f + s_d[p]; U member loads in flight
-      // per lane, consecutive lanes on consecutive f (coalesced). Long runs
-      // (32+ members per partition on average): lanes stride the block
-      // (f = t, t + kCB, ...) and walk the few boundaries each step crosses.
-      // Short runs: each wavefront takes U * 64 consecutive f per step; a
-      // wave-uniform cursor finds the partition of the step's first f by a
-      // ballot over 64 boundaries at a time; the next 64 boundaries are held
-      // one per lane, and for each 64-wide sub-block one ballot counts
-      // those before it while the few falling inside it are compared one by
-      // one (a wave-uniform readlane each), so the search costs a few
-      // instructions per boundary crossed and no LDS traffic (steps
-      // spanning more than 64 partitions walk instead).
-      if (tot >= 32 * P) {
+      const int c0i = (int)c0;
+      auto visit = [&](int32_t j, int32_t rk) {
+        const int jj = j - c0i;
+        Cnt::add(s_cnt, jj);
+        if (RANK) atomicMin(&s_rank[jj], (uint32_t)rk);
+      };
+      // Flattened member index f -> member position f + delta of its run; U
+      // member loads in flight per lane, consecutive lanes on consecutive f
+      // (coalesced). While the bitmap covers the window (up to 128 members
+      // per partition on average) each wavefront takes U * 64 consecutive f
+      // per step and f's run is the number of marks below f: those in the
+      // words before (one broadcast read with the word) plus a masked bit
+      // count. Longer windows: the flattened range is split evenly over the
+      // wavefronts and each walks its runs one after the other with
+      // wave-uniform bounds, U * 64 members of a run per step (on average
+      // at least two steps' worth of lanes per run, so few are idle, and no
+      // per-member search). Whole steps run without a bounds check.
+      if (tot > 64 * bmw) {
+        const int32_t share = (tot + kCB / kWave - 1) / (kCB / kWave);
+        const int32_t fa = wv * share, fb = fa + share < tot ? fa + share : tot;
         int p = 0;
-        for (int32_t f0 = t; f0 < tot; f0 += U * kCB) {
-          int32_t j[U];
-          int pu[U];
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int32_t f = f0 + u * kCB;
-            j[u] = -1;
-            if (f < tot) {
-              while (s_pre[p + 1] <= f) ++p;
-              j[u] = pl.members[f + s_d[p]];
-            }
-            pu[u] = p;
-          }
-#pragma unroll
-          for (int u = 0; u < U; ++u) {
-            if (j[u] < 0 || (full_rows && j[u] == (int32_t)i)) continue;
-            const int jj = (int)(j[u] - c0);
-            atomicAdd(&s_cnt[jj >> 1], 1u << (16 * (jj & 1)));
-            if (RANK) atomicMin(&s_rank[jj], (uint32_t)s_prank[pu[u]]);
+        if (fa < fb) {
+          int hi = P;  // s_pre[p] <= fa < s_pre[hi]
+          while (hi - p > 1) {
+            const int mid = (p + hi) >> 1;
+            if (s_pre[mid] <= fa) p = mid; else hi = mid;
           }
         }
-      } else {
-        // short runs: each wavefront takes U * 64 consecutive f per step;
-        // f's run = (run starts at or before f) - 1: the starts before its
-        // 64-bit bitmap word (prefix) plus a popcount of the word up to f
-        const int wv = t / kWave, ln = lane_id();
-        const uint64_t upto = ln == kWave - 1 ? ~0ull : ((2ull << ln) - 1ull);
-        for (int32_t base = wv * U * kWave; base < tot; base += U * kCB) {
+        for (int32_t f = fa; f < fb;) {
+          const int32_t re = __builtin_amdgcn_readfirstlane(s_pre[p + 1]);
+          const int32_t* __restrict__ mp =
+              pl.members + __builtin_amdgcn_readfirstlane(s_d[p]);
+          const int32_t rk = RANK ? s_prank[p] : 0;
+          const int32_t e = re < fb ? re : fb;
           int32_t j[U];
-          int32_t rk[U];
+          for (; f + U * kWave <= e; f += U * kWave) {
 #pragma unroll
-          for (int u = 0; u < U; ++u) {
-            const int32_t f0 = base + u * kWave, f = f0 + ln;
-            j[u] = -1;
-            rk[u] = 0;
-            if (f < tot) {
-              const int w = f0 >> 6;
-              const int r = s_wpre[w] + (int)__popcll(s_bm[w] & upto) - 1;
-              j[u] = pl.members[f + s_dr[r]];
-              if (RANK) rk[u] = s_rp[r];
+            for (int u = 0; u < U; ++u) j[u] = mp[f + u * kWave + ln];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (!full_rows || j[u] != self) visit(j[u], rk);
+          }
+          if (f < e) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+              const int32_t q = f + u * kWave + ln;
+              j[u] = q < e ? mp[q] : -1;
             }
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (j[u] >= 0 && j[u] != self) visit(j[u], rk);
           }
+          f = e;
+          ++p;
+        }
+      } else {
+        // member position and rank slot of flattened index base + 64 u + lane
+        auto place = [&](int32_t base, int u, int32_t& rk) {
+          const uint4 w = s_bm[(base >> 6) + u];
+          const uint32_t r = __builtin_amdgcn_mbcnt_hi(w.y, __builtin_amdgcn_mbcnt_lo(w.x, w.z));
+          if (RANK) rk = s_rp[r];
+          return base + u * kWave + ln + s_dr[r];
+        };
+        int32_t base = wv * U * kWave;
+        for (; base + U * kWave <= tot; base += U * kCB) {
+          int32_t j[U], rk[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) j[u] = pl.members[place(base, u, rk[u])];
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (!full_rows || j[u] != self) visit(j[u], rk[u]);
+        }
+        if (base < tot) {
+          int32_t j[U], rk[U];
 #pragma unroll
           for (int u = 0; u < U; ++u) {
-            if (j[u] < 0 || (full_rows && j[u] == (int32_t)i)) continue;
-            const int jj = (int)(j[u] - c0);
-            atomicAdd(&s_cnt[jj >> 1], 1u << (16 * (jj & 1)));
-            if (RANK) atomicMin(&s_rank[jj], (uint32_t)rk[u]);
+            j[u] = -1;
+            if (base + u * kWave + ln < tot) j[u] = pl.members[place(base, u, rk[u])];
           }
+#pragma unroll
+          for (int u = 0; u < U; ++u)
+            if (j[u] >= 0 && j[u] != self) visit(j[u], rk[u]);
         }
       }
       __syncthreads();
       for (int p2 = t; p2 < P; p2 += kCB) s_cur[p2] = s_hi[p2];
-      // read the window four words (eight columns) per lane and load, clearing
-      // the words it used; PASS 1 emits them in column order
+      // read the window 16 bytes of counters per lane and load (the groups
+      // past the window's width stay zero), clearing the groups it used
       const int width = (int)(c1 - c0);
-      const int words = (width + 1) >> 1;
-      const int groups = (words + 3) >> 2;  // 4-word groups, the last may be partial
-      uint4* s4 = reinterpret_cast<uint4*>(s_cnt);
-      // words 4g..4g+3 of group g (zeros past the window), cleared when used
-      auto read_group = [&](int g, uint32_t* xw) {
-        if (4 * g + 4 <= words) {
-          const uint4 x = s4[g];
-          xw[0] = x.x; xw[1] = x.y; xw[2] = x.z; xw[3] = x.w;
-          if (x.x | x.y | x.z | x.w) s4[g] = make_uint4(0u, 0u, 0u, 0u);
-        } else {
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int v = 4 * g + q;
-            xw[q] = v < words ? s_cnt[v] : 0u;
-            if (xw[q]) s_cnt[v] = 0u;
-          }
-        }
-      };
+      const int groups = (width + Cnt::kPerGroup - 1) / Cnt::kPerGroup;
+      uint4* s4w = reinterpret_cast<uint4*>(s_cnt);
       if (PASS == 0) {
-        uint32_t c = 0, mx = 0;
+        uint32_t c = 0;
         for (int g = t; g < groups; g += kCB) {
-          uint32_t xw[4];
-          read_group(g, xw);
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const uint32_t lo = xw[q] & 0xffffu, hi = xw[q] >> 16;
-            c += (lo != 0) + (hi != 0);
-            mx = lo > mx ? lo : mx;
-            mx = hi > mx ? hi : mx;
+          const uint4 x = s4[g];
+          if (x.x | x.y | x.z | x.w) {
+            s4w[g] = make_uint4(0u, 0u, 0u, 0u);
+            c += __popc(Cnt::mask(x));
+            mx_row = Cnt::max_of(x, mx_row);
           }
         }
         nnz_local += c;
-        if (mx) atomicMax(&s_max, mx);
       } else {  // PASS 1 and 2
-        // wave w emits groups [w*RG, (w+1)*RG) in column order
-        const int w = t / kWave, l = lane_id();
-        const int RG = ((groups + 4 * kWave - 1) / (4 * kWave)) * kWave;
-        const int ga = w * RG, gb = (w + 1) * RG < groups ? (w + 1) * RG : groups;
-        // non-zero 16-bit halves of a group: the high bit of each half of
-        // ((x & 0x7fff7fff) + 0x7fff7fff) | x is set iff the half is non-zero
-        auto nz_count = [](const uint32_t* xw) {
-          uint32_t c = 0;
-#pragma unroll
-          for (int q = 0; q < 4; ++q)
-            c += __popc((((xw[q] & 0x7fff7fffu) + 0x7fff7fffu) | xw[q]) & 0x80008000u);
-          return c;
-        };
+        // Wave w emits lane pieces (two groups each) [w*RG, (w+1)*RG) in
+        // column order. First the non-zero masks of its pieces (kept in
+        // registers: a window has few entries, about one column in twenty
+        // on the large ensembles, so reading the counters is most of the
+        // work), then per 64 pieces one prefix sum and a loop that takes the
+        // set bits of each lane's mask one by one, so the instructions
+        // follow the entries and not the columns.
+        const int pieces = (groups + 1) >> 1;
+        const int RG = ((pieces + 4 * kWave - 1) / (4 * kWave)) * kWave;
+        const int ga = wv * RG, gb = (wv + 1) * RG < pieces ? (wv + 1) * RG : pieces;
+        uint32_t mk[Cnt::kIters];
         uint32_t c = 0;
-        for (int g = ga + l; g < gb; g += kWave) {
-          uint32_t xw[4];
-          if (4 * g + 4 <= words) {
-            const uint4 x = s4[g];
-            xw[0] = x.x; xw[1] = x.y; xw[2] = x.z; xw[3] = x.w;
-          } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) xw[q] = 4 * g + q < words ? s_cnt[4 * g + q] : 0u;
+        for (int it = 0; it < Cnt::kIters; ++it) {
+          mk[it] = 0;
+          if (ga + it * kWave < gb) {  // uniform
+            const int g = 2 * (ga + it * kWave + ln);
+            if (g < groups) {
+              mk[it] = Cnt::mask(s4[g]);
+              if (g + 1 < groups) mk[it] |= Cnt::mask(s4[g + 1]) << Cnt::kPerGroup;
+            }
+            c += __popc(mk[it]);
           }
-          c += nz_count(xw);
         }
-        c = wave_sum(c);
-        if (l == 0) s_tmp[w] = c;
+        c = __builtin_amdgcn_readlane(wave_incl_scan_dpp(c), kWave - 1);
+        if (ln == 0) s_tmp[wv] = c;
         __syncthreads();
         int64_t o = row_base + written;
         uint32_t wtot = 0;
         for (int q = 0; q < kCB / kWave; ++q) {
-          if (q < w) o += s_tmp[q];
+          if (q < wv) o += s_tmp[q];
           wtot += s_tmp[q];
         }
         if (PASS == 2) {  // block-uniform: wtot, chunk_pos, chunk_end
@@ -532,51 +623,42 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
                 wtot ? ((uint64_t)chunk_pos << 16) | (uint64_t)wtot : 0ull;
           chunk_pos += wtot;
         }
-        for (int g0 = ga; g0 < gb; g0 += kWave) {
-          const int g = g0 + l;
-          uint32_t xw[4] = {0u, 0u, 0u, 0u};
-          if (g < gb) read_group(g, xw);
-          const uint32_t cnt = nz_count(xw);
-          if (__ballot(cnt != 0u) == 0ull) continue;  // wave-uniform: no entry in these groups
-          const uint32_t incl = wave_incl_scan(cnt);
-          int64_t at = o + (incl - cnt);
-          if (PASS == 2) {
+        uint32_t* __restrict__ po = PASS == 2 ? out.pool + o : nullptr;
+        int32_t* __restrict__ pc = PASS == 1 ? out_col + o : nullptr;
+        int32_t* __restrict__ pv = PASS == 1 ? out_val + o : nullptr;
+        int32_t* __restrict__ pr = PASS == 1 && RANK ? out_rank + o : nullptr;
+        uint32_t done = 0;  // entries this wave wrote before (uniform)
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-              const uint32_t lo = xw[q] & 0xffffu, hi = xw[q] >> 16;
-              const uint32_t cw = 2u * (uint32_t)(4 * g + q);  // column - c0
-              if (lo) out.pool[at++] = (lo << 16) | cw;
-              if (hi) out.pool[at++] = (hi << 16) | (cw + 1u);
-              mx_row = lo > mx_row ? lo : mx_row;
-              mx_row = hi > mx_row ? hi : mx_row;
-            }
-            o += __shfl(incl, kWave - 1, kWave);
-            continue;
-          }
-#pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const uint32_t lo = xw[q] & 0xffffu, hi = xw[q] >> 16;
-            const int32_t col = (int32_t)(c0 + 2 * (4 * g + q));
-            if (lo) {
-              out_col[at] = col;
-              out_val[at] = w_offset ? w_offset - (int32_t)lo : (int32_t)lo;
+        for (int it = 0; it < Cnt::kIters; ++it) {
+          if (ga + it * kWave >= gb) break;  // uniform
+          uint32_t m = mk[it];
+          if (__ballot(m != 0u) == 0ull) continue;
+          const uint32_t cnt = __popc(m);
+          const uint32_t incl = wave_incl_scan_dpp(cnt);
+          uint32_t at = done + incl - cnt;
+          done += __builtin_amdgcn_readlane(incl, kWave - 1);
+          const int g = 2 * (ga + it * kWave + ln);
+          const int colg = g * Cnt::kPerGroup;
+          const uint32_t m0 = m;
+          while (m) {
+            const int col = colg + __builtin_ctz(m);
+            m &= m - 1u;
+            const uint32_t v = s_ct[col];
+            if (PASS == 2) {
+              po[at] = (v << 16) | (uint32_t)col;
+              mx_row = max(mx_row, v);
+            } else {
+              pc[at] = c0i + col;
+              pv[at] = w_offset ? w_offset - (int32_t)v : (int32_t)v;
               if (RANK) {
-                out_rank[at] = (int32_t)s_rank[2 * (4 * g + q)];
-                s_rank[2 * (4 * g + q)] = ~0u;
+                pr[at] = (int32_t)s_rank[col];
+                s_rank[col] = ~0u;
               }
-              ++at;
             }
-            if (hi) {
-              out_col[at] = col + 1;
-              out_val[at] = w_offset ? w_offset - (int32_t)hi : (int32_t)hi;
-              if (RANK) {
-                out_rank[at] = (int32_t)s_rank[2 * (4 * g + q) + 1];
-                s_rank[2 * (4 * g + q) + 1] = ~0u;
-              }
-              ++at;
-            }
+            ++at;
           }
-          o += __shfl(incl, kWave - 1, kWave);
+          if (m0 & ((1u << Cnt::kPerGroup) - 1u)) s4w[g] = make_uint4(0u, 0u, 0u, 0u);
+          if (m0 >> Cnt::kPerGroup) s4w[g + 1] = make_uint4(0u, 0u, 0u, 0u);
         }
         written += wtot;
       }
@@ -588,13 +670,12 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
       if (t == 0) {
         out.row_nnz[i] = (int32_t)rt;
         if (out.nnz_sum) atomicAdd(out.nnz_sum, (unsigned long long)rt);
-        if (s_max) atomicMax(out.max_count, s_max);
       }
     }
     if (PASS == 2 && t == 0) out.row_nnz[i] = (int32_t)written;
     __syncthreads();
   }
-  if (PASS == 2) {
+  if (PASS == 0 || PASS == 2) {
     if (mx_row) atomicMax(&s_max, mx_row);
     __syncthreads();
     if (t == 0 && s_max) atomicMax(out.max_count, s_max);
@@ -654,7 +735,7 @@ struct CoBufs {
   int32_t* csize;
   int32_t* cstart;
   int32_t* row_nnz;
-  unsigned long long* ctr;  // [kCtrs]: row counters, [kMaxRanges] sampled nnz sum
+  unsigned long long* ctr;  // [kCtrs]: row counters, [kCtrSum] sampled nnz sum
   unsigned int* misc;  // [0] bad label, [1] max count
 };
 
@@ -700,12 +781,14 @@ int co_check(const int32_t* labels, int64_t n, const int64_t* h_koff, int32_t P)
 
 }  // namespace
 // Columns per LDS window (even, <= kWin): the whole row range when n is
-// small (fewer LDS bytes, more resident workgroups), else kWin, or the
-// EAC_TUNE_CO_WINDOW setting (the autotuner trades windows per row against
-// workgroups per compute unit).
+// small (fewer LDS bytes, more resident workgroups), else 16384 (16 KiB of
+// byte counters: seven workgroups per compute unit; 200,003 points x 64
+// partitions, whole build: 13.0 / 11.8 / 11.0 / 11.0 / 12.3 ms at 8192 /
+// 12288 / 16384 / 24576 / 32768), or the EAC_TUNE_CO_WINDOW setting (the
+// autotuner trades windows per row against workgroups per compute unit).
 int co_window(int64_t n) {
   int w = tune_value(EAC_TUNE_CO_WINDOW);
-  if (w <= 0) w = kWin;
+  if (w <= 0) w = 16384;
   if (w > kWin) w = kWin;
   const int64_t need = ((n + 63) / 64) * 64;
   if (need < w) w = (int)need;
@@ -714,19 +797,17 @@ int co_window(int64_t n) {
 // Member loads in flight per lane in the pair visits (EAC_TUNE_CO_UNROLL:
 // 4 by default, or 8).
 inline int co_unroll() { return tune_value(EAC_TUNE_CO_UNROLL) == 8 ? 8 : 4; }
-// Row ranges of the co-association row loop (EAC_TUNE_CO_RANGES: 1..8;
-// default one per XCD, or one range below 65536 rows: there every
-// workgroup takes few rows and the end of the pass, where each row fetch
-// tries every range's counter, dominates; 10,000 rows x 100 partitions:
-// the EAC pipeline's graph replay 1.51 ms with one range, 1.74 with eight).
+// Row ranges of the co-association row loop (EAC_TUNE_CO_RANGES: 1..8
+// contiguous ones; default one per XCD, or kStripes interleaved ranges below
+// 65536 rows, see the row kernel).
 inline int co_ranges(int64_t n) {
   const int r = tune_value(EAC_TUNE_CO_RANGES);
   if (r > 0 && r <= kMaxRanges) return r;
-  return n < 65536 ? 1 : kMaxRanges;
+  return n < 65536 ? -kStripes : kMaxRanges;
 }
 inline size_t co_lds(int win, int P, bool rank = false) {
-  return (size_t)(2 * co_bm_words(P) + win / 2 + (rank ? win : 0) + 9 * P + 1 +
-                  (P / 2 + 1)) * 4;
+  return (size_t)(4 * co_bm_words(P) + co_cnt_words(win, co_bytes(P) ? 1 : 2) +
+                  (rank ? win : 0) + 9 * P + 1) * 4;
 }
 // The ranked fill keeps a 4-byte rank per column next to the counters: its
 // window is at most half as wide.
@@ -745,18 +826,32 @@ int32_t* build_win_table(const CoBufs& B, int64_t n, int P, int64_t ktot, int wi
   if (hipGetLastError() != hipSuccess) return nullptr;
   return wtab;
 }
+// The row kernel with the counter width for P and the unroll knob.
+using CoRowsFn = void (*)(CoPlan, int, int, CoOut);
+template <int PASS, bool RANK = false>
+CoRowsFn co_rows_fn(int P) {
+  if constexpr (RANK) {
+    return co_bytes(P) ? k_coassoc_rows<PASS, true, 4, uint8_t>
+                       : k_coassoc_rows<PASS, true, 4, uint16_t>;
+  } else {
+    if (co_unroll() == 8)
+      return co_bytes(P) ? k_coassoc_rows<PASS, false, 8, uint8_t>
+                         : k_coassoc_rows<PASS, false, 8, uint16_t>;
+    return co_bytes(P) ? k_coassoc_rows<PASS, false, 4, uint8_t>
+                       : k_coassoc_rows<PASS, false, 4, uint16_t>;
+  }
+}
 // Every workgroup resident at once (rows are handed out dynamically).
-template <int PASS, bool RANK = false, int U = 4>
+template <int PASS, bool RANK = false>
 int co_grid(int win, int P) {
   int dev = 0, cus = 256, per = 1;
   if (hipGetDevice(&dev) == hipSuccess)
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
   // allow launch-time LDS beyond 64 KB (the window of large graphs)
   const size_t lds = co_lds(win, P, RANK);
-  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_coassoc_rows<PASS, RANK, U>),
-                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, k_coassoc_rows<PASS, RANK, U>, kCB,
-                                                   lds) != hipSuccess || per < 1)
+  const void* fn = reinterpret_cast<const void*>(co_rows_fn<PASS, RANK>(P));
+  (void)hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, fn, kCB, lds) != hipSuccess || per < 1)
     per = 1;
   return cus * per;
 }
@@ -826,15 +921,10 @@ int co_plan_build(const int32_t* labels, int64_t n, const int64_t* h_koff, int32
   return EAC_OK;
 }
 
-// Launches the row kernel for PASS 0 or 2 (unranked) with the unroll knob.
-template <int PASS>
+template <int PASS, bool RANK = false>
 int co_launch(const CoPlan& pl, int full_rows, int win, const CoOut& o, hipStream_t s) {
-  if (co_unroll() == 8)
-    k_coassoc_rows<PASS, false, 8><<<co_grid<PASS, false, 8>(win, pl.P), kCB,
-                                     co_lds(win, pl.P), s>>>(pl, full_rows, win, o);
-  else
-    k_coassoc_rows<PASS><<<co_grid<PASS>(win, pl.P), kCB, co_lds(win, pl.P), s>>>(pl, full_rows,
-                                                                                 win, o);
+  co_rows_fn<PASS, RANK>(pl.P)<<<co_grid<PASS, RANK>(win, pl.P), kCB, co_lds(win, pl.P, RANK),
+                                 s>>>(pl, full_rows, win, o);
   EAC_LAUNCH_CHECK();
   return EAC_OK;
 }
@@ -914,15 +1004,10 @@ int coassoc_fill(const int32_t* labels, int64_t n, const int64_t* h_koff, int32_
   if (rank) {
     k_first_partition<<<1, 256, 0, s>>>(B.cstart, B.k_off, P, d_first);
     EAC_LAUNCH_CHECK();
-    k_coassoc_rows<1, true><<<co_grid<1, true>(win, P), kCB, co_lds(win, P, true), s>>>(
-        pl, full_rows, win, o);
-  } else if (co_unroll() == 8) {
-    k_coassoc_rows<1, false, 8><<<co_grid<1, false, 8>(win, P), kCB, co_lds(win, P), s>>>(
-        pl, full_rows, win, o);
+    EAC_TRY((co_launch<1, true>(pl, full_rows, win, o, s)));
   } else {
-    k_coassoc_rows<1><<<co_grid<1>(win, P), kCB, co_lds(win, P), s>>>(pl, full_rows, win, o);
+    EAC_TRY(co_launch<1>(pl, full_rows, win, o, s));
   }
-  EAC_LAUNCH_CHECK();
   prof_end(pr, s);
   EAC_HIP_CHECK(hipStreamSynchronize(s));
   prof_flush();
@@ -1021,14 +1106,14 @@ extern "C" int eac_coassoc_estimate(const int32_t* labels, int64_t n, const int6
   o.row_ctr = B.ctr;
   o.row_nnz = B.row_nnz;
   o.max_count = B.misc + 1;
-  o.nnz_sum = B.ctr + kMaxRanges;
+  o.nnz_sum = B.ctr + kCtrSum;
   int pr = prof_begin(EAC_PROF_CO_COUNT, 0, s);
   EAC_TRY(co_launch<0>(pl, full_rows, win, o, s));
   prof_end(pr, s);
   unsigned int misc[4];
   EAC_TRY(d2h(misc, B.misc, sizeof(misc), s));
   unsigned long long sum = 0;
-  EAC_TRY(d2h(&sum, B.ctr + kMaxRanges, sizeof(sum), s));
+  EAC_TRY(d2h(&sum, B.ctr + kCtrSum, sizeof(sum), s));
   prof_flush();
   if (misc[0]) return fail(EAC_ERR_ARG, "coassoc: label >= k of its partition");
   const int64_t rows = (n + sample_stride - 1) / sample_stride;
@@ -1045,7 +1130,7 @@ extern "C" size_t eac_coassoc_stage_bytes(int64_t n, int32_t full_rows, int32_t 
   if (P < 1) P = 1;
   if (pool_entries < 0) pool_entries = 0;
   const StageLayout L = stage_layout(n, full_rows);
-  const int64_t grid = co_unroll() == 8 ? co_grid<2, false, 8>(L.win, P) : co_grid<2>(L.win, P);
+  const int64_t grid = co_grid<2>(L.win, P);
   return L.pool_at + (size_t)(pool_entries + (grid + 1) * L.chunk) * 4;
 }
 
