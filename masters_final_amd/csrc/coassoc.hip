@@ -14,7 +14,7 @@
 // reference's lossy matrix from the exact one plus per-entry partition ranks.
 //
 // MI355X design:
-//  * Plan: a stable radix sort of (global cluster id, point) turns labels
+//  * Plan: a stable counting sort by cluster (group.hip) turns labels
 //    [P][n] into member lists (ascending point id per cluster) plus each
 //    point's position in its list. A point's later co-members in partition p
 //    are then the suffix of its cluster's list after its own position: no
@@ -37,8 +37,8 @@
 #include <cstring>
 #include <vector>
 
+#include "group.hpp"
 #include "prims.hpp"
-#include "sort.hpp"
 
 namespace eac {
 namespace {
@@ -52,64 +52,24 @@ constexpr int kCtrPad = 16;    // row counters 128 bytes apart
 constexpr int kCtrSum = kStripes * kCtrPad;  // after the counters: the sampled nnz sum
 constexpr int kCtrs = kCtrSum + 2;
 
-// keys: global cluster id (unassigned points -> ktot, sorted last);
-// values: p * n + i
-__global__ void k_member_keys(const int32_t* __restrict__ labels, int64_t n, int P,
-                              const int64_t* __restrict__ k_off, int64_t ktot,
-                              uint32_t* __restrict__ key, uint32_t* __restrict__ val,
-                              int32_t* __restrict__ csize, unsigned int* __restrict__ bad) {
-  for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (int64_t)P * n;
-       t += (int64_t)gridDim.x * blockDim.x) {
-    int p = (int)(t / n);
-    int32_t l = labels[t];
-    int64_t kp = k_off[p + 1] - k_off[p];
-    uint32_t g;
-    if (l < 0) {
-      g = (uint32_t)ktot;
-    } else if (l >= kp) {
-      atomicOr(bad, 1u);
-      g = (uint32_t)ktot;
-    } else {
-      g = (uint32_t)(k_off[p] + l);
-    }
-    key[t] = g;
-    val[t] = (uint32_t)t;
-    atomicAdd(&csize[g], 1);
-  }
-}
-
-// members[q] = point id; pos[p*n + i] = q (or -1 when unassigned)
-__global__ void k_member_pos(const uint32_t* __restrict__ skey, const uint32_t* __restrict__ sval,
-                             int64_t total, int64_t n, int64_t ktot,
-                             int32_t* __restrict__ members, int32_t* __restrict__ pos) {
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total;
-       q += (int64_t)gridDim.x * blockDim.x) {
-    uint32_t v = sval[q];
-    members[q] = (int32_t)(v % (uint32_t)n);
-    pos[v] = skey[q] == (uint32_t)ktot ? -1 : (int32_t)q;
-  }
-}
-
 // Window table: wtab[g * (nw + 1) + w] = first position in cluster g's
 // member list whose member is >= w * win (windows aligned to multiples of
 // win), so a window's end in every partition is one load instead of a
-// search. Built from the sorted (cluster, point) keys: each position writes
-// the windows that start after its predecessor's member and up to its own,
-// the last member of a cluster also the windows after it.
-__global__ void k_win_table(const uint32_t* __restrict__ skey, const int32_t* __restrict__ members,
-                            const int32_t* __restrict__ cstart, int64_t total, int64_t ktot,
-                            int win, int nw, int32_t* __restrict__ wtab) {
+// search; one lower bound per entry over the cluster's ascending list.
+__global__ void k_win_table(const int32_t* __restrict__ members,
+                            const int32_t* __restrict__ cstart, int64_t ktot, int win, int nw,
+                            int32_t* __restrict__ wtab) {
   const int64_t ts = nw + 1;
-  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < total;
+  for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < ktot * ts;
        q += (int64_t)gridDim.x * blockDim.x) {
-    const uint32_t g = skey[q];
-    if (g >= (uint32_t)ktot) continue;  // unassigned points sort last
-    const int wq = members[q] / win;
-    const int wp = q == cstart[g] ? -1 : members[q - 1] / win;
-    int32_t* t = wtab + (int64_t)g * ts;
-    for (int w = wp + 1; w <= wq; ++w) t[w] = (int32_t)q;
-    if (q + 1 == cstart[g + 1])
-      for (int w = wq + 1; w <= nw; ++w) t[w] = (int32_t)(q + 1);
+    const int64_t g = q / ts;
+    const int64_t at = (q - g * ts) * win;
+    int32_t lo = cstart[g], hi = cstart[g + 1];
+    while (lo < hi) {
+      const int32_t mid = lo + ((hi - lo) >> 1);
+      if (members[mid] < at) lo = mid + 1; else hi = mid;
+    }
+    wtab[q] = lo;
   }
 }
 
@@ -726,13 +686,9 @@ __global__ __launch_bounds__(256) void k_coassoc_compact(
 
 struct CoBufs {
   int64_t* k_off;
-  uint32_t* key;
-  uint32_t* val;
-  uint32_t* skey;
-  uint32_t* sval;
+  int32_t* wtab;     // [items] window table, when it fits
   int32_t* members;
   int32_t* pos;
-  int32_t* csize;
   int32_t* cstart;
   int32_t* row_nnz;
   unsigned long long* ctr;  // [kCtrs]: row counters, [kCtrSum] sampled nnz sum
@@ -745,16 +701,11 @@ CoBufs carve_co(Arena& ar, int64_t n, int P, int64_t ktot) {
   b.k_off = ar.take<int64_t>(P + 1);
   b.members = ar.take<int32_t>(items);
   b.pos = ar.take<int32_t>(items);
-  b.csize = ar.take<int32_t>(ktot + 2);
   b.cstart = ar.take<int32_t>(ktot + 2);
   b.row_nnz = ar.take<int32_t>(n + 1);
-  b.ctr = ar.take<unsigned long long>(kCtrs);
-  b.misc = ar.take<unsigned int>(4);
-  // sort staging last: reused by later passes
-  b.key = ar.take<uint32_t>(items);
-  b.val = ar.take<uint32_t>(items);
-  b.skey = ar.take<uint32_t>(items);
-  b.sval = ar.take<uint32_t>(items);
+  b.ctr = ar.take<unsigned long long>(kCtrs + 2);  // one fill clears both
+  b.misc = reinterpret_cast<unsigned int*>(b.ctr + kCtrs);
+  b.wtab = ar.take<int32_t>(items);
   return b;
 }
 
@@ -813,18 +764,17 @@ inline size_t co_lds(int win, int P, bool rank = false) {
 // window is at most half as wide.
 constexpr int kWinRank = kWin / 2;
 
-// Builds the window table in the sort staging (free after the plan) when it
-// fits; returns nullptr otherwise (the rows then search their window ends).
+// Builds the window table when it fits its buffer; returns nullptr otherwise
+// (the rows then search their window ends).
 int32_t* build_win_table(const CoBufs& B, int64_t n, int P, int64_t ktot, int win, int* nw,
                          hipStream_t s) {
   *nw = (int)((n + win - 1) / win);
-  const int64_t items = (int64_t)P * n;
-  if (ktot * (int64_t)(*nw + 1) > items) return nullptr;
-  int32_t* wtab = reinterpret_cast<int32_t*>(B.key);
-  k_win_table<<<grid_for(items, 256, 16384), 256, 0, s>>>(B.skey, B.members, B.cstart, items,
-                                                          ktot, win, *nw, wtab);
+  const int64_t items = (int64_t)P * n, entries = ktot * (int64_t)(*nw + 1);
+  if (*nw < 2 || entries > items) return nullptr;  // one window needs no table
+  k_win_table<<<grid_for(entries, 256, 16384), 256, 0, s>>>(B.members, B.cstart, ktot, win, *nw,
+                                                            B.wtab);
   if (hipGetLastError() != hipSuccess) return nullptr;
-  return wtab;
+  return B.wtab;
 }
 // The row kernel with the counter width for P and the unroll knob.
 using CoRowsFn = void (*)(CoPlan, int, int, CoOut);
@@ -866,20 +816,16 @@ extern "C" size_t eac_coassoc_workspace_bytes(int64_t n, int32_t P, int64_t k_to
   if (P < 1) P = 1;
   Arena ar(nullptr, 0, true);
   (void)carve_co(ar, n, P, k_total);
-  size_t s1 = radix_sort_ws_bytes((int64_t)P * n, 4, 4);
-  size_t s2 = scan_ws_bytes(k_total + 2, 4);
-  size_t s3 = scan_ws_bytes(n + 1, 8);
-  size_t m = s1 > s2 ? s1 : s2;
-  m = m > s3 ? m : s3;
-  return ar.used + m + 4096;
+  const size_t s1 = group_ws_bytes(n, P, k_total);
+  const size_t s2 = scan_ws_bytes(n + 1, 8);
+  return ar.used + (s1 > s2 ? s1 : s2) + 4096;
 }
 
 namespace eac {
 namespace {
-// The member plan in ws (shared by every pass over the same labels):
-// global cluster keys, the stable sort of (cluster, point), cluster starts,
-// each point's position in its cluster's list; zeroes the row counters and
-// flags.
+// The member plan in ws (shared by every pass over the same labels): member
+// lists, cluster starts, each point's position in its cluster's list; zeroes
+// the row counters and flags.
 int co_plan_build(const int32_t* labels, int64_t n, const int64_t* h_koff, int32_t P,
                   void* ws, size_t ws_bytes, CoBufs* out, size_t* mark_out, Arena& ar,
                   hipStream_t s, const int64_t* d_koff = nullptr) {
@@ -895,26 +841,13 @@ int co_plan_build(const int32_t* labels, int64_t n, const int64_t* h_koff, int32
     EAC_HIP_CHECK(hipMemcpyAsync(B.k_off, d_koff, sizeof(int64_t) * (P + 1),
                                  hipMemcpyDeviceToDevice, s));
   } else {
-    EAC_HIP_CHECK(hipMemcpyAsync(B.k_off, h_koff, sizeof(int64_t) * (P + 1),
-                                 hipMemcpyHostToDevice, s));
-    EAC_HIP_CHECK(hipStreamSynchronize(s));
+    EAC_TRY(put_i64(B.k_off, h_koff, P + 1, s));
   }
-  EAC_TRY(fill<int32_t>(B.csize, ktot + 2, 0, s));
-  EAC_TRY(fill<int32_t>((int32_t*)B.misc, 4, 0, s));
-  EAC_TRY(fill<int64_t>((int64_t*)B.ctr, kCtrs, 0, s));
+  EAC_TRY(fill<int64_t>((int64_t*)B.ctr, kCtrs + 2, 0, s));
   int pr = prof_begin(EAC_PROF_CO_PLAN, 16 * items, s);
-  k_member_keys<<<grid_for(items, 256, 8192), 256, 0, s>>>(labels, n, P, B.k_off, ktot, B.key,
-                                                           B.val, B.csize, B.misc);
-  EAC_LAUNCH_CHECK();
-  const int bits = bits_for((uint64_t)ktot);
-  EAC_TRY((radix_sort<uint32_t, uint32_t>(B.key, B.skey, B.val, B.sval, items, 0,
-                                          bits < 1 ? 1 : bits, ar, s)));
+  EAC_TRY(group_by_cluster(labels, n, P, B.k_off, h_koff, reinterpret_cast<uint32_t*>(B.members),
+                           reinterpret_cast<uint32_t*>(B.cstart), B.pos, B.misc, ar, s));
   ar.used = mark;
-  EAC_TRY((scan_excl<int32_t, int32_t>(B.csize, B.cstart, ktot + 2, 0, nullptr, ar, s)));
-  ar.used = mark;
-  k_member_pos<<<grid_for(items, 256, 8192), 256, 0, s>>>(B.skey, B.sval, items, n, ktot,
-                                                          B.members, B.pos);
-  EAC_LAUNCH_CHECK();
   prof_end(pr, s);
   *out = B;
   *mark_out = mark;
@@ -1159,8 +1092,7 @@ extern "C" int eac_coassoc_stage(const int32_t* labels, int64_t n, const int64_t
   int64_t* hdr = reinterpret_cast<int64_t*>(st);
   k_stage_header<<<1, 64, 0, s>>>(hdr, SL.win, SL.nw, (int64_t)SL.pool_at, full_rows);
   EAC_LAUNCH_CHECK();
-  EAC_TRY(fill<int64_t>((int64_t*)B.ctr, kCtrs, 0, s));
-  EAC_TRY(fill<int32_t>((int32_t*)B.misc, 4, 0, s));
+  EAC_TRY(fill<int64_t>((int64_t*)B.ctr, kCtrs + 2, 0, s));
   int nw = 0;
   const int32_t* wtab = build_win_table(B, n, P, ktot, SL.win, &nw, s);
   CoPlan pl{labels, n, P, B.k_off, B.members, B.pos, B.cstart, wtab, nw, nullptr, co_ranges(n), 1};

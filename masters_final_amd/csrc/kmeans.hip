@@ -30,6 +30,7 @@
 #include <cstring>
 #include <vector>
 
+#include "group.hpp"
 #include "prims.hpp"
 #include "sort.hpp"
 
@@ -1056,21 +1057,23 @@ __global__ __launch_bounds__(kWave) void k_np_chunk_sums(const float* __restrict
   if (threadIdx.x == 0) csum[row * nchunks + c] = v[1];
 }
 
-// out[row] = ((0 + csum[row][0]) + csum[row][1]) + ...
+// ((0 + csum[0]) + csum[1]) + ...
+__device__ __forceinline__ float np_finish(const float* __restrict__ csum, int64_t nchunks) {
+  float r = 0.0f;
+  for (int64_t c = 0; c < nchunks; ++c) r = __fadd_rn(r, csum[c]);
+  return r;
+}
 __global__ void k_np_finish(const float* __restrict__ csum, int64_t nchunks, int64_t rows,
                             float* __restrict__ out) {
   const int64_t row = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (row >= rows) return;
-  float r = 0.0f;
-  for (int64_t c = 0; c < nchunks; ++c) r = __fadd_rn(r, csum[row * nchunks + c]);
-  out[row] = r;
+  out[row] = np_finish(csum + row * nchunks, nchunks);
 }
 
 int64_t np_chunks(int64_t n) { return n > 0 ? (n + kNpBuf - 1) / kNpBuf : 0; }
 
-// numpy float32 sums of `rows` rows of length n; csum holds rows * np_chunks(n)
-int np_sum_rows(const float* x, int64_t n, int64_t rows, float* csum, float* out,
-                hipStream_t s) {
+// chunk sums of `rows` rows of length n: csum holds rows * np_chunks(n)
+int np_chunk_sums(const float* x, int64_t n, int64_t rows, float* csum, hipStream_t s) {
   const int64_t nc = np_chunks(n);
   if (nc > 0) {
     for (int64_t r0 = 0; r0 < rows; r0 += 65535) {
@@ -1080,7 +1083,14 @@ int np_sum_rows(const float* x, int64_t n, int64_t rows, float* csum, float* out
       EAC_LAUNCH_CHECK();
     }
   }
-  k_np_finish<<<grid_for(rows, 256), 256, 0, s>>>(csum, nc, rows, out);
+  return EAC_OK;
+}
+
+// numpy float32 sums of `rows` rows of length n; csum holds rows * np_chunks(n)
+int np_sum_rows(const float* x, int64_t n, int64_t rows, float* csum, float* out,
+                hipStream_t s) {
+  EAC_TRY(np_chunk_sums(x, n, rows, csum, s));
+  k_np_finish<<<grid_for(rows, 256), 256, 0, s>>>(csum, np_chunks(n), rows, out);
   EAC_LAUNCH_CHECK();
   return EAC_OK;
 }
@@ -1104,147 +1114,175 @@ int launch_direct(const float* X, int64_t n, int d, const float* C, const int64_
 }
 
 // ------------------------------------------------------- centroid update
-// Sort keys (global centroid id) and point indices of every (partition,
-// point), and the member count of every centroid. Blocks cover a run of one
-// partition's points (grid.y over partitions); when that run is long next to
-// the partition's k, counts meet in LDS first (one global atomic per
-// centroid and block instead of one per point).
-constexpr int kKeyLds = 4096;
-__global__ __launch_bounds__(256) void k_label_keys(const int32_t* __restrict__ labels,
-                                                    int64_t n, int P,
-                                                    const int64_t* __restrict__ k_off,
-                                                    uint32_t* __restrict__ key,
-                                                    uint32_t* __restrict__ idx,
-                                                    int32_t* __restrict__ count) {
-  __shared__ int32_t s_cnt[kKeyLds];
-  const int64_t per_block = (n + gridDim.x - 1) / gridDim.x;
-  const int64_t i0 = (int64_t)blockIdx.x * per_block;
-  const int64_t i1 = i0 + per_block < n ? i0 + per_block : n;
-  for (int p = blockIdx.y; p < P; p += gridDim.y) {
-    const int64_t kb = k_off[p], kp = k_off[p + 1] - kb;
-    const bool lds = kp <= kKeyLds && 4 * kp <= i1 - i0;  // uniform over the block
-    if (lds) {
-      for (int c = threadIdx.x; c < kp; c += blockDim.x) s_cnt[c] = 0;
-      __syncthreads();
-    }
-    for (int64_t i = i0 + threadIdx.x; i < i1; i += blockDim.x) {
-      const int64_t t = (int64_t)p * n + i;
-      const int32_t l = labels[t];
-      key[t] = (uint32_t)(kb + l);
-      idx[t] = (uint32_t)i;
-      if (lds) atomicAdd(&s_cnt[l], 1);
-      else atomicAdd(&count[kb + l], 1);
-    }
-    if (lds) {
-      __syncthreads();
-      for (int c = threadIdx.x; c < kp; c += blockDim.x)
-        if (s_cnt[c]) atomicAdd(&count[kb + c], s_cnt[c]);
-      __syncthreads();
-    }
-  }
-}
-
 // new[c][j] = fp32 sequential sum over members in point order, / count in
-// double (KMeans.py:736-745). One single-wave block per centroid and group
-// of 128 dimensions: the lanes gather up to 2048 member coordinates at a
-// time into LDS (many loads in flight), then lane j adds dimension j's
-// values in member order (lane j + 64 too), so the serial chain runs on LDS
-// reads.
-constexpr int kSumStage = 2048;
+// double (KMeans.py:736-745). One workgroup per centroid and group of up to
+// 128 dimensions (grid.y over partitions). The members' rows are gathered by
+// all lanes, a stage of rows ahead in registers, and stored transposed in
+// LDS; lane j then adds dimension j's values in member order, four rows per
+// LDS read. The additions of one sum cannot be split (their order is part of
+// the result), so the longest cluster bounds the launch: LDS reads and adds
+// for it instead of a dependent gather per 16 members (500,000 x 16-d points,
+// 16 partitions of 32 to 2048 clusters: 612 -> 213 us). Small clusters take
+// one wavefront (BS = 64), so more of them are in flight (10,000 x 2-d, 100
+// partitions: 28 -> 15 us).
+// upd (nullable): partitions whose centroids stay. eflag (nullable): 1 for an
+// empty cluster; n_empty counts them.
+// V4: rows are read 16 bytes at a time (d a multiple of 4, X 16-byte aligned).
 constexpr int kSumDims = 2 * kWave;
-__global__ __launch_bounds__(kWave) void k_centroid_sums(const float* __restrict__ X, int d,
-                                                         const uint32_t* __restrict__ members,
-                                                         const int64_t* __restrict__ mstart,
-                                                         const int32_t* __restrict__ count,
-                                                         int64_t ktot, float* __restrict__ Cnew) {
-  __shared__ float s_x[kSumStage];
-  const int lane = threadIdx.x;
-  for (int64_t c = blockIdx.x; c < ktot; c += gridDim.x) {
-    const int32_t cnt = count[c];
-    if (cnt == 0) continue;  // uniform over the block
-    const uint32_t* m = members + mstart[c];
-    for (int j0 = 0; j0 < d; j0 += kSumDims) {
-      const int dd = d - j0 < kSumDims ? d - j0 : kSumDims;
-      const int q_max = kSumStage / dd;  // members per stage
-      float s0 = 0.f, s1 = 0.f;
-      for (int32_t b = 0; b < cnt; b += q_max) {
-        const int q = cnt - b < q_max ? cnt - b : q_max;
-        __syncthreads();
-        for (int v = lane; v < q * dd; v += kWave) {
-          const int r = v / dd;
-          s_x[v] = X[(int64_t)m[b + r] * d + j0 + (v - r * dd)];
-        }
-        __syncthreads();
-        if (lane < dd)
-          for (int r = 0; r < q; ++r) s0 = s0 + s_x[r * dd + lane];
-        if (lane + kWave < dd)
-          for (int r = 0; r < q; ++r) s1 = s1 + s_x[r * dd + lane + kWave];
-      }
-      if (lane < dd) Cnew[c * d + j0 + lane] = (float)((double)s0 / (double)cnt);
-      if (lane + kWave < dd)
-        Cnew[c * d + j0 + lane + kWave] = (float)((double)s1 / (double)cnt);
-    }
-  }
-}
-
-// The same sums for d <= 64 with L lanes per centroid (L = the power of two
-// >= d, at least 4; 64 / L centroids per wavefront): lane j of a group adds
-// dimension j of its centroid's members in point order straight from X, 16
-// member rows loaded ahead of the (in-order) additions. The one-wave-per-
-// centroid form above leaves 64 - d lanes idle and waits on LDS for every
-// member.
-template <int L>
-__global__ __launch_bounds__(256) void k_centroid_sums_narrow(
+template <int BS>
+struct SumStage {
+  static constexpr int kFloats = BS == kWave ? 1024 : 8192;
+  static constexpr int kRows = BS == kWave ? 256 : 1024;
+};
+template <int BS, bool V4>
+__global__ __launch_bounds__(BS) void k_centroid_sums(
     const float* __restrict__ X, int d, const uint32_t* __restrict__ members,
-    const int64_t* __restrict__ mstart, const int32_t* __restrict__ count, int64_t ktot,
-    float* __restrict__ Cnew) {
-  constexpr int U = 16;
-  const int j = threadIdx.x % L;
-  const int64_t groups = (int64_t)gridDim.x * (blockDim.x / L);
-  for (int64_t c = (int64_t)blockIdx.x * (blockDim.x / L) + threadIdx.x / L; c < ktot;
-       c += groups) {
-    const int32_t cnt = count[c];
-    if (cnt == 0 || j >= d) continue;
-    const uint32_t* m = members + mstart[c];
-    const float* xj = X + j;
-    float s = 0.f;
-    int32_t r = 0;
-    for (; r + U <= cnt; r += U) {
-      uint32_t mi[U];
-      float v[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) mi[u] = m[r + u];
-#pragma unroll
-      for (int u = 0; u < U; ++u) v[u] = xj[(int64_t)mi[u] * d];
-#pragma unroll
-      for (int u = 0; u < U; ++u) s = s + v[u];
-    }
-    for (; r < cnt; ++r) s = s + xj[(int64_t)m[r] * d];
-    Cnew[c * d + j] = (float)((double)s / (double)cnt);
-  }
-}
-
-// Copies the new centroids of the partitions still running (upd[p] != 0).
-__global__ void k_copy_running(float* __restrict__ C, const float* __restrict__ Cnew, int d,
-                               const int64_t* __restrict__ k_off, int P,
-                               const int32_t* __restrict__ upd) {
+    const uint32_t* __restrict__ start, const int64_t* __restrict__ k_off, int P,
+    const int32_t* __restrict__ upd, int32_t* __restrict__ eflag, int32_t* __restrict__ n_empty,
+    float* __restrict__ Cout) {
+  constexpr int kFloats = SumStage<BS>::kFloats, kRows = SumStage<BS>::kRows;
+  constexpr int W = V4 ? 4 : 1;
+  constexpr int NV = kFloats / W / BS;  // row pieces a lane holds
+  constexpr int NM = kRows / BS;        // member ids a lane holds
+  __shared__ __align__(16) float s_x[kFloats + 4 * kSumDims];
+  __shared__ uint32_t s_m[kRows];
+  const int t = threadIdx.x;
   for (int p = blockIdx.y; p < P; p += gridDim.y) {
-    if (!upd[p]) continue;
-    const int64_t a = k_off[p] * d, b = k_off[p + 1] * d;
-    for (int64_t t = a + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < b;
-         t += (int64_t)gridDim.x * blockDim.x)
-      C[t] = Cnew[t];
+    const int64_t kb = k_off[p], ke = k_off[p + 1];
+    const bool run = !upd || upd[p];
+    for (int64_t c = kb + blockIdx.x; c < ke; c += gridDim.x) {
+      const uint32_t m0 = start[c];
+      const uint32_t cnt = start[c + 1] - m0;
+      if (t == 0) {
+        if (eflag) eflag[c] = cnt == 0;
+        if (cnt == 0) atomicAdd(n_empty, 1);
+      }
+      if (cnt == 0 || !run) continue;  // uniform over the block
+      const uint32_t* m = members + m0;
+      for (int j0 = 0; j0 < d; j0 += kSumDims) {
+        const int dd = d - j0 < kSumDims ? d - j0 : kSumDims;
+        const int pw = dd / W;  // pieces per row
+        int rs = (kFloats / dd) & ~3;
+        if (rs > kRows) rs = kRows;
+        const int rsp = rs + 4;  // column stride: 16-byte aligned, columns on other banks
+        const int dr = BS / pw, dp = BS - dr * pw;  // a step of BS pieces: rows, pieces
+        uint32_t mi[NM];
+        float4 xv[V4 ? NV : 1];
+        float xs[V4 ? 1 : NV];
+        auto ids = [&](uint32_t b) {  // member ids of the stage at b
+#pragma unroll
+          for (int i = 0; i < NM; ++i) {
+            const uint32_t r = b + i * BS + t;
+            mi[i] = r < cnt ? m[r] : 0u;
+          }
+        };
+        auto keep_ids = [&]() {
+#pragma unroll
+          for (int i = 0; i < NM; ++i) s_m[i * BS + t] = mi[i];
+        };
+        auto rows = [&](int q) {  // q rows named by s_m, into registers
+          int r = t / pw, j = t - (t / pw) * pw;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            if (i * BS < q * pw) {  // uniform
+              if (r < q) {
+                const float* src = X + (int64_t)s_m[r] * d + j0 + j * W;
+                if constexpr (V4) xv[i] = *reinterpret_cast<const float4*>(src);
+                else xs[i] = *src;
+              }
+              r += dr;
+              j += dp;
+              if (j >= pw) {
+                j -= pw;
+                ++r;
+              }
+            }
+          }
+        };
+        auto keep_rows = [&](int q) {
+          int r = t / pw, j = t - (t / pw) * pw;
+#pragma unroll
+          for (int i = 0; i < NV; ++i) {
+            if (i * BS < q * pw) {
+              if (r < q) {
+                if constexpr (V4) {
+                  float* col = s_x + (j * 4) * rsp + r;
+                  col[0] = xv[i].x;
+                  col[rsp] = xv[i].y;
+                  col[2 * rsp] = xv[i].z;
+                  col[3 * rsp] = xv[i].w;
+                } else {
+                  s_x[j * rsp + r] = xs[i];
+                }
+              }
+              r += dr;
+              j += dp;
+              if (j >= pw) {
+                j -= pw;
+                ++r;
+              }
+            }
+          }
+        };
+        auto take = [&](uint32_t b) {
+          return (int)(cnt - b < (uint32_t)rs ? cnt - b : (uint32_t)rs);
+        };
+        float s0 = 0.f;
+        int q = take(0);
+        __syncthreads();  // the previous centroid's sums are done
+        ids(0);
+        keep_ids();
+        __syncthreads();
+        rows(q);
+        if (cnt > (uint32_t)rs) ids(rs);
+        for (uint32_t b = 0; b < cnt; b += rs) {
+          q = take(b);
+          keep_rows(q);
+          const bool more = b + rs < cnt;
+          if (more) {
+            __syncthreads();  // this stage's ids are consumed
+            keep_ids();
+          }
+          __syncthreads();  // the stage's rows and the next one's ids are in LDS
+          if (more) {
+            rows(take(b + rs));
+            if (b + 2 * rs < cnt) ids(b + 2 * rs);
+          }
+          if (t < dd) {
+            const float* col = s_x + t * rsp;
+            int r = 0;
+            for (; r + 16 <= q; r += 16) {
+              float4 v[4];
+#pragma unroll
+              for (int u = 0; u < 4; ++u) v[u] = *reinterpret_cast<const float4*>(col + r + 4 * u);
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                s0 = s0 + v[u].x;
+                s0 = s0 + v[u].y;
+                s0 = s0 + v[u].z;
+                s0 = s0 + v[u].w;
+              }
+            }
+            for (; r < q; ++r) s0 = s0 + col[r];
+          }
+          if (more) __syncthreads();  // the stage's rows are summed
+        }
+        if (t < dd) Cout[c * d + j0 + t] = (float)((double)s0 / (double)cnt);
+      }
+    }
   }
 }
 
 // KMeans.py:117-189 stopping rule of iteration `it` for every partition
-// still running: new_inertia = numpy float32 sum of the dists (inertia[p]),
+// still running: new_inertia = numpy float32 sum of the dists (the chunk sums
+// csum[p] added up in order),
 // err = |new_inertia - previous| in float32 (previous starts at +inf); stop
 // when err <= tol (compared in float32, as numpy compares a float32 scalar
 // with a Python float) or it >= max_iter, else mark the partition for a
-// centroid update. any[0] = some partition continues.
-__global__ void k_converge(const float* __restrict__ inertia, float* __restrict__ prev,
-                           int32_t* __restrict__ active, int32_t* __restrict__ iters,
+// centroid update. any[0] = some partition continues; any[1] (the update's
+// count of empty clusters) is cleared.
+__global__ void k_converge(const float* __restrict__ csum, int64_t nchunks,
+                           float* __restrict__ prev, int32_t* __restrict__ active, int32_t* __restrict__ iters,
                            int32_t* __restrict__ upd, int P, int it, int max_iter, float tol,
                            int32_t* __restrict__ any) {
   __shared__ int s_any;
@@ -1254,8 +1292,9 @@ __global__ void k_converge(const float* __restrict__ inertia, float* __restrict_
     upd[p] = 0;
     if (!active[p]) continue;
     iters[p] = it;
-    const float err = fabsf(__fsub_rn(inertia[p], prev[p]));
-    prev[p] = inertia[p];
+    const float inertia = np_finish(csum + p * nchunks, nchunks);
+    const float err = fabsf(__fsub_rn(inertia, prev[p]));
+    prev[p] = inertia;
     if (err <= tol || it >= max_iter) {
       active[p] = 0;
       continue;
@@ -1264,7 +1303,10 @@ __global__ void k_converge(const float* __restrict__ inertia, float* __restrict_
     s_any = 1;
   }
   __syncthreads();
-  if (threadIdx.x == 0) any[0] = s_any;
+  if (threadIdx.x == 0) {
+    any[0] = s_any;
+    any[1] = 0;
+  }
 }
 
 __global__ void k_fit_init(float* __restrict__ prev, int32_t* __restrict__ active,
@@ -1274,13 +1316,6 @@ __global__ void k_fit_init(float* __restrict__ prev, int32_t* __restrict__ activ
     active[p] = 1;
     iters[p] = 0;
   }
-}
-
-__global__ void k_empty_flags(const int32_t* __restrict__ count, int64_t ktot,
-                              int32_t* __restrict__ flag) {
-  for (int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; c < ktot;
-       c += (int64_t)gridDim.x * blockDim.x)
-    flag[c] = count[c] == 0;
 }
 
 // keys (dist bits << 32 | index) of one partition: ascending = (dist, index)
@@ -1294,13 +1329,15 @@ __global__ void k_dist_keys(const float* __restrict__ dists, int64_t n,
 // empty clusters c of one partition (ascending) take the points of the
 // smallest (dist, index), in that order
 __global__ void k_reseed(const float* __restrict__ X, int d, const uint64_t* __restrict__ sorted,
-                         const int32_t* __restrict__ count, const int32_t* __restrict__ erank,
-                         int64_t kbeg, int64_t kend, float* __restrict__ Cnew) {
+                         const int32_t* __restrict__ eflag, const int32_t* __restrict__ erank,
+                         int64_t kbeg, int64_t kend, const int32_t* __restrict__ upd,
+                         float* __restrict__ Cnew) {
+  if (upd && !*upd) return;  // a stopped partition keeps its centroids
   for (int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; t < (kend - kbeg) * d;
        t += (int64_t)gridDim.x * blockDim.x) {
     int64_t c = kbeg + t / d;
     int j = (int)(t % d);
-    if (count[c] != 0) continue;
+    if (!eflag[c]) continue;
     int32_t r = erank[c] - erank[kbeg];
     uint32_t src = (uint32_t)(sorted[r] & 0xffffffffu);
     Cnew[c * d + j] = X[(int64_t)src * d + j];
@@ -1390,8 +1427,9 @@ __global__ __launch_bounds__(256) void k_flag_bscatter(const uint64_t* __restric
 constexpr int kMaxReseed = 2048;
 __global__ __launch_bounds__(1024) void k_reseed_dev(
     const float* __restrict__ X, int d, const float* __restrict__ dists, int64_t n,
-    const int64_t* __restrict__ k_off, int P, const int32_t* __restrict__ count,
-    const int32_t* __restrict__ erank, float* __restrict__ Cnew, unsigned int* __restrict__ err) {
+    const int64_t* __restrict__ k_off, int P, const int32_t* __restrict__ eflag,
+    const int32_t* __restrict__ erank, const int32_t* __restrict__ upd,
+    float* __restrict__ Cnew, unsigned int* __restrict__ err) {
   __shared__ unsigned int hist[256];
   __shared__ unsigned long long s_sel[kMaxReseed];
   __shared__ int32_t s_emp[kMaxReseed];
@@ -1402,7 +1440,7 @@ __global__ __launch_bounds__(1024) void k_reseed_dev(
   for (int p = blockIdx.x; p < P; p += gridDim.x) {
     const int64_t kb = k_off[p], ke = k_off[p + 1];
     const int64_t e = (int64_t)erank[ke] - erank[kb];
-    if (e == 0) continue;
+    if (e == 0 || (upd && !upd[p])) continue;  // uniform over the block
     if (e > n || e > kMaxReseed) {
       if (t == 0) atomicOr(err, 2u);
       continue;
@@ -1435,7 +1473,7 @@ __global__ __launch_bounds__(1024) void k_reseed_dev(
     const unsigned long long T = s_prefix;  // the e-th smallest key (keys are unique)
     if (t == 0) s_nsel = 0;
     for (int64_t c = kb + t; c < ke; c += blockDim.x)
-      if (count[c] == 0) s_emp[erank[c] - erank[kb]] = (int32_t)c;
+      if (eflag[c]) s_emp[erank[c] - erank[kb]] = (int32_t)c;
     __syncthreads();
     for (int64_t i = t; i < n; i += blockDim.x) {
       const unsigned long long key =
@@ -1485,16 +1523,6 @@ int d2h(void* host, const void* dev, size_t bytes, hipStream_t s) {
   EAC_HIP_CHECK(hipMemcpyAsync(pin, dev, bytes, hipMemcpyDeviceToHost, s));
   EAC_HIP_CHECK(hipStreamSynchronize(s));
   memcpy(host, pin, bytes);
-  return EAC_OK;
-}
-
-int h2d(void* dev, const void* host, size_t bytes, hipStream_t s) {
-  void* pin = pinned_scratch(bytes);
-  if (!pin) return fail(EAC_ERR_HIP, "pinned host allocation failed");
-  EAC_HIP_CHECK(hipStreamSynchronize(s));
-  memcpy(pin, host, bytes);
-  EAC_HIP_CHECK(hipMemcpyAsync(dev, pin, bytes, hipMemcpyHostToDevice, s));
-  EAC_HIP_CHECK(hipStreamSynchronize(s));  // pinned buffer is reused
   return EAC_OK;
 }
 
@@ -1554,12 +1582,12 @@ struct KmGraph {
 };
 
 // Label all partitions; dists (nullable) receive FP64-exact distances for
-// the F64 / BF16X3 modes and fp32 distances for F32; inertia[p] (device,
-// nullable) their per-partition numpy float32 sums.
+// the F64 / BF16X3 modes and fp32 distances for F32; csum_out (nullable)
+// the numpy float32 chunk sums of each partition's dists.
 // With g (capturable calls) nothing is read back: the flag count stays on
 // the device and sizes the re-scoring from there.
 int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t* h_koff,
-                 int P, int mode, int32_t* labels, float* dists, float* inertia_out,
+                 int P, int mode, int32_t* labels, float* dists, const float** csum_out,
                  int64_t* n_rescored, Arena& ar, hipStream_t s,
                  const int64_t* d_koff = nullptr, const KmGraph* kg = nullptr) {
   const int64_t ktot = h_koff[P];
@@ -1568,9 +1596,7 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
   if (d_koff) {
     B.k_off = const_cast<int64_t*>(d_koff);  // read only
   } else {
-    EAC_HIP_CHECK(hipMemcpyAsync(B.k_off, h_koff, sizeof(int64_t) * (P + 1),
-                                 hipMemcpyHostToDevice, s));
-    EAC_HIP_CHECK(hipStreamSynchronize(s));  // h_koff may be a pageable stack array
+    EAC_TRY(put_i64(B.k_off, h_koff, P + 1, s));
   }
   if (n_rescored) *n_rescored = 0;
   if (mode == EAC_KM_F32 || mode == EAC_KM_F64 || mode == EAC_KM_F32_NUMPY ||
@@ -1583,9 +1609,10 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
     else
       EAC_TRY(launch_direct<double>(X, n, d, C, B.k_off, P, labels, dists, s));
     prof_end(pr, s);
-    if (inertia_out) {
+    if (csum_out) {
       if (!dists) return fail(EAC_ERR_ARG, "kmeans: inertia needs dists");
-      EAC_TRY(np_sum_rows(dists, n, P, B.csum, inertia_out, s));
+      EAC_TRY(np_chunk_sums(dists, n, P, B.csum, s));
+      *csum_out = B.csum;
     }
     return EAC_OK;
   }
@@ -1733,7 +1760,7 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
   }
   if (n_rescored) *n_rescored = (int64_t)nf;
   }  // read-back path
-  if (inertia_out && !dists) return fail(EAC_ERR_ARG, "kmeans: inertia needs dists");
+  if (csum_out && !dists) return fail(EAC_ERR_ARG, "kmeans: inertia needs dists");
   if (dists) {
     const int pgs = (P + kPG - 1) / kPG;
     const int py = pgs < 65535 ? pgs : 65535;
@@ -1741,124 +1768,101 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
                                                                         labels, dists);
     EAC_LAUNCH_CHECK();
   }
-  if (inertia_out) EAC_TRY(np_sum_rows(dists, n, P, B.csum, inertia_out, s));
+  if (csum_out) {
+    EAC_TRY(np_chunk_sums(dists, n, P, B.csum, s));
+    *csum_out = B.csum;
+  }
   return EAC_OK;
 }
 
+struct UpdateBufs {
+  int32_t* eflag;  // [ktot + 1]: 1 for an empty cluster (the last entry is 0)
+  int32_t* erank;  // [ktot + 1]
+  uint64_t* dk;
+  uint64_t* dks;
+  size_t mark;     // arena position of the scratch after these
+};
+
 size_t kmeans_update_ws_bytes(int64_t n, int d, int64_t ktot, int P) {
   Arena ar(nullptr, 0, true);
-  int64_t items = (int64_t)P * n;
   ar.take<int64_t>(P + 1);
-  ar.take<uint32_t>(items);
-  ar.take<uint32_t>(items);
-  ar.take<uint32_t>(items);
-  ar.take<uint32_t>(items);
-  ar.take<int32_t>(ktot + 1);
-  ar.take<int64_t>(ktot + 1);
+  ar.take<int32_t>(2);
+  ar.take<uint32_t>((int64_t)P * n);
+  ar.take<uint32_t>(ktot + 1);
   ar.take<int32_t>(ktot + 1);
   ar.take<int32_t>(ktot + 1);
   ar.take<uint64_t>(n);
   ar.take<uint64_t>(n);
   size_t a = ar.used;
-  size_t sort_a = radix_sort_ws_bytes(items, 4, 4);
+  size_t grp = group_ws_bytes(n, P, ktot);
   size_t sort_b = radix_sort_ws_bytes(n, 8, 0);
   size_t scan_b = scan_ws_bytes(ktot + 1, 8);
-  size_t m = sort_a > sort_b ? sort_a : sort_b;
+  size_t m = grp > sort_b ? grp : sort_b;
   m = m > scan_b ? m : scan_b;
   return a + m + 4096;
 }
 
-// New centroids for every partition (KMeans.py:709-754); empty clusters take
-// the points of smallest (dist, index) in ascending cluster order.
-// With g (capturable calls) the empty clusters are reseeded on the device.
-int kmeans_update(const float* X, int64_t n, int d, const int32_t* labels, const float* dists,
-                  const int64_t* h_koff, int P, float* Cnew, int64_t* n_empty, Arena& ar,
-                  hipStream_t s, const int64_t* d_koff = nullptr, const KmGraph* g = nullptr) {
+// New centroids of every partition (KMeans.py:709-754) into Cout, except
+// those of partitions with upd[p] == 0 (upd nullable); *n_empty (device,
+// cleared by the caller) += clusters without a point, which U->eflag marks
+// for the reseeding. Nothing is read back.
+int kmeans_update(const float* X, int64_t n, int d, const int32_t* labels, const int64_t* h_koff,
+                  const int64_t* d_koff, int P, float* Cout, const int32_t* upd, int32_t* n_empty,
+                  UpdateBufs* U, Arena& ar, hipStream_t s) {
   const int64_t ktot = h_koff[P];
   const int64_t items = (int64_t)P * n;
   if (items > (int64_t)UINT32_MAX || ktot >= (int64_t)UINT32_MAX)
     return fail(EAC_ERR_UNSUPPORTED, "kmeans update: P*n or k too large");
-  int64_t* k_off = ar.take<int64_t>(P + 1);
-  uint32_t* key = ar.take<uint32_t>(items);
-  uint32_t* idx = ar.take<uint32_t>(items);
-  uint32_t* skey = ar.take<uint32_t>(items);
   uint32_t* members = ar.take<uint32_t>(items);
-  int32_t* count = ar.take<int32_t>(ktot + 1);
-  int64_t* mstart = ar.take<int64_t>(ktot + 1);
-  int32_t* eflag = ar.take<int32_t>(ktot + 1);
-  int32_t* erank = ar.take<int32_t>(ktot + 1);
-  uint64_t* dk = ar.take<uint64_t>(n);
-  uint64_t* dks = ar.take<uint64_t>(n);
+  uint32_t* start = ar.take<uint32_t>(ktot + 1);
+  U->eflag = ar.take<int32_t>(ktot + 1);
+  U->erank = ar.take<int32_t>(ktot + 1);
+  U->dk = ar.take<uint64_t>(n);
+  U->dks = ar.take<uint64_t>(n);
+  U->mark = ar.used;
   if (ar.overflow()) return fail(EAC_ERR_WORKSPACE, "kmeans update: workspace too small");
-  if (d_koff) {
-    k_off = const_cast<int64_t*>(d_koff);  // read only
-  } else {
-    EAC_HIP_CHECK(hipMemcpyAsync(k_off, h_koff, sizeof(int64_t) * (P + 1),
-                                 hipMemcpyHostToDevice, s));
-    EAC_HIP_CHECK(hipStreamSynchronize(s));
-  }
-  EAC_TRY(fill<int32_t>(count, ktot + 1, 0, s));
-  {
-    // about 8192 blocks in all, each over a run of at least 1024 points
-    const int py = P < 65535 ? P : 65535;
-    int gx = grid_for(n, 1024, 8192 / py > 1 ? 8192 / py : 1);
-    k_label_keys<<<dim3(gx, py), 256, 0, s>>>(labels, n, P, k_off, key, idx, count);
-    EAC_LAUNCH_CHECK();
-  }
-  // stable by centroid: members of each centroid in ascending point order
-  const int bits = bits_for((uint64_t)ktot);
-  size_t mark = ar.used;
-  EAC_TRY((radix_sort<uint32_t, uint32_t>(key, skey, idx, members, items, 0, bits < 1 ? 1 : bits,
-                                          ar, s)));
-  ar.used = mark;
-  EAC_TRY((scan_excl<int32_t, int64_t>(count, mstart, ktot, 0, nullptr, ar, s)));
-  ar.used = mark;
-  auto narrow = [&](auto kern, int lanes) {
-    kern<<<grid_for(ktot, 256 / lanes, 65536), 256, 0, s>>>(X, d, members, mstart, count, ktot,
-                                                           Cnew);
+  EAC_TRY(group_by_cluster(labels, n, P, d_koff, h_koff, members, start, nullptr, nullptr, ar, s));
+  ar.used = U->mark;
+  int64_t kmax = 1;
+  for (int p = 0; p < P; ++p)
+    if (h_koff[p + 1] - h_koff[p] > kmax) kmax = h_koff[p + 1] - h_koff[p];
+  // small clusters (up to 1024 coordinates on average): one wavefront each
+  const bool small = d <= kWave && items / ktot * d <= SumStage<kWave>::kFloats;
+  const bool v4 = (d & 3) == 0 && (reinterpret_cast<uintptr_t>(X) & 15) == 0;
+  const dim3 grid((unsigned)(kmax < 65536 ? kmax : 65536), P < 65535 ? P : 65535);
+  auto go = [&](auto kern, int bs) {
+    kern<<<grid, bs, 0, s>>>(X, d, members, start, d_koff, P, upd, U->eflag, n_empty, Cout);
   };
-  if (d <= 4) narrow(k_centroid_sums_narrow<4>, 4);
-  else if (d <= 8) narrow(k_centroid_sums_narrow<8>, 8);
-  else if (d <= 16) narrow(k_centroid_sums_narrow<16>, 16);
-  else if (d <= 32) narrow(k_centroid_sums_narrow<32>, 32);
-  else if (d <= 64) narrow(k_centroid_sums_narrow<64>, 64);
-  else
-    k_centroid_sums<<<grid_for(ktot, 1, 65536), kWave, 0, s>>>(X, d, members, mstart, count, ktot,
-                                                                Cnew);
+  if (small && v4) go(k_centroid_sums<kWave, true>, kWave);
+  else if (small) go(k_centroid_sums<kWave, false>, kWave);
+  else if (v4) go(k_centroid_sums<256, true>, 256);
+  else go(k_centroid_sums<256, false>, 256);
   EAC_LAUNCH_CHECK();
-  // empty clusters
-  k_empty_flags<<<grid_for(ktot, 256, 4096), 256, 0, s>>>(count, ktot, eflag);
-  EAC_LAUNCH_CHECK();
-  EAC_TRY((scan_excl<int32_t, int32_t>(eflag, erank, ktot + 1, 0, nullptr, ar, s)));
-  ar.used = mark;
-  if (g) {
-    k_reseed_dev<<<P < 4096 ? P : 4096, 1024, 0, s>>>(X, d, dists, n, k_off, P, count, erank,
-                                                      Cnew, g->err);
-    EAC_LAUNCH_CHECK();
-    k_fit_tally<<<1, 64, 0, s>>>(g->info, nullptr, erank, ktot, g->any);
-    EAC_LAUNCH_CHECK();
-    if (n_empty) *n_empty = 0;
-    return EAC_OK;
-  }
+  return EAC_OK;
+}
+
+// Empty clusters (total of them, known on the host) take the points of
+// smallest (dist, index) of their partition in ascending cluster order.
+int kmeans_reseed(const float* X, int64_t n, int d, const float* dists, const int64_t* h_koff,
+                  int P, float* Cout, const int32_t* upd, int32_t total, const UpdateBufs& U,
+                  Arena& ar, hipStream_t s) {
+  if (total == 0) return EAC_OK;
+  const int64_t ktot = h_koff[P];
+  ar.used = U.mark;
+  EAC_TRY((scan_excl<int32_t, int32_t>(U.eflag, U.erank, ktot + 1, 0, nullptr, ar, s)));
+  ar.used = U.mark;
   std::vector<int32_t> er(ktot + 1);
-  {
-    // host needs only the per-partition empty counts
-    std::vector<int32_t> tmp(ktot + 1);
-    EAC_TRY(d2h(tmp.data(), erank, sizeof(int32_t) * (ktot + 1), s));
-    er.swap(tmp);
-  }
-  int64_t total_empty = er[ktot];
-  if (n_empty) *n_empty = total_empty;
-  for (int p = 0; p < P && total_empty > 0; ++p) {
-    int64_t e = er[h_koff[p + 1]] - er[h_koff[p]];
+  EAC_TRY(d2h(er.data(), U.erank, sizeof(int32_t) * (ktot + 1), s));
+  for (int p = 0; p < P; ++p) {
+    const int64_t e = er[h_koff[p + 1]] - er[h_koff[p]];
     if (e == 0) continue;
     if (e > n) return fail(EAC_ERR_ARG, "kmeans update: more empty clusters than points");
-    k_dist_keys<<<grid_for(n, 256, 4096), 256, 0, s>>>(dists + (int64_t)p * n, n, dk);
+    k_dist_keys<<<grid_for(n, 256, 4096), 256, 0, s>>>(dists + (int64_t)p * n, n, U.dk);
     EAC_LAUNCH_CHECK();
-    EAC_TRY((radix_sort<uint64_t, NoValue>(dk, dks, nullptr, nullptr, n, 0, 64, ar, s)));
-    ar.used = mark;
+    EAC_TRY((radix_sort<uint64_t, NoValue>(U.dk, U.dks, nullptr, nullptr, n, 0, 64, ar, s)));
+    ar.used = U.mark;
     k_reseed<<<grid_for((h_koff[p + 1] - h_koff[p]) * d, 256, 4096), 256, 0, s>>>(
-        X, d, dks, count, erank, h_koff[p], h_koff[p + 1], Cnew);
+        X, d, U.dks, U.eflag, U.erank, h_koff[p], h_koff[p + 1], upd ? upd + p : nullptr, Cout);
     EAC_LAUNCH_CHECK();
   }
   return EAC_OK;
@@ -1875,18 +1879,16 @@ extern "C" size_t eac_kmeans_workspace_bytes(int64_t n, int32_t d, int64_t k_tot
   if (P < 1) P = 1;
   size_t a = kmeans_label_ws_bytes(n, d, k_total, P);
   size_t b = kmeans_update_ws_bytes(n, d, k_total, P);
-  // fit: labels/dists are caller buffers; new centroids and the per-partition
-  // state (inertia, previous inertia, offsets, active, iterations, update
-  // flags, one flag), each rounded up to 256 bytes
+  // fit: labels/dists/centroids are caller buffers; the per-partition state
+  // (previous inertia, offsets, active, iterations, update flags, two
+  // counters), each rounded up to 256 bytes
   Arena fa(nullptr, 0, true);
-  fa.take<float>((size_t)k_total * d);
-  fa.take<float>(P);
   fa.take<float>(P);
   fa.take<int64_t>(P + 1);
   fa.take<int32_t>(P);
   fa.take<int32_t>(P);
   fa.take<int32_t>(P);
-  fa.take<int32_t>(1);
+  fa.take<int32_t>(2);
   size_t c = fa.used + 4096;
   return (a > b ? a : b) + c;
 }
@@ -1932,10 +1934,17 @@ extern "C" int eac_kmeans_update(const float* X, int64_t n, int32_t d, const int
     return fail(EAC_ERR_WORKSPACE, "kmeans update: workspace %zu < %zu bytes", ws_bytes, need);
   Arena ar(ws, ws_bytes);
   hipStream_t s = (hipStream_t)stream;
-  int64_t ne = 0;
-  EAC_TRY(kmeans_update(X, n, d, labels, dists, h_koff, P, C_new, &ne, ar, s));
+  int64_t* k_off = ar.take<int64_t>(P + 1);
+  int32_t* d_ctl = ar.take<int32_t>(2);
+  EAC_TRY(put_i64(k_off, h_koff, P + 1, s));
+  EAC_TRY(fill<int32_t>(d_ctl, 2, 0, s));
+  UpdateBufs U;
+  EAC_TRY(kmeans_update(X, n, d, labels, h_koff, k_off, P, C_new, nullptr, d_ctl + 1, &U, ar, s));
+  int32_t ctl[2];
+  EAC_TRY(d2h(ctl, d_ctl, sizeof(ctl), s));
+  EAC_TRY(kmeans_reseed(X, n, d, dists, h_koff, P, C_new, nullptr, ctl[1], U, ar, s));
   EAC_HIP_CHECK(hipStreamSynchronize(s));
-  if (h_out) h_out[0] = ne;
+  if (h_out) h_out[0] = ctl[1];
   return EAC_OK;
 }
 
@@ -1998,12 +2007,10 @@ extern "C" int eac_kmeans_fit_graph(const float* X, int64_t n, int32_t d, float*
   hipStream_t s = (hipStream_t)stream;
   Arena ar(ws, ws_bytes);
   KmGraph g = carve_graph(ar, n, P, d_info, d_err);
-  float* Cnew = ar.take<float>((size_t)ktot * d);
-  float* inertia = ar.take<float>(P);
   float* prev = ar.take<float>(P);
   int32_t* active = ar.take<int32_t>(P);
   int32_t* upd = ar.take<int32_t>(P);
-  int32_t* d_any = ar.take<int32_t>(1);
+  int32_t* d_any = ar.take<int32_t>(2);
   if (ar.overflow()) return fail(EAC_ERR_WORKSPACE, "kmeans fit graph: workspace too small");
   const size_t mark = ar.used;
   g.any = d_any;
@@ -2015,17 +2022,21 @@ extern "C" int eac_kmeans_fit_graph(const float* X, int64_t n, int32_t d, float*
   for (int it = 1; it <= max_iter; ++it) {
     ar.used = mark;
     int64_t nres = 0;
-    EAC_TRY(kmeans_label(X, n, d, C_inout, h_koff, P, mode, labels, dists, inertia, &nres, ar,
+    const float* csum = nullptr;
+    EAC_TRY(kmeans_label(X, n, d, C_inout, h_koff, P, mode, labels, dists, &csum, &nres, ar,
                          s, d_koff, &g));
-    k_converge<<<1, 1024, 0, s>>>(inertia, prev, active, d_iters, upd, P, it, max_iter,
+    k_converge<<<1, 1024, 0, s>>>(csum, np_chunks(n), prev, active, d_iters, upd, P, it, max_iter,
                                   (float)tol, d_any);
     EAC_LAUNCH_CHECK();
     if (it >= max_iter) break;
     ar.used = mark;
-    int64_t ne = 0;
-    EAC_TRY(kmeans_update(X, n, d, labels, dists, h_koff, P, Cnew, &ne, ar, s, d_koff, &g));
-    const dim3 gc(grid_for(ktot * d / P + 1, 256, 64), P < 65535 ? P : 65535);
-    k_copy_running<<<gc, 256, 0, s>>>(C_inout, Cnew, d, d_koff, P, upd);
+    UpdateBufs U;
+    EAC_TRY(kmeans_update(X, n, d, labels, h_koff, d_koff, P, C_inout, upd, d_any + 1, &U, ar, s));
+    EAC_TRY((scan_excl<int32_t, int32_t>(U.eflag, U.erank, ktot + 1, 0, nullptr, ar, s)));
+    k_reseed_dev<<<P < 4096 ? P : 4096, 1024, 0, s>>>(X, d, dists, n, d_koff, P, U.eflag, U.erank,
+                                                      upd, C_inout, g.err);
+    EAC_LAUNCH_CHECK();
+    k_fit_tally<<<1, 64, 0, s>>>(g.info, nullptr, U.erank, ktot, g.any);
     EAC_LAUNCH_CHECK();
   }
   return EAC_OK;
@@ -2070,19 +2081,19 @@ extern "C" int eac_kmeans_fit(const float* X, int64_t n, int32_t d, float* C_ino
     return fail(EAC_ERR_WORKSPACE, "kmeans fit: workspace %zu < %zu bytes", ws_bytes, need);
   hipStream_t s = (hipStream_t)stream;
   Arena ar(ws, ws_bytes);
-  float* Cnew = ar.take<float>((size_t)ktot * d);
-  float* inertia = ar.take<float>(P);
   float* prev = ar.take<float>(P);
   int64_t* d_koff = ar.take<int64_t>(P + 1);
   int32_t* active = ar.take<int32_t>(P);
   int32_t* d_iters = ar.take<int32_t>(P);
   int32_t* upd = ar.take<int32_t>(P);
-  int32_t* d_any = ar.take<int32_t>(1);
+  int32_t* d_any = ar.take<int32_t>(2);
   if (ar.overflow()) return fail(EAC_ERR_WORKSPACE, "kmeans fit: workspace too small");
   const size_t mark = ar.used;
-  // the partition offsets go up once; the stopping rule runs on the device,
-  // so an iteration costs one read-back (does any partition continue?)
-  EAC_TRY(h2d(d_koff, h_koff, sizeof(int64_t) * (P + 1), s));
+  // the partition offsets go up once; the stopping rule runs on the device
+  // and the update follows it unread (a stopped partition's centroids stay),
+  // so an iteration costs one read-back: does any partition continue, and
+  // did a cluster lose all its points?
+  EAC_TRY(put_i64(d_koff, h_koff, P + 1, s));
   k_fit_init<<<grid_for(P, 256, 1024), 256, 0, s>>>(prev, active, d_iters, P);
   EAC_LAUNCH_CHECK();
   int64_t tot_res = 0, tot_empty = 0;
@@ -2091,23 +2102,22 @@ extern "C" int eac_kmeans_fit(const float* X, int64_t n, int32_t d, float* C_ino
     // centroids, deterministic kernels)
     int64_t nres = 0;
     ar.used = mark;
-    EAC_TRY(kmeans_label(X, n, d, C_inout, h_koff, P, mode, labels, dists, inertia, &nres, ar,
-                         s, d_koff));
+    const float* csum = nullptr;
+    EAC_TRY(kmeans_label(X, n, d, C_inout, h_koff, P, mode, labels, dists, &csum, &nres, ar, s,
+                         d_koff));
     tot_res += nres;
-    k_converge<<<1, 1024, 0, s>>>(inertia, prev, active, d_iters, upd, P, it, max_iter,
+    k_converge<<<1, 1024, 0, s>>>(csum, np_chunks(n), prev, active, d_iters, upd, P, it, max_iter,
                                   (float)tol, d_any);
     EAC_LAUNCH_CHECK();
     if (it >= max_iter) break;  // every partition stops at max_iter
-    int32_t any = 0;
-    EAC_TRY(d2h(&any, d_any, sizeof(any), s));
-    if (!any) break;
     ar.used = mark;
-    int64_t ne = 0;
-    EAC_TRY(kmeans_update(X, n, d, labels, dists, h_koff, P, Cnew, &ne, ar, s, d_koff));
-    tot_empty += ne;
-    const dim3 gc(grid_for(ktot * d / P + 1, 256, 64), P < 65535 ? P : 65535);
-    k_copy_running<<<gc, 256, 0, s>>>(C_inout, Cnew, d, d_koff, P, upd);
-    EAC_LAUNCH_CHECK();
+    UpdateBufs U;
+    EAC_TRY(kmeans_update(X, n, d, labels, h_koff, d_koff, P, C_inout, upd, d_any + 1, &U, ar, s));
+    int32_t ctl[2];
+    EAC_TRY(d2h(ctl, d_any, sizeof(ctl), s));
+    if (!ctl[0]) break;
+    tot_empty += ctl[1];
+    EAC_TRY(kmeans_reseed(X, n, d, dists, h_koff, P, C_inout, upd, ctl[1], U, ar, s));
   }
   if (h_iters) EAC_TRY(d2h(h_iters, d_iters, sizeof(int32_t) * P, s));
   EAC_HIP_CHECK(hipStreamSynchronize(s));

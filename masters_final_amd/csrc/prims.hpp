@@ -18,6 +18,10 @@ template <typename Tin, typename Tout>
 int scan_excl(const Tin* in, Tout* out, int64_t n, Tout init, Tout* d_total,
               Arena& ar, hipStream_t s);
 
+// Copies a few host values to the device inside kernel arguments: no pinned
+// buffer, no copy engine and nothing to wait for before h_src is reused.
+int put_i64(int64_t* dst, const int64_t* h_src, int64_t n, hipStream_t s);
+
 // Fill kernel launcher (used instead of hipMemsetAsync so that callers may
 // capture the sequence in a graph).
 template <typename T>

@@ -10,13 +10,21 @@
 //
 // Layout: a tile is read coalesced (striped, 256 threads x 16 items), turned
 // blocked through padded LDS, scanned sequentially per thread, combined with
-// a wave64 shuffle scan across threads, and written back striped. Tile sums
-// are scanned recursively with the same kernels.
+// a wave64 shuffle scan across threads, and written back striped. Short
+// inputs take one workgroup and one launch; up to kDirectTiles tiles every
+// workgroup of the second launch adds up the sums of the tiles before its
+// own (a launch costs more than those reads); beyond that the tile sums are
+// scanned recursively with the same kernels.
 #include "prims.hpp"
 
 namespace eac {
 
 namespace {
+
+constexpr int kScanOne = 1024;          // threads of the one-workgroup scan
+constexpr int64_t kOneBlock = 32768;    // elements it takes: two of its tiles
+constexpr int64_t kDirectTiles = 8192;  // tile sums a workgroup adds up itself
+constexpr int kPutBatch = 448;          // values a k_put launch carries (3.5 KB of arguments)
 
 template <typename T>
 __device__ __forceinline__ int pad_idx(int i) {
@@ -47,7 +55,39 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const Tin* __restric
   }
 }
 
+// One workgroup scans up to kOneBlock elements, a tile of kScanOne threads x
+// 16 elements after the other. In place is allowed: a tile is read before
+// any of it is written.
 template <typename Tin, typename Tout>
+__global__ __launch_bounds__(kScanOne) void k_scan_one(const Tin* in, Tout* out, int64_t n,
+                                                       Tout init, Tout* __restrict__ d_total) {
+  __shared__ Tout wsum[kScanOne / kWave + 1];
+  const int t = threadIdx.x;
+  Tout off = init;
+  for (int64_t base = 0; base < n; base += kScanOne * kScanItems) {
+    const int64_t i0 = base + (int64_t)t * kScanItems;
+    Tout v[kScanItems];
+    Tout acc = 0;
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+      v[k] = i0 + k < n ? static_cast<Tout>(in[i0 + k]) : Tout(0);
+      acc += v[k];
+    }
+    Tout total;
+    Tout pre = off + block_excl_scan(acc, wsum, &total);
+#pragma unroll
+    for (int k = 0; k < kScanItems; ++k) {
+      if (i0 + k < n) out[i0 + k] = pre;
+      pre += v[k];
+    }
+    off += total;
+  }
+  if (d_total && t == 0) *d_total = off;
+}
+
+// RAW: offs holds the tiles' plain sums, and the workgroup adds up those
+// before its own.
+template <typename Tin, typename Tout, bool RAW = false>
 __global__ __launch_bounds__(kScanBlock) void k_scan_down(const Tin* in, Tout* out,
                                                           int64_t n,
                                                           const Tout* __restrict__ offs,
@@ -57,8 +97,20 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(const Tin* in, Tout* o
   __shared__ Tout tile[kScanTile + kPad];
   __shared__ Tout wsum[kScanBlock / kWave + 1];
   const int64_t base = (int64_t)blockIdx.x * kScanTile;
-  const Tout off = offs ? offs[blockIdx.x] : init;
   const int t = threadIdx.x;
+  Tout off = init;
+  if (RAW) {
+    Tout s = 0;
+    for (int j = t; j < (int)blockIdx.x; j += kScanBlock) s += offs[j];
+    s = wave_sum(s);
+    if (lane_id() == 0) wsum[t / kWave] = s;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kScanBlock / kWave; ++w) off += wsum[w];
+    __syncthreads();
+  } else if (offs) {
+    off = offs[blockIdx.x];
+  }
 #pragma unroll
   for (int j = 0; j < kScanItems; ++j) {
     int64_t i = base + j * kScanBlock + t;
@@ -86,6 +138,13 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_down(const Tin* in, Tout* o
     if (i < n) out[i] = tile[pad_idx<Tout>(j * kScanBlock + t)];
   }
   if (d_total && blockIdx.x == gridDim.x - 1 && t == 0) *d_total = off + total;
+}
+
+struct PutBatch {
+  int64_t v[kPutBatch];
+};
+__global__ void k_put(int64_t* __restrict__ dst, PutBatch b, int n) {
+  for (int i = threadIdx.x; i < n; i += blockDim.x) dst[i] = b.v[i];
 }
 
 template <typename T>
@@ -116,6 +175,18 @@ int fill(T* p, int64_t n, T value, hipStream_t s) {
   return EAC_OK;
 }
 
+int put_i64(int64_t* dst, const int64_t* h_src, int64_t n, hipStream_t s) {
+  for (int64_t i = 0; i < n; i += kPutBatch) {
+    PutBatch b;
+    const int m = (int)(n - i < kPutBatch ? n - i : kPutBatch);
+    for (int j = 0; j < m; ++j) b.v[j] = h_src[i + j];
+    for (int j = m; j < kPutBatch; ++j) b.v[j] = 0;
+    k_put<<<1, 256, 0, s>>>(dst + i, b, m);
+    EAC_LAUNCH_CHECK();
+  }
+  return EAC_OK;
+}
+
 template <typename Tin, typename Tout>
 int scan_excl(const Tin* in, Tout* out, int64_t n, Tout init, Tout* d_total,
               Arena& ar, hipStream_t s) {
@@ -131,10 +202,23 @@ int scan_excl(const Tin* in, Tout* out, int64_t n, Tout init, Tout* d_total,
     EAC_LAUNCH_CHECK();
     return EAC_OK;
   }
+  // in place with a narrower input a tile's outputs would cover inputs of
+  // the next one: those callers take the tiled kernels
+  if (n <= kOneBlock && ((const void*)in != (const void*)out || sizeof(Tin) == sizeof(Tout))) {
+    k_scan_one<Tin, Tout><<<1, kScanOne, 0, s>>>(in, out, n, init, d_total);
+    EAC_LAUNCH_CHECK();
+    return EAC_OK;
+  }
   Tout* sums = ar.take<Tout>(tiles);
   if (ar.overflow()) return fail(EAC_ERR_WORKSPACE, "scan: workspace too small");
   k_scan_reduce<Tin, Tout><<<(int)tiles, kScanBlock, 0, s>>>(in, n, sums);
   EAC_LAUNCH_CHECK();
+  if (tiles <= kDirectTiles) {
+    k_scan_down<Tin, Tout, true><<<(int)tiles, kScanBlock, 0, s>>>(in, out, n, sums, init,
+                                                                   d_total);
+    EAC_LAUNCH_CHECK();
+    return EAC_OK;
+  }
   EAC_TRY((scan_excl<Tout, Tout>(sums, sums, tiles, init, nullptr, ar, s)));
   k_scan_down<Tin, Tout><<<(int)tiles, kScanBlock, 0, s>>>(in, out, n, sums, init, d_total);
   EAC_LAUNCH_CHECK();
