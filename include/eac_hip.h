@@ -95,12 +95,12 @@ int eac_profile_read(int32_t slot, double* total_ms, int64_t* launches, int64_t*
  *                           4, up to 4 levels; 1 or -1 = one split only)
  *   EAC_TUNE_CO_UNROLL      co-association member loads in flight per lane
  *                           while counting (4 by default, or 8)
- *   EAC_TUNE_CO_RANGES      co-association row ranges with a row counter
- *                           each (1..8, default 8: one per XCD; 1 below
- *                           65536 rows)
- *   EAC_TUNE_KM_WAVES       waves per SIMD the split-BF16 labeling kernel
- *                           is compiled for (2, 3 or 4; default 3 for
- *                           d <= 64, else unconstrained) */
+ *   EAC_TUNE_CO_RANGES      contiguous co-association row ranges with a row
+ *                           counter each (1..8, default 8: one per XCD; 32
+ *                           interleaved ranges below 65536 rows)
+ *   EAC_TUNE_KM_WAVES       waves per SIMD the MFMA labeling kernel is
+ *                           compiled for (2, 3 or 4; for the layouts of
+ *                           d = 11..21 and d = 54..64) */
 #define EAC_TUNE_LIGHT_X10 0
 #define EAC_TUNE_FIRST_BATCH 1
 #define EAC_TUNE_FILTER_BPCU 2
@@ -293,10 +293,11 @@ int eac_radix_sort_u64(const uint64_t* keys_in, uint64_t* keys_out,
  *   EAC_KM_F64     FP64 direct difference, ascending dimensions, strict < ->
  *                  exactly MyML/MyML/cluster/KMeans.py:453-490 numba_label
  *                  evaluated in FP64 (the oracle);
- *   EAC_KM_BF16X3  split-BF16 MFMA contraction with fp32 accumulation, a
- *                  rigorous per-point error bound, FP64 re-scoring of every
- *                  point whose top-2 margin is within it -> labels and
- *                  distances equal EAC_KM_F64's (d < 16 runs EAC_KM_F64);
+ *   EAC_KM_BF16X3  MFMA contraction of operands split into two 16-bit halves
+ *                  with fp32 accumulation, a rigorous per-point error bound,
+ *                  FP64 re-scoring of every point whose margin is within it
+ *                  -> labels and distances equal EAC_KM_F64's (which runs
+ *                  for d < 4, and for d < 16 where it is the faster one);
  *   EAC_KM_F32_NUMPY numpy's float32 arithmetic of KMeans.py:493-522
  *                  np_label: ((x - c) ** 2).sum(axis=1) with a float32
  *                  difference and square and numpy's pairwise row sum,

@@ -7,8 +7,9 @@ or a given array, the label -> iteration count -> convergence check ->
 centroid update loop with tol on |sum(dists) - previous| (KMeans.py:154-186).
 Labeling and the centroid update run in libeac_hip.so; `precision` picks the
 labeling arithmetic:
-  "bf16x3" (default): split-BF16 MFMA distances, FP64 re-scoring of the points
-           a rigorous bound cannot certify -> labels equal the FP64 oracle's;
+  "bf16x3" (default): MFMA distances of operands split into 16-bit halves,
+           FP64 re-scoring of the points a rigorous bound cannot certify ->
+           labels equal the FP64 oracle's;
   "fp64":  FP64 direct difference (the oracle's arithmetic);
   "fp32":  plain FP32 direct difference (the reference GPU kernel's spirit,
            KMeans.py:586-629).

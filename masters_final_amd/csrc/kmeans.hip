@@ -14,20 +14,30 @@
 //  * F64: FP64 direct difference in ascending dimension order with strict <,
 //    i.e. the oracle's arithmetic; exact by construction.
 //  * BF16X3: the distance ||x||^2 - 2 x.c + ||c||^2 with the contraction on
-//    MFMA. Each operand is split into two bf16 halves (x = xh + xl + ex,
-//    xh = bf16(x), xl = bf16(x - xh)); three 16x16x32 bf16 MFMAs
-//    (xh.ch + xh.cl + xl.ch) accumulate in fp32. The epilogue keeps the two
-//    smallest distances per point. A rigorous per-point bound E on
+//    MFMA. Each operand is split into two 16-bit halves (x = xh + xl + ex);
+//    16x16x32 MFMAs of xh.ch + xh.cl + xl.ch accumulate in fp32. The halves
+//    are f16 after a power-of-two scaling: 22 bits of every coordinate
+//    against the 16 of two bf16 halves, at the same rate (2^-23 rather than
+//    2^-17 left over: 0.16% of a 500,000-point ensemble re-scored instead of
+//    0.33%, 0.19% of 4 M x 64-d points). The epilogue keeps the two best
+//    groups of four centroids per point. A rigorous per-point bound E on
 //    |approx - FP64 oracle| (split residuals, fp32 accumulation with a
-//    truncation-safe 2^-23 unit, epilogue rounding, oracle rounding) certifies
-//    the argmin when second - best > 2E; every other point is re-scored in
-//    FP64 against all centroids of its partition. Labels therefore equal the
-//    FP64 oracle's; distances are then recomputed in FP64 for every point
-//    (d flops) so they equal the oracle's too.
+//    truncation-safe 2^-23 unit, oracle rounding) certifies the group when the
+//    margin exceeds 2 E, and its four candidates are compared in FP64; every
+//    other point is re-scored in FP64 against all centroids of its partition.
+//    Labels and distances therefore equal the FP64 oracle's.
+//    Large single labelings of more than 32 dimensions run as a cascade: one
+//    product first (a third of the MFMAs, a wider bound), all three only for
+//    the rows it cannot certify (1% on the 64-d workload).
+//    4,194,304 x 64-d points, 2048 centroids: 4.00 -> 1.9 ms a pass (the
+//    single product 1.54, of which the group's FP64 comparison is a third;
+//    bound by vector issue), 300,007 x 37-d, 501 centroids: 239 -> 178 us.
+#include <algorithm>
 #include <cfloat>
 #include <climits>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "group.hpp"
@@ -37,396 +47,655 @@
 namespace eac {
 namespace {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
+// ------------------------------------------------- split-f16 MFMA labeling
+// Layout of the split rows (points in registers, centroids in memory and
+// LDS). Every operand is scaled by a power of two (a point by its own row's
+// largest coordinate, the centroids of a partition by theirs) into f16's
+// normal range and split into two f16 halves, v = h + l + e; halves below
+// f16's smallest normal value are zero, so no product meets a subnormal. Three
+// products h.h + h.l + l.h make the contraction. For d where it saves MFMA
+// steps the three pieces are laid end to end over one K axis of 3 d entries
+// (points: h, l, h; centroids: h, h, l), 32 entries a step: ceil(3 d / 32)
+// steps; otherwise (3 d close to a multiple of 96) h and l are kept as rows
+// of KB = ceil(d / 32) fragments and used twice: 3 KB steps from 2 KB
+// fragments.
+struct LabelLayout {
+  int KS;      // MFMA steps (32 entries each)
+  bool split;  // two rows of KS / 3 fragments
+  int NF;      // fragments per row (32 halves each)
+};
+inline LabelLayout label_layout(int d, bool want_split = false) {
+  LabelLayout L;
+  const int packed = (3 * d + 31) / 32, KB = (d + 31) / 32;
+  L.split = want_split || packed >= 3 * KB || packed == 3 || packed > 8 || packed == 6;
+  L.KS = L.split ? 3 * KB : packed;
+  L.NF = L.split ? 2 * KB : packed;
+  return L;
+}
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// LDS rows are written as 16-bit words and read as fragments
+typedef f16x8 f16x8_lds __attribute__((may_alias));
+typedef f32x4 f32x4_u __attribute__((aligned(4)));  // rows need no more than their own alignment
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+typedef u32x4 u32x4_lds __attribute__((may_alias));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef f16x4 f16x4_lds __attribute__((may_alias));
 
-__device__ __forceinline__ uint16_t bf16_rne(float f) {
-  uint32_t u = __float_as_uint(f);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// Power-of-two scale that takes a largest magnitude m into [2^14, 2^15)
+// (1 for 0, infinity and NaN; exponents are kept within 2^+-60, so products of
+// two scales and their inverses stay finite and normal).
+__device__ __forceinline__ float pow2_scale(float m) {
+  const int e = (int)((__float_as_uint(m) >> 23) & 255u);
+  if (e == 255 || m == 0.0f) return 1.0f;
+  int s = 127 + 14 - (e - 127);  // biased exponent of the scale
+  s = s < 127 - 60 ? 127 - 60 : s > 127 + 60 ? 127 + 60 : s;
+  return __uint_as_float((uint32_t)s << 23);
 }
-__device__ __forceinline__ float bf16_val(uint16_t h) { return __uint_as_float((uint32_t)h << 16); }
+__device__ __forceinline__ _Float16 f16_half(float v) {
+  return fabsf(v) < 6.103515625e-05f ? (_Float16)0.0f : (_Float16)v;
+}
+__device__ __forceinline__ uint16_t f16_bits(_Float16 h) { return __builtin_bit_cast(uint16_t, h); }
 
-// Partition of a global centroid index (k_off ascending, P small).
-__device__ __forceinline__ int part_of(const int64_t* k_off, int P, int64_t c) {
-  int lo = 0, hi = P;
-  while (lo + 1 < hi) {
-    int mid = (lo + hi) >> 1;
-    if (k_off[mid] <= c) lo = mid; else hi = mid;
+// Per-partition statistics of the centroids as float bits (non-negative
+// floats order like their bit patterns): maxima of ||c||, ||ch||, ||cl||,
+// ||ec|| (unscaled), and of |c_j| (the scale).
+constexpr int kStat = 5;
+
+// Largest |c_j| of each partition (grid.y over partitions).
+__global__ __launch_bounds__(256) void k_cent_max(const float* __restrict__ C, int d,
+                                                  const int64_t* __restrict__ k_off, int P,
+                                                  unsigned int* __restrict__ pstat) {
+  for (int p = blockIdx.y; p < P; p += gridDim.y) {
+    const int64_t a = k_off[p] * d, b = k_off[p + 1] * d;
+    unsigned int m = 0;
+    for (int64_t i = a + (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < b;
+         i += (int64_t)gridDim.x * blockDim.x)
+      m = max(m, __float_as_uint(C[i]) & 0x7fffffffu);
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) m = max(m, (unsigned)__shfl_xor(m, off, kWave));
+    if (lane_id() == 0 && m) atomicMax(&pstat[p * kStat + 4], m);
   }
-  return lo;
 }
 
-// Per-partition maxima of centroid norms, as float bits (non-negative floats
-// order like their bit patterns): [0] ||c||, [1] ||ch||, [2] ||cl||, [3] ||ec||.
-constexpr int kStat = 4;
-
-// Split every centroid into bf16 halves (row length KD, zero padded) and
-// record norms. The per-partition maxima are reduced over the wavefront
-// first when its lanes share one partition (one atomic per statistic instead
-// of one per centroid: same-address atomics serialise).
-__global__ void k_cent_prep(const float* __restrict__ C, int64_t ktot, int d, int KD,
-                            const int64_t* __restrict__ k_off, int P,
-                            uint16_t* __restrict__ Ch, uint16_t* __restrict__ Cl,
-                            float* __restrict__ Ct, float* __restrict__ ncf,
-                            unsigned int* __restrict__ pstat) {
-  const int64_t stride = (int64_t)gridDim.x * blockDim.x;
-  for (int64_t base = (int64_t)blockIdx.x * blockDim.x; base < ktot; base += stride) {
-    const int64_t c = base + threadIdx.x;
-    const bool valid = c < ktot;
-    double n2 = 0, h2 = 0, l2 = 0, e2 = 0;
-    int p = -1;
-    if (valid) {
-      for (int j = 0; j < KD; ++j) {
-        float x = j < d ? C[c * d + j] : 0.f;
-        uint16_t h = bf16_rne(x);
-        float r = x - bf16_val(h);  // exact
-        uint16_t l = bf16_rne(r);
-        float e = r - bf16_val(l);  // exact
-        Ch[c * KD + j] = h;
-        Cl[c * KD + j] = l;
-        if (j < d) Ct[(int64_t)j * ktot + c] = x;  // transposed copy for the re-scoring
+// Splits every centroid into its layout row Cf [ktot][NF * 32] (zero padded),
+// writes ||c||^2 and (Ct, nullable) the transposed copy, and reduces the norm
+// maxima. Sixteen lanes per centroid; grid.y over partitions.
+__global__ __launch_bounds__(256) void k_cent_prep(const float* __restrict__ C, int64_t ktot, int d,
+                                                   LabelLayout L,
+                                                   const int64_t* __restrict__ k_off, int P,
+                                                   uint16_t* __restrict__ Cf,
+                                                   float* __restrict__ Ct,
+                                                   float* __restrict__ ncf,
+                                                   unsigned int* __restrict__ pstat) {
+  __shared__ unsigned int s_v[256 / kWave][4];
+  const int sub = threadIdx.x & 15;
+  const int RH = L.NF * 32;
+  for (int p = blockIdx.y; p < P; p += gridDim.y) {
+    const int64_t kb = k_off[p], ke = k_off[p + 1];
+    const float sc = pow2_scale(__uint_as_float(pstat[p * kStat + 4])), inv = 1.0f / sc;
+    unsigned int v[4] = {0u, 0u, 0u, 0u};
+    for (int64_t c = kb + (int64_t)blockIdx.x * 16 + threadIdx.x / 16; c < ke;
+         c += (int64_t)gridDim.x * 16) {
+      double n2 = 0, h2 = 0, l2 = 0, e2 = 0;
+      uint16_t* row = Cf + c * RH;
+      for (int j = sub; j < d; j += 16) {
+        const float x = C[c * d + j], y = x * sc;
+        const _Float16 h = f16_half(y);
+        const float r = y - (float)h;  // exact
+        const _Float16 l = f16_half(r);
+        const float e = r - (float)l;  // exact
+        if (L.split) {
+          row[j] = f16_bits(h);
+          row[RH / 2 + j] = f16_bits(l);
+        } else {
+          row[j] = f16_bits(h);
+          row[d + j] = f16_bits(h);
+          row[2 * d + j] = f16_bits(l);
+        }
+        if (Ct) Ct[(int64_t)j * ktot + c] = x;  // transposed copy for the re-scoring
+        const double hd = (double)(float)h * inv, ld = (double)(float)l * inv;
+        const double ed = (double)e * inv;
         n2 += (double)x * x;
-        h2 += (double)bf16_val(h) * bf16_val(h);
-        l2 += (double)bf16_val(l) * bf16_val(l);
-        e2 += (double)e * e;
+        h2 += hd * hd;
+        l2 += ld * ld;
+        e2 += ed * ed;
       }
-      ncf[c] = (float)n2;
-      p = part_of(k_off, P, c);
+      if (L.split) {
+        for (int j = d + sub; j < RH / 2; j += 16) row[j] = row[RH / 2 + j] = 0;
+      } else {
+        for (int j = 3 * d + sub; j < RH; j += 16) row[j] = 0;
+      }
+#pragma unroll
+      for (int off = 1; off < 16; off <<= 1) {
+        n2 += __shfl_xor(n2, off, kWave);
+        h2 += __shfl_xor(h2, off, kWave);
+        l2 += __shfl_xor(l2, off, kWave);
+        e2 += __shfl_xor(e2, off, kWave);
+      }
+      if (sub == 0) ncf[c] = (float)n2;
+      // norms rounded up so the bound stays rigorous (a NaN or infinity
+      // keeps the largest bits: its partition's points are all re-scored)
+      v[0] = max(v[0], __float_as_uint((float)sqrt(n2) * (1.f + 1e-6f)) & 0x7fffffffu);
+      v[1] = max(v[1], __float_as_uint((float)sqrt(h2) * (1.f + 1e-6f)) & 0x7fffffffu);
+      v[2] = max(v[2], __float_as_uint((float)sqrt(l2) * (1.f + 1e-6f)) & 0x7fffffffu);
+      v[3] = max(v[3], __float_as_uint((float)sqrt(e2) * (1.f + 1e-6f)) & 0x7fffffffu);
     }
-    // norms rounded up so the bound stays rigorous; non-negative floats order
-    // like their bit patterns, and 0 is the identity of the maximum
-    unsigned int v[kStat] = {
-        valid ? __float_as_uint((float)sqrt(n2) * (1.f + 1e-6f)) : 0u,
-        valid ? __float_as_uint((float)sqrt(h2) * (1.f + 1e-6f)) : 0u,
-        valid ? __float_as_uint((float)sqrt(l2) * (1.f + 1e-6f)) : 0u,
-        valid ? __float_as_uint((float)sqrt(e2) * (1.f + 1e-6f)) : 0u};
-    int pmin = valid ? p : INT_MAX, pmax = p;
+    // one atomic per statistic and block (same-address atomics serialise)
 #pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      pmin = min(pmin, __shfl_xor(pmin, off, kWave));
-      pmax = max(pmax, __shfl_xor(pmax, off, kWave));
+    for (int q = 0; q < 4; ++q) {
+#pragma unroll
+      for (int off = 16; off < kWave; off <<= 1)
+        v[q] = max(v[q], (unsigned)__shfl_xor(v[q], off, kWave));
     }
-    if (pmin == pmax) {  // every valid lane in one partition (uniform)
+    __syncthreads();
+    if (lane_id() == 0)
 #pragma unroll
-      for (int q = 0; q < kStat; ++q)
-#pragma unroll
-        for (int off = kWave / 2; off > 0; off >>= 1) v[q] = max(v[q], __shfl_xor(v[q], off, kWave));
-      if (lane_id() == 0)
-#pragma unroll
-        for (int q = 0; q < kStat; ++q) atomicMax(&pstat[pmax * kStat + q], v[q]);
-    } else if (valid) {
-#pragma unroll
-      for (int q = 0; q < kStat; ++q) atomicMax(&pstat[p * kStat + q], v[q]);
+      for (int q = 0; q < 4; ++q) s_v[threadIdx.x / kWave][q] = v[q];
+    __syncthreads();
+    if (threadIdx.x < 4) {
+      unsigned int m = 0;
+      for (int u = 0; u < 256 / kWave; ++u) m = max(m, s_v[u][threadIdx.x]);
+      if (m) atomicMax(&pstat[p * kStat + threadIdx.x], m);
     }
   }
 }
 
 constexpr int kLB = 256;       // threads per labeling block (4 waves)
-constexpr int kRowsW = 32;     // points per wave
-constexpr int kBM = 128;       // points per block
 constexpr int kBN = 64;        // centroids per LDS tile
 constexpr int kFlagSlots = 64; // flag list regions (one counter each)
+constexpr int kGrp = 4;        // consecutive centroids of a candidate group
 
-// Rigorous bound on |approx - oracle| for one point and one partition.
-__device__ __forceinline__ float point_bound(float nx, float xn, float xhn, float xln, float exn,
-                                             const float* st, int KD, int d) {
+// Rigorous bound on |approx - oracle| for one point and one partition, for
+// D' = ||c||^2 - 2 x.c (||x||^2 is common to a point's centroids) accumulated
+// from ||c||^2 on: the three products of the split, or (TERMS = 1) only xh.ch,
+// where x.c - xh.ch = (x - xh).c + xh.(c - ch). rs: the point's ||x||, ||xh||,
+// ||xl|| and ||ex|| (TERMS = 1: ||x - xh||), st: the partition's maxima.
+template <int TERMS>
+__device__ __forceinline__ float point_bound(const float* rs, const float* st, int d) {
   const float u = 5.9604645e-08f;            // 2^-24
   const float ut = 1.1920929e-07f;           // 2^-23: fp32 accumulation, any rounding
+  const float xn = rs[0], xhn = rs[1], xln = rs[2], exn = rs[3];
   const float Cn = st[0], Chn = st[1], Cln = st[2], Cen = st[3];
-  // nonzero products per dot: 3 d (columns d..KD-1 are zero in both
-  // operands; adding an exact zero neither rounds nor truncates)
-  const float nterms = 3.f * (d < KD ? d : KD);
+  // nonzero products per dot and the starting value (the padding is zero in
+  // both operands; adding an exact zero neither rounds nor truncates)
+  const float nterms = (float)(TERMS * d + 1);
   const float gam = nterms * ut / (1.f - nterms * ut);
-  float cross = gam * (xhn * (Chn + Cln) + xln * Chn) + xhn * Cen + xln * (Cln + Cen) + exn * Cn;
-  float epi = 6.f * u * (nx + Cn * Cn);
-  float orc = 4.f * d * 1.1102230e-16f * (xn + Cn) * (xn + Cn);
+  const float cross =
+      TERMS == 1
+          ? gam * xhn * Chn + exn * Cn + xhn * (Cln + Cen)
+          : gam * (xhn * (Chn + Cln) + xln * Chn) + xhn * Cen + xln * (Cln + Cen) + exn * Cn;
+  const float epi = (gam + 6.f * u) * Cn * Cn + 6.f * u * xn * xn;
+  const float orc = 4.f * d * 1.1102230e-16f * (xn + Cn) * (xn + Cn);
   return (2.f * cross + epi + orc) * 1.0001f + 1e-30f;
 }
 
-// Waves per SIMD the compiler must fit (WPE): by default 3 for KD <= 64 (a
-// few values spill; measured faster than 2 waves without spills),
-// otherwise no constraint (1); the EAC_TUNE_KM_WAVES knob picks 2, 3 or 4.
-constexpr int label_waves(int KD) { return KD <= 64 ? 3 : 1; }
-template <int KD, int WPE = label_waves(KD)>
+// The nearest of a group's kGrp consecutive centroids for 16 points of a
+// wave, in the oracle's FP64 arithmetic (ascending dimensions, strict <, lowest
+// index on ties). Four lanes per point, one per candidate, each adding its own
+// chain in order; row and g are the lane's point and its group's first
+// centroid. The rows go through LDS, 16 dimensions at a time: a point's lanes
+// load its row and its candidates' rows 64 bytes a row, the next stage's
+// loads in flight during the current sums, and every lane reads back its own
+// row; straight from memory the lanes would take 16 bytes of 64 different
+// lines per load. sf: kRsLds floats of the wave; d >= 4. V4: d is a multiple
+// of four, so every piece lies on 16 bytes of LDS.
+constexpr int kRsD = 16;          // dimensions per stage
+constexpr int kRsS = kRsD + 4;    // LDS row stride: 16-byte reads of neighbouring rows on other banks
+constexpr int kRsLds = (kWave + kWave / kGrp) * kRsS + 4;
+template <bool V4>
+__device__ __forceinline__ void resolve16(const float* __restrict__ X, int d,
+                                          const float* __restrict__ C, int64_t kb, int64_t ke,
+                                          int64_t row, int32_t g, float* __restrict__ sf,
+                                          double& best, int32_t& bk) {
+#pragma clang fp contract(off)  // the oracle's separately rounded products and sums
+  using Piece = std::conditional_t<V4, f32x4, f32x4_u>;  // 16-byte LDS stores with V4
+  const int l = lane_id(), pt = l / kGrp, q = l % kGrp;
+  const int32_t k = (int32_t)(ke - kb);
+  // A point's four lanes load its rows together: lane q 16 bytes at 16 q of
+  // each candidate's row and of the point's, the last piece of a row moved
+  // back to end with it (its overlap with the piece before is the same
+  // values; it may start up to three floats before the stage, in the row
+  // before's padding). Byte offsets inside the partition's centroids
+  // (direct_f64 keeps them in range): half the registers of addresses.
+  float* sc = sf + 4;
+  float* sx = sc + kWave * kRsS;
+  const char* cb = reinterpret_cast<const char*>(C + kb * d);
+  const uint32_t d4 = (uint32_t)d * 4;
+  uint32_t cr[kGrp];
+#pragma unroll
+  for (int u = 0; u < kGrp; ++u) cr[u] = __umul24((uint32_t)min(g + u, k - 1), d4);
+  const float* xp = X + row * d;
+  f32x4 cv[kGrp], xv;
+  int at = 0;  // where the loaded pieces belong, relative to the stage
+  auto load = [&](int j0) {
+    const int j = min(j0 + 4 * q, d - 4);
+    at = j - j0;
+#pragma unroll
+    for (int u = 0; u < kGrp; ++u)
+      cv[u] = *reinterpret_cast<const f32x4_u*>(cb + (uint32_t)(cr[u] + 4 * j));
+    xv = *reinterpret_cast<const f32x4_u*>(xp + j);
+  };
+  load(0);
+  double acc = 0.0;
+  for (int j0 = 0; j0 < d; j0 += kRsD) {
+    const int dd = d - j0 < kRsD ? d - j0 : kRsD;
+    __builtin_amdgcn_wave_barrier();  // one wavefront: its LDS operations keep their order
+#pragma unroll
+    for (int u = 0; u < kGrp; ++u)
+      *reinterpret_cast<Piece*>(sc + (pt * kGrp + u) * kRsS + at) = cv[u];
+    *reinterpret_cast<Piece*>(sx + pt * kRsS + at) = xv;
+    __builtin_amdgcn_wave_barrier();
+    if (j0 + kRsD < d) load(j0 + kRsD);
+    const float* ca = sc + l * kRsS;
+    const float* xa = sx + pt * kRsS;
+    auto add = [&](float xe, float ce) {
+      const double e = (double)xe - (double)ce;
+      acc = acc + e * e;
+    };
+    if (dd == kRsD) {
+#pragma unroll 2
+      for (int j = 0; j < kRsD; j += 4) {
+        const f32x4 xe = *reinterpret_cast<const f32x4*>(xa + j);
+        const f32x4 ce = *reinterpret_cast<const f32x4*>(ca + j);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) add(xe[u], ce[u]);
+      }
+    } else {
+#pragma unroll 1
+      for (int j = 0; j < dd; ++j) add(xa[j], ca[j]);
+    }
+  }
+  // lanes hold ascending candidates: strictly smaller wins, else the lower
+  best = acc;
+  bk = g + q < k ? g + q : INT_MAX;
+#pragma unroll
+  for (int off = 1; off < kGrp; off <<= 1) {
+    const double ob = __shfl_xor(best, off, kWave);
+    const int32_t ok = __shfl_xor(bk, off, kWave);
+    if (ok != INT_MAX && (bk == INT_MAX || ob < best || (ob == best && ok < bk))) {
+      best = ob;
+      bk = ok;
+    }
+  }
+}
+
+// One wave labels MB blocks of 16 points against every centroid of the
+// block's partitions. The centroids are the rows of the MFMA result and the
+// points its columns, so a lane holds four consecutive centroids of one point
+// per 16 x 16 tile: their largest value (two operations) is all that enters
+// the running top two, with the group's number for an index, and the MFMAs
+// start from -||c||^2 / 2 (one value per row: a broadcast read of four), so the
+// accumulators are compared as they come. Per element that is 1.5 vector
+// operations (half a maximum, and a quarter of compare, med3 and two
+// selects), against 5 when every element adds its ||c||^2 and carries its own
+// index, and three registers of running state per point block instead of
+// twelve. The margin is then between groups: when the second group's maximum
+// is more than 2 E below the first's, the FP64 oracle's nearest centroid is
+// one of the first group's four, and resolve16 picks it in FP64; every other
+// point is flagged for the re-scoring. labels receives 4 x the group (FUSE:
+// the label).
+// Centroid tiles are double buffered in LDS and shared by the block's four
+// waves; each fragment read feeds MB MFMAs.
+// TERMS = 1: only xh.ch (from the h rows of a split layout), a third of the
+// MFMAs with point_bound1, for the first pass of a cascade. LIST: the points
+// are the rows of a flag list. FUSE (one partition): the group is resolved in
+// the kernel and labels and dists are final.
+constexpr uint64_t kFlagRow = (1ull << 40) - 1;
+template <int KS, bool SPLIT, int MB, int WPE, int TERMS = 3, bool FUSE = false,
+          bool LIST = false>
 __global__ __launch_bounds__(kLB) __attribute__((amdgpu_waves_per_eu(WPE)))
-void k_label_bf16x3(
-    const float* __restrict__ X, int64_t n, int d, const uint16_t* __restrict__ Ch,
-    const uint16_t* __restrict__ Cl, const float* __restrict__ ncf,
+void k_label_f16x3(
+    const float* __restrict__ X, int64_t row0, int64_t n, int d, const float* __restrict__ C,
+    const uint16_t* __restrict__ Cf, const float* __restrict__ ncf,
     const int64_t* __restrict__ k_off, int P, const unsigned int* __restrict__ pstat,
-    int32_t* __restrict__ labels, uint64_t* __restrict__ flags,
-    unsigned long long* __restrict__ nflag, int64_t region) {
-  constexpr int KB = KD / 32;
-  constexpr int LROW = KD + 8;  // padded LDS row (bf16 elements)
-  __shared__ uint16_t s_h[2][kBN * LROW];
-  __shared__ uint16_t s_l[2][kBN * LROW];
-  __shared__ float s_nc[2][kBN];
+    const uint64_t* __restrict__ list, int32_t* __restrict__ labels, float* __restrict__ dists,
+    uint64_t* __restrict__ flags, unsigned long long* __restrict__ nflag, int64_t region) {
+  static_assert(TERMS == 3 || SPLIT, "one product needs separate h rows");
+  constexpr int KB = KS / TERMS;                              // split: fragments of h
+  constexpr int NF = TERMS == 1 ? KS : SPLIT ? 2 * KB : KS;   // fragments per row
+  constexpr int RH = NF * 32;     // halves per centroid row
+  constexpr int LROW = RH + 8;    // padded LDS row
+  // two centroid tiles; with FUSE the resolving's rows afterwards
+  constexpr int kTiles = 2 * kBN * LROW * 2, kRs = FUSE ? (kLB / kWave) * kRsLds * 4 : 0;
+  __shared__ __align__(16) unsigned char s_raw[kTiles > kRs ? kTiles : kRs];
+  uint16_t* s_c = reinterpret_cast<uint16_t*>(s_raw);
+  __shared__ __align__(16) float s_nc[2][kBN];
+  __shared__ float s_st[4 * MB * 16][4];  // row statistics of point_bound
+  __shared__ float s_mx[kLB / kWave];
   const int t = threadIdx.x;
   const int w = t / kWave;
   const int l = lane_id();
-  const int lr = l & 15;  // row (A layout) / column (output layout) inside a 16-block
-  const int lq = l >> 4;  // k-group (A layout) / row quad (output layout)
-  const int64_t p0 = (int64_t)blockIdx.x * kBM + w * kRowsW;
+  const int lr = l & 15;  // point inside a 16-block / centroid row (A layout)
+  const int lq = l >> 4;  // k-group (operands) / centroid quad (result)
+  const int64_t p0 = row0 + ((int64_t)blockIdx.x * (kLB / kWave) + w) * (MB * 16);
+  auto row_id = [&](int64_t r) { return LIST ? (int64_t)(list[r] & kFlagRow) : r; };
+  // partitions of this block (grid.y splits them)
+  const int pa = (int)((int64_t)P * blockIdx.y / gridDim.y);
+  const int pz = (int)((int64_t)P * (blockIdx.y + 1) / gridDim.y);
 
-  // A fragments: rows p0 + rb*16 + lr, k = kb*32 + lq*8 .. +8 (hi and lo)
-  bf16x8 Ah[2][KB], Al[2][KB];
-  float nx_a[2], xn_a[2], xhn_a[2], xln_a[2], exn_a[2];
+  // Point fragments and row statistics, one block of 16 rows at a time: four
+  // lanes per row split its coordinates (scaled by one power of two for the
+  // block's points) into the wave's sixteen rows of the second centroid buffer (free until the first tile is done), from which
+  // the fragments are read back. (Split straight into the fragments, the
+  // loads and conditions of all blocks together spill.)
+  f16x8 pf[MB][NF];
+  float mx = 0.f;
+  // coordinates are loaded four at a time (the last piece of a row moved back
+  // to end with it), halves stored eight bytes at a time where d allows
+  const bool x4 = (d & 3) == 0;
+#pragma unroll 1
+  for (int pb = 0; pb < MB; ++pb) {
+    const int64_t row = p0 + pb * 16 + (l >> 2);
+    const float* xr = X + row_id(row < n ? row : n - 1) * d;
+    for (int j = 4 * (l & 3); j < d; j += 16) {
+      const f32x4 v = *reinterpret_cast<const f32x4_u*>(xr + min(j, d - 4));
+      mx = fmaxf(fmaxf(mx, fabsf(v[0])), fmaxf(fabsf(v[1]), fmaxf(fabsf(v[2]), fabsf(v[3]))));
+    }
+  }
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    int64_t row = p0 + rb * 16 + lr;
+  for (int off = kWave / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
+  if (l == 0) s_mx[w] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < kLB / kWave; ++u) mx = fmaxf(mx, s_mx[u]);
+  const float sx = pow2_scale(mx), isx = 1.0f / sx;  // exact: powers of two
+  uint16_t* sw = s_c + kBN * LROW + w * 16 * LROW;
+#pragma unroll
+  for (int pb = 0; pb < MB; ++pb) {
+    const int64_t row = p0 + pb * 16 + (l >> 2);
+    const bool ok = row < n;
+    const float* xr = X + row_id(ok ? row : n - 1) * d;
+    uint16_t* sr = sw + (l >> 2) * LROW;
     float s2 = 0, sh = 0, sl = 0, se = 0;
-    double s2d = 0;
-#pragma unroll
-    for (int kb = 0; kb < KB; ++kb) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        int col = kb * 32 + lq * 8 + j;
-        float x = (row < n && col < d) ? X[row * d + col] : 0.f;
-        uint16_t h = bf16_rne(x);
-        float r = x - bf16_val(h);
-        uint16_t lo = bf16_rne(r);
-        float e = r - bf16_val(lo);
-        Ah[rb][kb][j] = __builtin_bit_cast(__bf16, h);
-        Al[rb][kb][j] = __builtin_bit_cast(__bf16, lo);
-        s2d += (double)x * x;
-        sh += bf16_val(h) * bf16_val(h);
-        sl += bf16_val(lo) * bf16_val(lo);
+    const float sy = ok ? sx : 0.f;  // (rows past the end: zeros)
+    // one coordinate's halves, its share of the norms added
+    auto split = [&](float x, _Float16& h, _Float16& lo) {
+      const float y = x * sy;
+      h = f16_half(y);
+      const float r = y - (float)h;  // exact
+      s2 += y * y;
+      sh += (float)h * (float)h;
+      if constexpr (TERMS == 1) {
+        lo = (_Float16)0.f;
+        se += r * r;
+      } else {
+        lo = f16_half(r);
+        const float e = r - (float)lo;  // exact
+        sl += (float)lo * (float)lo;
         se += e * e;
       }
-    }
-    // the 4 lanes lr, lr+16, lr+32, lr+48 hold one row
+    };
+    if (x4) {
+      for (int j = 4 * (l & 3); j < d; j += 16) {
+        const f32x4 v = *reinterpret_cast<const f32x4_u*>(xr + j);
+        f16x4 h, lo;
 #pragma unroll
-    for (int off = 16; off < 64; off <<= 1) {
-      s2d += __shfl_xor(s2d, off, kWave);
+        for (int u = 0; u < 4; ++u) {
+          _Float16 a, b;
+          split(v[u], a, b);
+          h[u] = a;
+          lo[u] = b;
+        }
+        *reinterpret_cast<f16x4_lds*>(&sr[j]) = h;
+        if constexpr (TERMS == 3 && SPLIT) {
+          *reinterpret_cast<f16x4_lds*>(&sr[RH / 2 + j]) = lo;
+        } else if constexpr (TERMS == 3) {
+          *reinterpret_cast<f16x4_lds*>(&sr[d + j]) = lo;
+          *reinterpret_cast<f16x4_lds*>(&sr[2 * d + j]) = h;
+        }
+      }
+    } else {
+      for (int j = 4 * (l & 3); j < d; j += 16) {
+        const int jc = min(j, d - 4);
+        const f32x4 v = *reinterpret_cast<const f32x4_u*>(xr + jc);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int ju = jc + u;
+          if (ju < j) continue;  // the piece before has it
+          _Float16 h, lo;
+          split(v[u], h, lo);
+          sr[ju] = f16_bits(h);
+          if constexpr (TERMS == 3 && SPLIT) {
+            sr[RH / 2 + ju] = f16_bits(lo);
+          } else if constexpr (TERMS == 3) {
+            sr[d + ju] = f16_bits(lo);
+            sr[2 * d + ju] = f16_bits(h);
+          }
+        }
+      }
+    }
+    if constexpr (TERMS == 1) {
+      for (int j = d + (l & 3); j < RH; j += 4) sr[j] = 0;
+    } else if constexpr (SPLIT) {
+      for (int j = d + (l & 3); j < RH / 2; j += 4) sr[j] = sr[RH / 2 + j] = 0;
+    } else {
+      for (int j = 3 * d + (l & 3); j < RH; j += 4) sr[j] = 0;
+    }
+#pragma unroll
+    for (int off = 1; off < 4; off <<= 1) {
+      s2 += __shfl_xor(s2, off, kWave);
       sh += __shfl_xor(sh, off, kWave);
       sl += __shfl_xor(sl, off, kWave);
       se += __shfl_xor(se, off, kWave);
     }
-    nx_a[rb] = (float)s2d;
-    xn_a[rb] = (float)sqrt(s2d) * (1.f + 1e-6f);
-    xhn_a[rb] = sqrtf(sh) * (1.f + 1e-5f);
-    xln_a[rb] = sqrtf(sl) * (1.f + 1e-5f);
-    exn_a[rb] = sqrtf(se) * (1.f + 1e-5f);
+    if ((l & 3) == 0) {  // norms rounded up: the bound stays rigorous
+      float* st = s_st[w * MB * 16 + pb * 16 + (l >> 2)];
+      const float up = (1.f + 4e-5f) * isx;
+      st[0] = sqrtf(s2) * up;
+      st[1] = sqrtf(sh) * up;
+      st[2] = sqrtf(sl) * up;
+      st[3] = sqrtf(se) * up;
+    }
+#pragma unroll
+    for (int f = 0; f < NF; ++f)
+      pf[pb][f] = *reinterpret_cast<const f16x8_lds*>(&sw[lr * LROW + f * 32 + lq * 8]);
+    asm volatile("" ::: "memory");  // the next block overwrites the rows
   }
 
-  // Centroid tiles of every partition in sequence, double buffered in LDS:
-  // the next tile is fetched into registers before the current one is
+  // Centroid tiles of the block's partitions in sequence, double buffered in
+  // LDS: the next tile is fetched into registers before the current one is
   // multiplied and stored to the other buffer after it, so one barrier per
   // tile and the L2 latency overlaps the MFMAs.
-  constexpr int VPR = KD / 8;  // uint4 per row
+  constexpr int VPR = RH / 8;                       // uint4 per row
+  constexpr int VPG = (TERMS == 1 ? 2 : 1) * VPR;   // the same in memory (h and l rows)
   static_assert((kBN * VPR) % kLB == 0 && kBN <= kLB, "a tile splits evenly over the block");
   constexpr int NV = kBN * VPR / kLB;
-  uint4 ph[NV], pl[NV];
+  u32x4 pv[NV];
   float pnc;
+  float ncs = 0.f;  // -||c||^2 / 2 in the accumulators' scale
   // Rows past the partition repeat its last centroid (every partition has
-  // one; the host checks k >= 1) and get ||c||^2 = +inf, so their D is +inf
-  // and the epilogue never takes them. Fetch and store are branch-free: the
-  // loads are unconditional, every thread loads a norm (kLB / kBN threads
-  // store the same value to each entry) and the +inf default is chosen when
-  // the tile is stored. A register write to a load's destination next to
-  // the load, or a load skipped on some lanes, would make the wave wait for
-  // the new tile there, before the MFMAs, and undo the double buffering.
-  // Row indices are 32-bit offsets from the tile's first centroid.
+  // one; the host checks k >= 1) and start from -inf, so the epilogue never
+  // takes them. Fetch and store
+  // are branch-free: the loads are unconditional, every thread loads a norm
+  // (kLB / kBN threads store the same value to each entry) and the defaults
+  // are chosen when the tile is stored. A register write to a load's
+  // destination next to the load, or a load skipped on some lanes, would make
+  // the wave wait for the new tile there, before the MFMAs, and undo the
+  // double buffering. Row indices are 32-bit offsets from the tile's first
+  // centroid.
   int32_t f_rem = 0;
   auto fetch = [&](int64_t c0, int64_t kend) {
-    const int32_t rem = (int32_t)(kend - c0);  // >= 1 rows left in the range
-    const uint4* bh = reinterpret_cast<const uint4*>(Ch + c0 * KD);
-    const uint4* bl = reinterpret_cast<const uint4*>(Cl + c0 * KD);
+    const int32_t rem = (int32_t)(kend - c0 < kBN ? kend - c0 : kBN);  // >= 1 rows left
+    const u32x4* bh = reinterpret_cast<const u32x4*>(Cf + c0 * (VPG * 8));
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int v = t + i * kLB;
       const int32_t r = min(v / VPR, rem - 1);
-      ph[i] = bh[r * VPR + v % VPR];
-      pl[i] = bl[r * VPR + v % VPR];
+      pv[i] = bh[r * VPG + v % VPR];
     }
     pnc = ncf[c0 + min(t % kBN, rem - 1)];
     f_rem = rem;
   };
-  // (the stored values pass through a mask: stored straight from the load
-  // registers, the compiler keeps the prefetched tile in scratch memory)
-  auto masked = [](uint4 a, uint32_t m) { return make_uint4(a.x & m, a.y & m, a.z & m, a.w & m); };
   auto stash = [&](int b) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int v = t + i * kLB;
-      const uint32_t m = v / VPR < f_rem ? ~0u : 0u;
-      *reinterpret_cast<uint4*>(&s_h[b][(v / VPR) * LROW + (v % VPR) * 8]) = masked(ph[i], m);
-      *reinterpret_cast<uint4*>(&s_l[b][(v / VPR) * LROW + (v % VPR) * 8]) = masked(pl[i], m);
+      *reinterpret_cast<u32x4_lds*>(&s_c[b * kBN * LROW + (v / VPR) * LROW + (v % VPR) * 8]) =
+          pv[i];
     }
-    s_nc[b][t % kBN] = (t % kBN) < f_rem ? pnc : INFINITY;
+    s_nc[b][t % kBN] = (t % kBN) < f_rem ? pnc * ncs : -INFINITY;
   };
-  int p = 0, buf = 0;
-  int64_t c0 = k_off[0];
-  fetch(c0, k_off[1]);
+  auto part_scale = [&](int q) { return pow2_scale(__uint_as_float(pstat[q * kStat + 4])); };
+  int p = pa, buf = 0;
+  if (pa >= pz) return;  // uniform over the block
+  int64_t c0 = k_off[pa];
+  float scp = part_scale(pa);
+  ncs = -0.5f * sx * scp;
+  fetch(c0, k_off[pa + 1]);
   stash(0);
   __syncthreads();
-  for (; p < P; ++p) {
+  for (; p < pz; ++p) {
     const int64_t kbeg = k_off[p], kend = k_off[p + 1];
-    float d1[2][4], d2[2][4];
-    int32_t k1[2][4];
+    const float isc = 1.0f / scp;
+    float d1[MB], d2[MB];
+    int32_t k1[MB];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { d1[rb][i] = FLT_MAX; d2[rb][i] = FLT_MAX; k1[rb][i] = -1; }
+    for (int pb = 0; pb < MB; ++pb) {
+      d1[pb] = -FLT_MAX;
+      d2[pb] = -FLT_MAX;
+      k1[pb] = -kGrp;
+    }
     for (c0 = kbeg; c0 < kend; c0 += kBN) {
       // the next tile: this partition's, else the next partition's first
       int64_t nc0 = c0 + kBN, nend = kend;
-      if (nc0 >= kend && p + 1 < P) {
+      if (nc0 >= kend && p + 1 < pz) {
         nc0 = kend;
         nend = k_off[p + 2];
+        scp = part_scale(p + 1);
+        ncs = -0.5f * sx * scp;
       }
       const bool more = nc0 < nend;
       if (more) fetch(nc0, nend);
-      f32x4 acc[2][4];
+      const uint16_t* sc = s_c + buf * kBN * LROW;
+      const int32_t gb = __builtin_amdgcn_readfirstlane((int32_t)(c0 - kbeg));
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
+      for (int cb = 0; cb < kBN / 16; ++cb) {
+        f16x8 af[NF];
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) acc[rb][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
-      const uint16_t* sh = s_h[buf];
-      const uint16_t* sl = s_l[buf];
-      // per 32-wide K block: its B fragments (8 LDS reads), then the MFMAs
-      // in rounds of 8 independent accumulators, so no MFMA waits on the one
-      // before it (fragments of one K block at a time keep the register count
-      // within 3 waves per SIMD)
+        for (int f = 0; f < NF; ++f)
+          af[f] = *reinterpret_cast<const f16x8_lds*>(&sc[(cb * 16 + lr) * LROW + f * 32 + lq * 8]);
+        const f32x4 nc = *reinterpret_cast<const f32x4*>(&s_nc[buf][cb * 16 + lq * 4]);
+        f32x4 acc[MB];
 #pragma unroll
-      for (int kb = 0; kb < KB; ++kb) {
-        bf16x8 Bh[4], Bl[4];
+        for (int pb = 0; pb < MB; ++pb) acc[pb] = nc;  // (the first MFMA's addend)
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb) {
-          const int r = cb * 16 + lr;
-          Bh[cb] = *reinterpret_cast<const bf16x8*>(&sh[r * LROW + kb * 32 + lq * 8]);
-          Bl[cb] = *reinterpret_cast<const bf16x8*>(&sl[r * LROW + kb * 32 + lq * 8]);
+        for (int s = 0; s < KS; ++s) {
+          // split rows: h.h, h.l, l.h per fragment
+          const int a = SPLIT && TERMS == 3 ? (s % 3 == 1 ? KB + s / 3 : s / 3) : s;
+          const int b = SPLIT && TERMS == 3 ? (s % 3 == 2 ? KB + s / 3 : s / 3) : s;
+#pragma unroll
+          for (int pb = 0; pb < MB; ++pb)
+            acc[pb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[a], pf[pb][b], acc[pb], 0, 0, 0);
         }
+        // x.c - ||c||^2 / 2 of four consecutive centroids, their maximum, and
+        // the running top two of the groups
+        const int32_t id = gb + cb * 16;  // uniform; the lane's quad comes at the end
 #pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb)
-            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ah[rb][kb], Bh[cb],
-                                                                  acc[rb][cb], 0, 0, 0);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb)
-            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Ah[rb][kb], Bl[cb],
-                                                                  acc[rb][cb], 0, 0, 0);
-#pragma unroll
-        for (int cb = 0; cb < 4; ++cb)
-#pragma unroll
-          for (int rb = 0; rb < 2; ++rb)
-            acc[rb][cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(Al[rb][kb], Bh[cb],
-                                                                  acc[rb][cb], 0, 0, 0);
-      }
-      __builtin_amdgcn_sched_barrier(0);
-      // epilogue: lane holds column cb*16 + lr, rows 4*lq + i. The running
-      // top two per row compare D' = ||c||^2 - 2 x.c (the row's ||x||^2 is
-      // common to all columns, so it changes neither the argmin nor the
-      // margin); columns past the partition carry ||c||^2 = +inf. Five VALU
-      // operations per element: fma, compare, med3 (new second) and two
-      // selects (best value, best column).
-      const int32_t colb = (int32_t)(c0 - kbeg) + lr;
-#pragma unroll
-      for (int cb = 0; cb < 4; ++cb) {
-        const float nc = s_nc[buf][cb * 16 + lr];
-        const int32_t col = colb + cb * 16;
-#pragma unroll
-        for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            const float D = fmaf(-2.f, acc[rb][cb][i], nc);
-            const bool take = D < d1[rb][i];
-            d2[rb][i] = __builtin_amdgcn_fmed3f(d1[rb][i], d2[rb][i], D);
-            d1[rb][i] = take ? D : d1[rb][i];
-            k1[rb][i] = take ? col : k1[rb][i];
-          }
+        for (int pb = 0; pb < MB; ++pb) {
+          // (the NaN-propagating maximum: the other one costs an instruction
+          // per accumulator that quiets signalling NaNs)
+          const float m3 = __builtin_elementwise_maximum(
+              __builtin_elementwise_maximum(acc[pb][0], acc[pb][1]), acc[pb][2]);
+          const float m = __builtin_elementwise_maximum(m3, acc[pb][3]);
+          const bool take = m > d1[pb];
+          d2[pb] = __builtin_amdgcn_fmed3f(d1[pb], d2[pb], m);
+          d1[pb] = take ? m : d1[pb];
+          k1[pb] = take ? id : k1[pb];
+        }
       }
       // the epilogue stays ahead of the tile store: its VALU work covers the
       // latency of the next tile's loads (left alone, the compiler sinks it
       // below the store and the barrier, which then wait right after the MFMAs)
 #pragma unroll
-      for (int rb = 0; rb < 2; ++rb)
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-          asm volatile("" : "+v"(d1[rb][i]), "+v"(d2[rb][i]), "+v"(k1[rb][i])::"memory");
+      for (int pb = 0; pb < MB; ++pb)
+        asm volatile("" : "+v"(d1[pb]), "+v"(d2[pb]), "+v"(k1[pb])::"memory");
       if (more) {
         stash(buf ^ 1);  // last read in the previous tile, before its barrier
         __syncthreads();
         buf ^= 1;
       }
     }
-    // merge the 16 lanes that share rows (same lq)
+    // merge the four lanes of a point (lower group on equal maxima), then lane
+    // (lq, lr) finishes point block lq
+    float st[4];
 #pragma unroll
-    for (int rb = 0; rb < 2; ++rb)
+    for (int q = 0; q < 4; ++q) st[q] = __uint_as_float(pstat[p * kStat + q]);
+    float D1 = 0.f, D2 = 0.f;
+    int32_t K1 = -1;
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
+    for (int pb = 0; pb < MB; ++pb) {
+      float a1 = d1[pb], a2 = d2[pb];
+      int32_t k = k1[pb] < 0 ? INT_MAX : k1[pb] + kGrp * lq;
 #pragma unroll
-        for (int off = 1; off < 16; off <<= 1) {
-          float od1 = __shfl_xor(d1[rb][i], off, kWave);
-          float od2 = __shfl_xor(d2[rb][i], off, kWave);
-          int32_t ok1 = __shfl_xor(k1[rb][i], off, kWave);
-          float hi1 = fmaxf(d1[rb][i], od1);
-          float nd2 = fminf(fminf(d2[rb][i], od2), hi1);
-          bool take = od1 < d1[rb][i] || (od1 == d1[rb][i] && ok1 >= 0 &&
-                                          (k1[rb][i] < 0 || ok1 < k1[rb][i]));
-          if (take) { d1[rb][i] = od1; k1[rb][i] = ok1; }
-          d2[rb][i] = nd2;
-        }
+      for (int off = 16; off < 64; off <<= 1) {
+        const float o1 = __shfl_xor(a1, off, kWave);
+        const float o2 = __shfl_xor(a2, off, kWave);
+        const int32_t ok = __shfl_xor(k, off, kWave);
+        a2 = fmaxf(fmaxf(a2, o2), fminf(a1, o1));
+        const bool take = o1 > a1 || (o1 == a1 && ok < k);
+        a1 = take ? o1 : a1;
+        k = take ? ok : k;
       }
-    // Bounds in output layout, then write. After the merge the 16 lanes of a
-    // row group hold the same top two for each of the group's 8 rows; lane
-    // lr < 8 finishes row slot (rb, i) = (lr / 4, lr % 4), so each lane
-    // computes one bound instead of the group's first lane computing eight.
-    float st[kStat];
-#pragma unroll
-    for (int q = 0; q < kStat; ++q) st[q] = __uint_as_float(pstat[p * kStat + q]);
-    const int rs = lr & 7, rbs = rs >> 2, is = rs & 3;
-    float D1 = d1[0][0], D2 = d2[0][0];
-    int32_t K1 = k1[0][0];
-#pragma unroll
-    for (int q = 1; q < 8; ++q)
-      if (rs == q) {
-        D1 = d1[q >> 2][q & 3];
-        D2 = d2[q >> 2][q & 3];
-        K1 = k1[q >> 2][q & 3];
+      if (lq == pb) {
+        D1 = a1;
+        D2 = a2;
+        K1 = k;
       }
-    // row statistics: lanes lr' = lq * 4 + i hold row lq * 4 + i of each block
-    const int src = lq * 4 + is;
-    float xs[2][5];
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      xs[rb][0] = __shfl(nx_a[rb], src, kWave);
-      xs[rb][1] = __shfl(xn_a[rb], src, kWave);
-      xs[rb][2] = __shfl(xhn_a[rb], src, kWave);
-      xs[rb][3] = __shfl(xln_a[rb], src, kWave);
-      xs[rb][4] = __shfl(exn_a[rb], src, kWave);
     }
-    const int64_t row = p0 + rbs * 16 + lq * 4 + is;
+    const bool mine = l < MB * 16 && p0 + l < n;
+    const int64_t row = row_id(mine ? p0 + l : row0);
+    const int32_t g = K1 == INT_MAX ? 0 : K1;  // first centroid of the group
     bool flagged = false;
-    if (lr < 8 && row < n && K1 >= 0) {
-      const float E = rbs ? point_bound(xs[1][0], xs[1][1], xs[1][2], xs[1][3], xs[1][4], st, KD, d)
-                          : point_bound(xs[0][0], xs[0][1], xs[0][2], xs[0][3], xs[0][4], st, KD, d);
-      labels[(int64_t)p * n + row] = K1;
-      flagged = !(D2 - D1 > 2.f * E);
+    if (mine) {
+      const float E = point_bound<TERMS>(s_st[w * MB * 16 + l], st, d);
+      const float margin = (D1 - D2) * (2.f * isx * isc);  // in squared distance
+      // no group taken (all values infinite or NaN): re-scored as well
+      flagged = !(margin > 2.f * E) || K1 == INT_MAX;
+      if (!FUSE) labels[(int64_t)p * n + row] = g;
     }
     // append flagged (p, row) pairs: one atomic per wave
-    const uint32_t cnt = flagged ? 1u : 0u;
-    const uint32_t incl = wave_incl_scan(cnt);
-    const uint32_t tot = __shfl(incl, kWave - 1, kWave);
-    unsigned long long base = 0;
-    // flags go to one of kFlagSlots regions (by block): counters on one
-    // address would serialise one atomic per wave and partition
-    const int slot = blockIdx.x % kFlagSlots;
-    if (l == kWave - 1 && tot) base = atomicAdd(&nflag[slot], (unsigned long long)tot);
-    base = __shfl(base, kWave - 1, kWave);
-    if (flagged) {
-      const unsigned long long o = base + incl - 1;
-      if (o < (unsigned long long)region)
-        flags[(int64_t)slot * region + (int64_t)o] = ((uint64_t)p << 40) | (uint64_t)row;
+    const uint64_t fm = __ballot(flagged);
+    if (fm) {
+      // flags go to one of kFlagSlots regions (by block): counters on one
+      // address would serialise one atomic per wave and partition
+      const int slot = blockIdx.x % kFlagSlots;
+      unsigned long long base = 0;
+      if (l == 0) base = atomicAdd(&nflag[slot], (unsigned long long)__popcll(fm));
+      base = __shfl(base, 0, kWave);
+      if (flagged) {
+        const unsigned long long o = base + __popcll(fm & lanemask_lt());
+        if (o < (unsigned long long)region)
+          flags[(int64_t)slot * region + (int64_t)o] = ((uint64_t)p << 40) | (uint64_t)row;
+      }
+    }
+    if constexpr (FUSE) {
+      // one partition: pick the nearest of the group right here, 16 points at
+      // a time, while the other waves multiply (the rows were read when the
+      // wave started and come from the last-level cache)
+      __syncthreads();  // the centroid tiles are consumed: their LDS is free
+      float* sf = reinterpret_cast<float*>(s_raw) + w * kRsLds;
+#pragma unroll 1
+      for (int it = 0; it < MB; ++it) {
+        const int src = it * 16 + l / kGrp;
+        const int32_t gi = __shfl(g, src, kWave);
+        const int64_t ri = __shfl(row, src, kWave);
+        const bool ok = __shfl((int)mine, src, kWave);
+        double best;
+        int32_t bk;
+        if (x4) resolve16<true>(X, d, C, kbeg, kend, ri, gi, sf, best, bk);
+        else resolve16<false>(X, d, C, kbeg, kend, ri, gi, sf, best, bk);
+        if (ok && l % kGrp == 0) {
+          labels[ri] = bk;
+          if (dists) dists[ri] = (float)best;
+        }
+      }
+      return;  // (the only partition: the fragments need not outlive the tiles)
     }
   }
 }
 
-// FP64 re-scoring of flagged points: one wave per (p, row), lanes stride the
-// partition's centroids; strict < in ascending k, lowest k on ties.
 // acc + diff^2 with separately rounded multiply and add in FP64 (the
 // oracle's arithmetic: no fused multiply-add), plain expression otherwise.
 // HIP's __dmul_rn / __dadd_rn are plain operators that the compiler may
@@ -454,88 +723,238 @@ __device__ __forceinline__ double dist2_f64(const float* __restrict__ x,
       acc = sq_acc(acc, (double)xv.w - (double)cv.w);
     }
   } else {
-    for (int j = 0; j < d; ++j) {
-      acc = sq_acc(acc, (double)x[j] - (double)c[j]);
+    int j = 0;
+    for (; j + 8 <= d; j += 8) {  // eight loads in flight, then the chain
+      float xv[8], cv[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        xv[u] = x[j + u];
+        cv[u] = c[j + u];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) acc = sq_acc(acc, (double)xv[u] - (double)cv[u]);
     }
+    for (; j < d; ++j) acc = sq_acc(acc, (double)x[j] - (double)c[j]);
   }
   return acc;
 }
 
-// The lanes stride the partition's centroids and read them from the
-// transposed copy Ct [d][ktot] (64 consecutive floats per load, the point's
-// coordinates are wave-uniform). A wave takes F flagged points of one
-// partition at a time (F > 1 only for single-partition calls, where every
-// flag shares the centroids): each centroid value loaded serves F
-// independent FP64 chains (on 4M x 64 points, k = 2048, 6263 flags: 225 us
-// with 2 per wave against 254 with 1).
+// The screen's bounds: R (relative, as a factor on the smallest screened
+// value) and A (absolute underflow slack), see k_rescore_tiled.
+__device__ __forceinline__ void screen_bounds(int d, float& R, float& A) {
+  const double ug = 1.1920928955078125e-07, u64 = 1.1102230246251565e-16;
+  const double gs = (d + 2) * ug / (1.0 - (d + 2) * ug);
+  const double g64 = (d + 2) * 2 * u64 / (1.0 - (d + 2) * 2 * u64);
+  R = (float)((1.0 + gs) * (1.0 + g64) / ((1.0 - gs) * (1.0 - g64)) * (1.0 + 1e-6));
+  A = (float)d * 4.7e-38f;  // >= d * 2^-124
+}
+
+// Re-scoring of few flagged points (d <= 128): a block takes up to F flags of
+// one partition at a time. Its threads hold U centroids each, read from the
+// transposed copy Ct [d][ktot] (64 consecutive floats per load), and walk the
+// dimensions with the F points' coordinates broadcast from LDS, so each
+// centroid value loaded serves F points and each coordinate U centroids. FP32
+// screen, then FP64 for the candidates, by the bounds of k_rescore_tiled; a
+// thread that may hold more candidates than it kept makes the block score
+// every centroid in FP64.
+// The flags are a list (nflag or *d_nflag of them), or (cnt) still lie in the
+// regions of the labeling; then more than kFewMax are left alone.
+constexpr int kRfF = 4;
+constexpr int64_t kFewMax = 65536;
 template <int F>
-__global__ __launch_bounds__(256) void k_rescore_f64(const float* __restrict__ X, int64_t n,
-                                                     int d, const float* __restrict__ Ct,
-                                                     int64_t ktot,
-                                                     const int64_t* __restrict__ k_off,
-                                                     const uint64_t* __restrict__ flags,
-                                                     int64_t nflag, int32_t* __restrict__ labels,
-                                                     const int64_t* __restrict__ d_nflag = nullptr) {
-  const int l = lane_id();
+__global__ __launch_bounds__(256, 4) void k_rescore_few(
+    const float* __restrict__ X, int64_t n, int d, const float* __restrict__ C,
+    const float* __restrict__ Ct, int64_t ktot, const int64_t* __restrict__ k_off,
+    const uint64_t* __restrict__ list, int64_t nflag, int32_t* __restrict__ labels,
+    float* __restrict__ dists, const int64_t* __restrict__ d_nflag,
+    const unsigned long long* __restrict__ cnt, int64_t region) {
+  constexpr int U = 4;  // centroids per thread and pass
+  constexpr int NW = 256 / kWave;
+  __shared__ float s_x[128 * F];
+  __shared__ uint64_t s_f[F];
+  __shared__ float s_min[F][NW];
+  __shared__ double s_best[F][NW];
+  __shared__ int32_t s_bk[F][NW];
+  __shared__ unsigned long long s_pre[kFlagSlots + 1];
+  const int t = threadIdx.x, w = t / kWave, l = lane_id();
   if (d_nflag) nflag = *d_nflag;  // count left on the device (capturable calls)
-  const int64_t ngroups = (nflag + F - 1) / F;
-  for (int64_t gi = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave; gi < ngroups;
-       gi += ((int64_t)gridDim.x * blockDim.x) / kWave) {
-    const float* x[F];
-    int64_t row[F];
-    bool has[F];
-    int p = 0;
-#pragma unroll
-    for (int q = 0; q < F; ++q) {
-      const int64_t f = gi * F + q;
-      has[q] = f < nflag;
-      const uint64_t fl = flags[has[q] ? f : gi * F];  // a missing flag repeats the first
-      if (q == 0) p = (int)(fl >> 40);
-      row[q] = (int64_t)(fl & ((1ull << 40) - 1));
-      x[q] = X + row[q] * d;
+  if (cnt) {  // the flags lie in their regions: entries before each
+    if (t < kWave) {
+      const uint32_t c = (uint32_t)cnt[l];
+      const uint32_t incl = wave_incl_scan(c);
+      s_pre[l] = incl - c;
+      if (l == kWave - 1) s_pre[kFlagSlots] = incl;
     }
-    const int64_t kbeg = k_off[p], kend = k_off[p + 1];
-    double best[F];
-    int64_t bk[F];
-#pragma unroll
-    for (int q = 0; q < F; ++q) { best[q] = DBL_MAX; bk[q] = -1; }
-    for (int64_t c = kbeg + l; c < kend; c += kWave) {
-      const float* ct = Ct + c;
-      double acc[F];
-#pragma unroll
-      for (int q = 0; q < F; ++q) acc[q] = 0.0;
-      int j = 0;
-      for (; j + 8 <= d; j += 8) {  // eight loads in flight, then the chains
-        float cv[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u) cv[u] = ct[(int64_t)(j + u) * ktot];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-#pragma unroll
-          for (int q = 0; q < F; ++q) acc[q] = sq_acc(acc[q], (double)x[q][j + u] - (double)cv[u]);
-      }
-      for (; j < d; ++j) {
-        const float cj = ct[(int64_t)j * ktot];
-#pragma unroll
-        for (int q = 0; q < F; ++q) acc[q] = sq_acc(acc[q], (double)x[q][j] - (double)cj);
-      }
-#pragma unroll
-      for (int q = 0; q < F; ++q)
-        if (bk[q] < 0 || acc[q] < best[q]) { best[q] = acc[q]; bk[q] = c; }
+    __syncthreads();
+    nflag = (int64_t)s_pre[kFlagSlots];
+    if (nflag >= kFewMax) return;  // left to the host (uniform over the grid)
+  }
+  auto flag_at = [&](int64_t f) {
+    if (!cnt) return list[f];
+    int lo = 0, hi = kFlagSlots;  // slot with s_pre[lo] <= f < s_pre[lo + 1]
+    while (hi - lo > 1) {
+      const int mid = (lo + hi) >> 1;
+      if (s_pre[mid] <= (unsigned long long)f) lo = mid; else hi = mid;
     }
+    return list[(int64_t)lo * region + (f - (int64_t)s_pre[lo])];
+  };
+  float R, A;
+  screen_bounds(d, R, A);
+  for (int64_t f0 = (int64_t)blockIdx.x * F; f0 < nflag; f0 += (int64_t)gridDim.x * F) {
+    const int nf = nflag - f0 < F ? (int)(nflag - f0) : F;
+    if (t < nf) s_f[t] = flag_at(f0 + t);
+    __syncthreads();
+    for (int done = 0; done < nf;) {  // runs of one partition (block-uniform)
+      const int p = (int)(s_f[done] >> 40);
+      int end = done + 1;
+      while (end < nf && (int)(s_f[end] >> 40) == p) ++end;
+      const int64_t kbeg = k_off[p], kend = k_off[p + 1];
+      const float* x[F];
 #pragma unroll
-    for (int q = 0; q < F; ++q) {
+      for (int q = 0; q < F; ++q) {
+        const int f = done + q < end ? done + q : done;  // a missing flag repeats one
+        x[q] = X + (int64_t)(s_f[f] & kFlagRow) * d;
+      }
+      __syncthreads();  // the previous run's rows and results are consumed
+      for (int j = t; j < d; j += 256)
 #pragma unroll
-      for (int off = kWave / 2; off > 0; off >>= 1) {
-        double ob = __shfl_xor(best[q], off, kWave);
-        int64_t ok = __shfl_xor(bk[q], off, kWave);
-        if (ok >= 0 && (bk[q] < 0 || ob < best[q] || (ob == best[q] && ok < bk[q]))) {
-          best[q] = ob;
-          bk[q] = ok;
+        for (int q = 0; q < F; ++q) s_x[j * F + q] = x[q][j];
+      __syncthreads();
+      float v1[F], v2[F];
+      int32_t k1[F];
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+        v1[q] = INFINITY;
+        v2[q] = INFINITY;
+        k1[q] = -1;
+      }
+      const bool any = kbeg + t < kend;  // this thread has a centroid
+      for (int64_t c0 = kbeg; c0 < kend; c0 += 256 * U) {
+        // U centroids a thread, every coordinate of theirs for all F points
+        float a[U][F];
+        const float* ct[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t c = c0 + u * 256 + t;
+          ct[u] = Ct + (c < kend ? c : kend - 1);
+#pragma unroll
+          for (int q = 0; q < F; ++q) a[u][q] = 0.f;
+        }
+        const int nu = kend - c0 >= 256 * U ? U : (int)((kend - c0 + 255) / 256);  // uniform
+        auto pass = [&](auto full_u) {
+#pragma unroll 4
+          for (int j = 0; j < d; ++j) {
+            float cv[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (full_u.value || u < nu) cv[u] = ct[u][(int64_t)j * ktot];
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+              if (full_u.value || u < nu) {
+#pragma unroll
+                for (int q = 0; q < F; ++q) {
+                  const float e = s_x[j * F + q] - cv[u];
+                  a[u][q] = fmaf(e, e, a[u][q]);
+                }
+              }
+          }
+        };
+        if (nu == U) pass(std::true_type{});
+        else pass(std::false_type{});
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int64_t c = c0 + u * 256 + t;
+          if (c < kend) {
+#pragma unroll
+            for (int q = 0; q < F; ++q) {
+              const bool lt1 = a[u][q] < v1[q];
+              v2[q] = __builtin_amdgcn_fmed3f(v1[q], v2[q], a[u][q]);
+              k1[q] = lt1 ? (int32_t)(c - kbeg) : k1[q];
+              v1[q] = lt1 ? a[u][q] : v1[q];
+            }
+          }
         }
       }
-      if (l == 0 && has[q]) labels[(int64_t)p * n + row[q]] = (int32_t)(bk[q] - kbeg);
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+        float m = v1[q];
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) m = fminf(m, __shfl_xor(m, off, kWave));
+        if (l == 0) s_min[q][w] = m;
+      }
+      __syncthreads();
+      double best[F];
+      int32_t bk[F];
+      bool full = false;
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+        float m = s_min[q][0];
+#pragma unroll
+        for (int u = 1; u < NW; ++u) m = fminf(m, s_min[q][u]);
+        const float T = (m + A) * R + A;
+        best[q] = DBL_MAX;
+        bk[q] = -1;
+        if (k1[q] >= 0 && v1[q] <= T) {
+          best[q] = dist2_f64(x[q], C + (kbeg + k1[q]) * d, d, false);
+          bk[q] = k1[q];
+        }
+        // (NaN screens take the full pass)
+        full = full || (any && (k1[q] < 0 || !(v2[q] > T)));
+      }
+      if (__syncthreads_or(full)) {
+#pragma unroll
+        for (int q = 0; q < F; ++q) {
+          best[q] = DBL_MAX;
+          bk[q] = -1;
+        }
+        for (int64_t c = kbeg + t; c < kend; c += 256) {
+#pragma unroll
+          for (int q = 0; q < F; ++q) {
+            const double a = dist2_f64(x[q], C + c * d, d, false);
+            if (bk[q] < 0 || a < best[q]) {
+              best[q] = a;
+              bk[q] = (int32_t)(c - kbeg);
+            }
+          }
+        }
+      }
+#pragma unroll
+      for (int q = 0; q < F; ++q) {
+#pragma unroll
+        for (int off = kWave / 2; off > 0; off >>= 1) {
+          const double ob = __shfl_xor(best[q], off, kWave);
+          const int32_t ok = __shfl_xor(bk[q], off, kWave);
+          if (ok >= 0 && (bk[q] < 0 || ob < best[q] || (ob == best[q] && ok < bk[q]))) {
+            best[q] = ob;
+            bk[q] = ok;
+          }
+        }
+        if (l == 0) {
+          s_best[q][w] = best[q];
+          s_bk[q][w] = bk[q];
+        }
+      }
+      __syncthreads();
+      if (t < end - done) {
+        double b = s_best[t][0];
+        int32_t k = s_bk[t][0];
+        for (int u = 1; u < NW; ++u) {
+          const double ob = s_best[t][u];
+          const int32_t ok = s_bk[t][u];
+          if (ok >= 0 && (k < 0 || ob < b || (ob == b && ok < k))) {
+            b = ob;
+            k = ok;
+          }
+        }
+        const int64_t o =
+            (int64_t)p * n + (int64_t)(s_f[done + t] & kFlagRow);
+        labels[o] = k;
+        if (dists) dists[o] = (float)b;
+      }
+      __syncthreads();  // the shared results are consumed
+      done = end;
     }
+    __syncthreads();  // and the flags
   }
 }
 
@@ -575,7 +994,8 @@ template <int DX>
 __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
     const float* __restrict__ X, int64_t n, int d, const float* __restrict__ C,
     const int64_t* __restrict__ k_off, const uint64_t* __restrict__ flags, int64_t nflag,
-    int32_t* __restrict__ labels, const int64_t* __restrict__ d_nflag = nullptr) {
+    int32_t* __restrict__ labels, float* __restrict__ dists,
+    const int64_t* __restrict__ d_nflag = nullptr) {
   extern __shared__ __align__(16) float s_dyn[];
   __shared__ double s_best[kRtS][kRtF];
   __shared__ int32_t s_bk[kRtS][kRtF];
@@ -589,12 +1009,8 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
   if (d_nflag) nflag = *d_nflag;  // count left on the device: tiles in a loop
   for (int64_t f0 = (int64_t)blockIdx.x * kRtF; f0 < nflag; f0 += (int64_t)gridDim.x * kRtF) {
   const int cnt = nflag - f0 < kRtF ? (int)(nflag - f0) : kRtF;
-  // screen bounds (double, then rounded up into float)
-  const double ug = 1.1920928955078125e-07, u64 = 1.1102230246251565e-16;
-  const double gs = (d + 2) * ug / (1.0 - (d + 2) * ug);
-  const double g64 = (d + 2) * 2 * u64 / (1.0 - (d + 2) * 2 * u64);
-  const float R = (float)((1.0 + gs) * (1.0 + g64) / ((1.0 - gs) * (1.0 - g64)) * (1.0 + 1e-6));
-  const float A = (float)d * 4.7e-38f;  // >= d * 2^-124
+  float R, A;
+  screen_bounds(d, R, A);
   for (int done = 0; done < cnt;) {  // runs of one partition (block-uniform)
     const int p = (int)(flags[f0 + done] >> 40);
     int end = done + 1;
@@ -718,7 +1134,9 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
         const int32_t ok = s_bk[q][g];
         if (ok >= 0 && (k < 0 || ob < b || (ob == b && ok < k))) { b = ob; k = ok; }
       }
-      labels[(int64_t)p * n + (int64_t)(flags[f0 + g] & kRowMask)] = k;
+      const int64_t o = (int64_t)p * n + (int64_t)(flags[f0 + g] & kRowMask);
+      labels[o] = k;
+      if (dists) dists[o] = (float)b;
     }
     __syncthreads();
     done = end;
@@ -753,79 +1171,40 @@ __global__ void k_gather_flags(const uint64_t* __restrict__ regions, int64_t reg
   }
 }
 
-// FP64 distance of every point to its labelled centroid (oracle arithmetic),
-// stored as float32 like the reference's dists array. LPP = 4 lanes share a
-// point (the addition chain has d/4 steps whatever LPP is, and fewer lanes
-// per point run more points per wave: on 4M x 64 points, 303 us against 342
-// with 8 lanes, 500 with 16, 416 with 2 and 785 with 1):
-// lane s loads dimensions 4s..4s+3 of each (4 LPP)-dimension chunk of the
-// point's row and its centroid's row (coalesced) and squares the
-// differences in parallel; the running sum then visits the lanes in order
-// (4 adds in lane s, then a shuffle to lane s+1), so the additions happen in
-// ascending dimension order exactly as in the oracle. Padding dimensions add
-// exact zeros. A block takes kPG partitions (grid.y over partition groups)
-// with the partitions innermost, so a point's row is read from memory once
-// per group and from cache for the other partitions.
+// resolve16 for every (point, partition): labels holds the group's first
+// centroid and receives the label, dists (nullable) its distance as float32
+// like the reference's dists array. A block takes kPG partitions (grid.y over
+// partition groups) with the partitions innermost, so a point's row is read
+// from memory once per group and from cache for the other partitions.
 constexpr int kPG = 8;
-template <int LPP>
-__global__ __launch_bounds__(256) void k_exact_dists(const float* __restrict__ X, int64_t n,
-                                                     int d, const float* __restrict__ C,
-                                                     const int64_t* __restrict__ k_off, int P,
-                                                     const int32_t* __restrict__ labels,
-                                                     float* __restrict__ dists) {
-#pragma clang fp contract(off)  // the oracle's separately rounded products and sums
-  constexpr int PPB = 256 / LPP;  // points per block and step
-  const int lane = lane_id(), sub = lane & (LPP - 1), base = lane & ~(LPP - 1);
-  const int64_t groups = (int64_t)gridDim.x * PPB;
-  const bool v4 = (d & 3) == 0 && ((reinterpret_cast<uintptr_t>(X) |
-                                    reinterpret_cast<uintptr_t>(C)) & 15) == 0;
+template <bool V4>
+__global__ __launch_bounds__(256) void k_resolve(const float* __restrict__ X, int64_t n, int d,
+                                                 const float* __restrict__ C,
+                                                 const int64_t* __restrict__ k_off, int P,
+                                                 int32_t* __restrict__ labels,
+                                                 float* __restrict__ dists) {
+  constexpr int PW = kWave / kGrp;  // points per wave
+  __shared__ __align__(16) float s_rs[256 / kWave][kRsLds];
+  const int w = threadIdx.x / kWave, l = lane_id();
+  const int64_t step = (int64_t)gridDim.x * (256 / kGrp);
   for (int pg = blockIdx.y * kPG; pg < P; pg += gridDim.y * kPG) {
-    const int np = P - pg < kPG ? P - pg : kPG;
-    // wave-uniform trip count (the shuffles need every lane)
-    const int64_t g0 = (int64_t)blockIdx.x * PPB + threadIdx.x / LPP;
-    const int64_t first = g0 - (threadIdx.x & (kWave - 1)) / LPP;  // group of lane 0
-    for (int64_t gb = first; gb < n; gb += groups) {
-      const int64_t i = gb + base / LPP;
+    const int pe = P - pg < kPG ? P : pg + kPG;
+    // wave-uniform trip count
+    for (int64_t i0 = ((int64_t)blockIdx.x * (256 / kWave) + w) * PW; i0 < n; i0 += step) {
+      const int64_t i = i0 + l / kGrp;
       const bool valid = i < n;
-      const float* xr = X + (valid ? i : 0) * d;
-#pragma unroll
-      for (int q = 0; q < kPG; ++q) {
-        if (q >= np) break;  // uniform
-        const int p = pg + q;
-        const int64_t kbeg = k_off[p];
-        const int64_t c = valid ? kbeg + labels[(int64_t)p * n + i] : kbeg;
-        const float* cr = C + c * d;
-        double acc = 0.0;
-        for (int j0 = 0; j0 < d; j0 += 4 * LPP) {
-          double sq[4];
-          const int jb = j0 + 4 * sub;
-          if (v4 && jb + 4 <= d) {  // one 16-byte load per row
-            const float4 xv = *reinterpret_cast<const float4*>(xr + jb);
-            const float4 cv = *reinterpret_cast<const float4*>(cr + jb);
-            const double e0 = (double)xv.x - (double)cv.x, e1 = (double)xv.y - (double)cv.y;
-            const double e2 = (double)xv.z - (double)cv.z, e3 = (double)xv.w - (double)cv.w;
-            sq[0] = e0 * e0;
-            sq[1] = e1 * e1;
-            sq[2] = e2 * e2;
-            sq[3] = e3 * e3;
-          } else {
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-              const int j = jb + u;
-              const double diff = j < d ? (double)xr[j] - (double)cr[j] : 0.0;
-              sq[u] = diff * diff;
-            }
-          }
-          const int steps = d - j0 >= 4 * LPP ? LPP : (d - j0 + 3) / 4;
-          for (int st = 0; st < steps; ++st) {
-            if (sub == st) {
-#pragma unroll
-              for (int u = 0; u < 4; ++u) acc = acc + sq[u];
-            }
-            acc = __shfl(acc, base + st, kWave);
-          }
+      const int64_t row = valid ? i : n - 1;
+      int32_t g = labels[(int64_t)pg * n + row];
+      for (int p = pg; p < pe; ++p) {
+        const int32_t gn = p + 1 < pe ? labels[(int64_t)(p + 1) * n + row] : 0;  // in flight
+        double best;
+        int32_t bk;
+        resolve16<V4>(X, d, C, k_off[p], k_off[p + 1], row, g, s_rs[w], best, bk);
+        if (valid && l % kGrp == 0) {
+          labels[(int64_t)p * n + i] = bk;
+          if (dists) dists[(int64_t)p * n + i] = (float)best;
         }
-        if (valid && sub == 0) dists[(int64_t)p * n + i] = (float)acc;
+        g = gn;
       }
     }
   }
@@ -1366,19 +1745,19 @@ __global__ void k_flags_total(const unsigned long long* __restrict__ cnt, int64_
 // Counting sort of the flags by partition (flag = partition << 40 | row),
 // stable-free but deterministic: kSortBlocks workgroups each take the same
 // grid-stride share of the flags in both passes; pass 1 counts its share's
-// flags per partition in LDS (bcount[p][b]); one workgroup scans bcount in
-// (partition, workgroup) order into offsets; pass 2 places the share's flags
+// flags per partition in LDS (bcount[p][b]); a scan of bcount in (partition,
+// workgroup) order gives offsets; pass 2 places the share's flags
 // from LDS cursors started at those offsets. No global atomics (their
 // serialisation on a few hot partitions dominated).
 constexpr int kSortBlocks = 256;
 constexpr int kSortMaxP = 4096;  // partitions counted in LDS
 __global__ __launch_bounds__(256) void k_flag_bcount(const uint64_t* __restrict__ flags,
-                                                     const int64_t* __restrict__ d_nf, int P,
-                                                     int32_t* __restrict__ bcount) {
+                                                     int64_t nf, const int64_t* __restrict__ d_nf,
+                                                     int P, int32_t* __restrict__ bcount) {
   __shared__ int32_t h[kSortMaxP];
   for (int p = threadIdx.x; p < P; p += blockDim.x) h[p] = 0;
   __syncthreads();
-  const int64_t nf = *d_nf;
+  if (d_nf) nf = *d_nf;
   for (int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; f < nf;
        f += (int64_t)gridDim.x * blockDim.x) {
     const int p = (int)(flags[f] >> 40);
@@ -1387,20 +1766,8 @@ __global__ __launch_bounds__(256) void k_flag_bcount(const uint64_t* __restrict_
   __syncthreads();
   for (int p = threadIdx.x; p < P; p += blockDim.x) bcount[(int64_t)p * gridDim.x + blockIdx.x] = h[p];
 }
-__global__ __launch_bounds__(1024) void k_flag_bscan(int32_t* __restrict__ bcount, int64_t len) {
-  __shared__ int32_t s_tmp[1024 / kWave + 1];
-  int32_t carry = 0;
-  for (int64_t i0 = 0; i0 < len; i0 += 1024) {
-    const int64_t i = i0 + threadIdx.x;
-    const int32_t v = i < len ? bcount[i] : 0;
-    int32_t tot;
-    const int32_t pre = block_excl_scan<int32_t>(v, s_tmp, &tot);
-    if (i < len) bcount[i] = carry + pre;
-    carry += tot;
-    __syncthreads();
-  }
-}
 __global__ __launch_bounds__(256) void k_flag_bscatter(const uint64_t* __restrict__ flags,
+                                                       int64_t nf,
                                                        const int64_t* __restrict__ d_nf, int P,
                                                        const int32_t* __restrict__ boff,
                                                        uint64_t* __restrict__ out) {
@@ -1408,7 +1775,7 @@ __global__ __launch_bounds__(256) void k_flag_bscatter(const uint64_t* __restric
   for (int p = threadIdx.x; p < P; p += blockDim.x)
     cur[p] = boff[(int64_t)p * gridDim.x + blockIdx.x];
   __syncthreads();
-  const int64_t nf = *d_nf;
+  if (d_nf) nf = *d_nf;
   for (int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; f < nf;
        f += (int64_t)gridDim.x * blockDim.x) {
     const uint64_t fl = flags[f];
@@ -1510,13 +1877,6 @@ __global__ void k_fit_tally(int64_t* __restrict__ info, const int64_t* __restric
   }
 }
 
-int kd_for(int d) {
-  if (d <= 32) return 32;
-  if (d <= 64) return 64;
-  if (d <= 128) return 128;
-  return 0;
-}
-
 int d2h(void* host, const void* dev, size_t bytes, hipStream_t s) {
   void* pin = pinned_scratch(bytes);
   if (!pin) return fail(EAC_ERR_HIP, "pinned host allocation failed");
@@ -1528,14 +1888,14 @@ int d2h(void* host, const void* dev, size_t bytes, hipStream_t s) {
 
 struct LabelBufs {
   int64_t* k_off;
-  uint16_t* Ch;
-  uint16_t* Cl;
+  uint16_t* Cf;  // split rows of the centroids
   float* Ct;  // centroids transposed: [d][ktot]
   float* ncf;
-  unsigned int* pstat;
+  unsigned int* pstat;        // [P][kStat]; cleared with nflag, which follows it
   uint64_t* flags_r;  // kFlagSlots regions of `region` flags
   uint64_t* flags;    // the flags of all regions, contiguous
   unsigned long long* nflag;  // per-region counts
+  int32_t* bcount;            // [P][kSortBlocks] flags per (partition, sorting workgroup)
   float* csum;                // numpy-order chunk sums of the dists
   int64_t flag_cap;
   int64_t region;
@@ -1543,20 +1903,20 @@ struct LabelBufs {
 
 LabelBufs carve_label(Arena& ar, int64_t n, int d, int64_t ktot, int P) {
   LabelBufs b;
-  int KD = kd_for(d) ? kd_for(d) : 32;
+  const int NF = std::max(label_layout(d).NF, label_layout(d, true).NF);
   b.k_off = ar.take<int64_t>(P + 1);
-  b.Ch = ar.take<uint16_t>((size_t)ktot * KD + 64);
-  b.Cl = ar.take<uint16_t>((size_t)ktot * KD + 64);
+  b.Cf = ar.take<uint16_t>((size_t)ktot * NF * 32 + 64);
   b.Ct = ar.take<float>((size_t)ktot * d);
   b.ncf = ar.take<float>(ktot);
-  b.pstat = ar.take<unsigned int>((size_t)P * kStat);
+  b.nflag = ar.take<unsigned long long>(kFlagSlots + ((size_t)P * kStat + 1) / 2);
+  b.pstat = reinterpret_cast<unsigned int*>(b.nflag + kFlagSlots);
   b.flag_cap = (int64_t)P * n;
   // a region holds every (partition, row) its blocks can flag
-  const int64_t nblocks = (n + kBM - 1) / kBM;
-  b.region = ((nblocks + kFlagSlots - 1) / kFlagSlots) * kBM * (int64_t)P;
+  const int64_t nblocks = (n + kLB - 1) / kLB;
+  b.region = ((nblocks + kFlagSlots - 1) / kFlagSlots) * kLB * (int64_t)P;
   b.flags_r = ar.take<uint64_t>((size_t)kFlagSlots * b.region);
   b.flags = ar.take<uint64_t>(b.flag_cap);
-  b.nflag = ar.take<unsigned long long>(kFlagSlots);
+  b.bcount = ar.take<int32_t>((size_t)std::min(P, kSortMaxP) * kSortBlocks);
   b.csum = ar.take<float>((size_t)P * np_chunks(n) + 1);
   return b;
 }
@@ -1566,20 +1926,168 @@ LabelBufs carve_label(Arena& ar, int64_t n, int d, int64_t ktot, int P) {
 size_t kmeans_label_ws_bytes(int64_t n, int d, int64_t ktot, int P) {
   Arena ar(nullptr, 0, true);
   (void)carve_label(ar, n, d, ktot, P);
-  return ar.used + 4096;
+  return ar.used + scan_ws_bytes((int64_t)std::min(P, kSortMaxP) * kSortBlocks, 4) + 4096;
 }
 
-// Device-side state of a capturable fit: flag count, per-partition flag
-// counts and cursors, flags sorted by partition, running totals (info[0]
+// Device-side state of a capturable fit: flag count, running totals (info[0]
 // flags re-scored, info[1] clusters reseeded), error bits.
 struct KmGraph {
   const int32_t* any;  // some partition still runs (the labeling counts only then)
   int64_t* d_nf;
-  int32_t* bcount;     // [P][kSortBlocks] flags per (partition, sorting workgroup)
-  uint64_t* sorted;
   int64_t* info;
   unsigned int* err;
 };
+
+// The labeling kernel for a layout: point blocks per wave (four where the
+// point fragments leave the registers for it, two for wide rows and for
+// inputs of too few points to fill the chip otherwise) and waves per SIMD
+// (EAC_TUNE_KM_WAVES, or the built-in choice, for the layouts of d = 11 ... 21 and
+// d = 54 ... 64).
+struct LabelCall {
+  const float* X;
+  int64_t row0, n;  // rows [row0, n), or entries of `list`
+  int d;
+  const float* C;
+  const uint16_t* Cf;
+  const float* ncf;
+  const int64_t* k_off;
+  int P;
+  const unsigned int* pstat;
+  const uint64_t* list;
+  int32_t* labels;
+  float* dists;
+  uint64_t* flags;
+  unsigned long long* nflag;
+  int64_t region;
+};
+template <int KS, bool SPLIT, int MB, int WPE, int TERMS = 3, bool FUSE = false,
+          bool LIST = false>
+void label_go(const LabelCall& a, hipStream_t s) {
+  const int64_t gx = (a.n - a.row0 + 64 * MB - 1) / (64 * MB);
+  int64_t gy = FUSE || gx >= 1536 ? 1 : (1536 + gx - 1) / gx;
+  if (gy > a.P) gy = a.P;
+  if (gy > 65535) gy = 65535;
+  k_label_f16x3<KS, SPLIT, MB, WPE, TERMS, FUSE, LIST>
+      <<<dim3((unsigned)gx, (unsigned)gy), kLB, 0, s>>>(a.X, a.row0, a.n, a.d, a.C, a.Cf, a.ncf,
+                                                        a.k_off, a.P, a.pstat, a.list, a.labels,
+                                                        a.dists, a.flags, a.nflag, a.region);
+}
+template <int KS, bool SPLIT, bool FUSE>
+void label_sized(const LabelCall& a, bool wide, hipStream_t s) {
+  if constexpr (KS == 2 || (KS == 6 && SPLIT)) {
+    switch (tune_value(EAC_TUNE_KM_WAVES)) {
+      case 2: return wide ? label_go<KS, SPLIT, 4, 2, 3, FUSE>(a, s)
+                          : label_go<KS, SPLIT, 2, 2, 3, FUSE>(a, s);
+      case 3: return wide ? label_go<KS, SPLIT, 4, 3, 3, FUSE>(a, s)
+                          : label_go<KS, SPLIT, 2, 3, 3, FUSE>(a, s);
+      case 4: return wide ? label_go<KS, SPLIT, 4, 4, 3, FUSE>(a, s)
+                          : label_go<KS, SPLIT, 2, 4, 3, FUSE>(a, s);
+    }
+  }
+  constexpr int W = KS <= 3 ? 4 : 3;
+  return wide ? label_go<KS, SPLIT, 4, W, 3, FUSE>(a, s)
+              : label_go<KS, SPLIT, 2, W, 3, FUSE>(a, s);
+}
+template <bool FUSE>
+int launch_label(const LabelLayout& L, const LabelCall& a, hipStream_t s) {
+  const bool wide = (a.n - a.row0) * a.P >= 256 * 1536;
+  if (L.split) {
+    switch (L.KS) {
+      case 3: label_sized<3, true, FUSE>(a, wide, s); break;
+      case 6: label_sized<6, true, FUSE>(a, wide, s); break;
+      case 9: label_go<9, true, 2, 2, 3, FUSE>(a, s); break;
+      default: label_go<12, true, 2, 2, 3, FUSE>(a, s); break;
+    }
+  } else {
+    switch (L.KS) {
+      case 1: label_sized<1, false, FUSE>(a, wide, s); break;
+      case 2: label_sized<2, false, FUSE>(a, wide, s); break;
+      case 4: label_sized<4, false, FUSE>(a, wide, s); break;
+      case 5: label_sized<5, false, FUSE>(a, wide, s); break;
+      case 7: label_go<7, false, 2, 2, 3, FUSE>(a, s); break;
+      default: label_go<8, false, 2, 2, 3, FUSE>(a, s); break;
+    }
+  }
+  EAC_LAUNCH_CHECK();
+  return EAC_OK;
+}
+// The cascade's passes (split layouts of two to four fragments, one
+// partition): the single product over rows, and all three over a list.
+int launch_single(const LabelLayout& L, const LabelCall& a, hipStream_t s) {
+  switch (L.KS) {
+    case 6: label_go<2, true, 4, 4, 1, true>(a, s); break;
+    case 9: label_go<3, true, 4, 3, 1, true>(a, s); break;
+    default: label_go<4, true, 4, 3, 1, true>(a, s); break;
+  }
+  EAC_LAUNCH_CHECK();
+  return EAC_OK;
+}
+int launch_listed(const LabelLayout& L, const LabelCall& a, hipStream_t s) {
+  switch (L.KS) {
+    case 6: label_go<6, true, 2, 3, 3, true, true>(a, s); break;
+    case 9: label_go<9, true, 2, 2, 3, true, true>(a, s); break;
+    default: label_go<12, true, 2, 2, 3, true, true>(a, s); break;
+  }
+  EAC_LAUNCH_CHECK();
+  return EAC_OK;
+}
+
+// Flags in all regions (read back).
+int read_flags(const LabelBufs& B, unsigned long long* nf, hipStream_t s) {
+  unsigned long long hcnt[kFlagSlots];
+  EAC_TRY(d2h(hcnt, B.nflag, sizeof(hcnt), s));
+  *nf = 0;
+  for (int q = 0; q < kFlagSlots; ++q) {
+    if ((int64_t)hcnt[q] > B.region) return fail(EAC_ERR_HIP, "kmeans: flag list overflow");
+    *nf += hcnt[q];
+  }
+  if ((int64_t)*nf > B.flag_cap) return fail(EAC_ERR_HIP, "kmeans: flag list overflow");
+  return EAC_OK;
+}
+// The gathered flags (their number on the host, or at d_nf) sorted by
+// partition into the regions, which the gathering has emptied.
+int sort_flags(const LabelBufs& B, int P, int64_t nf, const int64_t* d_nf, Arena& ar,
+               hipStream_t s) {
+  k_flag_bcount<<<kSortBlocks, 256, 0, s>>>(B.flags, nf, d_nf, P, B.bcount);
+  EAC_LAUNCH_CHECK();
+  const size_t mark = ar.used;
+  EAC_TRY((scan_excl<int32_t, int32_t>(B.bcount, B.bcount, (int64_t)P * kSortBlocks, 0, nullptr,
+                                       ar, s)));
+  ar.used = mark;
+  k_flag_bscatter<<<kSortBlocks, 256, 0, s>>>(B.flags, nf, d_nf, P, B.bcount, B.flags_r);
+  EAC_LAUNCH_CHECK();
+  return EAC_OK;
+}
+int gather_flags(const LabelBufs& B, unsigned long long nf, hipStream_t s) {
+  k_gather_flags<<<grid_for((int64_t)nf, 256, 65536), 256, 0, s>>>(B.flags_r, B.region, B.nflag,
+                                                                   B.flags, (int64_t)nf);
+  EAC_LAUNCH_CHECK();
+  return EAC_OK;
+}
+
+// Whether BF16X3 takes the plain FP64 labeling (the same labels and
+// distances). It must where resolve16 does not reach: fewer than four
+// dimensions, or a partition beyond its 32-bit offsets (2^23 rows of up to 512
+// bytes). From 16 dimensions on it never does (it pays only for toy sizes
+// there). In between the cheaper one, from measured times: a thread of the
+// direct kernel walks its partition's centroids in sequence (c1 us each,
+// whatever n is; 40 us a call with no centroid to speak of), a full chip does
+// a (point, centroid) pair in c2 us; the MFMA path costs 28 us more a call
+// (60 with several partitions: sorted flags, a separate resolving) and about
+// 0.075e-6 us a pair and MFMA step. E.g. d = 8: 30,000 points, k = 100: 51 us
+// direct, 68 MFMA; k = 500: 101 and 73; 300,000 points, k = 2000: 631 and 149.
+bool direct_f64(int64_t n, int d, const int64_t* h_koff, int P) {
+  if (d < 4) return true;
+  int64_t kmax = 1;
+  for (int p = 0; p < P; ++p) kmax = std::max(kmax, h_koff[p + 1] - h_koff[p]);
+  if (kmax >= (int64_t)1 << 23) return true;
+  if (d >= 16) return false;
+  const int dx = d <= 4 ? 0 : d <= 8 ? 1 : 2;
+  const double c1[] = {0.083, 0.125, 0.29}, c2[] = {0.59e-6, 0.99e-6, 1.9e-6};
+  const double pairs = (double)n * (double)h_koff[P];
+  const double direct = std::max((double)kmax * c1[dx], pairs * c2[dx]);
+  return direct <= (P == 1 ? 28.0 : 60.0) + pairs * 0.075e-6 * label_layout(d).KS;
+}
 
 // Label all partitions; dists (nullable) receive FP64-exact distances for
 // the F64 / BF16X3 modes and fp32 distances for F32; csum_out (nullable)
@@ -1599,8 +2107,10 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
     EAC_TRY(put_i64(B.k_off, h_koff, P + 1, s));
   }
   if (n_rescored) *n_rescored = 0;
-  if (mode == EAC_KM_F32 || mode == EAC_KM_F64 || mode == EAC_KM_F32_NUMPY ||
-      (mode == EAC_KM_BF16X3 && d < 16)) {
+  if (mode != EAC_KM_F32 && mode != EAC_KM_F64 && mode != EAC_KM_F32_NUMPY &&
+      mode != EAC_KM_BF16X3)
+    return fail(EAC_ERR_ARG, "kmeans: unknown mode %d", mode);
+  if (mode != EAC_KM_BF16X3 || direct_f64(n, d, h_koff, P)) {
     int pr = prof_begin(EAC_PROF_KM_LABEL, 2 * n * (int64_t)d * ktot, s);
     if (mode == EAC_KM_F32_NUMPY)
       EAC_TRY(launch_np(X, n, d, C, B.k_off, P, labels, dists, s));
@@ -1616,42 +2126,67 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
     }
     return EAC_OK;
   }
-  if (mode != EAC_KM_BF16X3) return fail(EAC_ERR_ARG, "kmeans: unknown mode %d", mode);
-  const int KD = kd_for(d);
-  if (!KD) return fail(EAC_ERR_UNSUPPORTED, "kmeans bf16x3: d=%d > 128", d);
-  EAC_TRY(fill<int32_t>((int32_t*)B.pstat, (int64_t)P * kStat, 0, s));
-  EAC_TRY(fill<uint64_t>((uint64_t*)B.nflag, kFlagSlots, 0ull, s));
-  k_cent_prep<<<grid_for(ktot, 256, 8192), 256, 0, s>>>(C, ktot, d, KD, B.k_off, P, B.Ch, B.Cl,
-                                                        B.Ct, B.ncf, B.pstat);
-  EAC_LAUNCH_CHECK();
-  int g = (int)((n + kBM - 1) / kBM);
-  int pr = prof_begin(EAC_PROF_KM_LABEL, 2 * n * (int64_t)d * ktot, s);
+  if (d > 128) return fail(EAC_ERR_UNSUPPORTED, "kmeans bf16x3: d=%d > 128", d);
+  if (csum_out && !dists) return fail(EAC_ERR_ARG, "kmeans: inertia needs dists");
+  // The cascade pays where the three products take long (its read-backs
+  // cost about 40 us) and two thirds of the MFMAs are to be saved: one
+  // partition of more than 32 dimensions.
+  const bool cascade = !kg && P == 1 && d > 32 && n * ktot * ((d + 31) / 32) >= (int64_t)5e8;
+  const LabelLayout L = label_layout(d, cascade);
+  EAC_TRY(fill<uint64_t>((uint64_t*)B.nflag, kFlagSlots + ((int64_t)P * kStat + 1) / 2, 0ull, s));
   {
-    // waves per SIMD the kernel is compiled for: the built-in choice, or
-    // EAC_TUNE_KM_WAVES (2, 3 or 4; the same labels, other register
-    // budgets and occupancy)
-    const int wk = tune_value(EAC_TUNE_KM_WAVES);
-    const int w = (wk >= 2 && wk <= 4) ? wk : 0;
-    auto go = [&](auto kern) {
-      kern<<<g, kLB, 0, s>>>(X, n, d, B.Ch, B.Cl, B.ncf, B.k_off, P, B.pstat, labels, B.flags_r,
-                             B.nflag, B.region);
-    };
-    if (KD == 32) {
-      if (w == 2) go(k_label_bf16x3<32, 2>);
-      else if (w == 4) go(k_label_bf16x3<32, 4>);
-      else go(k_label_bf16x3<32, 3>);
-    } else if (KD == 64) {
-      if (w == 2) go(k_label_bf16x3<64, 2>);
-      else if (w == 4) go(k_label_bf16x3<64, 4>);
-      else go(k_label_bf16x3<64, 3>);
-    } else {
-      if (w == 2) go(k_label_bf16x3<128, 2>);
-      else if (w == 3) go(k_label_bf16x3<128, 3>);
-      else go(k_label_bf16x3<128, 1>);
-    }
+    const int py = P < 65535 ? P : 65535;
+    const int gm = grid_for(ktot * d / P, 4096, 64), gp = grid_for(ktot / P, 64, 256);
+    k_cent_max<<<dim3(gm, py), 256, 0, s>>>(C, d, B.k_off, P, B.pstat);
+    EAC_LAUNCH_CHECK();
+    k_cent_prep<<<dim3(gp, py), 256, 0, s>>>(C, ktot, d, L, B.k_off, P, B.Cf, B.Ct, B.ncf,
+                                             B.pstat);
+    EAC_LAUNCH_CHECK();
   }
-  EAC_LAUNCH_CHECK();
+  int pr = prof_begin(EAC_PROF_KM_LABEL, 2 * n * (int64_t)d * ktot, s);
+  LabelCall call{X,       0,      n,        d,      C,     B.Cf,      B.ncf,   B.k_off,
+                 P,       B.pstat, nullptr, labels, dists, B.flags_r, B.nflag, B.region};
+  if (cascade) {
+    // The single product first, on a sample: when it certifies most points
+    // the rest follow it and only the flagged rows take the three products.
+    const int64_t ns = n < 65536 ? n : 65536;
+    unsigned long long nf1 = 0;
+    call.n = ns;
+    EAC_TRY(launch_single(L, call, s));
+    EAC_TRY(read_flags(B, &nf1, s));
+    const bool single = nf1 * 4 <= (unsigned long long)ns;
+    call.n = n;
+    if (single) {
+      call.row0 = ns;
+      if (ns < n) {
+        EAC_TRY(launch_single(L, call, s));
+        EAC_TRY(read_flags(B, &nf1, s));
+      }
+      if (nf1 > 0) {
+        EAC_TRY(gather_flags(B, nf1, s));
+        EAC_TRY(fill<uint64_t>((uint64_t*)B.nflag, kFlagSlots, 0ull, s));
+        call.row0 = 0;
+        call.n = (int64_t)nf1;
+        call.list = B.flags;
+        EAC_TRY(launch_listed(L, call, s));
+      }
+    } else {
+      EAC_TRY(fill<uint64_t>((uint64_t*)B.nflag, kFlagSlots, 0ull, s));
+      EAC_TRY(launch_label<true>(L, call, s));
+    }
+  } else if (P == 1) {
+    EAC_TRY(launch_label<true>(L, call, s));
+  } else {
+    EAC_TRY(launch_label<false>(L, call, s));
+  }
   prof_end(pr, s);
+  if (P > 1) {
+    const int pgs = (P + kPG - 1) / kPG;
+    const dim3 gr(grid_for(n, 256 / kGrp, 16384), pgs < 65535 ? pgs : 65535);
+    if ((d & 3) == 0) k_resolve<true><<<gr, 256, 0, s>>>(X, n, d, C, B.k_off, P, labels, dists);
+    else k_resolve<false><<<gr, 256, 0, s>>>(X, n, d, C, B.k_off, P, labels, dists);
+    EAC_LAUNCH_CHECK();
+  }
   if (kg) {
     // flags gathered, sorted by partition and re-scored with device counts
     // (grids sized for the whole list, blocks past the count exit at once)
@@ -1663,13 +2198,8 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
     const uint64_t* fl = B.flags;
     const bool tiled = rescore_tiled_lds(d) <= 64 * 1024;
     if (tiled && P > 1 && P <= kSortMaxP) {
-      k_flag_bcount<<<kSortBlocks, 256, 0, s>>>(B.flags, kg->d_nf, P, kg->bcount);
-      EAC_LAUNCH_CHECK();
-      k_flag_bscan<<<1, 1024, 0, s>>>(kg->bcount, (int64_t)P * kSortBlocks);
-      EAC_LAUNCH_CHECK();
-      k_flag_bscatter<<<kSortBlocks, 256, 0, s>>>(B.flags, kg->d_nf, P, kg->bcount, kg->sorted);
-      EAC_LAUNCH_CHECK();
-      fl = kg->sorted;
+      EAC_TRY(sort_flags(B, P, 0, kg->d_nf, ar, s));
+      fl = B.flags_r;
     }
     int pr2 = prof_begin(EAC_PROF_KM_RESCORE, 0, s);
     if (tiled) {
@@ -1684,56 +2214,48 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
       auto go = [&](auto kern) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        kern<<<nb, kRtF * kRtS, lds, s>>>(X, n, d, C, B.k_off, fl, 0, labels, kg->d_nf);
+        kern<<<nb, kRtF * kRtS, lds, s>>>(X, n, d, C, B.k_off, fl, 0, labels, dists, kg->d_nf);
       };
       if (d <= 16) go(k_rescore_tiled<16>);
       else if (d <= 32) go(k_rescore_tiled<32>);
       else if (d <= 64) go(k_rescore_tiled<64>);
       else go(k_rescore_tiled<0>);
     } else {
-      if (P == 1)
-        k_rescore_f64<2><<<grid_for(B.flag_cap * kWave / 2, 256, 16384), 256, 0, s>>>(
-            X, n, d, B.Ct, ktot, B.k_off, B.flags, 0, labels, kg->d_nf);
-      else
-        k_rescore_f64<1><<<grid_for(B.flag_cap * kWave, 256, 16384), 256, 0, s>>>(
-            X, n, d, B.Ct, ktot, B.k_off, B.flags, 0, labels, kg->d_nf);
+      const int gr = grid_for(B.flag_cap, kRfF, 16384);
+      k_rescore_few<kRfF><<<gr, 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, B.flags, 0, labels,
+                                             dists, kg->d_nf, nullptr, 0);
     }
     EAC_LAUNCH_CHECK();
     prof_end(pr2, s);
     k_fit_tally<<<1, 64, 0, s>>>(kg->info, kg->d_nf, nullptr, 0, kg->any);
     EAC_LAUNCH_CHECK();
   } else {
-  unsigned long long hcnt[kFlagSlots];
-  EAC_TRY(d2h(hcnt, B.nflag, sizeof(hcnt), s));
-  unsigned long long nf = 0;
-  for (int q = 0; q < kFlagSlots; ++q) {
-    if ((int64_t)hcnt[q] > B.region) return fail(EAC_ERR_HIP, "kmeans: flag list overflow");
-    nf += hcnt[q];
-  }
-  if ((int64_t)nf > B.flag_cap) return fail(EAC_ERR_HIP, "kmeans: flag list overflow");
-  if (nf > 0) {
-    k_gather_flags<<<grid_for((int64_t)nf, 256, 65536), 256, 0, s>>>(B.flags_r, B.region, B.nflag,
-                                                                     B.flags, (int64_t)nf);
+  // One partition: the re-scoring of up to kFewMax flags needs no sorting and
+  // follows without a read-back, straight from the regions.
+  if (P == 1) {
+    int pr2 = prof_begin(EAC_PROF_KM_RESCORE, 0, s);
+    k_rescore_few<kRfF><<<1024, 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, B.flags_r, 0,
+                                             labels, dists, nullptr, B.nflag, B.region);
     EAC_LAUNCH_CHECK();
+    prof_end(pr2, s);
+  }
+  unsigned long long nf = 0;
+  EAC_TRY(read_flags(B, &nf, s));
+  if (nf > 0 && (P > 1 || nf >= (unsigned long long)kFewMax)) {
+    EAC_TRY(gather_flags(B, nf, s));
     int pr2 = prof_begin(EAC_PROF_KM_RESCORE, 3 * (int64_t)nf * d * (ktot / P), s);
     // Many flags (at least 1024 blocks of 64) and d <= 127 (LDS tiles up to
-    // 64 KiB): flags sorted by partition (one radix pass for up to 256
-    // partitions) feed the LDS-tiled re-scoring. Few flags, or no room for the sort: one wavefront per flag
-    // over the transposed centroids (more parallelism per flag).
+    // 64 KiB): the LDS-tiled re-scoring. Few flags: a block per kRfF of them
+    // over the transposed centroids (more parallelism per flag). Both want
+    // neighbouring flags in one partition: from 4096 flags on they are
+    // sorted by partition.
     const uint64_t* fl = B.flags;
     bool tiled = nf >= (unsigned long long)kRtF * 1024 && rescore_tiled_lds(d) <= 64 * 1024;
-    if (tiled && P > 1) {
-      const size_t mark2 = ar.used;
-      uint64_t* sorted = ar.take<uint64_t>(nf);
-      if (ar.overflow() || ar.cap - ar.used < radix_sort_ws_bytes((int64_t)nf, 8, 0)) {
-        tiled = false;
-        ar.used = mark2;
-      } else {
-        const int pb = bits_for((uint64_t)(P - 1));
-        EAC_TRY((radix_sort<uint64_t, NoValue>(B.flags, sorted, nullptr, nullptr, (int64_t)nf, 40,
-                                               40 + (pb < 1 ? 1 : pb), ar, s)));
-        fl = sorted;
-      }
+    bool sorted_flags = P == 1;
+    if (P > 1 && P <= kSortMaxP && nf >= 4096) {
+      EAC_TRY(sort_flags(B, P, (int64_t)nf, nullptr, ar, s));
+      fl = B.flags_r;
+      sorted_flags = true;
     }
     if (tiled) {
       const size_t lds = rescore_tiled_lds(d);
@@ -1741,33 +2263,27 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
       auto go = [&](auto kern) {
         (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern),
                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
-        kern<<<nb, kRtF * kRtS, lds, s>>>(X, n, d, C, B.k_off, fl, (int64_t)nf, labels, nullptr);
+        kern<<<nb, kRtF * kRtS, lds, s>>>(X, n, d, C, B.k_off, fl, (int64_t)nf, labels, dists,
+                                          nullptr);
       };
       if (d <= 16) go(k_rescore_tiled<16>);
       else if (d <= 32) go(k_rescore_tiled<32>);
       else if (d <= 64) go(k_rescore_tiled<64>);
       else go(k_rescore_tiled<0>);
     } else {
-      if (P == 1)
-        k_rescore_f64<2><<<grid_for((int64_t)(nf + 1) / 2 * kWave, 256, 65536), 256, 0, s>>>(
-            X, n, d, B.Ct, ktot, B.k_off, B.flags, (int64_t)nf, labels, nullptr);
-      else
-        k_rescore_f64<1><<<grid_for((int64_t)nf * kWave, 256, 65536), 256, 0, s>>>(
-            X, n, d, B.Ct, ktot, B.k_off, B.flags, (int64_t)nf, labels, nullptr);
+      auto go = [&](auto kern, int f) {
+        kern<<<grid_for((int64_t)nf, f, 65536), 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, fl,
+                                                             (int64_t)nf, labels, dists, nullptr,
+                                                             nullptr, 0);
+      };
+      if (sorted_flags) go(k_rescore_few<kRfF>, kRfF);
+      else go(k_rescore_few<1>, 1);
     }
     EAC_LAUNCH_CHECK();
     prof_end(pr2, s);
   }
   if (n_rescored) *n_rescored = (int64_t)nf;
   }  // read-back path
-  if (csum_out && !dists) return fail(EAC_ERR_ARG, "kmeans: inertia needs dists");
-  if (dists) {
-    const int pgs = (P + kPG - 1) / kPG;
-    const int py = pgs < 65535 ? pgs : 65535;
-    k_exact_dists<4><<<dim3(grid_for(n, 64, 16384), py), 256, 0, s>>>(X, n, d, C, B.k_off, P,
-                                                                        labels, dists);
-    EAC_LAUNCH_CHECK();
-  }
   if (csum_out) {
     EAC_TRY(np_chunk_sums(dists, n, P, B.csum, s));
     *csum_out = B.csum;
@@ -1951,13 +2467,11 @@ extern "C" int eac_kmeans_update(const float* X, int64_t n, int32_t d, const int
 // ------------------------------------------------- capturable batched fit
 namespace eac {
 namespace {
-// KmGraph buffers (flag count, per-partition counts and cursors, flags
-// sorted by partition); info and err are the caller's device arrays.
+// KmGraph buffers (the flag count); info and err are the caller's device
+// arrays.
 KmGraph carve_graph(Arena& ar, int64_t n, int P, int64_t* info, unsigned int* err) {
   KmGraph g;
   g.d_nf = ar.take<int64_t>(1);
-  g.bcount = ar.take<int32_t>((size_t)P * kSortBlocks);
-  g.sorted = ar.take<uint64_t>((size_t)P * n);
   g.info = info;
   g.err = err;
   g.any = nullptr;
