@@ -89,7 +89,7 @@ int eac_profile_read(int32_t slot, double* total_ms, int64_t* launches, int64_t*
  *                           resident); -1: one 1024-thread block per unit
  *   EAC_TUNE_CO_WINDOW      co-association LDS window in columns (even,
  *                           <= 32768; default: the row range when n is
- *                           smaller, else 32768)
+ *                           smaller, else 16384)
  *   EAC_TUNE_LEVEL_STEP     growth of the light edges per vertex from one
  *                           weight level of the split to the next (default
  *                           4, up to 4 levels; 1 or -1 = one split only)
@@ -479,9 +479,16 @@ int eac_coassoc_cap(const int64_t* indptr, const int32_t* indices, const int32_t
  * numba_update_condensed_coassoc_with_cluster :155-166): out[i, j] = number
  * of partitions with labels[p][i] == labels[p][j] >= 0, in the matrix dtype
  * (uint8 wraps as the reference's += 1 does); *h_max (host, nullable)
- * receives the largest stored value. ws: 256 bytes.
+ * receives the largest stored value. ws: 256 bytes; with
+ * eac_coassoc_dense_workspace_bytes the labels are transposed to bit planes
+ * once instead of in every tile.
+ * eac_coassoc_dense_add: the same counts added to the matrix (same types,
+ * integer types wrap), without a second matrix.
  * eac_dense_diassoc replaces full.py:98-112 make_diassoc (_1d / _2d):
  * mat[i] = val - mat[i] over len elements (integer types wrap).
+ * eac_dense_diassoc_max: the same with val = the matrix's largest value + 1,
+ * taken on the device (integer types only: a float's maximum may not be a
+ * number); len >= 1, ws: 256 bytes.
  * eac_dense_degree replaces full.py:83-95 get_degree: degree[i] = non-zero
  * entries of row i (condensed: its columns j > i only), *h_nnz the total.
  * eac_full_sl_lifetime replaces MyML/MyML/EAC/eac.py:337-364
@@ -500,10 +507,15 @@ int eac_coassoc_cap(const int64_t* indptr, const int32_t* indices, const int32_t
  * eac_labels_from_Z replaces linkage.py:303-357 labels_from_Z_numba for any
  * valid Z: the first n - n_clusters merges, clusters numbered by first
  * occurrence. n <= 65536 for the single-linkage calls. */
+size_t eac_coassoc_dense_workspace_bytes(int64_t n, int32_t P);
 int eac_coassoc_dense(const int32_t* labels, int64_t n, int32_t P, int32_t condensed,
                       int32_t dtype, void* out, int64_t* h_max, void* ws, size_t ws_bytes,
                       void* stream);
+int eac_coassoc_dense_add(const int32_t* labels, int64_t n, int32_t P, int32_t condensed,
+                          int32_t dtype, void* inout, void* ws, size_t ws_bytes, void* stream);
 int eac_dense_diassoc(void* mat, int64_t len, int32_t dtype, double val, void* stream);
+int eac_dense_diassoc_max(void* mat, int64_t len, int32_t dtype, void* ws, size_t ws_bytes,
+                          void* stream);
 int eac_dense_degree(const void* mat, int32_t dtype, int64_t n, int32_t condensed,
                      int32_t* degree, int64_t* h_nnz, void* ws, size_t ws_bytes, void* stream);
 size_t eac_dense_sl_workspace_bytes(int64_t n, int32_t dtype, int32_t condensed);

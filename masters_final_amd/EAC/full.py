@@ -49,7 +49,7 @@ def coassoc_dense_device(labels, condensed=True, dtype=np.uint8):
     shape = (n * (n - 1) // 2,) if condensed else (n, n)
     out = t.empty(shape, dtype=tdt, device=dl.device)
     mx = C.c_int64()
-    ws = L.workspace(256)
+    ws = L.workspace(lib.eac_coassoc_dense_workspace_bytes(n, P))
     L.check(lib.eac_coassoc_dense(L.ptr(dl), n, P, 1 if condensed else 0, _DT[dt], L.ptr(out),
                                   C.byref(mx), L.ptr(ws), ws.numel(), L.stream_ptr()))
     return out, mx.value
@@ -127,8 +127,27 @@ class EAC_FULL:
 
     def update_labels(self, labels):
         """Device entry: labels [P, n] (-1 = not listed)."""
-        add, _ = coassoc_dense_device(labels, condensed=self.condensed, dtype=self.dtype)
-        self.coassoc += add  # uint8 wraps, as the reference's in-place += does
+        t = L.torch()
+        m = self.coassoc
+        dl = L.as_device(labels, t.int32)
+        if dl.dim() == 1:
+            dl = dl[None]
+        P, n = dl.shape
+        # The counts go straight into the matrix (uint8 wraps, as the
+        # reference's in-place += does) where it is still this object's own
+        # form; anything else is added as a tensor.
+        if (P and n == self.n_samples and m.dtype in (t.uint8, t.int32, t.float32)
+                and m.dtype == self._tdt and m.device == dl.device and m.is_contiguous()
+                and not m.requires_grad
+                and m.shape == ((n * (n - 1) // 2,) if self.condensed else (n, n))):
+            lib = L.load_library()
+            ws = L.workspace(lib.eac_coassoc_dense_workspace_bytes(n, P))
+            L.check(lib.eac_coassoc_dense_add(
+                L.ptr(dl), n, P, 1 if self.condensed else 0, _wcode(m), L.ptr(m), L.ptr(ws),
+                ws.numel(), L.stream_ptr()))
+        else:
+            add, _ = coassoc_dense_device(dl, condensed=self.condensed, dtype=self.dtype)
+            self.coassoc += add
         self.n_updates += int(np.prod(np.shape(labels)[:-1])) if np.ndim(labels) > 1 else 1
 
     def todense(self):
@@ -162,6 +181,16 @@ class EAC_FULL:
             if self.max_val is not None:
                 max_val = self.max_val + 1
             else:
+                t = L.torch()
+                m = self.coassoc
+                if m.dtype in (t.uint8, t.int32) and m.numel() and m.is_contiguous():
+                    # the maximum stays on the device: no copy to the host and
+                    # back between the two kernels
+                    ws = L.workspace(256)
+                    L.check(L.load_library().eac_dense_diassoc_max(
+                        L.ptr(m), m.numel(), _wcode(m), L.ptr(ws), ws.numel(), L.stream_ptr()))
+                    self.is_diassoc = True
+                    return
                 max_val = int(self.coassoc.max().item()) + 1
         lib = L.load_library()
         L.check(lib.eac_dense_diassoc(L.ptr(self.coassoc), self.coassoc.numel(),
