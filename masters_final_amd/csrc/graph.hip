@@ -600,6 +600,21 @@ struct RoundCtl {
   int overflow_rounds;  // stopped at the round limit
 };
 
+// Device state counters of one MST call.
+struct MstState {
+  unsigned int overflow;
+  unsigned int missing;
+  int32_t n_f;  // forest edges (k_mst_one)
+  MstPlan plan;
+  RoundCtl ctl[2];
+  unsigned int had_edge[kMaxRounds + 1];
+  unsigned long long tot0[2][kLogSlots];                 // round-0 light / heavy keys
+  unsigned long long rlog[kMaxRounds][2][kLogSlots];     // per round: keys in / kept
+  unsigned int cand[kMaxRounds + 1];  // cand[r]: filter(r - 1) listed a candidate
+};
+constexpr size_t kStateHead = sizeof(MstState);
+constexpr size_t kCtlHead = offsetof(MstState, tot0);  // what the round loop reads
+
 // A level ends when a hook finds no candidate: the next level (if its lower
 // threshold is finite) starts with a routing pass over the heavy list.
 __device__ __forceinline__ RoundCtl next_ctl(RoundCtl c, int r, unsigned int had,
@@ -1526,20 +1541,6 @@ int weight_bytes(int32_t dt) {
   }
 }
 
-// Device state counters of one MST call.
-struct MstState {
-  unsigned int overflow;
-  unsigned int missing;
-  MstPlan plan;
-  RoundCtl ctl[2];
-  unsigned int had_edge[kMaxRounds + 1];
-  unsigned long long tot0[2][kLogSlots];                 // round-0 light / heavy keys
-  unsigned long long rlog[kMaxRounds][2][kLogSlots];     // per round: keys in / kept
-  unsigned int cand[kMaxRounds + 1];  // cand[r]: filter(r - 1) listed a candidate
-};
-constexpr size_t kStateHead = sizeof(MstState);
-constexpr size_t kCtlHead = offsetof(MstState, tot0);  // what the round loop reads
-
 inline unsigned long long fold_slots(const unsigned long long* v) {
   unsigned long long t = 0;
   for (int i = 0; i < kLogSlots; ++i) t += v[i];
@@ -1804,6 +1805,432 @@ int mst_rounds(MstBuffers& B, int32_t n, int r0, int count, MstRecs& rec, hipStr
   return r;
 }
 
+// ------------------------------------------------------- small graphs
+// The rounds of a graph with n <= kOneN and m <= kOneM in one workgroup:
+// every vertex's parent and candidate slot sit in LDS (2 + 8 bytes: what it
+// holds is the limit on n), the key lists stay where round 0 put them, and a
+// wavefront packs its share's survivors as it filters them. The rounds are
+// those of k_hook and k_round, level by level, so every forest key lands in
+// the same slot. Only roots hook: a wavefront keeps the list of its own.
+// A small graph's rounds are launches and round trips to memory, not work: a
+// mesh of 15,606 vertices and degree 6 needs 11 rounds, 22 launches. Here a
+// round costs three microseconds and what its keys take in LDS accesses. The
+// whole call, launches against this: 600 vertices of degree 6 207 -> 81 us,
+// the mesh 346 -> 201, 15,900 vertices of degree 12 (191,000 entries) 349 ->
+// 242; at degree 24 (382,000 entries) launches take 280, this took 347: one
+// compute unit then has too many keys.
+constexpr int32_t kOneN = 16000;
+constexpr int64_t kOneM = 1 << 18;
+constexpr int kOneT = 1024, kOneW = kOneT / kWave;
+inline size_t one_lds(int32_t n) { return (size_t)n * 8 + ((size_t)n * 2 + 15) / 16 * 16; }
+
+// 2 * vb <= 28: both ends sit in the key's low word.
+__device__ __forceinline__ void one_ends(uint64_t key, int vb, uint32_t* lo, uint32_t* hi) {
+  const uint32_t x = (uint32_t)key, mask = (1u << vb) - 1u;
+  *hi = x & mask;
+  *lo = (x >> vb) & mask;
+}
+__device__ __forceinline__ int ones_below(uint64_t m) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+}
+// A wavefront's keys: of every 16 slices of kOneSlice slots that the chunks
+// divide into it owns one, in turn another (a chunk's first slices are the
+// full ones), in this order, as one list. Survivors are packed at its front,
+// so a pass never writes past what it has read, and after the first pass the
+// list has no gaps.
+constexpr int kOneQ = 4, kOneSlice = kOneQ * kWave;
+__device__ __forceinline__ int64_t one_slice(int w, int32_t j) {
+  return (int64_t)kOneW * j + ((w + j) & (kOneW - 1));
+}
+__device__ __forceinline__ int64_t one_slot(int w, int32_t i) {
+  return one_slice(w, i / kOneSlice) * kOneSlice + i % kOneSlice;
+}
+
+// One pass over the wavefront's list of `from`: with cnt (a list still in its
+// chunks) the keys of every chunk's count, else nk packed keys. FLAT: every
+// key end's parent is its root (routing; the first round); else that root's
+// parent is, and a kept key's ends are made to point at it. ROUTE: keys below
+// limk become candidates and go to `to`, heavier cross keys stay. Returns
+// the keys read; *out, *out_to are the survivors' counts. Bound by the LDS
+// (40 accesses at random banks for 256 keys kept) and, in the first pass, by
+// the lists' latency: two slices are in flight.
+template <bool ROUTE, bool FLAT>
+__device__ __forceinline__ int32_t one_filter(uint64_t* from, const int32_t* cnt, int32_t nk,
+                                              int64_t nchunks, uint64_t* to, uint64_t limk, int vb,
+                                              uint16_t* s_par, unsigned long long* s_best,
+                                              int32_t* out, int32_t* out_to, bool* any_cand) {
+  const int lane = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  constexpr int Q = kOneQ, kPer = kGTile / kOneSlice;
+  int32_t read = 0, o = 0, ot = 0;
+  const int32_t total =  // slices
+      (int32_t)(cnt ? (nchunks * kPer + kOneW - 1) / kOneW : (nk + kOneSlice - 1) / kOneSlice);
+  int32_t held = 0;  // lane j: keys of the slice (batch of 64) + j
+  auto slice_keys = [&](int32_t j) {
+    if (!cnt) return nk - j * kOneSlice < kOneSlice ? nk - j * kOneSlice : kOneSlice;
+    return __builtin_amdgcn_readlane(held, j % kWave);
+  };
+  auto fetch_counts = [&](int32_t j) {  // j: a multiple of 64
+    if (!cnt) return;
+    const int64_t sl = one_slice(w, j + lane);
+    int32_t h = 0;
+    if (sl < nchunks * kPer) h = cnt[sl / kPer] - (int32_t)(sl % kPer) * kOneSlice;
+    held = h < 0 ? 0 : (h > kOneSlice ? kOneSlice : h);
+  };
+  auto load = [&](uint64_t (&k)[Q], int32_t j, int32_t have) {
+    const uint64_t* f = from + one_slot(w, j * kOneSlice);
+#pragma unroll
+    for (int q = 0; q < Q; ++q) k[q] = q * kWave + lane < have ? f[q * kWave + lane] : kInf;
+  };
+  auto filter = [&](const uint64_t (&k)[Q]) {
+    uint32_t x[2 * Q], p[2 * Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+      one_ends(k[q] != kInf ? k[q] : 0ull, vb, &x[2 * q], &x[2 * q + 1]);
+#pragma unroll
+    for (int i = 0; i < 2 * Q; ++i) p[i] = s_par[x[i]];
+    if (!FLAT) {
+      uint32_t rt[2 * Q];
+#pragma unroll
+      for (int i = 0; i < 2 * Q; ++i) rt[i] = s_par[p[i]];
+#pragma unroll
+      for (int i = 0; i < 2 * Q; ++i) {
+        if (k[i / 2] != kInf && rt[i & ~1] != rt[i | 1] && rt[i] != p[i])
+          s_par[x[i]] = (uint16_t)rt[i];
+        p[i] = rt[i];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      const bool keep = k[q] != kInf && p[2 * q] != p[2 * q + 1];
+      const bool cand = keep && (!ROUTE || k[q] < limk);
+      if (cand) {  // (a read first: atomics on one word serialise)
+        unsigned long long* b0 = &s_best[p[2 * q]];
+        unsigned long long* b1 = &s_best[p[2 * q + 1]];
+        if (k[q] < *(volatile unsigned long long*)b0) atomicMin(b0, k[q]);
+        if (k[q] < *(volatile unsigned long long*)b1) atomicMin(b1, k[q]);
+      }
+      *any_cand |= cand;
+      const uint64_t m = __ballot(cand);
+      if (ROUTE) {
+        const uint64_t ms = __ballot(keep && !cand);
+        if (cand) to[one_slot(w, ot + ones_below(m))] = k[q];
+        if (keep && !cand) from[one_slot(w, o + ones_below(ms))] = k[q];
+        ot += __popcll(m);
+        o += __popcll(ms);
+      } else {
+        if (cand) from[one_slot(w, o + ones_below(m))] = k[q];
+        o += __popcll(m);
+      }
+    }
+  };
+  // the keys of two slices ahead are loaded before this slice's are filtered:
+  // they lie past every write
+  uint64_t k0[Q], k1[Q];
+  fetch_counts(0);
+  int32_t h0 = total > 0 ? slice_keys(0) : 0, h1 = total > 1 ? slice_keys(1) : 0;
+  if (total > 0) load(k0, 0, h0);
+  if (total > 1) load(k1, 1, h1);
+  for (int32_t j = 0; j < total; ++j) {
+    uint64_t k[Q];
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      k[q] = k0[q];
+      k0[q] = k1[q];
+    }
+    const int32_t h = h0;
+    h0 = h1;
+    h1 = 0;
+    if (j + 2 < total) {
+      if ((j + 2) % kWave == 0) fetch_counts(j + 2);
+      h1 = slice_keys(j + 2);
+      load(k1, j + 2, h1);
+    }
+    read += h;
+    if (h > 0) filter(k);
+  }
+  *out = o;
+  if (ROUTE) *out_to = ot;
+  return read;
+}
+
+// Each vx[i] (vertex, hooked to: high half) of a lane that hooked: its parent
+// becomes its tree's root, four walks side by side, at most 16 steps (others
+// may store a nearer ancestor meanwhile: either is one). *more: a walk did
+// not end; *cycle: one came back. Returns the bits of the walks that ended.
+__device__ __forceinline__ uint32_t one_walks(uint16_t* s_par, const uint32_t* vx, bool* more,
+                                              bool* cycle) {
+  uint32_t x[4], y[4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = vx[i] >> 16;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) x[i] = s_par[x[i]];
+#pragma unroll
+  for (int i = 0; i < 4; ++i) y[i] = s_par[x[i]];
+  for (int step = 0; step < 16; ++step) {
+    bool go = false;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) go |= x[i] != y[i];
+    if (!go) break;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) x[i] = y[i];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) y[i] = s_par[x[i]];
+  }
+  uint32_t done = 0;
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const uint32_t v = vx[i] & 0xffffu;
+    if (v == vx[i] >> 16) continue;  // a root
+    done |= x[i] == y[i] ? 1u << i : 0u;
+    *more |= x[i] != y[i];
+    *cycle |= x[i] == v;
+    s_par[v] = (uint16_t)x[i];
+  }
+  return done;
+}
+
+// enq: rounds allowed (the control word of round enq is written as the rounds
+// left it). labels (nullable): first-occurrence component numbers. roots:
+// scratch of n words.
+__global__ __launch_bounds__(kOneT) void k_mst_one(
+    int32_t n, int vb, uint64_t* light, uint64_t* heavy, const int32_t* __restrict__ cnt_light,
+    const int32_t* __restrict__ cnt_heavy, int64_t nchunks,
+    const unsigned long long* __restrict__ best, uint64_t* mst_key, uint32_t* roots, MstState* st,
+    int enq, uint64_t* __restrict__ fkeys, int32_t* __restrict__ d_nf,
+    int32_t* __restrict__ labels, unsigned long long* __restrict__ rlog) {
+  extern __shared__ __align__(16) unsigned long long s_best[];
+  uint16_t* s_par = reinterpret_cast<uint16_t*>(s_best + n);
+  __shared__ int32_t s_tmp[kOneW + 1];
+  const int t = threadIdx.x, lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(t / kWave);
+  // this wavefront's vertices [a0, a1) and the list of its roots
+  const int seg = (n + kOneW - 1) / kOneW;
+  const int a0 = w * seg < n ? w * seg : n, a1 = a0 + seg < n ? a0 + seg : n;
+  uint32_t* const ra = roots + a0;
+  int nr = a1 - a0;
+  bool any = false;
+  for (int b = a0; b < a1; b += 4 * kWave) {
+    unsigned long long k[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int v = b + q * kWave + lane;
+      k[q] = v < a1 ? best[v] : kInf;
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int v = b + q * kWave + lane;
+      if (v >= a1) continue;
+      s_best[v] = k[q];
+      s_par[v] = (uint16_t)v;
+      ra[v - a0] = (uint32_t)v << 16 | (uint32_t)v;
+      any |= k[q] != kInf;
+    }
+  }
+  int32_t nl = 0, nh = -1;  // keys of the packed lists, -1: still in their chunks
+  int had = __syncthreads_or(any);
+  RoundCtl c;
+  c.phase = 0;
+  c.active = 1;
+  c.rounds = 0;
+  c.overflow_rounds = 0;
+  for (int r = 0; r < enq; ++r) {
+    if (had) {
+      for (int b = 0; b < nr; b += 4 * kWave) {
+        uint32_t vx[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int e = b + i * kWave + lane;
+          vx[i] = e < nr ? ra[e] : 0u;
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int e = b + i * kWave + lane;
+          if (e >= nr) continue;
+          const uint32_t v = vx[i] & 0xffffu;
+          uint32_t x = v;
+          const unsigned long long k = s_best[v];
+          if (k != kInf) {
+            uint32_t a, c2;
+            one_ends(k, vb, &a, &c2);
+            const uint32_t pa = s_par[a], pb = s_par[c2];
+            x = pa == v ? pb : pa;
+            // of a mirror pair (both picked k) the smaller id stays the root
+            if (s_best[x] == k && v < x) x = v;
+            if (x != v) mst_key[v] = k;
+          }
+          ra[e] = v | x << 16;
+        }
+      }
+      __syncthreads();
+      for (int b = 0; b < nr; b += 4 * kWave) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int e = b + i * kWave + lane;
+          if (e >= nr) continue;
+          const uint32_t vx = ra[e], v = vx & 0xffffu, x = vx >> 16;
+          if (x != v) s_par[v] = (uint16_t)x;
+          s_best[v] = kInf;
+        }
+      }
+      __syncthreads();
+      // every hooked root to its tree's root (a pick chain may hold all of
+      // them). Only a graph passed as symmetric that is not has a cycle.
+      bool cycle = false;
+      int left = nr;
+      for (int pass = 0;; ++pass) {
+        bool more = false;
+        int out = 0;
+        for (int b = 0; b < left; b += 4 * kWave) {
+          uint32_t vx[4];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int e = b + i * kWave + lane;
+            vx[i] = e < left ? ra[e] : 0u;
+          }
+          uint32_t done = one_walks(s_par, vx, &more, &cycle);
+          // what stays a root, and the walks that go on, are listed again
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const bool stay = b + i * kWave + lane < left && !(done & (1u << i));
+            const uint64_t m = __ballot(stay);
+            if (stay) ra[out + ones_below(m)] = vx[i];
+            out += __popcll(m);
+          }
+        }
+        left = out;
+        if (!__syncthreads_or(more)) break;
+        if (pass == 32) {
+          cycle = true;
+          break;
+        }
+      }
+      if (cycle) atomicOr(&st->overflow, 4u);
+      nr = left;
+    } else {  // the level is done: every vertex to its root
+      for (int pass = 0; pass <= 32; ++pass) {
+        bool more = false, cycle = false;
+        for (int b = a0; b < a1; b += 4 * kWave) {
+          uint32_t f[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int v = b + q * kWave + lane;
+            f[q] = v < a1 ? (uint32_t)s_par[v] << 16 | (uint32_t)v : 0u;
+          }
+          (void)one_walks(s_par, f, &more, &cycle);
+        }
+        if (!__syncthreads_or(more)) break;
+      }
+    }
+    if (rlog && t == 0) st->had_edge[r] = had;
+    const int phase = c.phase;
+    c = next_ctl(c, r, had, kMaxRounds, &st->plan);
+    if (!c.active) break;
+    bool cand = false;
+    int32_t in, ol = 0, oh = 0;
+    if (c.phase != phase) {
+      const uint64_t lim = st->plan.lim[c.phase], limk = lim == kInf ? kInf : lim << (2 * vb);
+      in = one_filter<true, true>(heavy, nh < 0 ? cnt_heavy : nullptr, nh, nchunks, light, limk, vb,
+                                  s_par, s_best, &oh, &ol, &cand);
+      nh = oh;
+    } else if (r == 0) {
+      in = one_filter<false, true>(light, cnt_light, 0, nchunks, nullptr, 0, vb, s_par, s_best, &ol,
+                                   &oh, &cand);
+    } else {
+      in = one_filter<false, false>(light, nullptr, nl, nchunks, nullptr, 0, vb, s_par, s_best, &ol,
+                                    &oh, &cand);
+    }
+    nl = ol;
+    if (rlog && lane == 0) {
+      atomicAdd(&rlog[(2 * r) * kLogSlots + w], (unsigned long long)in);
+      atomicAdd(&rlog[(2 * r + 1) * kLogSlots + w], (unsigned long long)(ol + oh));
+    }
+    had = __syncthreads_or(cand);
+  }
+  if (t == 0) st->ctl[enq & 1] = c;
+  __syncthreads();
+  // forest keys in vertex order, the slots past their count empty
+  int32_t cnt = 0, nf = 0, o = 0;
+  auto keys4 = [&](int b, uint64_t (&k)[4]) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int v = b + q * kWave + lane;
+      k[q] = v < a1 ? mst_key[v] : kInf;
+    }
+  };
+  for (int b = a0; b < a1; b += 4 * kWave) {
+    uint64_t k[4];
+    keys4(b, k);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) cnt += __popcll(__ballot(k[q] != kInf));
+  }
+  if (lane == 0) s_tmp[w] = cnt;
+  __syncthreads();
+  for (int q = 0; q < kOneW; ++q) {
+    o += q < w ? s_tmp[q] : 0;
+    nf += s_tmp[q];
+  }
+  for (int b = a0; b < a1; b += 4 * kWave) {
+    uint64_t k[4];
+    keys4(b, k);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const uint64_t m = __ballot(k[q] != kInf);
+      if (k[q] != kInf) fkeys[o + ones_below(m)] = k[q];
+      o += __popcll(m);
+    }
+  }
+  for (int q = nf + t; q < n; q += kOneT) fkeys[q] = kInf;
+  if (t == 0) {
+    *d_nf = nf;
+    st->n_f = nf;
+  }
+  if (!labels) return;
+  // components numbered by their smallest vertex (every parent is a root:
+  // the last round hooked nothing)
+  int32_t* s_first = reinterpret_cast<int32_t*>(s_best);
+  int32_t* s_rank = s_first + n;
+  for (int v = t; v < n; v += kOneT) s_first[v] = INT32_MAX;
+  __syncthreads();
+  for (int v = t; v < n; v += kOneT) {
+    int32_t* f = &s_first[s_par[v]];
+    if (v < *(volatile int32_t*)f) atomicMin(f, v);
+  }
+  __syncthreads();
+  cnt = 0;
+  for (int v = a0 + lane; v - lane < a1; v += kWave)
+    cnt += __popcll(__ballot(v < a1 && s_first[s_par[v < a1 ? v : a0]] == v));
+  if (lane == 0) s_tmp[w] = cnt;
+  __syncthreads();
+  o = 0;
+  for (int q = 0; q < w; ++q) o += s_tmp[q];
+  for (int v = a0 + lane; v - lane < a1; v += kWave) {
+    const bool is = v < a1 && s_first[s_par[v < a1 ? v : a0]] == v;
+    const uint64_t m = __ballot(is);
+    if (is) s_rank[v] = o + ones_below(m);
+    o += __popcll(m);
+  }
+  __syncthreads();
+  for (int v = t; v < n; v += kOneT) labels[v] = s_rank[s_first[s_par[v]]];
+}
+
+inline bool one_fits(int32_t n, int64_t m) { return n <= kOneN && m <= kOneM; }
+
+// All rounds, the forest keys and the labels of a small graph.
+int mst_one(MstBuffers& B, int32_t n, int enq, int32_t* d_nf, int32_t* labels, MstRecs& rec,
+            hipStream_t s) {
+  const size_t lds = one_lds(n);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_mst_one),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  rec.round.push_back(prof_begin(EAC_PROF_MST_ROUND, 0, s));
+  k_mst_one<<<1, kOneT, lds, s>>>(n, vbits_for(n), B.light, B.heavy, B.cnt_light, B.cnt_heavy,
+                                  B.nchunks, B.best[0], B.mst_key,
+                                  reinterpret_cast<uint32_t*>(B.roots[0]), B.st, enq, B.fkeys,
+                                  d_nf, labels, prof_on() ? &B.st->rlog[0][0][0] : nullptr);
+  EAC_LAUNCH_CHECK();
+  prof_end(rec.round.back(), s);
+  return EAC_OK;
+}
+
 // Errors recorded on the device, and whether rounds are still running.
 int mst_check(const MstState& hs, int enq, int vb, bool* active) {
   if (hs.plan.err)
@@ -1832,6 +2259,14 @@ void mst_prof_bytes(const MstState& hs, int enq, int32_t n, int64_t nchunks, Mst
                    hs.had_edge[r], fold_slots(hs.rlog[r][0]), fold_slots(hs.rlog[r][1]));
   }
   prof_set_bytes(rec.pr0, rec.round0_bytes + 8 * (int64_t)(l0 + h0));
+  if (rec.hook.empty() && !rec.round.empty()) {  // one launch for all rounds
+    int64_t in = 0, out = 0;
+    for (int r = 0; r < hs.ctl[enq & 1].rounds && r < kMaxRounds; ++r) {
+      in += (int64_t)fold_slots(hs.rlog[r][0]);
+      out += (int64_t)fold_slots(hs.rlog[r][1]);
+    }
+    prof_set_bytes(rec.round[0], 8 * (in + out) + 24 * (int64_t)n);
+  }
   for (int r = 0; r < (int)rec.hook.size(); ++r) {
     const bool ran = r < hs.ctl[enq & 1].rounds;
     const int64_t in = ran ? (int64_t)fold_slots(hs.rlog[r][0]) : 0;
@@ -1857,12 +2292,15 @@ int mst_forest(MstBuffers& B, int32_t n, int32_t* d_nf, hipStream_t s) {
   return EAC_OK;
 }
 
-inline int first_batch(int32_t n) {
-  // about the rounds a graph of this size needs (idle rounds cost a few
-  // microseconds, a host read tens)
+// Rounds enqueued before the first read-back: about what a graph of this size
+// needs, and one more for every further weight level (each ends with a round
+// that finds nothing). One round too few costs the tail once more and two
+// host reads (100 us of 1,200 at a million vertices of degree 40, which need
+// 16), one too many the few microseconds of two launches that return at once.
+inline int first_batch(int32_t n, int64_t m, int symmetric) {
   if (tune_value(EAC_TUNE_FIRST_BATCH) > 0) return tune_value(EAC_TUNE_FIRST_BATCH);
-  const int vb = vbits_for(n);
-  return vb * 3 / 4 > 6 ? vb * 3 / 4 : 6;
+  const int vb = vbits_for(n), base = vb * 3 / 4 > 6 ? vb * 3 / 4 : 6;
+  return base + split_plan(n, m, symmetric).levels - 1;
 }
 
 // Boruvka rounds up to the forest key list (shared by the lifetime cut and
@@ -1879,9 +2317,21 @@ int mst_core(const int32_t* dest, const W* weight, const int64_t* fe, const int3
   MstRecs rec;
   EAC_TRY((mst_begin<W, HAS_OD>(dest, weight, fe, od, n, m, symmetric, B, rec, s)));
   const int fixed_rounds = graph_rounds < kMaxRounds ? graph_rounds : kMaxRounds;
-  int enq = 0, batch = graph_mode ? fixed_rounds : first_batch(n);
+  int enq = 0, batch = graph_mode ? fixed_rounds : first_batch(n, m, symmetric);
+  const int64_t ftiles = (n + kGTile - 1) / kGTile;
+  int32_t* d_nf = B.tile_cnt + ftiles;
   MstState hs;
-  for (;;) {
+  const bool one = one_fits(n, m);
+  if (one) {
+    enq = graph_mode ? fixed_rounds : kMaxRounds;
+    EAC_TRY(mst_one(B, n, enq, d_nf, nullptr, rec, s));
+    if (!graph_mode) {
+      EAC_TRY(d2h_sync(&hs, B.st, prof_on() ? kStateHead : kCtlHead, s));
+      bool active = false;
+      EAC_TRY(mst_check(hs, enq, vb, &active));
+    }
+  }
+  for (; !one;) {
     enq = mst_rounds(B, n, enq, batch, rec, s);
     if (graph_mode) break;
     EAC_TRY(d2h_sync(&hs, B.st, prof_on() ? kStateHead : kCtlHead, s));
@@ -1891,9 +2341,7 @@ int mst_core(const int32_t* dest, const W* weight, const int64_t* fe, const int3
     batch = 4;
   }
   if (!graph_mode) mst_prof_bytes(hs, enq, n, B.nchunks, rec);
-  const int64_t ftiles = (n + kGTile - 1) / kGTile;
-  int32_t* d_nf = B.tile_cnt + ftiles;
-  EAC_TRY(mst_forest(B, n, d_nf, s));
+  if (!one) EAC_TRY(mst_forest(B, n, d_nf, s));
   fi->vb = vb;
   fi->d_nf = d_nf;
   fi->plan = &B.st->plan;
@@ -1906,8 +2354,8 @@ int mst_core(const int32_t* dest, const W* weight, const int64_t* fe, const int3
     fi->rounds = fixed_rounds;
     return EAC_OK;
   }
-  int32_t n_f = 0;
-  EAC_TRY(d2h_sync(&n_f, d_nf, sizeof(int32_t), s));
+  int32_t n_f = hs.n_f;
+  if (!one) EAC_TRY(d2h_sync(&n_f, d_nf, sizeof(int32_t), s));
   fi->n_f = n_f;
   fi->wbits = hs.plan.wbits;
   fi->wlo = hs.plan.wlo;
@@ -2022,7 +2470,33 @@ int mst_impl(const int32_t* dest, const W* weight, const int64_t* fe, const int3
   int32_t* d_nf = B.tile_cnt + ftiles;
   MstRecs rec;
   EAC_TRY((mst_begin<W, HAS_OD>(dest, weight, fe, od, n, m, symmetric, B, rec, s)));
-  int enq = mst_rounds(B, n, 0, first_batch(n), rec, s);
+  if (one_fits(n, m)) {
+    const int enq = kMaxRounds;
+    EAC_TRY(mst_one(B, n, enq, d_nf, labels, rec, s));
+    if (n > 1 && (ids || wout)) {
+      k_tail_pos<W, HAS_OD><<<grid_for(8 * (int64_t)(n - 1), kGB,
+                                       resident_grid(k_tail_pos<W, HAS_OD>, kGB)),
+                              kGB, 0, s>>>(B.fkeys, n - 1, d_nf, dest, weight, fe, od, vb,
+                                           symmetric, &B.st->plan, ids, wout, &B.st->missing,
+                                           nullptr, 0, nullptr);
+      EAC_LAUNCH_CHECK();
+    }
+    MstState hs;
+    EAC_TRY(d2h_sync(&hs, B.st, prof_on() ? kStateHead : kCtlHead, s));
+    bool active = false;
+    EAC_TRY(mst_check(hs, enq, vb, &active));
+    mst_prof_bytes(hs, enq, n, B.nchunks, rec);
+    prof_flush();
+    if (hs.missing) return fail(EAC_ERR_HIP, "boruvka: forest edge not found in its row");
+    if (h_out) {
+      h_out[0] = hs.n_f;
+      h_out[1] = n - hs.n_f;
+      h_out[2] = hs.ctl[enq & 1].rounds;
+      h_out[3] = hs.plan.wbits;
+    }
+    return EAC_OK;
+  }
+  int enq = mst_rounds(B, n, 0, first_batch(n, m, symmetric), rec, s);
   MstTail ht;
   for (int attempt = 0;; ++attempt) {
     ar.used = mark;
