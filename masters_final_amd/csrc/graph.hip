@@ -1359,15 +1359,9 @@ __global__ void k_iota(int32_t* p, int32_t n) {
     p[i] = (int32_t)i;
 }
 
-// Unites the endpoints of keys[0 : nk], or of keys[0 : min(nk, *d_cnt)]
-// when the count lives on the device.
+// Unites the endpoints of keys[0 : nk].
 __global__ __launch_bounds__(kGB) void k_unite_keys(const uint64_t* __restrict__ keys,
-                                                    int64_t nk, const int32_t* __restrict__ d_cnt,
-                                                    int vb, int32_t* P) {
-  if (d_cnt) {
-    const int64_t c = *d_cnt;
-    nk = c < nk ? c : nk;
-  }
+                                                    int64_t nk, int vb, int32_t* P) {
   for (int64_t i = (int64_t)blockIdx.x * kGB + threadIdx.x; i < nk;
        i += (int64_t)gridDim.x * kGB) {
     int32_t a, b;
@@ -1598,12 +1592,11 @@ MstBuffers carve_mst(Arena& ar, int32_t n, int64_t m, int symmetric) {
 // union-find labels over a key list, numbered by first occurrence
 int labels_from_keys(const uint64_t* keys, int64_t nk, int vb, int32_t n, int32_t* parent,
                      int32_t* root, int32_t* flag, int32_t* rank, int32_t* labels,
-                     int32_t* d_ncomp, Arena& ar, hipStream_t s,
-                     const int32_t* d_nk = nullptr) {
+                     int32_t* d_ncomp, Arena& ar, hipStream_t s) {
   k_iota<<<grid_for(n, 256, 4096), 256, 0, s>>>(parent, n);
   EAC_LAUNCH_CHECK();
   if (nk > 0) {
-    k_unite_keys<<<grid_for(nk, kGB, persistent_blocks()), kGB, 0, s>>>(keys, nk, d_nk, vb,
+    k_unite_keys<<<grid_for(nk, kGB, persistent_blocks()), kGB, 0, s>>>(keys, nk, vb,
                                                                         parent);
     EAC_LAUNCH_CHECK();
   }
@@ -2671,7 +2664,8 @@ template <typename W>
 __device__ CutOut cut_decide(const uint64_t* __restrict__ sk, int64_t nf, int64_t n, int vb,
                              uint64_t wlo, uint64_t gmax_word, int rule, double max_dist,
                              int32_t n_clusters, unsigned long long max_lt_bits,
-                             unsigned long long min_lt_bits, unsigned long long argmax) {
+                             unsigned long long min_lt_bits, unsigned long long argmax,
+                             int64_t known_above = -1) {
   CutOut o{nf, 0, 0, 0, 0.0};
   const double gmax = weight_value<W>(gmax_word);  // largest graph weight
   if (nf < 2 && (rule == 1 || n_clusters == 0)) { o.err = 1; return o; }
@@ -2692,13 +2686,16 @@ __device__ CutOut cut_decide(const uint64_t* __restrict__ sk, int64_t nf, int64_
   int64_t nc_stable;
   if (n_clusters == 0) {
     // lifetime_n_clusters, eac.py:366-391
-    double wa = weight_value<W>((sk[a] >> (2 * vb)) + wlo);
-    int64_t lo = a, hi = nf;  // first index with w > w[a]
-    while (lo < hi) {
-      int64_t mid = (lo + hi) >> 1;
-      if (weight_value<W>((sk[mid] >> (2 * vb)) + wlo) > wa) hi = mid; else lo = mid + 1;
+    int64_t above = known_above;  // edges heavier than edge a
+    if (above < 0) {
+      double wa = weight_value<W>((sk[a] >> (2 * vb)) + wlo);
+      int64_t lo = a, hi = nf;  // first index with w > w[a]
+      while (lo < hi) {
+        int64_t mid = (lo + hi) >> 1;
+        if (weight_value<W>((sk[mid] >> (2 * vb)) + wlo) > wa) hi = mid; else lo = mid + 1;
+      }
+      above = nf - lo;
     }
-    int64_t above = nf - lo;
     int64_t cont = above == 0 ? 1 : above + 1;
     double mn = __longlong_as_double((long long)min_lt_bits);
     if (!(mn <= 1e-8)) { o.err = 1; return o; }  // np.min over an empty selection
@@ -2849,106 +2846,304 @@ __global__ __launch_bounds__(kGB) void k_graph_wmax(const W* __restrict__ weight
 }
 
 // Lifetime statistics and the cut decision of every graph: one block per
-// graph over its segment sk[seg[g] : seg[g+1]] (sorted by key).
+// graph over its segment sk[seg[g] : seg[g+1]] (sorted by key), read once for
+// the largest lifetime with its first index and the smallest, and once more
+// for the edges heavier than that one. gmax (null: max_dist is given, so no
+// rule asks for it): the graphs' largest weight words.
 struct GraphCut {
   long long keep, nc_stable, err, labels_empty;
 };
+constexpr int kSegT = 1024;
+constexpr int kSegN = 1 << 16, kSegMin = 64;  // see k_seg_label
 template <typename W>
-__global__ __launch_bounds__(kGB) void k_seg_cut(const uint64_t* __restrict__ sk,
-                                                 const int64_t* __restrict__ seg,
-                                                 const int64_t* __restrict__ goff, int G, int vb,
-                                                 const MstPlan* __restrict__ plan,
-                                                 const unsigned long long* __restrict__ gmax,
-                                                 int rule, double max_dist, int32_t n_clusters,
-                                                 GraphCut* __restrict__ out) {
+__global__ __launch_bounds__(kSegT) void k_seg_cut(const uint64_t* __restrict__ sk,
+                                                   const int64_t* __restrict__ seg,
+                                                   const int64_t* __restrict__ goff, int G, int vb,
+                                                   const MstPlan* __restrict__ plan,
+                                                   const unsigned long long* __restrict__ gmax,
+                                                   int rule, double max_dist, int32_t n_clusters,
+                                                   GraphCut* __restrict__ out,
+                                                   int32_t* __restrict__ big) {
   const uint64_t wlo = plan->wlo;
-  __shared__ unsigned long long s_a[kGB / kWave], s_b[kGB / kWave];
-  __shared__ unsigned long long s_mx, s_mn, s_arg;
+  constexpr int kNW = kSegT / kWave;
+  __shared__ unsigned long long s_mx[kNW], s_mn[kNW], s_arg[kNW];
+  __shared__ unsigned int s_above[kNW];
+  const int w = threadIdx.x / kWave;
   for (int g = blockIdx.x; g < G; g += gridDim.x) {
     const uint64_t* k = sk + seg[g];
     const int64_t nf = seg[g + 1] - seg[g];
-    unsigned long long mx = 0, mn = ~0ull;
-    for (int64_t i = threadIdx.x; i + 1 < nf; i += kGB) {
+    unsigned long long mx = 0, mn = ~0ull, arg = ~0ull;
+#pragma unroll 4
+    for (int64_t i = threadIdx.x; i + 1 < nf; i += kSegT) {
       double wi = weight_value<W>((k[i] >> (2 * vb)) + wlo);
       double wj = weight_value<W>((k[i + 1] >> (2 * vb)) + wlo);
       unsigned long long b = (unsigned long long)__double_as_longlong(wj - wi);
-      mx = b > mx ? b : mx;
-      mn = b < mn ? b : mn;
-    }
-#pragma unroll
-    for (int off = kWave / 2; off > 0; off >>= 1) {
-      unsigned long long a = __shfl_xor(mx, off, kWave), b = __shfl_xor(mn, off, kWave);
-      mx = a > mx ? a : mx;
-      mn = b < mn ? b : mn;
-    }
-    if (lane_id() == 0) { s_a[threadIdx.x / kWave] = mx; s_b[threadIdx.x / kWave] = mn; }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      for (int q = 1; q < kGB / kWave; ++q) {
-        mx = s_a[q] > mx ? s_a[q] : mx;
-        mn = s_b[q] < mn ? s_b[q] : mn;
+      if (b > mx || arg == ~0ull) {
+        mx = b;
+        arg = (unsigned long long)i;
       }
-      s_mx = mx;
-      s_mn = mn;
-      s_arg = ~0ull;
+      mn = b < mn ? b : mn;
+    }
+    auto fold = [&](unsigned long long a, unsigned long long ai, unsigned long long b) {
+      if (ai != ~0ull && (arg == ~0ull || a > mx || (a == mx && ai < arg))) {
+        mx = a;
+        arg = ai;
+      }
+      mn = b < mn ? b : mn;
+    };
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1)
+      fold(__shfl_xor(mx, off, kWave), __shfl_xor(arg, off, kWave), __shfl_xor(mn, off, kWave));
+    if (lane_id() == 0) {
+      s_mx[w] = mx;
+      s_mn[w] = mn;
+      s_arg[w] = arg;
     }
     __syncthreads();
-    for (int64_t i = threadIdx.x; i + 1 < nf; i += kGB) {
-      double wi = weight_value<W>((k[i] >> (2 * vb)) + wlo);
-      double wj = weight_value<W>((k[i + 1] >> (2 * vb)) + wlo);
-      if ((unsigned long long)__double_as_longlong(wj - wi) == s_mx)
-        atomicMin(&s_arg, (unsigned long long)i);
+    for (int q = 0; q < kNW; ++q) fold(s_mx[q], s_arg[q], s_mn[q]);
+    unsigned int above = 0;
+    if (arg != ~0ull) {
+      const double wa = weight_value<W>((k[arg] >> (2 * vb)) + wlo);
+#pragma unroll 4
+      for (int64_t i = threadIdx.x; i < nf; i += kSegT)
+        above += weight_value<W>((k[i] >> (2 * vb)) + wlo) > wa;
     }
+    above = wave_sum(above);
+    if (lane_id() == 0) s_above[w] = above;
     __syncthreads();
     if (threadIdx.x == 0) {
-      CutOut o = cut_decide<W>(k, nf, goff[g + 1] - goff[g], vb, wlo, gmax[g], rule, max_dist,
-                               n_clusters, s_mx, s_mn, s_arg);
+      int64_t heavier = 0;
+      for (int q = 0; q < kNW; ++q) heavier += s_above[q];
+      CutOut o = cut_decide<W>(k, nf, goff[g + 1] - goff[g], vb, wlo, gmax ? gmax[g] : 0ull, rule,
+                               max_dist, n_clusters, mx, mn, arg, arg != ~0ull ? heavier : -1);
       out[g].keep = o.keep;
       out[g].nc_stable = o.nc_stable;
       out[g].err = o.err;
       out[g].labels_empty = o.labels_empty;
+      if (goff[g + 1] - goff[g] > kSegN && nf > 0 && o.keep > 0) *big = 1;
     }
     __syncthreads();
   }
 }
 
-__global__ void k_seg_keep_flags(const uint32_t* __restrict__ gid, int64_t nf, int G,
-                                 const int64_t* __restrict__ seg,
-                                 const GraphCut* __restrict__ cut, int32_t* __restrict__ flag) {
-  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < nf;
-       i += (int64_t)gridDim.x * blockDim.x) {
-    uint32_t g = gid[i];
-    flag[i] = g < (uint32_t)G && (i - seg[g]) < cut[g].keep;
+// ---- labels of the batch: union of every graph's kept edges, components
+// numbered by first occurrence inside the graph.
+//
+// k_seg_label: one workgroup per graph of up to kSegN vertices, the forest in
+// LDS (16-bit parents). Rounds: every edge between two roots hooks the larger
+// under the smaller (any of several: the others come again), then every
+// vertex goes to its root; an edge within a component is dropped, the rest
+// are packed as pairs of roots. 64 graphs of 1,000 to 50,000 vertices: the
+// lock-free union-find over the union, its flattening and numbering (the
+// k_batch_* kernels) took 420 us, bound by dependent reads of memory; this 70.
+// They remain for larger graphs (`big`: one with kept edges; without any, as
+// the padding of a recorded batch has it, a graph of any size is numbered
+// here), and where the graphs are so small (fewer than kSegMin vertices on
+// average) that most of a workgroup would be idle.
+__global__ __launch_bounds__(kSegT) void k_seg_label(const uint64_t* __restrict__ sk,
+                                                     const int64_t* __restrict__ seg,
+                                                     const int64_t* __restrict__ goff, int G,
+                                                     int vb, const GraphCut* __restrict__ cut,
+                                                     const int32_t* __restrict__ big,
+                                                     uint32_t* __restrict__ pairs,
+                                                     int32_t* __restrict__ labels,
+                                                     int32_t* __restrict__ count) {
+  if (*big) return;
+  extern __shared__ __align__(16) uint16_t s_up[];
+  constexpr int kNW = kSegT / kWave;
+  __shared__ int32_t s_cnt[kNW];
+  const int t = threadIdx.x, lane = lane_id();
+  const int w = __builtin_amdgcn_readfirstlane(t / kWave);
+  for (int g = blockIdx.x; g < G; g += gridDim.x) {
+    const int64_t v0 = goff[g];
+    const int nv = goff[g + 1] > v0 ? (int)(goff[g + 1] - v0) : 0;
+    const int64_t have = seg[g + 1] - seg[g];
+    const int64_t kept = cut[g].keep < 0 ? 0 : (cut[g].keep < have ? cut[g].keep : have);
+    if (kept == 0) {  // uniform
+#pragma unroll 4
+      for (int v = t; v < nv; v += kSegT) labels[v0 + v] = v;
+      if (t == 0) count[g] = nv;
+      continue;
+    }
+    for (int v = t; v < nv; v += kSegT) s_up[v] = (uint16_t)v;
+    __syncthreads();
+    // this wavefront's edges
+    const int64_t per = (kept + kNW - 1) / kNW;
+    const int64_t e0 = w * per < kept ? w * per : kept;
+    int32_t ne = (int32_t)((e0 + per < kept ? e0 + per : kept) - e0);
+    const uint64_t* keys = sk + seg[g] + e0;
+    uint32_t* list = pairs + seg[g] + e0;
+    for (bool first = true;; first = false) {
+      int32_t out = 0;
+      for (int b = 0; b < ne; b += 4 * kWave) {
+        uint32_t x[4], y[4];
+        bool on[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int e = b + q * kWave + lane;
+          on[q] = e < ne;
+          x[q] = y[q] = 0;
+          if (!on[q]) continue;
+          if (first) {
+            int32_t lo, hi;
+            unpack_ends(keys[e], vb, &lo, &hi);
+            on[q] = lo >= v0 && hi - v0 < nv;  // (an edge out of its graph joins nothing)
+            x[q] = (uint32_t)(lo - v0);
+            y[q] = (uint32_t)(hi - v0);
+          } else {
+            x[q] = list[e] & 0xffffu;
+            y[q] = list[e] >> 16;
+          }
+        }
+        if (!first) {
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            if (!on[q]) continue;
+            x[q] = s_up[x[q]];
+            y[q] = s_up[y[q]];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const bool go = on[q] && x[q] != y[q];
+          const uint32_t lo = x[q] < y[q] ? x[q] : y[q], hi = x[q] < y[q] ? y[q] : x[q];
+          if (go) s_up[hi] = (uint16_t)lo;
+          const uint64_t m = __ballot(go);
+          if (go) list[out + ones_below(m)] = hi << 16 | lo;
+          out += __popcll(m);
+        }
+      }
+      ne = out;
+      if (!__syncthreads_or(ne > 0)) break;
+      for (;;) {  // parents fall, so every walk ends; 16 steps at a time
+        bool more = false, cycle = false;
+        for (int b = w * kWave; b < nv; b += 4 * kSegT) {
+          uint32_t f[4];
+#pragma unroll
+          for (int q = 0; q < 4; ++q) {
+            const int v = b + q * kSegT + lane;
+            f[q] = v < nv ? (uint32_t)s_up[v] << 16 | (uint32_t)v : 0u;
+          }
+          (void)one_walks(s_up, f, &more, &cycle);
+        }
+        if (!__syncthreads_or(more)) break;
+      }
+    }
+    // roots are their components' smallest vertices
+    const int part = ((nv + kNW - 1) / kNW + kWave - 1) / kWave * kWave;
+    const int a0 = w * part < nv ? w * part : nv, a1 = a0 + part < nv ? a0 + part : nv;
+    int32_t cnt = 0;
+    for (int v = a0 + lane; v - lane < a1; v += kWave)
+      cnt += __popcll(__ballot(v < a1 && s_up[v] == v));
+    if (lane == 0) s_cnt[w] = cnt;
+    __syncthreads();
+    int32_t o = 0;
+    for (int q = 0; q < w; ++q) o += s_cnt[q];
+    for (int v = a0 + lane; v - lane < a1; v += kWave) {
+      const bool root = v < a1 && s_up[v] == v;
+      const uint64_t m = __ballot(root);
+      if (root) labels[v0 + v] = o + ones_below(m);
+      o += __popcll(m);
+    }
+    if (w == kNW - 1 && lane == 0) count[g] = o;
+    __syncthreads();
+#pragma unroll 4
+    for (int v = t; v < nv; v += kSegT)
+      if (s_up[v] != v) labels[v0 + v] = labels[v0 + s_up[v]];
+    __syncthreads();
   }
 }
 
-// per-graph labels from union labels numbered by first occurrence (graphs
-// occupy consecutive vertex ranges, so graph g's labels start at the label of
-// its first vertex): base[g] = label of the first vertex, base[G] = total.
-__global__ void k_graph_base(const int32_t* __restrict__ lab, const int64_t* __restrict__ goff,
-                             int G, const int32_t* __restrict__ total,
-                             int32_t* __restrict__ base) {
-  for (int g = blockIdx.x * blockDim.x + threadIdx.x; g <= G; g += gridDim.x * blockDim.x) {
-    if (g == G) { base[g] = *total; continue; }
-    base[g] = goff[g + 1] > goff[g] ? lab[goff[g]] : -1;
+// The same over the whole union in memory: a lock-free union-find, roots
+// flattened and ranked over all vertices. big null: always.
+__global__ __launch_bounds__(kGB) void k_batch_unite(const uint64_t* __restrict__ sk,
+                                                     const uint32_t* __restrict__ gid, int64_t nf,
+                                                     int G, int vb,
+                                                     const int64_t* __restrict__ seg,
+                                                     const GraphCut* __restrict__ cut,
+                                                     const int32_t* __restrict__ big,
+                                                     int32_t* P) {
+  if (big && !*big) return;
+  for (int64_t i = (int64_t)blockIdx.x * kGB + threadIdx.x; i < nf;
+       i += (int64_t)gridDim.x * kGB) {
+    const uint32_t g = gid[i];
+    if (g >= (uint32_t)G || i - seg[g] >= cut[g].keep) continue;
+    int32_t a, b;
+    unpack_ends(sk[i], vb, &a, &b);
+    uf_unite(P, a, b);
   }
 }
-__global__ void k_graph_sub(int32_t* __restrict__ lab, const int64_t* __restrict__ goff, int G,
-                            const int32_t* __restrict__ base, const GraphCut* __restrict__ cut,
-                            int64_t* __restrict__ gout) {
-  for (int g = blockIdx.x; g < G; g += gridDim.x) {
-    const int64_t v0 = goff[g], v1 = goff[g + 1];
-    const int32_t b = base[g];
-    for (int64_t v = v0 + threadIdx.x; v < v1; v += blockDim.x) lab[v] -= b;
-    if (threadIdx.x == 0) {
-      int32_t nb = -1;
-      for (int q = g + 1; q <= G; ++q)
-        if (base[q] >= 0) { nb = base[q]; break; }
-      gout[4 * g + 0] = v1 > v0 ? (int64_t)(nb - b) : 0;
-      gout[4 * g + 1] = cut[g].labels_empty;
-      gout[4 * g + 2] = cut[g].nc_stable;
-      gout[4 * g + 3] = cut[g].err ? -1 : cut[g].keep;
+__global__ void k_batch_iota(int32_t* __restrict__ p, int32_t n, const int32_t* __restrict__ big) {
+  if (big && !*big) return;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x)
+    p[i] = (int32_t)i;
+}
+__global__ void k_batch_flatten(int32_t* P, int32_t n, const int32_t* __restrict__ big,
+                                int32_t* __restrict__ root, int32_t* __restrict__ flag) {
+  if (big && !*big) return;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    int32_t r = uf_find(P, (int32_t)i);
+    root[i] = r;
+    flag[i] = (r == (int32_t)i);
+  }
+}
+__global__ void k_batch_labels(const int32_t* __restrict__ root, const int32_t* __restrict__ rank,
+                               int32_t n, const int64_t* __restrict__ goff, int G,
+                               const int32_t* __restrict__ big, int32_t* __restrict__ labels) {
+  if (big && !*big) return;
+  for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    int lo = 0, hi = G;  // last graph that starts at or before i
+    while (lo + 1 < hi) {
+      const int mid = (lo + hi) >> 1;
+      if (goff[mid] <= i) lo = mid; else hi = mid;
     }
+    const int64_t v0 = goff[lo];
+    labels[i] = rank[root[i]] - (v0 < n ? rank[v0] : 0);
+  }
+}
+
+// gout of every graph and the batch's totals: tot[0] kept edges, tot[2]
+// components (one atomic per workgroup; cleared by the caller).
+__global__ __launch_bounds__(256) void k_batch_out(int G, const int64_t* __restrict__ goff,
+                                                   const int64_t* __restrict__ seg,
+                                                   const GraphCut* __restrict__ cut, int in_lds,
+                                                   const int32_t* __restrict__ big,
+                                                   const int32_t* __restrict__ count, int32_t n,
+                                                   const int32_t* __restrict__ rank,
+                                                   const int32_t* __restrict__ total,
+                                                   int64_t* __restrict__ gout,
+                                                   int32_t* __restrict__ tot) {
+  __shared__ int32_t s_k[256 / kWave], s_c[256 / kWave];
+  const int g = blockIdx.x * 256 + threadIdx.x;
+  int32_t kept = 0, comps = 0;
+  if (g < G) {
+    const int64_t v0 = goff[g], v1 = goff[g + 1], have = seg[g + 1] - seg[g];
+    if (v1 > v0)
+      comps = in_lds && !*big ? count[g] : (v1 < n ? rank[v1] : *total) - rank[v0];
+    const int64_t k = cut[g].keep;
+    kept = (int32_t)(k < 0 ? 0 : (k < have ? k : have));
+    gout[4 * (int64_t)g + 0] = comps;
+    gout[4 * (int64_t)g + 1] = cut[g].labels_empty;
+    gout[4 * (int64_t)g + 2] = cut[g].nc_stable;
+    gout[4 * (int64_t)g + 3] = cut[g].err ? -1 : k;
+  }
+  kept = wave_sum(kept);
+  comps = wave_sum(comps);
+  if (lane_id() == 0) {
+    s_k[threadIdx.x / kWave] = kept;
+    s_c[threadIdx.x / kWave] = comps;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int q = 1; q < 256 / kWave; ++q) {
+      kept += s_k[q];
+      comps += s_c[q];
+    }
+    if (kept) atomicAdd(&tot[0], kept);
+    if (comps) atomicAdd(&tot[2], comps);
   }
 }
 
@@ -3052,14 +3247,15 @@ int sl_impl(const int32_t* dest, const W* weight, const int64_t* fe, const int32
 // where the reference raises ValueError}.
 // Graph offsets as the batched kernels read them: each clamped to [0, N]
 // (so no kernel indexes outside the union); bad[0] = 1 when the input was
-// not 0 = goff[0] <= ... <= goff[G] = N.
+// not 0 = goff[0] <= ... <= goff[G] = N (then also big[0], see k_seg_label).
 __global__ void k_goff_prep(const int64_t* __restrict__ in, int G, int32_t N,
-                            int64_t* __restrict__ out, int32_t* __restrict__ bad) {
+                            int64_t* __restrict__ out, int32_t* __restrict__ bad,
+                            int32_t* __restrict__ big) {
   for (int g = blockIdx.x * blockDim.x + threadIdx.x; g <= G; g += gridDim.x * blockDim.x) {
     const int64_t v = in[g];
     out[g] = v < 0 ? 0 : (v > N ? N : v);
     const bool ok = (g > 0 || v == 0) && (g < G || v == N) && (g == 0 || in[g - 1] <= v);
-    if (!ok) *bad = 1;
+    if (!ok) *bad = *big = 1;
   }
 }
 
@@ -3069,11 +3265,10 @@ __global__ void k_goff_prep(const int64_t* __restrict__ in, int G, int32_t N,
 // 4 graph passed as symmetric is not, 8 key wider than 64 bits,
 // 16 rounds not converged, 32 bad graph offsets.
 __global__ void k_batch_summary(const MstState* __restrict__ st, int enq,
-                                const int32_t* __restrict__ d_ncomp,
                                 const int64_t* __restrict__ seg_total,
                                 const int32_t* __restrict__ misc, int64_t* __restrict__ out) {
   if (threadIdx.x != 0 || blockIdx.x != 0) return;
-  out[0] = *d_ncomp;
+  out[0] = misc[2];
   out[1] = *seg_total;
   const RoundCtl c = st->ctl[enq & 1];
   out[2] = c.rounds;
@@ -3136,12 +3331,18 @@ int sl_batched_impl(const int32_t* dest, const W* weight, const int64_t* fe, con
   if (ar.overflow()) return fail(EAC_ERR_WORKSPACE, "sl_batched: workspace too small");
   if (!summary) summary = sum_ws;
   const size_t mark0 = ar.used;
-  EAC_TRY(fill<int32_t>(misc, 2, 0, s));
+  // misc: [0] kept edges, [1] bad offsets, [2] components, [3] a big graph
+  EAC_TRY(fill<int32_t>(misc, 4, 0, s));
+  const bool in_lds = N >= (int64_t)kSegMin * G;  // see k_seg_label
+  int64_t most = N;  // vertices of a graph, at most
   if (d_goff) {
-    k_goff_prep<<<grid_for(G + 1, 256), 256, 0, s>>>(d_goff, G, N, goff_ws, misc + 1);
+    k_goff_prep<<<grid_for(G + 1, 256), 256, 0, s>>>(d_goff, G, N, goff_ws, misc + 1, misc + 3);
     EAC_LAUNCH_CHECK();
   } else {
     if (graph_mode) return fail(EAC_ERR_ARG, "sl_batched: graph mode needs device goff");
+    most = 0;
+    for (int g = 0; g < G; ++g)
+      most = h_goff[g + 1] - h_goff[g] > most ? h_goff[g + 1] - h_goff[g] : most;
     EAC_HIP_CHECK(hipMemcpyAsync(goff_ws, h_goff, sizeof(int64_t) * (G + 1),
                                  hipMemcpyHostToDevice, s));
     EAC_HIP_CHECK(hipStreamSynchronize(s));  // h_goff may be pageable
@@ -3180,32 +3381,50 @@ int sl_batched_impl(const int32_t* dest, const W* weight, const int64_t* fe, con
   // seg[G] = present forest keys; they lead sk2, grouped by graph
   k_seg_bounds<<<grid_for(G + 1, 256), 256, 0, s>>>(gid_s, nf, G, seg);
   EAC_LAUNCH_CHECK();
-  EAC_TRY(fill<uint64_t>((uint64_t*)gmax, G, 0ull, s));
-  k_graph_wmax<W, HAS_OD><<<HAS_OD ? (G < 4096 ? G : 4096)
-                                    : grid_for(M, 1, resident_grid(k_graph_wmax<W, HAS_OD>, kGB)),
-                            kGB, 0, s>>>(weight, fe, od, goff, G, M, gmax);
-  EAC_LAUNCH_CHECK();
-  k_seg_cut<W><<<G < 4096 ? G : 4096, kGB, 0, s>>>(sk2, seg, goff, G, vb, fi.plan, gmax, rule,
-                                                  max_dist, n_clusters, cut);
-  EAC_LAUNCH_CHECK();
-  EAC_TRY(fill<int32_t>(misc, 1, 0, s));
-  if (nf > 0) {
-    k_seg_keep_flags<<<g1, kGB, 0, s>>>(gid_s, nf, G, seg, cut, B.flag);
-    EAC_LAUNCH_CHECK();
-    EAC_TRY((scan_excl<int32_t, int32_t>(B.flag, B.rank, nf, 0, misc, ar, s)));
-    ar.used = mark0;
-    k_compact_flagged<<<g1, kGB, 0, s>>>(sk2, B.flag, B.rank, nf, B.fkeys);
+  const bool want_max = max_dist < 0;
+  if (want_max) {
+    EAC_TRY(fill<uint64_t>((uint64_t*)gmax, G, 0ull, s));
+    k_graph_wmax<W, HAS_OD><<<HAS_OD ? (G < 4096 ? G : 4096)
+                                      : grid_for(M, 1, resident_grid(k_graph_wmax<W, HAS_OD>, kGB)),
+                              kGB, 0, s>>>(weight, fe, od, goff, G, M, gmax);
     EAC_LAUNCH_CHECK();
   }
+  k_seg_cut<W><<<G < 4096 ? G : 4096, kSegT, 0, s>>>(sk2, seg, goff, G, vb, fi.plan,
+                                                    want_max ? gmax : nullptr, rule, max_dist,
+                                                    n_clusters, cut, misc + 3);
+  EAC_LAUNCH_CHECK();
+  int32_t* const big = misc + 3;
   const int64_t ftiles = (N + kGTile - 1) / kGTile;
   int32_t* d_ncomp = B.tile_cnt + ftiles;
-  EAC_TRY(labels_from_keys(B.fkeys, nf, vb, N, B.hook, B.comp, B.flag, B.rank, labels, d_ncomp,
-                           ar, s, misc));
-  k_graph_base<<<grid_for(G + 1, 256), 256, 0, s>>>(labels, goff, G, d_ncomp, base);
+  if (in_lds) {
+    const size_t lds = 2 * (size_t)(most < 8 ? 8 : (most > kSegN ? kSegN : most));
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_seg_label),
+                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    // (the keys sorted by weight alone are not needed any more: room for pairs)
+    k_seg_label<<<G < 65536 ? G : 65536, kSegT, lds, s>>>(
+        sk2, seg, goff, G, vb, cut, big, reinterpret_cast<uint32_t*>(sk), labels, base);
+    EAC_LAUNCH_CHECK();
+  }
+  if (!in_lds || most > kSegN) {  // whether a graph is too big shows on the device
+    const int32_t* cond = in_lds ? big : nullptr;
+    const int gn = grid_for(N, 256, 4096);
+    k_batch_iota<<<gn, 256, 0, s>>>(B.hook, N, cond);
+    EAC_LAUNCH_CHECK();
+    if (nf > 0) {
+      k_batch_unite<<<g1, kGB, 0, s>>>(sk2, gid_s, nf, G, vb, seg, cut, cond, B.hook);
+      EAC_LAUNCH_CHECK();
+    }
+    k_batch_flatten<<<gn, 256, 0, s>>>(B.hook, N, cond, B.comp, B.flag);
+    EAC_LAUNCH_CHECK();
+    EAC_TRY((scan_excl<int32_t, int32_t>(B.flag, B.rank, N, 0, d_ncomp, ar, s)));
+    ar.used = mark0;
+    k_batch_labels<<<gn, 256, 0, s>>>(B.comp, B.rank, N, goff, G, cond, labels);
+    EAC_LAUNCH_CHECK();
+  }
+  k_batch_out<<<grid_for(G, 256), 256, 0, s>>>(G, goff, seg, cut, in_lds, big, base, N, B.rank,
+                                               d_ncomp, gout, misc + 0);
   EAC_LAUNCH_CHECK();
-  k_graph_sub<<<G < 4096 ? G : 4096, 256, 0, s>>>(labels, goff, G, base, cut, gout);
-  EAC_LAUNCH_CHECK();
-  k_batch_summary<<<1, 64, 0, s>>>(B.st, fi.enq, d_ncomp, seg + G, misc, summary);
+  k_batch_summary<<<1, 64, 0, s>>>(B.st, fi.enq, seg + G, misc, summary);
   EAC_LAUNCH_CHECK();
   if (graph_mode) return EAC_OK;
   int64_t hs[5];
