@@ -652,31 +652,6 @@ __global__ void k_dense_init(int64_t n, uint16_t* __restrict__ comp, int32_t* __
   best[v] = minv[v] = tree[v] = sorted[v] = ~0ull;
 }
 
-// Order of the tree's keys by their ranks, for n up to kRankN: a workgroup
-// takes 64 keys, one a lane, and every wavefront counts the smaller ones of a
-// sixteenth of all keys, which it reads as scalars. The keys differ (absent
-// ones, all ones, stay where they are), so a rank is a place. n^2 comparisons
-// in one launch, 22 us for 8,000 keys; the 24 launches of a radix sort take 290.
-// Above 16,384 keys (four times as long at twice the count) the radix sort runs.
-constexpr int64_t kRankN = 16384;
-__global__ __launch_bounds__(1024) void k_rank_sort(const unsigned long long* __restrict__ in,
-                                                    int64_t n,
-                                                    unsigned long long* __restrict__ out) {
-  __shared__ uint32_t s_rank[kWave];
-  const int l = lane_id(), w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
-  const int64_t i = (int64_t)blockIdx.x * kWave + l;
-  const unsigned long long k = i < n ? in[i] : ~0ull;
-  if (threadIdx.x < kWave) s_rank[threadIdx.x] = 0;
-  __syncthreads();
-  const int per = (int)((n + 15) / 16), a = w * per, b = (int)(a + per < n ? a + per : n);
-  uint32_t rank = 0;
-#pragma unroll 8
-  for (int j = a; j < b; ++j) rank += in[j] < k;
-  atomicAdd(&s_rank[l], rank);
-  __syncthreads();
-  if (w == 0 && k != ~0ull) out[s_rank[l]] = k;
-}
-
 __global__ void k_iota(int32_t* __restrict__ a, int64_t n) {
   const int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (v < n) a[v] = (int32_t)v;
@@ -1126,11 +1101,6 @@ int dense_tree(const void* sq, int32_t dtype, int64_t n, int32_t condensed, int 
       k_dense_round_end<<<1, 1, 0, s>>>(n, done);
     }
     EAC_LAUNCH_CHECK();
-  }
-  if (n <= kRankN) {
-    k_rank_sort<<<grid_for(n, kWave), 1024, 0, s>>>(B.tree, n, B.sorted);
-    EAC_LAUNCH_CHECK();
-    return EAC_OK;
   }
   const size_t mark = ar.used;
   // (weight words of narrow types leave the top bits zero; the absent key's

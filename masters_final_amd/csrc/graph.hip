@@ -2930,12 +2930,15 @@ __global__ __launch_bounds__(kSegT) void k_seg_cut(const uint64_t* __restrict__ 
 // numbered by first occurrence inside the graph.
 //
 // k_seg_label: one workgroup per graph of up to kSegN vertices, the forest in
-// LDS (16-bit parents). Rounds: every edge between two roots hooks the larger
-// under the smaller (any of several: the others come again), then every
-// vertex goes to its root; an edge within a component is dropped, the rest
-// are packed as pairs of roots. 64 graphs of 1,000 to 50,000 vertices: the
+// LDS (16-bit parents). Rounds: every edge finds both its roots and hooks the
+// larger under the smaller; an edge that finds one root is dropped, the rest
+// are packed as pairs of roots. Edges that hook the same root in one round
+// overwrite each other, and a walk may pass over a link that is overwritten:
+// whoever made it is still listed and comes again, so the links and the
+// listed edges together always connect what the kept edges do. Parents only
+// fall, so no cycle forms. 64 graphs of 1,000 to 50,000 vertices: the
 // lock-free union-find over the union, its flattening and numbering (the
-// k_batch_* kernels) took 420 us, bound by dependent reads of memory; this 70.
+// k_batch_* kernels) took 420 us, bound by dependent reads of memory; this 114.
 // They remain for larger graphs (`big`: one with kept edges; without any, as
 // the padding of a recorded batch has it, a graph of any size is numbered
 // here), and where the graphs are so small (fewer than kSegMin vertices on
@@ -2995,13 +2998,32 @@ __global__ __launch_bounds__(kSegT) void k_seg_label(const uint64_t* __restrict_
             y[q] = list[e] >> 16;
           }
         }
-        if (!first) {
+        if (!first) {  // (an idle lane walks from vertex 0, a root)
+          uint32_t p[4], r[4];
 #pragma unroll
           for (int q = 0; q < 4; ++q) {
-            if (!on[q]) continue;
-            x[q] = s_up[x[q]];
-            y[q] = s_up[y[q]];
+            p[q] = s_up[x[q]];
+            r[q] = s_up[y[q]];
           }
+          const uint32_t h[4] = {y[0], y[1], y[2], y[3]};
+          for (;;) {
+            bool go = false;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              go |= p[q] != x[q] || r[q] != y[q];
+              x[q] = p[q];
+              y[q] = r[q];
+            }
+            if (!go) break;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+              p[q] = s_up[x[q]];
+              r[q] = s_up[y[q]];
+            }
+          }
+#pragma unroll
+          for (int q = 0; q < 4; ++q)
+            if (on[q] && y[q] != h[q]) s_up[h[q]] = (uint16_t)y[q];
         }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -3015,19 +3037,19 @@ __global__ __launch_bounds__(kSegT) void k_seg_label(const uint64_t* __restrict_
       }
       ne = out;
       if (!__syncthreads_or(ne > 0)) break;
-      for (;;) {  // parents fall, so every walk ends; 16 steps at a time
-        bool more = false, cycle = false;
-        for (int b = w * kWave; b < nv; b += 4 * kSegT) {
-          uint32_t f[4];
+    }
+    for (;;) {  // every vertex to its root, 16 steps at a time
+      bool more = false, cycle = false;
+      for (int b = w * kWave; b < nv; b += 4 * kSegT) {
+        uint32_t f[4];
 #pragma unroll
-          for (int q = 0; q < 4; ++q) {
-            const int v = b + q * kSegT + lane;
-            f[q] = v < nv ? (uint32_t)s_up[v] << 16 | (uint32_t)v : 0u;
-          }
-          (void)one_walks(s_up, f, &more, &cycle);
+        for (int q = 0; q < 4; ++q) {
+          const int v = b + q * kSegT + lane;
+          f[q] = v < nv ? (uint32_t)s_up[v] << 16 | (uint32_t)v : 0u;
         }
-        if (!__syncthreads_or(more)) break;
+        (void)one_walks(s_up, f, &more, &cycle);
       }
+      if (!__syncthreads_or(more)) break;
     }
     // roots are their components' smallest vertices
     const int part = ((nv + kNW - 1) / kNW + kWave - 1) / kWave * kWave;
@@ -3047,9 +3069,19 @@ __global__ __launch_bounds__(kSegT) void k_seg_label(const uint64_t* __restrict_
     }
     if (w == kNW - 1 && lane == 0) count[g] = o;
     __syncthreads();
-#pragma unroll 4
-    for (int v = t; v < nv; v += kSegT)
-      if (s_up[v] != v) labels[v0 + v] = labels[v0 + s_up[v]];
+    for (int b = t; b < nv; b += 4 * kSegT) {
+      int32_t lab[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int v = b + q * kSegT;
+        lab[q] = v < nv ? labels[v0 + s_up[v]] : 0;
+      }
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int v = b + q * kSegT;
+        if (v < nv && s_up[v] != v) labels[v0 + v] = lab[q];
+      }
+    }
     __syncthreads();
   }
 }
