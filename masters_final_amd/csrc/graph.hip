@@ -640,21 +640,25 @@ __device__ __forceinline__ RoundCtl next_ctl(RoundCtl c, int r, unsigned int had
 // Per-block table of (root, lightest key) pairs: cross edges of one block
 // that share a root meet in LDS, and each distinct root costs one global
 // atomicMin per block (a component touching most edges -- the giant one --
-// would otherwise take one serialised atomic per edge). A root whose slot
-// is taken goes straight to the global atomic: while components are many
-// (the first rounds, the routing passes) the table is crowded, and probing
-// further slots costs more LDS atomics than the global ones it saves
-// (measured on the 1M-vertex k-NN graph: 8 probes 0.83 ms per call, 1 probe
-// 0.79; 512 to 1024 slots are equal, 256 or 2048 and more are slower).
+// would otherwise take one serialised atomic per edge). While components are
+// many (the first rounds) the table is crowded, and a root whose slot is taken
+// goes straight to the global atomic: probing further slots costs more LDS
+// atomics than the global ones it saves (1M-vertex k-NN graph, 8 probes in
+// every round 0.83 ms per call, 1 probe 0.79; 512 to 1024 slots are equal, 256
+// or 2048 and more are slower). From round kProbeRound on components are few
+// and the table has room, but two of them that share a slot and touch most
+// edges would send every edge of one to its single word in memory: there a
+// taken slot is passed over (such a round of 83,000 keys: 59 -> 26 us). A
+// routing pass meets many components again.
 // The table has four slots per thread (1024 for the 256-thread filter
 // block, 4096 for the 1024-thread one).
-constexpr int kMinProbes = 1;  // table slots tried before the direct atomic
+constexpr int kProbeRound = 3, kMinProbes = 4;
 template <int LOGS>
 __device__ __forceinline__ void min_insert(int32_t* s_root, unsigned long long* s_min,
                                            int32_t root, uint64_t key,
-                                           unsigned long long* best) {
+                                           unsigned long long* best, int probes) {
   uint32_t h = ((uint32_t)root * 2654435761u) >> (32 - LOGS);
-  for (int p = 0; p < kMinProbes; ++p, h = (h + 1) & ((1u << LOGS) - 1)) {
+  for (int p = 0; p < probes; ++p, h = (h + 1) & ((1u << LOGS) - 1)) {
     const int32_t k = atomicCAS(&s_root[h], -1, root);
     if (k == -1 || k == root) {
       atomicMin(&s_min[h], (unsigned long long)key);
@@ -671,7 +675,7 @@ __device__ __forceinline__ void min_insert(int32_t* s_root, unsigned long long* 
 template <int LOGS>
 __device__ __forceinline__ void wave_min_insert(int32_t* s_root, unsigned long long* s_min,
                                                 int32_t root, uint64_t key, bool active,
-                                                unsigned long long* best) {
+                                                unsigned long long* best, int probes) {
   uint64_t pend = __ballot(active);
   for (int it = 0; it < 2 && pend; ++it) {
     const int leader = __ffsll((unsigned long long)pend) - 1;
@@ -686,11 +690,11 @@ __device__ __forceinline__ void wave_min_insert(int32_t* s_root, unsigned long l
       const uint64_t o = __shfl_xor(v, off, kWave);
       v = o < v ? o : v;
     }
-    if (lane_id() == leader) min_insert<LOGS>(s_root, s_min, R, v, best);
+    if (lane_id() == leader) min_insert<LOGS>(s_root, s_min, R, v, best, probes);
     pend &= ~__ballot(mine);
     if (mine) active = false;
   }
-  if (active) min_insert<LOGS>(s_root, s_min, root, key, best);
+  if (active) min_insert<LOGS>(s_root, s_min, root, key, best, probes);
 }
 
 // Keys per lane per step of the filter (their root lookups in flight together).
@@ -698,6 +702,82 @@ __device__ __forceinline__ void wave_min_insert(int32_t* s_root, unsigned long l
 #define EAC_FILTER_KEYS 4
 #endif
 constexpr int kFilterKeys = EAC_FILTER_KEYS;
+
+// One step of a light list: the roots x[2 q], x[2 q + 1] of the ends of the Q
+// keys after this round's hooks, keep[q] where they differ, the kept keys as
+// candidates of their roots. P[x] is x's root when the round started (the
+// ends of a listed key are written back here) and that root's parent is its
+// root after this round's hooks.
+template <int LOGS>
+__device__ __forceinline__ void light_step(const uint64_t (&k)[kFilterKeys], int vb, int32_t* P,
+                                           int32_t* s_root, unsigned long long* s_min,
+                                           unsigned long long* __restrict__ best, int probes,
+                                           bool (&keep)[kFilterKeys], bool* any_cand) {
+  constexpr int Q = kFilterKeys;
+  int32_t x[2 * Q], p[2 * Q], rt[2 * Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    int32_t a = 0, b = 0;
+    if (k[q] != kInf) unpack_ends(k[q], vb, &a, &b);
+    x[2 * q] = a;
+    x[2 * q + 1] = b;
+  }
+#pragma unroll
+  for (int i = 0; i < 2 * Q; ++i) p[i] = P[x[i]];
+#pragma unroll
+  for (int i = 0; i < 2 * Q; ++i) rt[i] = P[p[i]];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) keep[q] = k[q] != kInf && rt[2 * q] != rt[2 * q + 1];
+  // a kept key's ends point at their roots: the next round's hook reads
+  // them with one load
+#pragma unroll
+  for (int i = 0; i < 2 * Q; ++i)
+    if (keep[i / 2] && rt[i] != p[i]) P[x[i]] = rt[i];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) *any_cand |= keep[q];
+#pragma unroll
+  for (int i = 0; i < 2 * Q; ++i)
+    wave_min_insert<LOGS>(s_root, s_min, rt[i], k[i / 2], keep[i / 2], best, probes);
+}
+
+// Filters up to kFilterKeys chunks of at most 64 keys each, a chunk per key
+// of a lane. After a round or two most chunks of a graph with many heavy
+// entries hold a few dozen light keys, and a wavefront that takes one at a
+// time has most of its lanes and nearly all of its loads in flight idle.
+template <int LOGS>
+__device__ __forceinline__ void filter_small(uint64_t* __restrict__ list, int32_t* __restrict__ cnt,
+                                             const int32_t* s_work, const int32_t* s_work_n,
+                                             int at, int end, int64_t first, int64_t G, int vb,
+                                             int32_t* P, int32_t* s_root,
+                                             unsigned long long* s_min,
+                                             unsigned long long* __restrict__ best, int probes,
+                                             unsigned long long* sum_in,
+                                             unsigned long long* sum_out, bool* any_cand) {
+  const int lane = lane_id();
+  constexpr int Q = kFilterKeys;
+  uint64_t k[Q];
+  int64_t cc[Q];
+  bool keep[Q];
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    const bool in = at + q < end;  // uniform
+    cc[q] = first + (int64_t)s_work[in ? at + q : at] * G;
+    k[q] = in && lane < s_work_n[in ? at + q : at]
+               ? __builtin_nontemporal_load(list + cc[q] * kGTile + lane) : kInf;
+  }
+  light_step<LOGS>(k, vb, P, s_root, s_min, best, probes, keep, any_cand);
+#pragma unroll
+  for (int q = 0; q < Q; ++q) {
+    if (at + q >= end) continue;  // uniform
+    const uint64_t m = __ballot(keep[q]);
+    if (keep[q]) list[cc[q] * kGTile + __popcll(m & ((1ull << lane) - 1ull))] = k[q];
+    if (lane == 0) {
+      cnt[cc[q]] = __popcll(m);
+      *sum_in += (unsigned long long)s_work_n[at + q];
+      *sum_out += (unsigned long long)__popcll(m);
+    }
+  }
+}
 
 // Filters one chunk `cc` (n_in keys) of `list` with one wavefront. ROUTE
 // (the first round of a weight level): `list` is the heavy list, whose cross
@@ -712,7 +792,7 @@ __device__ __forceinline__ void filter_chunk(uint64_t* __restrict__ list,
                                              int32_t* __restrict__ cnt_to, int64_t cc,
                                              int32_t n_in, uint64_t lim, int vb, int32_t* P,
                                              int32_t* s_root, unsigned long long* s_min,
-                                             unsigned long long* __restrict__ best,
+                                             unsigned long long* __restrict__ best, int probes,
                                              unsigned long long* sum_in,
                                              unsigned long long* sum_out, bool* any_cand) {
   const int lane = lane_id();
@@ -738,20 +818,18 @@ __device__ __forceinline__ void filter_chunk(uint64_t* __restrict__ list,
       const int e = base + Q * kWave + q * kWave + lane;
       kn[q] = e < n_in ? __builtin_nontemporal_load(lc + e) : kInf;
     }
-    int32_t x[2 * Q];  // roots of the endpoints of the Q keys
-#pragma unroll
-    for (int q = 0; q < Q; ++q) {
-      int32_t a = 0, b = 0;
-      if (k[q] != kInf) unpack_ends(k[q], vb, &a, &b);
-      x[2 * q] = a;
-      x[2 * q + 1] = b;
-    }
-    // Light keys: P[x] is x's root when the round started (their ends are
-    // written back below) and that root's parent is its root after this
-    // round's hooks. A routing pass follows a round without hooks, whose
-    // hook pass left P flat.
+    // A routing pass follows a round without hooks, whose hook pass left P
+    // flat.
     bool keep[Q], cand[Q];
     if (ROUTE) {
+      int32_t x[2 * Q];  // roots of the endpoints of the Q keys
+#pragma unroll
+      for (int q = 0; q < Q; ++q) {
+        int32_t a = 0, b = 0;
+        if (k[q] != kInf) unpack_ends(k[q], vb, &a, &b);
+        x[2 * q] = a;
+        x[2 * q + 1] = b;
+      }
 #pragma unroll
       for (int i = 0; i < 2 * Q; ++i) x[i] = P[x[i]];
 #pragma unroll
@@ -759,31 +837,14 @@ __device__ __forceinline__ void filter_chunk(uint64_t* __restrict__ list,
         keep[q] = k[q] != kInf && x[2 * q] != x[2 * q + 1];
         cand[q] = keep[q] && (k[q] >> (2 * vb)) < lim;
       }
+#pragma unroll
+      for (int q = 0; q < Q; ++q) *any_cand |= cand[q];
+#pragma unroll
+      for (int i = 0; i < 2 * Q; ++i)
+        wave_min_insert<LOGS>(s_root, s_min, x[i], k[i / 2], cand[i / 2], best, probes);
     } else {
-      int32_t p[2 * Q];
-#pragma unroll
-      for (int i = 0; i < 2 * Q; ++i) p[i] = P[x[i]];
-      int32_t rt[2 * Q];
-#pragma unroll
-      for (int i = 0; i < 2 * Q; ++i) rt[i] = P[p[i]];
-#pragma unroll
-      for (int q = 0; q < Q; ++q) {
-        keep[q] = k[q] != kInf && rt[2 * q] != rt[2 * q + 1];
-        cand[q] = keep[q];
-      }
-      // a kept key's ends point at their roots: the next round's hook
-      // reads them with one load
-#pragma unroll
-      for (int i = 0; i < 2 * Q; ++i) {
-        if (keep[i / 2] && rt[i] != p[i]) P[x[i]] = rt[i];
-        x[i] = rt[i];
-      }
+      light_step<LOGS>(k, vb, P, s_root, s_min, best, probes, keep, any_cand);
     }
-#pragma unroll
-    for (int q = 0; q < Q; ++q) *any_cand |= cand[q];
-#pragma unroll
-    for (int i = 0; i < 2 * Q; ++i)
-      wave_min_insert<LOGS>(s_root, s_min, x[i], k[i / 2], cand[i / 2], best);
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
       if (ROUTE) {
@@ -831,7 +892,7 @@ __global__ __launch_bounds__(RB) void k_round(int r, uint64_t* __restrict__ ligh
   __shared__ unsigned long long s_min[kSlots];
   __shared__ unsigned long long s_io[2 * (RB / kWave)];
   __shared__ int32_t s_work[kOwnBatch], s_work_n[kOwnBatch];
-  __shared__ int s_take, s_nwork;
+  __shared__ int s_take, s_nwork, s_nsmall;
   const RoundCtl prev = ctl[r & 1];
   const unsigned int had = had_edge[r];
   // The first batch of chunk counts of both lists is read with the control
@@ -857,45 +918,58 @@ __global__ __launch_bounds__(RB) void k_round(int r, uint64_t* __restrict__ ligh
   // Workgroup b owns chunks b, b + G, b + 2G, ... (G = grid): the key
   // density of the list varies along it, and interleaving gives every
   // workgroup a sample of the whole list. Per batch of up to 64 owned
-  // chunks, the first wavefront lists the non-empty ones in LDS and the
-  // wavefronts take them one at a time from an LDS counter, so a wavefront
-  // that drew light chunks takes more and empty chunks cost nothing.
+  // chunks, the first wavefront lists the non-empty ones in LDS (the small
+  // ones of a light list first) and the wavefronts take one, or kFilterKeys
+  // small ones, at a time from an LDS counter, so a wavefront that drew light
+  // chunks takes more and empty chunks cost nothing.
   uint64_t* const list = route ? heavy : light;
   int32_t* const cnt = route ? cnt_heavy : cnt_light;
   const uint64_t lim = route ? plan->lim[c.phase] : kInf;
   unsigned long long sum_in = 0, sum_out = 0;
   bool any_cand = false;
+  const int probes = r >= kProbeRound && !route ? kMinProbes : 1;
   for (int64_t b0 = 0; b0 < owned; b0 += kOwnBatch) {
     if (threadIdx.x < kWave) {
       const int64_t j = b0 + lane;
       const int64_t cc = blockIdx.x + j * G;
       int32_t nk = b0 == 0 ? (route ? pre_h : pre_l) : (j < owned ? cnt[cc] : 0);
       nk = nk < 0 ? 0 : (nk > kGTile ? kGTile : nk);
-      const uint64_t m = __ballot(nk > 0);
+      const bool small = !route && nk > 0 && nk <= kWave;
+      const uint64_t ms = __ballot(small), mb = __ballot(nk > 0 && !small);
       if (nk > 0) {
-        const int at = __popcll(m & ((1ull << lane) - 1ull));
+        const uint64_t below = (1ull << lane) - 1ull;
+        const int at = small ? __popcll(ms & below) : __popcll(ms) + __popcll(mb & below);
         s_work[at] = (int32_t)j;
         s_work_n[at] = nk;
       }
       if (lane == 0) {
         s_take = 0;
-        s_nwork = __popcll(m);
+        s_nsmall = __popcll(ms);
+        s_nwork = __popcll(ms) + __popcll(mb);
       }
     }
     __syncthreads();
+    const int nsmall = s_nsmall, nbig = s_nwork - nsmall;
     for (;;) {
       int w = 0;
       if (lane == 0) w = atomicAdd(&s_take, 1);
       w = __builtin_amdgcn_readfirstlane(w);
-      if (w >= s_nwork) break;
+      if (w >= nbig) {  // the large ones first
+        const int at = (w - nbig) * kFilterKeys;
+        if (at >= nsmall) break;
+        filter_small<LOGS>(list, cnt, s_work, s_work_n, at, nsmall, blockIdx.x, G, vb, P, s_root,
+                           s_min, best, probes, &sum_in, &sum_out, &any_cand);
+        continue;
+      }
+      w += nsmall;
       const int64_t cc = blockIdx.x + (int64_t)s_work[w] * G;
       const int32_t n_in = s_work_n[w];
       if (route)
         filter_chunk<true, LOGS>(list, cnt, light, cnt_light, cc, n_in, lim, vb, P, s_root,
-                                 s_min, best, &sum_in, &sum_out, &any_cand);
+                                 s_min, best, probes, &sum_in, &sum_out, &any_cand);
       else
         filter_chunk<false, LOGS>(list, cnt, nullptr, nullptr, cc, n_in, lim, vb, P, s_root,
-                                  s_min, best, &sum_in, &sum_out, &any_cand);
+                                  s_min, best, probes, &sum_in, &sum_out, &any_cand);
     }
     __syncthreads();
   }
