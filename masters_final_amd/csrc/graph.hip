@@ -2361,13 +2361,15 @@ int mst_forest(MstBuffers& B, int32_t n, int32_t* d_nf, hipStream_t s) {
 
 // Rounds enqueued before the first read-back: about what a graph of this size
 // needs, and one more for every further weight level (each ends with a round
-// that finds nothing). One round too few costs the tail once more and two
+// that finds nothing; a graph dense enough for four, a co-association matrix
+// say, needs three more: 15 rounds at 10,000 vertices). One round too few costs the tail once more and two
 // host reads (100 us of 1,200 at a million vertices of degree 40, which need
 // 16), one too many the few microseconds of two launches that return at once.
 inline int first_batch(int32_t n, int64_t m, int symmetric) {
   if (tune_value(EAC_TUNE_FIRST_BATCH) > 0) return tune_value(EAC_TUNE_FIRST_BATCH);
   const int vb = vbits_for(n), base = vb * 3 / 4 > 6 ? vb * 3 / 4 : 6;
-  return base + split_plan(n, m, symmetric).levels - 1;
+  const int levels = split_plan(n, m, symmetric).levels;
+  return base + levels - 1 + (levels > 3 ? 3 : 0);
 }
 
 // Boruvka rounds up to the forest key list (shared by the lifetime cut and
@@ -3024,7 +3026,7 @@ __global__ __launch_bounds__(kSegT) void k_seg_label(const uint64_t* __restrict_
                                                      const int32_t* __restrict__ big,
                                                      uint32_t* __restrict__ pairs,
                                                      int32_t* __restrict__ labels,
-                                                     int32_t* __restrict__ count) {
+                                                     int32_t* __restrict__ count, int quiet) {
   if (*big) return;
   extern __shared__ __align__(16) uint16_t s_up[];
   constexpr int kNW = kSegT / kWave;
@@ -3036,6 +3038,7 @@ __global__ __launch_bounds__(kSegT) void k_seg_label(const uint64_t* __restrict_
     const int nv = goff[g + 1] > v0 ? (int)(goff[g + 1] - v0) : 0;
     const int64_t have = seg[g + 1] - seg[g];
     const int64_t kept = cut[g].keep < 0 ? 0 : (cut[g].keep < have ? cut[g].keep : have);
+    if (quiet && (cut[g].err || cut[g].labels_empty)) continue;  // (uniform) no labels then
     if (kept == 0) {  // uniform
 #pragma unroll 4
       for (int v = t; v < nv; v += kSegT) labels[v0 + v] = v;
@@ -3343,6 +3346,119 @@ int sl_impl(const int32_t* dest, const W* weight, const int64_t* fe, const int32
   return EAC_OK;
 }
 
+// One graph of up to kSegN vertices: the same cut from the batch's kernels
+// (a batch of one), enqueued behind the rounds without a read-back. The form
+// above reads five times between its kernels, 14 us each (the whole EAC of
+// 10,000 points: 1175 -> 1083 us); it stays for larger graphs, whose forest
+// one workgroup would take too long over.
+struct SlRecord {
+  GraphCut cut;
+  int64_t goff[2], seg[2];
+  int32_t misc[4];  // [3]: never set here (see k_seg_label)
+  int32_t count, pad;
+};
+// seg = {0, keys before the first absent one}: one wavefront, 64 probes a step.
+__global__ __launch_bounds__(kWave) void k_key_bounds(const uint64_t* __restrict__ sk, int32_t n,
+                                                      SlRecord* __restrict__ rec) {
+  int lo = 0, hi = n;  // sk[lo - 1] present, sk[hi] absent
+  while (lo < hi) {
+    const int step = (hi - lo + kWave - 1) / kWave, at = lo + lane_id() * step;
+    const bool in = at < hi && sk[at] != kInf;
+    const int k = __popcll(__ballot(in));  // the probes before the bound
+    const int next = k ? lo + (k - 1) * step + 1 : lo;
+    hi = lo + k * step < hi ? lo + k * step : hi;
+    lo = next;
+  }
+  if (lane_id() == 0) {
+    rec->goff[0] = 0;
+    rec->goff[1] = n;
+    rec->seg[0] = 0;
+    rec->seg[1] = lo;
+    rec->misc[3] = 0;
+    rec->count = 0;
+  }
+}
+
+template <typename W, bool HAS_OD>
+int sl_small(const int32_t* dest, const W* weight, const int64_t* fe, const int32_t* od,
+             int32_t n, int64_t m, int symmetric, int rule, double max_dist, int32_t n_clusters,
+             int32_t* labels, int64_t* h_out, void* ws, size_t ws_bytes, hipStream_t s) {
+  Arena ar(ws, ws_bytes);
+  MstBuffers B = carve_mst(ar, n, m, symmetric);
+  uint64_t* sk = ar.take<uint64_t>(n);
+  SlRecord* rec = ar.take<SlRecord>(1);
+  if (ar.overflow()) return fail(EAC_ERR_WORKSPACE, "sl_lifetime: workspace too small");
+  const size_t mark = ar.used;
+  const int vb = vbits_for(n);
+  const int64_t ftiles = (n + kGTile - 1) / kGTile;
+  int32_t* d_nf = B.tile_cnt + ftiles;
+  MstRecs recs;
+  EAC_TRY((mst_begin<W, HAS_OD>(dest, weight, fe, od, n, m, symmetric, B, recs, s)));
+  const bool one = one_fits(n, m);
+  int key_bits = 8 * (int)sizeof(W) + 2 * vb;
+  key_bits = key_bits < 64 ? key_bits : 64;
+  const size_t lds = 2 * (size_t)(n < 8 ? 8 : n);
+  (void)hipFuncSetAttribute(reinterpret_cast<const void*>(k_seg_label),
+                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  MstState hs;
+  SlRecord hr;
+  int enq = 0;
+  for (int batch = first_batch(n, m, symmetric);; batch = 4) {
+    if (one) {
+      enq = kMaxRounds;
+      EAC_TRY(mst_one(B, n, enq, d_nf, nullptr, recs, s));
+    } else {
+      enq = mst_rounds(B, n, enq, batch, recs, s);
+      EAC_TRY(mst_forest(B, n, d_nf, s));
+    }
+    if (rule == 0) {
+      k_drop_zero<W><<<grid_for(n, kGB), kGB, 0, s>>>(B.fkeys, n, vb, &B.st->plan);
+      EAC_LAUNCH_CHECK();
+    }
+    ar.used = mark;
+    // canonical (w, min, max) order = ascending key order, absent keys last
+    EAC_TRY((radix_sort<uint64_t, NoValue>(B.fkeys, sk, nullptr, nullptr, n, 0, key_bits, ar, s)));
+    ar.used = mark;
+    k_key_bounds<<<1, kWave, 0, s>>>(sk, n, rec);
+    EAC_LAUNCH_CHECK();
+    k_seg_cut<W><<<1, kSegT, 0, s>>>(sk, rec->seg, rec->goff, 1, vb, &B.st->plan,
+                                     max_dist < 0 ? &B.st->plan.whi : nullptr, rule, max_dist,
+                                     n_clusters, &rec->cut, &rec->misc[3]);
+    EAC_LAUNCH_CHECK();
+    k_seg_label<<<1, kSegT, lds, s>>>(sk, rec->seg, rec->goff, 1, vb, &rec->cut, &rec->misc[3],
+                                      reinterpret_cast<uint32_t*>(B.fkeys), labels, &rec->count,
+                                      1);
+    EAC_LAUNCH_CHECK();
+    const size_t head = prof_on() ? kStateHead : kCtlHead, at = (head + 15) & ~size_t(15);
+    char* pin = static_cast<char*>(pinned_scratch(at + sizeof(hr)));
+    if (!pin) return fail(EAC_ERR_HIP, "pinned host allocation failed");
+    EAC_HIP_CHECK(hipMemcpyAsync(pin, B.st, head, hipMemcpyDeviceToHost, s));
+    EAC_HIP_CHECK(hipMemcpyAsync(pin + at, rec, sizeof(hr), hipMemcpyDeviceToHost, s));
+    EAC_HIP_CHECK(hipStreamSynchronize(s));
+    memcpy(&hs, pin, head);
+    memcpy(&hr, pin + at, sizeof(hr));
+    bool active = false;
+    EAC_TRY(mst_check(hs, enq, vb, &active));
+    if (!active) break;
+  }
+  mst_prof_bytes(hs, enq, n, B.nchunks, recs);
+  prof_flush();
+  if (hr.cut.err)
+    return fail(EAC_ERR_VALUE, rule == 1 ? "sl_mst_lifetime: fewer than 2 forest edges "
+                                           "(numpy argmax of an empty array)"
+                                         : "sp_sl_lifetime: lifetime rule undefined (fewer "
+                                           "than 2 forest edges or no zero lifetime)");
+  if (h_out) {
+    h_out[0] = hr.cut.labels_empty ? 1 : hr.count;
+    h_out[1] = hr.cut.labels_empty;
+    h_out[2] = hr.cut.nc_stable;
+    h_out[3] = hr.cut.keep;
+    h_out[4] = hr.seg[1];
+    h_out[5] = hs.ctl[enq & 1].rounds;
+  }
+  return EAC_OK;
+}
+
 // Many independent graphs given as one disjoint union (graph g owns the
 // vertex range [goff[g], goff[g+1]) and its rows): one Boruvka run over the
 // union (keys on global ids keep each graph's own (w, min, max) order, so
@@ -3508,7 +3624,7 @@ int sl_batched_impl(const int32_t* dest, const W* weight, const int64_t* fe, con
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     // (the keys sorted by weight alone are not needed any more: room for pairs)
     k_seg_label<<<G < 65536 ? G : 65536, kSegT, lds, s>>>(
-        sk2, seg, goff, G, vb, cut, big, reinterpret_cast<uint32_t*>(sk), labels, base);
+        sk2, seg, goff, G, vb, cut, big, reinterpret_cast<uint32_t*>(sk), labels, base, 0);
     EAC_LAUNCH_CHECK();
   }
   if (!in_lds || most > kSegN) {  // whether a graph is too big shows on the device
@@ -3605,6 +3721,9 @@ struct SlRun {
                  int32_t n, int64_t m, int symmetric, int rule, double max_dist,
                  int32_t n_clusters, int32_t* labels, int64_t* h_out, void* ws, size_t ws_bytes,
                  hipStream_t s) {
+    if (n <= kSegN)
+      return sl_small<W, HAS_OD>(dest, (const W*)weight, fe, od, n, m, symmetric, rule, max_dist,
+                                 n_clusters, labels, h_out, ws, ws_bytes, s);
     return sl_impl<W, HAS_OD>(dest, (const W*)weight, fe, od, n, m, symmetric, rule, max_dist,
                               n_clusters, labels, h_out, ws, ws_bytes, s);
   }
@@ -3662,7 +3781,7 @@ extern "C" int eac_boruvka_mst(const int32_t* dest, const void* weight, int32_t 
 extern "C" size_t eac_sl_lifetime_workspace_bytes(int32_t n, int64_t m) {
   size_t b = eac_boruvka_workspace_bytes(n, m);
   b += ((size_t)(n < 1 ? 1 : n) * 8 + 255) & ~size_t(255);
-  b += 512 + radix_sort_ws_bytes(n < 1 ? 1 : n, 8, 0);
+  b += 1024 + radix_sort_ws_bytes(n < 1 ? 1 : n, 8, 0);
   return b;
 }
 

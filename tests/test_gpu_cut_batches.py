@@ -82,3 +82,36 @@ def test_batches(torch, sizes, deg, rule, max_dist):
         assert np.array_equal(go.cpu().numpy(), want_g)
         assert inf["kept_edges"] == info["kept_edges"]
     cg.close()
+
+
+@pytest.mark.parametrize("n", [2, 3, 64, 16_000, 16_001, 65_536, 65_537])
+def test_single_graph_forms(torch, n):
+    """One graph at the limits of the forms, with zero weights, against the
+    oracle's rules."""
+    from masters_final_amd._lib import EACError
+    from masters_final_amd.graph.singlelink import lifetime_cut
+    from oracle import oracle as O
+    g = synth.random_graph(n, 3, n, wmax=6, n_isolated=n // 50, n_parts=1 + n // 3000)
+    rows = np.repeat(np.arange(n), np.diff(g["indptr"]))
+    g["weight"][(rows + g["dest"]) % 11 == 0] = 0
+    u, v, w, _ = O.csr_edges(g["dest"], g["weight"], g["indptr"][:-1], np.diff(g["indptr"]))
+    if not len(u):
+        return
+    for rule, md in ((1, None), (1, 4.0), (0, None)):
+        try:
+            if rule == 1:
+                want, nc, kept = O.sl_mst_lifetime(u, v, w, n, disconnect_weight=md)
+            else:
+                nc, want = O.sp_sl_lifetime(u, v, w, n)
+                kept = None
+        except ValueError:
+            with pytest.raises((EACError, ValueError)):
+                lifetime_cut(g["dest"], g["weight"], g["indptr"], None, rule=rule, max_dist=md)
+            continue
+        lab, info = lifetime_cut(g["dest"], g["weight"], g["indptr"], None, rule=rule, max_dist=md)
+        if kept is not None:
+            assert info["kept_edges"] == kept
+        if want.size == 0:
+            assert lab is None and info["n_components"] == 1
+        else:
+            assert info["n_components"] == nc and np.array_equal(lab.cpu().numpy(), want)
