@@ -123,6 +123,23 @@ __device__ __forceinline__ uint32_t wave_incl_scan_dpp(uint32_t v) {
   return v;
 }
 
+// 64-bit values the same way, the two halves shifted together.
+__device__ __forceinline__ uint64_t wave_incl_scan_dpp(uint64_t v) {
+#define EAC_DPP_STEP(ctrl, rows)                                                              \
+  v += (uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)v, ctrl, rows, 0xf,  \
+                                                       false) |                               \
+       (uint64_t)(uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(v >> 32), ctrl, rows, \
+                                                       0xf, false) << 32
+  EAC_DPP_STEP(0x111, 0xf);
+  EAC_DPP_STEP(0x112, 0xf);
+  EAC_DPP_STEP(0x114, 0xf);
+  EAC_DPP_STEP(0x118, 0xf);
+  EAC_DPP_STEP(0x142, 0xa);
+  EAC_DPP_STEP(0x143, 0xc);
+#undef EAC_DPP_STEP
+  return v;
+}
+
 template <typename T>
 __device__ __forceinline__ T wave_sum(T v) {
 #pragma unroll

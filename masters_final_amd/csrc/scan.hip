@@ -65,7 +65,18 @@ __global__ __launch_bounds__(kScanBlock) void k_scan_reduce(const Tin* __restric
 template <typename T>
 __device__ __forceinline__ T incl_scan64(T v) {
   if constexpr (sizeof(T) == 4) return (T)wave_incl_scan_dpp((uint32_t)v);
-  else return wave_incl_scan(v);
+  else return (T)wave_incl_scan_dpp((uint64_t)v);
+}
+// Lane 63's value, for every lane.
+template <typename T>
+__device__ __forceinline__ T last_lane(T v) {
+  const uint32_t lo = __builtin_amdgcn_readlane((int)(uint32_t)v, kWave - 1);
+  if constexpr (sizeof(T) == 4) {
+    return (T)lo;
+  } else {
+    const uint32_t hi = __builtin_amdgcn_readlane((int)(uint32_t)((uint64_t)v >> 32), kWave - 1);
+    return (T)((uint64_t)hi << 32 | lo);
+  }
 }
 template <typename Tin, typename Tout>
 __global__ __launch_bounds__(kScanOne) void k_scan_one(const Tin* in, Tout* out, int64_t n,
@@ -86,7 +97,7 @@ __global__ __launch_bounds__(kScanOne) void k_scan_one(const Tin* in, Tout* out,
     for (int k = 0; k < kScanItems; ++k) {
       const Tout inc = incl_scan64<Tout>(v[k]);
       pre[k] = run + inc - v[k];
-      run += __shfl(inc, kWave - 1, kWave);
+      run += last_lane(inc);
     }
     if (l == 0) wsum[turn][w] = run;
     __syncthreads();
