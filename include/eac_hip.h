@@ -418,11 +418,15 @@ int eac_coassoc_fill_ranked(const int32_t* labels, int64_t n, const int64_t* h_k
  *   eac_coassoc_stage (same ws, unchanged): indptr[n+1], h_nnz, largest
  *     count; h_nnz = -1 when the pool was too small (then build with
  *     eac_coassoc_count + eac_coassoc_fill);
+ *   eac_coassoc_plan: the plan alone, in place of eac_coassoc_estimate
+ *     where the pool holds every pair anyway;
  *   eac_coassoc_compact: indices[nnz], data[nnz] as eac_coassoc_fill writes
  *     them, from the staging buffer (its header holds the layout). */
 int eac_coassoc_estimate(const int32_t* labels, int64_t n, const int64_t* h_koff,
                          int32_t P, int32_t full_rows, int64_t sample_stride,
                          int64_t* h_estimate, void* ws, size_t ws_bytes, void* stream);
+int eac_coassoc_plan(const int32_t* labels, int64_t n, const int64_t* h_koff, int32_t P, void* ws,
+                     size_t ws_bytes, void* stream);
 size_t eac_coassoc_stage_bytes(int64_t n, int32_t full_rows, int32_t P, int64_t pool_entries);
 int eac_coassoc_stage(const int32_t* labels, int64_t n, const int64_t* h_koff, int32_t P,
                       int32_t full_rows, int64_t* indptr, void* stage, size_t stage_bytes,

@@ -718,6 +718,26 @@ int d2h(void* host, const void* dev, size_t bytes, hipStream_t s) {
   return EAC_OK;
 }
 
+// Several small reads behind one wait (a wait costs 10 us, a copy 2).
+struct HostRead {
+  void* host;
+  const void* dev;
+  size_t bytes;
+};
+template <int N>
+int d2h_all(const HostRead (&r)[N], hipStream_t s) {
+  constexpr size_t kSlot = 64;
+  char* pin = static_cast<char*>(pinned_scratch(N * kSlot));
+  if (!pin) return fail(EAC_ERR_HIP, "pinned host allocation failed");
+  for (int i = 0; i < N; ++i) {
+    if (r[i].bytes > kSlot) return fail(EAC_ERR_ARG, "coassoc: host read too long");
+    EAC_HIP_CHECK(hipMemcpyAsync(pin + i * kSlot, r[i].dev, r[i].bytes, hipMemcpyDeviceToHost, s));
+  }
+  EAC_HIP_CHECK(hipStreamSynchronize(s));
+  for (int i = 0; i < N; ++i) memcpy(r[i].host, pin + i * kSlot, r[i].bytes);
+  return EAC_OK;
+}
+
 int co_check(const int32_t* labels, int64_t n, const int64_t* h_koff, int32_t P) {
   if (n < 1 || P < 1) return fail(EAC_ERR_ARG, "coassoc: need n, P >= 1");
   if (P > kMaxP) return fail(EAC_ERR_UNSUPPORTED, "coassoc: more than %d partitions", kMaxP);
@@ -891,9 +911,8 @@ extern "C" int eac_coassoc_count(const int32_t* labels, int64_t n, const int64_t
   EAC_TRY((scan_excl<int32_t, int64_t>(B.row_nnz, indptr, n + 1, 0, nullptr, ar, s)));
   ar.used = mark;
   unsigned int misc[4];
-  EAC_TRY(d2h(misc, B.misc, sizeof(misc), s));
   int64_t nnz = 0;
-  EAC_TRY(d2h(&nnz, indptr + n, sizeof(int64_t), s));
+  EAC_TRY(d2h_all<2>({{misc, B.misc, sizeof(misc)}, {&nnz, indptr + n, sizeof(nnz)}}, s));
   prof_flush();
   if (misc[0]) return fail(EAC_ERR_ARG, "coassoc: label >= k of its partition");
   if (h_nnz) *h_nnz = nnz;
@@ -1017,6 +1036,20 @@ StageLayout stage_layout(int64_t n, int full_rows) {
 // Plan (as eac_coassoc_count) plus the count pass over rows 0, stride,
 // 2 * stride, ...: h_estimate = their nnz sum x (rows / sampled rows),
 // rounded up. Keep ws for eac_coassoc_stage.
+extern "C" int eac_coassoc_plan(const int32_t* labels, int64_t n, const int64_t* h_koff,
+                                int32_t P, void* ws, size_t ws_bytes, void* stream) {
+  EAC_TRY(co_check(labels, n, h_koff, P));
+  hipStream_t s = (hipStream_t)stream;
+  Arena ar(ws, ws_bytes);
+  CoBufs B;
+  size_t mark = 0;
+  EAC_TRY(co_plan_build(labels, n, h_koff, P, ws, ws_bytes, &B, &mark, ar, s));
+  unsigned int misc[4];
+  EAC_TRY(d2h(misc, B.misc, sizeof(misc), s));
+  if (misc[0]) return fail(EAC_ERR_ARG, "coassoc: label >= k of its partition");
+  return EAC_OK;
+}
+
 extern "C" int eac_coassoc_estimate(const int32_t* labels, int64_t n, const int64_t* h_koff,
                                     int32_t P, int32_t full_rows, int64_t sample_stride,
                                     int64_t* h_estimate, void* ws, size_t ws_bytes,
@@ -1044,9 +1077,8 @@ extern "C" int eac_coassoc_estimate(const int32_t* labels, int64_t n, const int6
   EAC_TRY(co_launch<0>(pl, full_rows, win, o, s));
   prof_end(pr, s);
   unsigned int misc[4];
-  EAC_TRY(d2h(misc, B.misc, sizeof(misc), s));
   unsigned long long sum = 0;
-  EAC_TRY(d2h(&sum, B.ctr + kCtrSum, sizeof(sum), s));
+  EAC_TRY(d2h_all<2>({{misc, B.misc, sizeof(misc)}, {&sum, B.ctr + kCtrSum, sizeof(sum)}}, s));
   prof_flush();
   if (misc[0]) return fail(EAC_ERR_ARG, "coassoc: label >= k of its partition");
   const int64_t rows = (n + sample_stride - 1) / sample_stride;
@@ -1112,11 +1144,12 @@ extern "C" int eac_coassoc_stage(const int32_t* labels, int64_t n, const int64_t
   EAC_TRY((scan_excl<int32_t, int64_t>(B.row_nnz, indptr, n + 1, 0, nullptr, ar, s)));
   ar.used = mark;
   unsigned int misc[4];
-  EAC_TRY(d2h(misc, B.misc, sizeof(misc), s));
   int64_t tail[2] = {0, 0};  // overflow flag (hdr[3])
-  EAC_TRY(d2h(tail, hdr + 2, sizeof(tail), s));
   int64_t nnz = 0;
-  EAC_TRY(d2h(&nnz, indptr + n, sizeof(int64_t), s));
+  EAC_TRY(d2h_all<3>({{misc, B.misc, sizeof(misc)},
+                      {tail, hdr + 2, sizeof(tail)},
+                      {&nnz, indptr + n, sizeof(nnz)}},
+                     s));
   prof_flush();
   *h_nnz = tail[1] ? -1 : nnz;
   if (h_max_count) *h_max_count = (int32_t)misc[1];
