@@ -1210,14 +1210,18 @@ __global__ __launch_bounds__(256) void k_resolve(const float* __restrict__ X, in
   }
 }
 
-// Direct-difference labeling: one thread per (point, partition), blocks of
-// 256 points x one partition (grid.y over partitions, so a small data set
+// Direct-difference labeling: one thread per (PT points, partition), blocks of
+// 256 PT points x one partition (grid.y over partitions, so a small data set
 // with many partitions still fills the chip). The point sits in registers
 // (DX = d exactly for d <= 4, else zero padded to DX: padding adds exact
 // zeros) and the partition's centroids are staged in LDS, already converted
 // to T, a tile of at most 16 KiB at a time. T = float: plain FP32; T =
 // double: the oracle's FP64 arithmetic (ascending dimensions, strict <).
-template <typename T, int DX>
+// PT points a lane (i and i + 256): a centroid read from LDS serves them all,
+// and their chains of rounded operations overlap. 10,000 points, 100
+// partitions of 50 to 100 centroids in 2-D in FP64: 35 us with one point, 31
+// with two.
+template <typename T, int DX, int PT>
 __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ X, int64_t n,
                                                       int d, const float* __restrict__ C,
                                                       const int64_t* __restrict__ k_off, int P,
@@ -1226,15 +1230,22 @@ __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ 
   constexpr int kTileRaw = 16384 / (DX * (int)sizeof(T));
   constexpr int kTile = kTileRaw > 256 ? 256 : kTileRaw;
   __shared__ T s_c[kTile * DX];
-  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = i < n;
-  T xr[DX];
+  const int64_t i0 = (int64_t)blockIdx.x * (256 * PT) + threadIdx.x;
+  T xr[PT][DX];
 #pragma unroll
-  for (int j = 0; j < DX; ++j) xr[j] = (valid && j < d) ? (T)X[i * d + j] : T(0);
+  for (int q = 0; q < PT; ++q)
+#pragma unroll
+    for (int j = 0; j < DX; ++j)
+      xr[q][j] = (i0 + q * 256 < n && j < d) ? (T)X[(i0 + q * 256) * d + j] : T(0);
   for (int p = blockIdx.y; p < P; p += gridDim.y) {
     const int64_t kbeg = k_off[p], kend = k_off[p + 1];
-    T best = 0;
-    int32_t bl = -1;
+    T best[PT];
+    int32_t bl[PT];
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+      best[q] = 0;
+      bl[q] = -1;
+    }
     for (int64_t c0 = kbeg; c0 < kend; c0 += kTile) {
       const int rows = (int)((kend - c0) < kTile ? (kend - c0) : kTile);
       __syncthreads();
@@ -1243,18 +1254,39 @@ __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ 
         s_c[v] = j < d ? (T)C[(c0 + r) * d + j] : T(0);
       }
       __syncthreads();
-      if (valid) {
-        for (int r = 0; r < rows; ++r) {
+      int r = 0;
+      if (c0 == kbeg) {  // the first centroid wins whatever its distance is (a NaN stays)
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
           T dist = 0;
 #pragma unroll
-          for (int j = 0; j < DX; ++j) dist = sq_acc(dist, xr[j] - s_c[r * DX + j]);
-          if (bl < 0 || dist < best) { best = dist; bl = (int32_t)(c0 + r - kbeg); }
+          for (int j = 0; j < DX; ++j) dist = sq_acc(dist, xr[q][j] - s_c[j]);
+          best[q] = dist;
+          bl[q] = 0;
+        }
+        r = 1;
+      }
+      const int base = (int)(c0 - kbeg);
+#pragma unroll 2
+      for (; r < rows; ++r) {
+#pragma unroll
+        for (int q = 0; q < PT; ++q) {
+          T dist = 0;
+#pragma unroll
+          for (int j = 0; j < DX; ++j) dist = sq_acc(dist, xr[q][j] - s_c[r * DX + j]);
+          const bool less = dist < best[q];
+          best[q] = less ? dist : best[q];
+          bl[q] = less ? base + r : bl[q];
         }
       }
     }
-    if (valid) {
-      labels[(int64_t)p * n + i] = bl;
-      if (dists) dists[(int64_t)p * n + i] = (float)best;
+#pragma unroll
+    for (int q = 0; q < PT; ++q) {
+      const int64_t i = i0 + q * 256;
+      if (i < n) {
+        labels[(int64_t)p * n + i] = bl[q];
+        if (dists) dists[(int64_t)p * n + i] = (float)best[q];
+      }
     }
   }
 }
@@ -1477,16 +1509,27 @@ int np_sum_rows(const float* x, int64_t n, int64_t rows, float* csum, float* out
 template <typename T>
 int launch_direct(const float* X, int64_t n, int d, const float* C, const int64_t* k_off, int P,
                   int32_t* labels, float* dists, hipStream_t s) {
-  const dim3 g(grid_for(n, 256), P < 65535 ? P : 65535);
-  if (d == 1) k_label_direct<T, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d == 2) k_label_direct<T, 2><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d == 3) k_label_direct<T, 3><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d == 4) k_label_direct<T, 4><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d <= 8) k_label_direct<T, 8><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d <= 16) k_label_direct<T, 16><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d <= 32) k_label_direct<T, 32><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d <= 64) k_label_direct<T, 64><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
-  else if (d <= 128) k_label_direct<T, 128><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  const int py = P < 65535 ? P : 65535;
+  const dim3 g(grid_for(n, 256), py);
+  // two points a lane while that still leaves every unit two workgroups
+  if (d <= 4 && (int64_t)grid_for(n, 512) * py >= 512) {
+    const dim3 g2(grid_for(n, 512), py);
+    if (d == 1) k_label_direct<T, 1, 2><<<g2, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+    else if (d == 2) k_label_direct<T, 2, 2><<<g2, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+    else if (d == 3) k_label_direct<T, 3, 2><<<g2, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+    else k_label_direct<T, 4, 2><<<g2, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+    EAC_LAUNCH_CHECK();
+    return EAC_OK;
+  }
+  if (d == 1) k_label_direct<T, 1, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d == 2) k_label_direct<T, 2, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d == 3) k_label_direct<T, 3, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d == 4) k_label_direct<T, 4, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d <= 8) k_label_direct<T, 8, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d <= 16) k_label_direct<T, 16, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d <= 32) k_label_direct<T, 32, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d <= 64) k_label_direct<T, 64, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
+  else if (d <= 128) k_label_direct<T, 128, 1><<<g, 256, 0, s>>>(X, n, d, C, k_off, P, labels, dists);
   else return fail(EAC_ERR_UNSUPPORTED, "kmeans direct: d=%d > 128", d);
   EAC_LAUNCH_CHECK();
   return EAC_OK;

@@ -62,3 +62,24 @@ def test_cascade_equals_fp64(torch, d, k, ties):
     assert n * k * ((d + 31) // 32) >= 5e8
     nres = _same(torch, X, C)
     assert (nres > n // 2) == ties
+
+
+@pytest.mark.parametrize("n", [255, 256, 257, 511, 512, 513, 2570])
+@pytest.mark.parametrize("d", [1, 2, 3, 4])
+def test_direct_points_per_lane(torch, n, d):
+    """The FP64 form with one and with two points a lane (enough partitions):
+    the same labels and distances, bit for bit, NaN rows included."""
+    from masters_final_amd.cluster.KMeans import label_device
+    rng = np.random.default_rng(n + d)
+    X = rng.standard_normal((n, d)).astype(np.float32)
+    X[n // 2] = np.nan
+    C = rng.standard_normal((5, d)).astype(np.float32)
+    a, da, _ = label_device(X, C, precision="fp64")
+    P = 600
+    b, db, _ = label_device(X, np.tile(C, (P, 1)), [5] * P, precision="fp64")
+    assert torch.equal(b, a.expand(P, n))
+    assert torch.equal(db.view(torch.int32), da.expand(P, n).contiguous().view(torch.int32))
+    with np.errstate(invalid="ignore"):
+        D = ((X[:, None].astype(np.float64) - C[None].astype(np.float64)) ** 2).sum(-1)
+    want = np.where(np.isnan(D).any(1), 0, D.argmin(1))
+    assert np.array_equal(a[0].cpu().numpy(), want)
