@@ -169,7 +169,7 @@ def autotune_coassoc(labels, ks, windows=(4096, 8192, 16384, 32768), unrolls=(4,
 
 
 def autotune_kmeans(X, centroids, k_list=None, waves=(0, 2, 3, 4), reps=3, use_cache=True):
-    """Picks the waves per SIMD the split-BF16 labeling kernel is compiled
+    """Picks the waves per SIMD the split-f16 labeling kernel is compiled
     for (km_waves; 0 = built-in) on this data shape: timed label passes,
     identical labels checked. Returns dict(knobs, ms, cached, candidates)."""
     from .cluster.KMeans import label_device
