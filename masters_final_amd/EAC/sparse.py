@@ -97,10 +97,17 @@ def coassoc_device(labels, k_list, full_rows=False, w_offset=0, one_pass=None,
                                       L.stream_ptr()))
         if info is not None:
             info.update(estimate=est.value, pool_entries=pool, sample_stride=stride)
+        indices = data = None
         if nnz.value >= 0:
             m = max(nnz.value, 1)
-            indices = t.empty(m, dtype=t.int32, device=dl.device)
-            data = t.empty(m, dtype=t.int32, device=dl.device)
+            try:
+                indices = t.empty(m, dtype=t.int32, device=dl.device)
+                data = t.empty(m, dtype=t.int32, device=dl.device)
+            except t.cuda.OutOfMemoryError:  # beside a pool for every pair
+                if not bound:
+                    raise
+                indices = data = None
+        if data is not None:
             if w_offset == "max+1":
                 w_offset = mx.value + 1
             L.check(lib.eac_coassoc_compact(n, L.ptr(indptr), L.ptr(stage), nb, int(w_offset),
@@ -110,7 +117,7 @@ def coassoc_device(labels, k_list, full_rows=False, w_offset=0, one_pass=None,
             return indptr, indices[: nnz.value], data[: nnz.value], mx.value
         del stage
         if info is not None:
-            info["path"] = "one-pass overflow, two-pass"
+            info["path"] = "one-pass overflow, two-pass" if nnz.value < 0 else "two-pass"
     L.check(lib.eac_coassoc_count(L.ptr(dl), n, koff.ctypes.data_as(C.c_void_p), P,
                                   1 if full_rows else 0, L.ptr(indptr), C.byref(nnz), C.byref(mx),
                                   L.ptr(ws), ws.numel(), L.stream_ptr()))

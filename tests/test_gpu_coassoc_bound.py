@@ -42,3 +42,31 @@ def test_bound_build_reports_bad_labels(torch):
     labels[1, 4999] = 3
     with pytest.raises(EACError, match="label >= k"):
         coassoc_device(labels, [1, 3])
+
+
+@pytest.mark.parametrize("fails", [(0,), (1,), (2,)])
+def test_bound_build_without_room(torch, monkeypatch, fails):
+    """The pool (allocation 0), the columns (1) or the values (2) do not fit
+    beside each other: the two visits, which need no pool, take over."""
+    from masters_final_amd.EAC.sparse import coassoc_device
+    n, P = 5000, 6
+    labels = np.random.default_rng(5).integers(0, 40, (P, n)).astype(np.int32)
+    want = coassoc_device(labels, [40] * P, w_offset="max+1", one_pass=False)
+    dl = torch.from_numpy(labels).cuda()
+    empty, seen = torch.empty, []
+
+    def scarce(*a, **kw):
+        if kw.get("dtype") in (torch.uint8, torch.int32):
+            seen.append(a)
+            if len(seen) - 1 in fails:
+                raise torch.cuda.OutOfMemoryError("none left")
+        return empty(*a, **kw)
+
+    coassoc_device(labels, [40] * P)  # the shared workspace is there
+    monkeypatch.setattr(torch, "empty", scarce)
+    info = {}
+    got = coassoc_device(dl, [40] * P, w_offset="max+1", info=info)
+    assert info["path"] == "two-pass" and len(seen) == fails[0] + 3
+    assert got[3] == want[3]
+    for x, y in zip(got[:3], want[:3]):
+        assert torch.equal(x, y)
