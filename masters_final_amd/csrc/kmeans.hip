@@ -1405,67 +1405,79 @@ int launch_np(const float* X, int64_t n, int d, const float* C, const int64_t* k
 // PW_BLOCKSIZE 128): a range of len < 8 is summed sequentially from 0; len
 // <= 128 keeps eight partial sums over a[j], a[j+8], ... combined as
 // ((r0+r1)+(r2+r3))+((r4+r5)+(r6+r7)), then adds the tail in order; longer
-// ranges split at n2 = len/2 rounded down to a multiple of 8. The tree of a
-// chunk is a pure function of its length, so one wavefront evaluates it
-// bottom-up: heap node h at depth t has its range found by descending from
-// the root along the bits of h, each level's nodes are computed in parallel
-// from the level below (held in LDS), and leaves (len <= 128) sum their
-// range directly. Every addition is a float32 addition, so the result is
-// numpy's to the bit.
+// ranges split at n2 = len/2 rounded down to a multiple of 8. Every addition
+// is a float32 addition, so the result is numpy's to the bit.
+//
+// The tree of a chunk is a pure function of its length. The shorter half n2
+// grows with len, so the leftmost node of a depth is its shortest, and T, the
+// first depth at which that one is a leaf (len <= 128), has all its 2^T <= 64
+// nodes. Halves differ by at most 15, so the lengths of a depth by less than
+// 30, and a node of depth T that is no leaf (len < 158) has two leaves: depth
+// T is computed node by node and the rest is a full binary tree.
 constexpr int kNpBuf = 8192;
-constexpr int kNpDepth = 8;  // chunk trees of len <= 8192 are at most 7 deep
 
-__device__ __forceinline__ bool np_node(int len0, int h, int t, int& off, int& len) {
-  off = 0;
-  len = len0;
-  for (int q = t - 1; q >= 0; --q) {
-    if (len <= 128) return false;  // an ancestor is a leaf
-    int n2 = len >> 1;
-    n2 -= n2 & 7;
-    if ((h >> q) & 1) { off += n2; len -= n2; } else { len = n2; }
-  }
-  return true;
-}
-
-__device__ __forceinline__ float np_leaf(const float* __restrict__ a, int len) {
-  if (len < 8) {
-    float res = 0.0f;
-    for (int i = 0; i < len; ++i) res = __fadd_rn(res, a[i]);
-    return res;
-  }
-  float r[8];
+// A leaf's sum by eight lanes (lane j holds the partial sum over a[j],
+// a[j+8], ...), all of a lane's loads in flight at once; the result is that of
+// lane 0, whose additions take their operands in numpy's order.
+__device__ __forceinline__ float np_leaf(const float* __restrict__ a, int len, int j) {
+  float res = 0.0f;
+  if (len >= 8) {
+    constexpr int Q = 128 / 8;
+    const int m = len >> 3;
+    float e[Q];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) r[j] = a[j];
-  int i = 8;
-  for (; i < len - (len & 7); i += 8) {
+    for (int q = 0; q < Q; ++q) e[q] = q < m ? a[8 * q + j] : 0.0f;
+    res = e[0];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) r[j] = __fadd_rn(r[j], a[i + j]);
+    for (int q = 1; q < Q; ++q)
+      if (q < m) res = __fadd_rn(res, e[q]);
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) res = __fadd_rn(res, __shfl_xor(res, o));
   }
-  float res = __fadd_rn(__fadd_rn(__fadd_rn(r[0], r[1]), __fadd_rn(r[2], r[3])),
-                        __fadd_rn(__fadd_rn(r[4], r[5]), __fadd_rn(r[6], r[7])));
-  for (; i < len; ++i) res = __fadd_rn(res, a[i]);
+  for (int i = len & ~7; i < len; ++i) res = __fadd_rn(res, a[i]);
   return res;
 }
 
-// One wavefront per (chunk, row): csum[row * nchunks + chunk].
-__global__ __launch_bounds__(kWave) void k_np_chunk_sums(const float* __restrict__ x, int64_t n,
-                                                         int64_t nchunks,
-                                                         float* __restrict__ csum) {
-  __shared__ float v[2 << kNpDepth];
+// One workgroup per (chunk, row): csum[row * nchunks + chunk]. Eight lanes a
+// node of depth T, so that a full chunk is read at once, 32 bytes a node, and
+// its sum waits for one round trip to memory; the 2^T sums are one
+// wavefront's. 100 rows of 10,000: 4.5 us (a lane a leaf and a walk of the
+// tree in LDS: 9.8).
+constexpr int kNpT = 512;
+__global__ __launch_bounds__(kNpT) void k_np_chunk_sums(const float* __restrict__ x, int64_t n,
+                                                        int64_t nchunks,
+                                                        float* __restrict__ csum) {
+  __shared__ float v[kWave];
   const int64_t c = blockIdx.x;
   const int64_t row = blockIdx.y;
   const int64_t base = c * kNpBuf;
   const int len0 = (int)(n - base < kNpBuf ? n - base : kNpBuf);
   const float* a = x + row * n + base;
-  for (int t = kNpDepth; t >= 0; --t) {
-    for (int h = (1 << t) + (int)threadIdx.x; h < (2 << t); h += kWave) {
-      int off, len;
-      if (!np_node(len0, h, t, off, len)) continue;
-      v[h] = len <= 128 ? np_leaf(a + off, len) : __fadd_rn(v[2 * h], v[2 * h + 1]);
+  int T = 0;
+  for (int l = len0; l > 128; l = (l >> 1) & ~7) ++T;
+  const int g = threadIdx.x >> 3, j = threadIdx.x & 7;
+  if (g < 1 << T) {
+    int len = len0;
+    for (int q = T - 1; q >= 0; --q) {
+      const int n2 = (len >> 1) & ~7;
+      if ((g >> q) & 1) {
+        a += n2;
+        len -= n2;
+      } else {
+        len = n2;
+      }
     }
-    __syncthreads();
+    const int n2 = len > 128 ? (len >> 1) & ~7 : len;
+    float r = np_leaf(a, n2, j);
+    if (len > n2) r = __fadd_rn(r, np_leaf(a + n2, len - n2, j));
+    if (j == 0) v[g] = r;
   }
-  if (threadIdx.x == 0) csum[row * nchunks + c] = v[1];
+  __syncthreads();
+  if (threadIdx.x < kWave) {
+    float r = (int)threadIdx.x < 1 << T ? v[threadIdx.x] : 0.0f;
+    for (int o = 1; o < 1 << T; o <<= 1) r = __fadd_rn(r, __shfl_xor(r, o));
+    if (threadIdx.x == 0) csum[row * nchunks + c] = r;
+  }
 }
 
 // ((0 + csum[0]) + csum[1]) + ...
@@ -1489,7 +1501,7 @@ int np_chunk_sums(const float* x, int64_t n, int64_t rows, float* csum, hipStrea
   if (nc > 0) {
     for (int64_t r0 = 0; r0 < rows; r0 += 65535) {
       const int64_t rr = rows - r0 < 65535 ? rows - r0 : 65535;
-      k_np_chunk_sums<<<dim3((unsigned)nc, (unsigned)rr), kWave, 0, s>>>(x + r0 * n, n, nc,
+      k_np_chunk_sums<<<dim3((unsigned)nc, (unsigned)rr), kNpT, 0, s>>>(x + r0 * n, n, nc,
                                                                           csum + r0 * nc);
       EAC_LAUNCH_CHECK();
     }
