@@ -704,7 +704,9 @@ __device__ __forceinline__ double sq_acc(double acc, double diff) {
 #pragma clang fp contract(off)
   return acc + diff * diff;
 }
-__device__ __forceinline__ float sq_acc(float acc, float diff) { return acc + diff * diff; }
+__device__ __forceinline__ float sq_acc(float acc, float diff) {
+  return __builtin_fmaf(diff, diff, acc);
+}
 
 // Squared distance of two float rows in FP64, accumulated in ascending
 // dimension order (the oracle's arithmetic); 16-byte loads when both rows
@@ -1210,6 +1212,10 @@ __global__ __launch_bounds__(256) void k_resolve(const float* __restrict__ X, in
   }
 }
 
+// The smaller one, a NaN left out.
+__device__ __forceinline__ float min_of(float a, float b) { return __builtin_fminf(a, b); }
+__device__ __forceinline__ double min_of(double a, double b) { return __builtin_fmin(a, b); }
+
 // Direct-difference labeling: one thread per (PT points, partition), blocks of
 // 256 PT points x one partition (grid.y over partitions, so a small data set
 // with many partitions still fills the chip). The point sits in registers
@@ -1218,9 +1224,16 @@ __global__ __launch_bounds__(256) void k_resolve(const float* __restrict__ X, in
 // to T, a tile of at most 16 KiB at a time. T = float: plain FP32; T =
 // double: the oracle's FP64 arithmetic (ascending dimensions, strict <).
 // PT points a lane (i and i + 256): a centroid read from LDS serves them all,
-// and their chains of rounded operations overlap. 10,000 points, 100
-// partitions of 50 to 100 centroids in 2-D in FP64: 35 us with one point, 31
-// with two.
+// and their chains of rounded operations overlap.
+// Vector issue bounds it. Up to four dimensions the comparison costs as much
+// as the distance, so it is made on the minimum of four (NaN rows fill the
+// last four; a minimum leaves NaNs out, as the strict < does), and the best
+// four of a tile are computed once more for the lowest index that gives the
+// minimum. 10,000 points, 100 partitions of 50 to 100 centroids in 2-D in
+// FP64: 35 us with one point a lane, 31 with two, 26 in fours. 300,000 points
+// and 300 centroids, a call in FP64 (FP32), one by one and in fours: 62 and 51
+// us in 1-D (53 and 47), 94 and 85 in 4-D (61 and 58), but 124 and 136 in 8-D,
+// 223 and 234 in 16-D (111 and 128), where the loads of four rows stall.
 template <typename T, int DX, int PT>
 __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ X, int64_t n,
                                                       int d, const float* __restrict__ C,
@@ -1229,6 +1242,7 @@ __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ 
                                                       float* __restrict__ dists) {
   constexpr int kTileRaw = 16384 / (DX * (int)sizeof(T));
   constexpr int kTile = kTileRaw > 256 ? 256 : kTileRaw;
+  constexpr bool kFours = DX <= 4;
   __shared__ T s_c[kTile * DX];
   const int64_t i0 = (int64_t)blockIdx.x * (256 * PT) + threadIdx.x;
   T xr[PT][DX];
@@ -1237,6 +1251,12 @@ __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ 
 #pragma unroll
     for (int j = 0; j < DX; ++j)
       xr[q][j] = (i0 + q * 256 < n && j < d) ? (T)X[(i0 + q * 256) * d + j] : T(0);
+  auto dist_to = [&](int q, int r) {  // point q to the tile's row r
+    T v = 0;
+#pragma unroll
+    for (int j = 0; j < DX; ++j) v = sq_acc(v, xr[q][j] - s_c[r * DX + j]);
+    return v;
+  };
   for (int p = blockIdx.y; p < P; p += gridDim.y) {
     const int64_t kbeg = k_off[p], kend = k_off[p + 1];
     T best[PT];
@@ -1248,35 +1268,58 @@ __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ 
     }
     for (int64_t c0 = kbeg; c0 < kend; c0 += kTile) {
       const int rows = (int)((kend - c0) < kTile ? (kend - c0) : kTile);
+      const int stored = kFours ? (rows + 3) & ~3 : rows;
       __syncthreads();
-      for (int v = threadIdx.x; v < rows * DX; v += blockDim.x) {
+      for (int v = threadIdx.x; v < stored * DX; v += blockDim.x) {
         const int r = v / DX, j = v - (v / DX) * DX;
-        s_c[v] = j < d ? (T)C[(c0 + r) * d + j] : T(0);
+        s_c[v] = r < rows ? (j < d ? (T)C[(c0 + r) * d + j] : T(0)) : (T)__builtin_nanf("");
       }
       __syncthreads();
       int r = 0;
       if (c0 == kbeg) {  // the first centroid wins whatever its distance is (a NaN stays)
 #pragma unroll
         for (int q = 0; q < PT; ++q) {
-          T dist = 0;
-#pragma unroll
-          for (int j = 0; j < DX; ++j) dist = sq_acc(dist, xr[q][j] - s_c[j]);
-          best[q] = dist;
+          best[q] = dist_to(q, 0);
           bl[q] = 0;
         }
-        r = 1;
+        r = kFours ? 0 : 1;
       }
       const int base = (int)(c0 - kbeg);
+      if constexpr (kFours) {
+        int bg[PT];  // the tile's best four, -1: none better than before
+#pragma unroll
+        for (int q = 0; q < PT; ++q) bg[q] = -1;
+        for (; r < rows; r += 4) {
+#pragma unroll
+          for (int q = 0; q < PT; ++q) {
+            T v[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) v[u] = dist_to(q, r + u);
+            const T m = min_of(min_of(v[0], v[1]), min_of(v[2], v[3]));
+            const bool less = m < best[q];
+            best[q] = less ? m : best[q];
+            bg[q] = less ? r : bg[q];
+          }
+        }
+#pragma unroll
+        for (int q = 0; q < PT; ++q)
+          if (bg[q] >= 0) {
+            int at = 0;
+#pragma unroll
+            for (int u = 3; u > 0; --u) at = dist_to(q, bg[q] + u) == best[q] ? u : at;
+            at = dist_to(q, bg[q]) == best[q] ? 0 : at;
+            bl[q] = base + bg[q] + at;
+          }
+      } else {
 #pragma unroll 2
-      for (; r < rows; ++r) {
+        for (; r < rows; ++r) {
 #pragma unroll
-        for (int q = 0; q < PT; ++q) {
-          T dist = 0;
-#pragma unroll
-          for (int j = 0; j < DX; ++j) dist = sq_acc(dist, xr[q][j] - s_c[r * DX + j]);
-          const bool less = dist < best[q];
-          best[q] = less ? dist : best[q];
-          bl[q] = less ? base + r : bl[q];
+          for (int q = 0; q < PT; ++q) {
+            const T v = dist_to(q, r);
+            const bool less = v < best[q];
+            best[q] = less ? v : best[q];
+            bl[q] = less ? base + r : bl[q];
+          }
         }
       }
     }

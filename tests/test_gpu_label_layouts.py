@@ -83,3 +83,35 @@ def test_direct_points_per_lane(torch, n, d):
         D = ((X[:, None].astype(np.float64) - C[None].astype(np.float64)) ** 2).sum(-1)
     want = np.where(np.isnan(D).any(1), 0, D.argmin(1))
     assert np.array_equal(a[0].cpu().numpy(), want)
+
+
+@pytest.mark.parametrize("d", [1, 2, 3, 4, 7, 8, 16, 17])
+@pytest.mark.parametrize("k", [1, 3, 4, 5, 8, 127, 128, 255, 256, 257, 515])
+@pytest.mark.parametrize("P", [1, 300])
+def test_direct_fours(torch, d, k, P):
+    """The plain labeling's groups of four at the edges of groups and of
+    centroid tiles, with one and with two points a lane: ties go to the lowest
+    index, NaN centroids lose unless they come first, in the oracle's FP64
+    arithmetic (ascending dimensions, strict <)."""
+    from masters_final_amd.cluster.KMeans import label_device
+    rng = np.random.default_rng(1000 * d + k)
+    n = 600 if P > 1 else 517
+    X = rng.integers(-3, 4, (n, d)).astype(np.float32)  # coarse: many equal distances
+    C = rng.integers(-3, 4, (k, d)).astype(np.float32)
+    X[5], X[6] = 1e30, np.nan
+    if k > 4:
+        C[3], C[k - 1] = np.nan, np.inf
+    got, dist, _ = label_device(X, np.tile(C, (P, 1)), [k] * P, precision="fp64")
+    f32, _, _ = label_device(X, np.tile(C, (P, 1)), [k] * P, precision="fp32")
+    D = np.zeros((n, k))
+    with np.errstate(all="ignore"):
+        for j in range(d):
+            t = X[:, j, None].astype(np.float64) - C[None, :, j].astype(np.float64)
+            D = D + t * t
+    want = np.where(np.isnan(D[:, 0]), 0, np.where(np.isnan(D), np.inf, D).argmin(1))
+    assert np.array_equal(got.cpu().numpy(), np.broadcast_to(want, (P, n)))
+    ref = D[np.arange(n), want].astype(np.float32)
+    assert np.array_equal(dist.cpu().numpy(), np.broadcast_to(ref, (P, n)), equal_nan=True)
+    small = np.ones(n, bool)
+    small[5] = False  # whose squares leave float32's range
+    assert np.array_equal(f32.cpu().numpy()[:, small], np.broadcast_to(want[small], (P, n - 1)))
