@@ -144,8 +144,8 @@ def eac_compare(n=10_000, P=100, kmin=50, kmax=100, iters=3, seed=0, reps=3, cpu
     rr, tr = timed(lambda: rec.run(dinit), reps, 1, torch)
     rp, tp = timed(plain, reps, 1, torch)
     out = {"n": n, "partitions": P, "k_range": [kmin, kmax], "iters": iters,
-           "batched_labeling": "FP64 direct difference: d = 2 is below the d >= 16 where the "
-                               "split-f16 MFMA path applies, so precision 'bf16x3' runs the "
+           "batched_labeling": "FP64 direct difference: d = 2 is below the 4 dimensions from which "
+                               "the split-f16 MFMA path applies, so precision 'bf16x3' runs the "
                                "FP64 labeler here; the gain is from batching the partitions",
            "plain_labeling": "FP32 direct difference, one K-Means call per partition",
            "batched_bf16_ms": tb, "plain_fp32_ms": tp, "speedup": tp / tb,
