@@ -49,9 +49,9 @@ namespace {
 
 // ------------------------------------------------- split-f16 MFMA labeling
 // Layout of the split rows (points in registers, centroids in memory and
-// LDS). Every operand is scaled by a power of two (a point by its own row's
-// largest coordinate, the centroids of a partition by theirs) into f16's
-// normal range and split into two f16 halves, v = h + l + e; halves below
+// LDS). Every operand is scaled by a power of two (the centroids of a partition
+// by their largest coordinate, the points of a workgroup by that of most of
+// its rows, see kApart) into f16's normal range and split into two f16 halves, v = h + l + e; halves below
 // f16's smallest normal value are zero, so no product meets a subnormal. Three
 // products h.h + h.l + l.h make the contraction. For d where it saves MFMA
 // steps the three pieces are laid end to end over one K axis of 3 d entries
@@ -342,6 +342,34 @@ __device__ __forceinline__ void resolve16(const float* __restrict__ X, int d,
 // MFMAs with point_bound1, for the first pass of a cascade. LIST: the points
 // are the rows of a flag list. FUSE (one partition): the group is resolved in
 // the kernel and labels and dists are final.
+//
+// The points' scale: one for the workgroup, so that a tile's accumulators start
+// from one value per centroid, whatever the point. Where the rows' largest
+// coordinates lie within 2^kApart of each other (ordinary data) it is the
+// largest row's. f16's smallest normal value cuts low halves off at 2^-14; the
+// largest coordinate of the smallest such row is 2^2 or more, so 2^-16 of it
+// stay, what two bf16 halves would leave. Where some lie further apart (a fill
+// value, a heavy tail) the scale is the one that leaves the fewest rows to the
+// re-scoring, by scale_cost: rows below it have wider bounds, rows above it
+// overflow to infinite halves, so that their norms and bounds are infinite or
+// NaN. An outlier then costs itself and not the rows beside it: with one row in
+// 128 2^40 times the others, 300,007 x 37-d and 501 centroids take 196 us (168
+// without; 1633 when the largest row's scale served all), 1,000,000 x 64-d and
+// 2048 centroids 1.7 ms (0.72; 27.7).
+constexpr int kApart = 12;
+// The cost of a scale with exponent e for the rows' own exponents (hist: rows
+// by exponent, upto: rows with this exponent or a smaller one): the share of
+// 256 rows like it that the bound cannot certify, 2^(k - 13) of them for a row
+// whose own scale is 2^k times this one (300,007 x 37-d: 0.2% at k = 0, 1% at
+// 14). A row that overflows counts twice: it is far from everything, and the
+// re-scoring's screen seldom spares such a row a centroid.
+template <typename U32>
+__device__ __forceinline__ uint32_t scale_cost(int e, const U32* hist, const U32* upto) {
+  uint32_t cost = e > 1 ? 512u * upto[e - 2] : 0u;
+  for (int k = kApart + 1; k <= kApart + 8; ++k)
+    if (e + k < 256) cost += hist[e + k] << (k - 13);
+  return cost + 256u * (upto[255] - upto[min(e + kApart + 8, 255)]);
+}
 constexpr uint64_t kFlagRow = (1ull << 40) - 1;
 template <int KS, bool SPLIT, int MB, int WPE, int TERMS = 3, bool FUSE = false,
           bool LIST = false>
@@ -363,7 +391,14 @@ void k_label_f16x3(
   uint16_t* s_c = reinterpret_cast<uint16_t*>(s_raw);
   __shared__ __align__(16) float s_nc[2][kBN];
   __shared__ float s_st[4 * MB * 16][4];  // row statistics of point_bound
-  __shared__ float s_mx[kLB / kWave];
+  constexpr int kRows = (kLB / kWave) * MB * 16;  // rows of a workgroup
+  __shared__ uint32_t s_rng[kLB / kWave], s_key[2][kLB / kWave];
+  // the exponents of the scales the rows would have alone, how many have each
+  // and how many up to each (before the tiles need the room)
+  static_assert((kRows + 512) * 4 <= kTiles && kLB == 256, "an exponent a thread");
+  typedef uint32_t __attribute__((may_alias)) u32_lds;
+  u32_lds* s_ex = reinterpret_cast<u32_lds*>(s_raw);
+  u32_lds *s_hist = s_ex + kRows, *s_upto = s_hist + 256;
   const int t = threadIdx.x;
   const int w = t / kWave;
   const int l = lane_id();
@@ -376,12 +411,13 @@ void k_label_f16x3(
   const int pz = (int)((int64_t)P * (blockIdx.y + 1) / gridDim.y);
 
   // Point fragments and row statistics, one block of 16 rows at a time: four
-  // lanes per row split its coordinates (scaled by one power of two for the
-  // block's points) into the wave's sixteen rows of the second centroid buffer (free until the first tile is done), from which
+  // lanes per row split its scaled coordinates into the wave's sixteen rows of the second centroid buffer (free until the first tile is done), from which
   // the fragments are read back. (Split straight into the fragments, the
   // loads and conditions of all blocks together spill.)
   f16x8 pf[MB][NF];
-  float mx = 0.f;
+  // largest exponent and largest 255 - exponent of the rows' scales
+  typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+  u16x2 rng = {0, 0};
   // coordinates are loaded four at a time (the last piece of a row moved back
   // to end with it), halves stored eight bytes at a time where d allows
   const bool x4 = (d & 3) == 0;
@@ -389,18 +425,55 @@ void k_label_f16x3(
   for (int pb = 0; pb < MB; ++pb) {
     const int64_t row = p0 + pb * 16 + (l >> 2);
     const float* xr = X + row_id(row < n ? row : n - 1) * d;
+    float mx = 0.f;
     for (int j = 4 * (l & 3); j < d; j += 16) {
       const f32x4 v = *reinterpret_cast<const f32x4_u*>(xr + min(j, d - 4));
       mx = fmaxf(fmaxf(mx, fabsf(v[0])), fmaxf(fabsf(v[1]), fmaxf(fabsf(v[2]), fabsf(v[3]))));
     }
+    // the four lanes of a row (quad permutations: lane ^ 1, lane ^ 2)
+    mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0xb1, 0xf,
+                                                              0xf, true)));
+    mx = fmaxf(mx, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(mx), 0x4e, 0xf,
+                                                              0xf, true)));
+    // (0: zeros, which any scale takes)
+    const uint32_t ex = mx == 0.f ? 0u : __float_as_uint(pow2_scale(mx)) >> 23;
+    if ((l & 3) == 0) s_ex[(w * MB + pb) * 16 + (l >> 2)] = ex;
+    if (ex) rng = __builtin_elementwise_max(rng, u16x2{(uint16_t)ex, (uint16_t)(255u - ex)});
   }
 #pragma unroll
-  for (int off = kWave / 2; off > 0; off >>= 1) mx = fmaxf(mx, __shfl_xor(mx, off, kWave));
-  if (l == 0) s_mx[w] = mx;
+  for (int off = 4; off < kWave; off <<= 1)
+    rng = __builtin_elementwise_max(
+        rng, __builtin_bit_cast(
+                 u16x2, __shfl_xor(__builtin_bit_cast(uint32_t, rng), off, kWave)));
+  if (l == 0) s_rng[w] = __builtin_bit_cast(uint32_t, rng);
   __syncthreads();
 #pragma unroll
-  for (int u = 0; u < kLB / kWave; ++u) mx = fmaxf(mx, s_mx[u]);
-  const float sx = pow2_scale(mx), isx = 1.0f / sx;  // exact: powers of two
+  for (int u = 0; u < kLB / kWave; ++u)
+    rng = __builtin_elementwise_max(rng, __builtin_bit_cast(u16x2, s_rng[u]));
+  uint32_t ex = rng.x ? 255u - rng.y : 127u;
+  if (rng.x > ex + kApart) {  // uniform over the block
+    s_hist[t] = 0;
+    __syncthreads();
+    if (t < kRows && s_ex[t]) atomicAdd((uint32_t*)&s_hist[s_ex[t]], 1u);
+    __syncthreads();
+    uint32_t upto = wave_incl_scan_dpp((uint32_t)s_hist[t]);
+    if (l == kWave - 1) s_key[0][w] = upto;
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < kLB / kWave; ++u) upto += u < w ? s_key[0][u] : 0u;
+    s_upto[t] = upto;
+    __syncthreads();
+    uint32_t key = s_hist[t] ? scale_cost(t, s_hist, s_upto) << 8 | (uint32_t)t : ~0u;
+#pragma unroll
+    for (int off = kWave / 2; off > 0; off >>= 1) key = min(key, __shfl_xor(key, off, kWave));
+    if (l == 0) s_key[1][w] = key;
+    __syncthreads();  // (and the tiles may have their room)
+#pragma unroll
+    for (int u = 0; u < kLB / kWave; ++u) key = min(key, s_key[1][u]);
+    ex = key & 255u;
+  }
+  const float sx = __uint_as_float(ex << 23);
+  const float isx = 1.0f / sx;  // exact: powers of two
   uint16_t* sw = s_c + kBN * LROW + w * 16 * LROW;
 #pragma unroll
   for (int pb = 0; pb < MB; ++pb) {
@@ -483,10 +556,12 @@ void k_label_f16x3(
     if ((l & 3) == 0) {  // norms rounded up: the bound stays rigorous
       float* st = s_st[w * MB * 16 + pb * 16 + (l >> 2)];
       const float up = (1.f + 4e-5f) * isx;
-      st[0] = sqrtf(s2) * up;
-      st[1] = sqrtf(sh) * up;
-      st[2] = sqrtf(sl) * up;
-      st[3] = sqrtf(se) * up;
+      // d squares that went to zero (below the smallest normal value) are less
+      const float gone = (float)d * 1.17549435e-38f;
+      st[0] = sqrtf(s2 + gone) * up;
+      st[1] = sqrtf(sh + gone) * up;
+      st[2] = sqrtf(sl + gone) * up;
+      st[3] = sqrtf(se + gone) * up;
     }
 #pragma unroll
     for (int f = 0; f < NF; ++f)
