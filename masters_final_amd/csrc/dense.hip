@@ -117,9 +117,10 @@ __global__ __launch_bounds__(256, PLANES ? 4 : 2) void k_dense_counts(
     const int32_t* __restrict__ labels, int64_t n, int P, int condensed,
     const uint32_t* __restrict__ planes, const int32_t* __restrict__ bits, int64_t npad,
     T* __restrict__ out, unsigned int* __restrict__ max_count) {
-  // workgroups go to the XCDs in turn: rows of tiles up and down over them
-  const int cols = (int)((n + kCC - 1) / kCC), xcd = blockIdx.x % 8, at = blockIdx.x / 8;
-  const int turn = at / cols, ti = turn * 8 + (turn & 1 ? 7 - xcd : xcd), tj = at % cols;
+  // workgroups go to the XCDs in turn (eight a column of tiles): rows of tiles
+  // up and down over them
+  const int turn = blockIdx.y, xcd = blockIdx.x % 8, tj = blockIdx.x / 8;
+  const int ti = turn * 8 + (turn & 1 ? 7 - xcd : xcd);
   const int64_t i0 = (int64_t)ti * kDT, j0 = (int64_t)tj * kCC;
   if (i0 >= n || j0 + kCC <= i0) return;  // below the diagonal (block-uniform)
   __shared__ __align__(16) uint32_t s_r[kPlanes][kDT];
@@ -1187,7 +1188,8 @@ void launch_counts(const int32_t* labels, int64_t n, int32_t P, int32_t condense
                    const uint32_t* planes, const int32_t* bits, void* out, unsigned int* mx,
                    hipStream_t s) {
   const int64_t tiles = (n + kDT - 1) / kDT;
-  const unsigned g = (unsigned)((tiles + 7) / 8 * 8 * ((n + kCC - 1) / kCC));
+  // (two dimensions: one takes fewer than 2^32 threads, n = 370,727)
+  const dim3 g((unsigned)(8 * ((n + kCC - 1) / kCC)), (unsigned)((tiles + 7) / 8));
   auto f = planes ? k_dense_counts<T, ADD, true> : k_dense_counts<T, ADD, false>;
   f<<<g, 256, 0, s>>>(labels, n, P, condensed, planes, bits, tiles * kDT, static_cast<T*>(out), mx);
 }
