@@ -39,7 +39,8 @@ __global__ __launch_bounds__(kGH) void k_group_hist(const int32_t* __restrict__ 
                                                     int64_t chunk, int64_t nch,
                                                     int32_t* __restrict__ T, int64_t last,
                                                     unsigned int* __restrict__ bad) {
-  extern __shared__ int32_t s_g[];
+  extern __shared__ int32_t s_dyn[];
+  int32_t* const s_g = s_dyn;
   const int64_t i0 = (int64_t)blockIdx.x * chunk;
   const int64_t i1 = i0 + chunk < n ? i0 + chunk : n;
   const int32_t z0 = (int32_t)blockIdx.z * kGRange;
@@ -73,7 +74,10 @@ __global__ __launch_bounds__(kWave) void k_group_place(
     const int32_t* __restrict__ labels, int64_t n, int P, const int64_t* __restrict__ k_off,
     int64_t chunk, int64_t nch, const int32_t* __restrict__ T, int64_t last,
     uint32_t* __restrict__ members, uint32_t* __restrict__ start, int32_t* __restrict__ pos) {
-  extern __shared__ int32_t s_g[];  // next position of each cluster
+  extern __shared__ int32_t s_dyn[];
+  // next position of each cluster: lanes read what other lanes of the wavefront
+  // wrote a step before, so every access is made, in order
+  volatile int32_t* const s_g = s_dyn;
   const int ln = threadIdx.x;
   const int64_t i0 = (int64_t)blockIdx.x * chunk;
   const int64_t i1 = i0 + chunk < n ? i0 + chunk : n;
@@ -122,7 +126,7 @@ __global__ __launch_bounds__(kWave) void k_group_place(
           at = (uint32_t)s_g[c] + rank;
           // the lane ranked last moves the cluster's position on (the reads
           // of this step come first: one wavefront's LDS operations complete
-          // in order)
+          // in the order they are made)
           if ((peers >> ln) == 1ull) s_g[c] = (int32_t)at + 1;
           members[at] = (uint32_t)i;
         }
