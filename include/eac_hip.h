@@ -414,7 +414,8 @@ int eac_coassoc_fill_ranked(const int32_t* labels, int64_t n, const int64_t* h_k
  *   the caller allocates a staging buffer of
  *     eac_coassoc_stage_bytes(n, full_rows, P, pool_entries) bytes: room
  *     for pool_entries staged entries (the estimate plus a margin) beyond
- *     the workgroups' partly used chunks;
+ *     the workgroups' partly used chunks, or, from n (n - 1) / 2 entries on
+ *     (full rows: n (n - 1)), a place for every pair and no more;
  *   eac_coassoc_stage (same ws, unchanged): indptr[n+1], h_nnz, largest
  *     count; h_nnz = -1 when the pool was too small (then build with
  *     eac_coassoc_count + eac_coassoc_fill);

@@ -103,16 +103,16 @@ struct CoPlan {
 // Outputs of the row kernel (pointers a pass does not use are null).
 struct CoOut {
   unsigned long long* row_ctr;  // row counters kCtrPad apart, zeroed
-  int32_t* row_nnz;             // PASS 0 / 2: nnz of each row
-  unsigned int* max_count;      // PASS 0 / 2: largest count
+  int32_t* row_nnz;             // PASS 0, 2, 3: nnz of each row
+  unsigned int* max_count;      // PASS 0, 2, 3: largest count
   unsigned long long* nnz_sum;  // PASS 0: sum of the visited rows' nnz
   const int64_t* indptr;        // PASS 1: row offsets
   int32_t w_offset;             // PASS 1: data = w_offset - count when non-zero
   int32_t* col;                 // PASS 1: columns
   int32_t* val;                 // PASS 1: counts (or w_offset - count)
   int32_t* rank;                // PASS 1 with RANK: first partition rank
-  uint32_t* pool;               // PASS 2: staged entries (count << 16 | column - c0)
-  uint64_t* seg;                // PASS 2: per (row, window) offset << 16 | entries
+  uint32_t* pool;               // PASS 2, 3: staged entries (count << 16 | column - c0)
+  uint64_t* seg;                // PASS 2, 3: per (row, window) offset << 16 | entries
   unsigned long long* pool_ctr; // PASS 2: next free pool chunk
   int64_t pool_cap;             // PASS 2: pool entries
   int64_t pool_chunk;           // PASS 2: entries per chunk (>= win)
@@ -120,8 +120,17 @@ struct CoOut {
 };
 
 // Staged entries are taken from the pool in chunks (one global atomic per
-// chunk) of up to this many, or 16 windows when that is more.
+// chunk) of up to this many, or 16 windows when that is more. A pool of
+// co_pairs entries needs no chunks: row i's entries of columns from c on start
+// at co_pair_at(i, c), after a place for every pair before them.
 constexpr int64_t kPoolChunk = 65536;
+__host__ __device__ inline int64_t co_pairs(int64_t n, int full_rows) {
+  return full_rows ? n * (n - 1) : n * (n - 1) / 2;
+}
+__host__ __device__ inline int64_t co_pair_at(int64_t i, int64_t c, int64_t n, int full_rows) {
+  if (full_rows) return i * (n - 1) + c - (c > i ? 1 : 0);
+  return i * (n - 1) - i * (i - 1) / 2 + (c > i + 1 ? c - (i + 1) : 0);
+}
 
 // Segment-table slot of (row i, first window of the row): rows keep the
 // windows from w0(i) = (i + 1) / win on (every window with full rows), so
@@ -220,11 +229,13 @@ struct CoCnt {
 // (count << 16 | column - c0), the window's (pool offset, entries) to the
 // segment table, and the row's nnz and the max count as in PASS 0; a
 // workgroup that finds the pool used up sets the overflow flag and stops.
+// PASS 3: the same with a place for every pair in the pool (co_pair_at).
 // U: member loads in flight per lane while visiting (4 or 8, a tuning knob).
 template <int PASS, bool RANK, int U, typename CT>
 __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, int win,
                                                       CoOut out) {
   using Cnt = CoCnt<CT>;
+  constexpr bool STAGE = PASS >= 2;
   unsigned long long* __restrict__ row_ctr = out.row_ctr;
   const int64_t* __restrict__ indptr = out.indptr;
   const int32_t w_offset = out.w_offset;
@@ -345,7 +356,7 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
     int64_t written = 0;
     // PASS 2: the row's first segment-table slot and its first window
     const int64_t w_first = full_rows ? 0 : (i + 1) / win;
-    const int64_t seg0 = PASS == 2 ? seg_base(i, win, pl.nw, full_rows) : 0;
+    const int64_t seg0 = STAGE ? seg_base(i, win, pl.nw, full_rows) : 0;
     uint32_t nnz_local = 0;
     const int self = full_rows ? (int)i : -1;  // full rows skip the diagonal
     // windows aligned to multiples of win (columns <= i get no counts)
@@ -532,7 +543,7 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
           }
         }
         nnz_local += c;
-      } else {  // PASS 1 and 2
+      } else {  // PASS 1, 2 and 3
         // Wave w emits lane pieces (two groups each) [w*RG, (w+1)*RG) in
         // column order. First the non-zero masks of its pieces (kept in
         // registers: a window has few entries, about one column in twenty
@@ -566,8 +577,10 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
           if (q < wv) o += s_tmp[q];
           wtot += s_tmp[q];
         }
-        if (PASS == 2) {  // block-uniform: wtot, chunk_pos, chunk_end
-          if (chunk_pos + (int64_t)wtot > chunk_end) {
+        if (STAGE) {  // block-uniform: wtot, chunk_pos, chunk_end
+          if (PASS == 3) {
+            chunk_pos = co_pair_at(i, c0, n, full_rows);
+          } else if (chunk_pos + (int64_t)wtot > chunk_end) {
             if (t == 0) s_chunk = atomicAdd(out.pool_ctr, (unsigned long long)out.pool_chunk);
             __syncthreads();
             chunk_pos = (int64_t)s_chunk;
@@ -583,7 +596,7 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
                 wtot ? ((uint64_t)chunk_pos << 16) | (uint64_t)wtot : 0ull;
           chunk_pos += wtot;
         }
-        uint32_t* __restrict__ po = PASS == 2 ? out.pool + o : nullptr;
+        uint32_t* __restrict__ po = STAGE ? out.pool + o : nullptr;
         int32_t* __restrict__ pc = PASS == 1 ? out_col + o : nullptr;
         int32_t* __restrict__ pv = PASS == 1 ? out_val + o : nullptr;
         int32_t* __restrict__ pr = PASS == 1 && RANK ? out_rank + o : nullptr;
@@ -604,7 +617,7 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
             const int col = colg + __builtin_ctz(m);
             m &= m - 1u;
             const uint32_t v = s_ct[col];
-            if (PASS == 2) {
+            if (STAGE) {
               po[at] = (v << 16) | (uint32_t)col;
               mx_row = max(mx_row, v);
             } else {
@@ -632,10 +645,10 @@ __global__ __launch_bounds__(kCB) void k_coassoc_rows(CoPlan pl, int full_rows, 
         if (out.nnz_sum) atomicAdd(out.nnz_sum, (unsigned long long)rt);
       }
     }
-    if (PASS == 2 && t == 0) out.row_nnz[i] = (int32_t)written;
+    if (STAGE && t == 0) out.row_nnz[i] = (int32_t)written;
     __syncthreads();
   }
-  if (PASS == 0 || PASS == 2) {
+  if (PASS != 1) {
     if (mx_row) atomicMax(&s_max, mx_row);
     __syncthreads();
     if (t == 0 && s_max) atomicMax(out.max_count, s_max);
@@ -1030,6 +1043,15 @@ StageLayout stage_layout(int64_t n, int full_rows) {
   L.chunk = c < 16 * (int64_t)L.win ? 16 * (int64_t)L.win : c;
   return L;
 }
+// Entries per chunk for a staging buffer of these bytes, -1: it does not hold
+// one. 0: a place for every pair (PASS 3), for the bytes
+// eac_coassoc_stage_bytes gives for that, or rounded up to a page (a larger
+// buffer was sized as entries and chunks).
+int64_t stage_chunk(const StageLayout& L, int64_t n, int full_rows, size_t stage_bytes) {
+  const size_t all = L.pool_at + (size_t)co_pairs(n, full_rows) * 4;
+  if (stage_bytes >= all && stage_bytes < all + 4096) return 0;
+  return stage_bytes >= L.pool_at + (size_t)L.chunk * 4 ? L.chunk : -1;
+}
 }  // namespace
 }  // namespace eac
 
@@ -1087,14 +1109,17 @@ extern "C" int eac_coassoc_estimate(const int32_t* labels, int64_t n, const int6
 }
 
 // Bytes of the staging buffer with room for pool_entries staged entries
-// beyond the partly used chunks of the workgroups (the segment table and
-// the chunk size depend on n, full_rows and the window knob).
+// beyond the partly used chunks of the workgroups, or for every pair and no
+// more (the segment table and the chunk size depend on n, full_rows and the
+// window knob).
 extern "C" size_t eac_coassoc_stage_bytes(int64_t n, int32_t full_rows, int32_t P,
                                           int64_t pool_entries) {
   if (n < 1) n = 1;
   if (P < 1) P = 1;
   if (pool_entries < 0) pool_entries = 0;
   const StageLayout L = stage_layout(n, full_rows);
+  const int64_t pairs = co_pairs(n, full_rows);
+  if (pool_entries >= pairs) return L.pool_at + (size_t)pairs * 4;
   const int64_t grid = co_grid<2>(L.win, P);
   return L.pool_at + (size_t)(pool_entries + (grid + 1) * L.chunk) * 4;
 }
@@ -1113,7 +1138,8 @@ extern "C" int eac_coassoc_stage(const int32_t* labels, int64_t n, const int64_t
   if (!ws || ws_bytes < need)
     return fail(EAC_ERR_WORKSPACE, "coassoc: workspace %zu < %zu bytes", ws_bytes, need);
   const StageLayout SL = stage_layout(n, full_rows);
-  if (stage_bytes < SL.pool_at + (size_t)SL.chunk * 4)
+  const int64_t chunk = stage_chunk(SL, n, full_rows, stage_bytes);
+  if (chunk < 0)
     return fail(EAC_ERR_WORKSPACE, "coassoc: staging buffer %zu < %zu bytes", stage_bytes,
                 SL.pool_at + (size_t)SL.chunk * 4);
   hipStream_t s = (hipStream_t)stream;
@@ -1136,10 +1162,12 @@ extern "C" int eac_coassoc_stage(const int32_t* labels, int64_t n, const int64_t
   o.pool = reinterpret_cast<uint32_t*>(st + SL.pool_at);
   o.pool_ctr = reinterpret_cast<unsigned long long*>(hdr + 2);
   o.pool_cap = (int64_t)((stage_bytes - SL.pool_at) / 4);
-  o.pool_chunk = SL.chunk;
+  o.pool_chunk = chunk;
   o.overflow = reinterpret_cast<unsigned int*>(hdr + 3);
   int pr = prof_begin(EAC_PROF_CO_STAGE, 0, s);
-  EAC_TRY(co_launch<2>(pl, full_rows, SL.win, o, s));
+  // (PASS 3 apart: the choice inside PASS 2 cost its emission 1.7%)
+  EAC_TRY(chunk ? co_launch<2>(pl, full_rows, SL.win, o, s)
+                : co_launch<3>(pl, full_rows, SL.win, o, s));
   prof_end(pr, s);
   EAC_TRY((scan_excl<int32_t, int64_t>(B.row_nnz, indptr, n + 1, 0, nullptr, ar, s)));
   ar.used = mark;
@@ -1222,7 +1250,8 @@ extern "C" int eac_coassoc_graph(const int32_t* labels, int64_t n, const int64_t
   if (w_offset < -1) return fail(EAC_ERR_ARG, "coassoc graph: w_offset < -1");
   const int64_t ktot = h_koff[P];
   const StageLayout SL = stage_layout(n, full_rows);
-  if (stage_bytes < SL.pool_at + (size_t)SL.chunk * 4)
+  const int64_t chunk = stage_chunk(SL, n, full_rows, stage_bytes);
+  if (chunk < 0)
     return fail(EAC_ERR_WORKSPACE, "coassoc graph: staging buffer %zu < %zu bytes", stage_bytes,
                 SL.pool_at + (size_t)SL.chunk * 4);
   hipStream_t s = (hipStream_t)stream;
@@ -1245,10 +1274,12 @@ extern "C" int eac_coassoc_graph(const int32_t* labels, int64_t n, const int64_t
   o.pool = reinterpret_cast<uint32_t*>(st + SL.pool_at);
   o.pool_ctr = reinterpret_cast<unsigned long long*>(hdr + 2);
   o.pool_cap = (int64_t)((stage_bytes - SL.pool_at) / 4);
-  o.pool_chunk = SL.chunk;
+  o.pool_chunk = chunk;
   o.overflow = reinterpret_cast<unsigned int*>(hdr + 3);
   int pr = prof_begin(EAC_PROF_CO_STAGE, 0, s);
-  EAC_TRY(co_launch<2>(pl, full_rows, SL.win, o, s));
+  // (PASS 3 apart: the choice inside PASS 2 cost its emission 1.7%)
+  EAC_TRY(chunk ? co_launch<2>(pl, full_rows, SL.win, o, s)
+                : co_launch<3>(pl, full_rows, SL.win, o, s));
   prof_end(pr, s);
   EAC_TRY((scan_excl<int32_t, int64_t>(B.row_nnz, indptr, n + 1, 0, nullptr, ar, s)));
   ar.used = mark;
