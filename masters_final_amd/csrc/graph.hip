@@ -3346,11 +3346,14 @@ int sl_impl(const int32_t* dest, const W* weight, const int64_t* fe, const int32
   return EAC_OK;
 }
 
-// One graph of up to kSegN vertices: the same cut from the batch's kernels
+// One graph of up to kOneCutN vertices: the same cut from the batch's kernels
 // (a batch of one), enqueued behind the rounds without a read-back. The form
 // above reads five times between its kernels, 14 us each (the whole EAC of
-// 10,000 points: 1175 -> 1083 us); it stays for larger graphs, whose forest
-// one workgroup would take too long over.
+// 10,000 points: 1175 -> 1083 us); it stays for larger graphs, over whose
+// forest one workgroup takes longer than that: geometric graphs of degree 6
+// to 30, this against the other, 10,000 vertices 229 and 275 us, 20,000 408
+// and 461, 30,000 444 and 479, 45,000 490 and 510, 65,000 555 and 530.
+constexpr int kOneCutN = 49152;
 struct SlRecord {
   GraphCut cut;
   int64_t goff[2], seg[2];
@@ -3721,7 +3724,7 @@ struct SlRun {
                  int32_t n, int64_t m, int symmetric, int rule, double max_dist,
                  int32_t n_clusters, int32_t* labels, int64_t* h_out, void* ws, size_t ws_bytes,
                  hipStream_t s) {
-    if (n <= kSegN)
+    if (n <= kOneCutN)
       return sl_small<W, HAS_OD>(dest, (const W*)weight, fe, od, n, m, symmetric, rule, max_dist,
                                  n_clusters, labels, h_out, ws, ws_bytes, s);
     return sl_impl<W, HAS_OD>(dest, (const W*)weight, fe, od, n, m, symmetric, rule, max_dist,
