@@ -1308,7 +1308,9 @@ __device__ __forceinline__ double min_of(double a, double b) { return __builtin_
 // FP64: 35 us with one point a lane, 31 with two, 26 in fours. 300,000 points
 // and 300 centroids, a call in FP64 (FP32), one by one and in fours: 62 and 51
 // us in 1-D (53 and 47), 94 and 85 in 4-D (61 and 58), but 124 and 136 in 8-D,
-// 223 and 234 in 16-D (111 and 128), where the loads of four rows stall.
+// 223 and 234 in 16-D (111 and 128), where the loads of four rows stall. Beyond
+// 64 dimensions the point alone fills the registers and a centroid is taken at a
+// time: 200,000 x 128-d and 500 centroids in FP64 5.42 ms, two at a time 5.64.
 template <typename T, int DX, int PT>
 __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ X, int64_t n,
                                                       int d, const float* __restrict__ C,
@@ -1386,7 +1388,7 @@ __global__ __launch_bounds__(256) void k_label_direct(const float* __restrict__ 
             bl[q] = base + bg[q] + at;
           }
       } else {
-#pragma unroll 2
+#pragma unroll (DX > 64 ? 1 : 2)
         for (; r < rows; ++r) {
 #pragma unroll
           for (int q = 0; q < PT; ++q) {
