@@ -1885,9 +1885,12 @@ int mst_rounds(MstBuffers& B, int32_t n, int r0, int count, MstRecs& rec, hipStr
 // whole call, launches against this: 600 vertices of degree 6 207 -> 81 us,
 // the mesh 346 -> 201, 15,900 vertices of degree 12 (191,000 entries) 349 ->
 // 242; at degree 24 (382,000 entries) launches take 280, this took 347: one
-// compute unit then has too many keys.
+// compute unit then has too many keys. A graph whose entries are all keys (not
+// passed as symmetric) has twice as many: up to kOneMAll entries, where both
+// take as long (16,000 vertices: 151,000 entries 0.79 of the launches' time,
+// 179,000 0.83 to 1.00, 214,000 0.98 to 1.11, 249,000 1.05 to 1.18).
 constexpr int32_t kOneN = 16000;
-constexpr int64_t kOneM = 1 << 18;
+constexpr int64_t kOneM = 1 << 18, kOneMAll = 176 << 10;
 constexpr int kOneT = 1024, kOneW = kOneT / kWave;
 inline size_t one_lds(int32_t n) { return (size_t)n * 8 + ((size_t)n * 2 + 15) / 16 * 16; }
 
@@ -2280,7 +2283,9 @@ __global__ __launch_bounds__(kOneT) void k_mst_one(
   for (int v = t; v < n; v += kOneT) labels[v] = s_rank[s_first[s_par[v]]];
 }
 
-inline bool one_fits(int32_t n, int64_t m) { return n <= kOneN && m <= kOneM; }
+inline bool one_fits(int32_t n, int64_t m, int symmetric) {
+  return n <= kOneN && m <= (symmetric ? kOneM : kOneMAll);
+}
 
 // All rounds, the forest keys and the labels of a small graph.
 int mst_one(MstBuffers& B, int32_t n, int enq, int32_t* d_nf, int32_t* labels, MstRecs& rec,
@@ -2390,7 +2395,7 @@ int mst_core(const int32_t* dest, const W* weight, const int64_t* fe, const int3
   const int64_t ftiles = (n + kGTile - 1) / kGTile;
   int32_t* d_nf = B.tile_cnt + ftiles;
   MstState hs;
-  const bool one = one_fits(n, m);
+  const bool one = one_fits(n, m, symmetric);
   if (one) {
     enq = graph_mode ? fixed_rounds : kMaxRounds;
     EAC_TRY(mst_one(B, n, enq, d_nf, nullptr, rec, s));
@@ -2539,7 +2544,7 @@ int mst_impl(const int32_t* dest, const W* weight, const int64_t* fe, const int3
   int32_t* d_nf = B.tile_cnt + ftiles;
   MstRecs rec;
   EAC_TRY((mst_begin<W, HAS_OD>(dest, weight, fe, od, n, m, symmetric, B, rec, s)));
-  if (one_fits(n, m)) {
+  if (one_fits(n, m, symmetric)) {
     const int enq = kMaxRounds;
     EAC_TRY(mst_one(B, n, enq, d_nf, labels, rec, s));
     if (n > 1 && (ids || wout)) {
@@ -3408,7 +3413,7 @@ int sl_small(const int32_t* dest, const W* weight, const int64_t* fe, const int3
   int32_t* d_nf = B.tile_cnt + ftiles;
   MstRecs recs;
   EAC_TRY((mst_begin<W, HAS_OD>(dest, weight, fe, od, n, m, symmetric, B, recs, s)));
-  const bool one = one_fits(n, m);
+  const bool one = one_fits(n, m, symmetric);
   int key_bits = 8 * (int)sizeof(W) + 2 * vb;
   key_bits = key_bits < 64 ? key_bits : 64;
   const size_t lds = 2 * (size_t)(n < 8 ? 8 : n);
