@@ -835,18 +835,26 @@ __device__ __forceinline__ void screen_bounds(int d, float& R, float& A) {
 // thread that may hold more candidates than it kept makes the block score
 // every centroid in FP64.
 // The flags are a list (nflag or *d_nflag of them), or (cnt) still lie in the
-// regions of the labeling; then more than kFewMax are left alone.
+// regions of the labeling; then kFewMax or more are left alone.
+// BS threads: 256 while flags are few, and the workgroups for them too; many
+// flags of partitions of up to kRfOneK centroids, most of which would leave
+// lanes of four wavefronts idle, go by one wavefront each, four times as many
+// workgroups at a time. 30,000 x 100-d points with 14,000 to 27,000 flags, 10
+// partitions of 30 centroids: a call 366 and 263 us, 150: 486 and 374, 600: 756
+// and 626, 1500: 1138 and 1219; one of 100,000 x 64-d with 22,000 to 47,000
+// flags, 40: 210 and 128, 500: 385 and 224, 1000: 407 and 388; but with 200
+// flags, 100 centroids 102 and 114, 500 123 and 136.
 constexpr int kRfF = 4;
-constexpr int64_t kFewMax = 65536;
-template <int F>
-__global__ __launch_bounds__(256, 4) void k_rescore_few(
+constexpr int64_t kFewMax = 8192, kRfOneK = 600;
+template <int F, int BS>
+__global__ __launch_bounds__(BS, 4) void k_rescore_few(
     const float* __restrict__ X, int64_t n, int d, const float* __restrict__ C,
     const float* __restrict__ Ct, int64_t ktot, const int64_t* __restrict__ k_off,
     const uint64_t* __restrict__ list, int64_t nflag, int32_t* __restrict__ labels,
     float* __restrict__ dists, const int64_t* __restrict__ d_nflag,
     const unsigned long long* __restrict__ cnt, int64_t region) {
   constexpr int U = 4;  // centroids per thread and pass
-  constexpr int NW = 256 / kWave;
+  constexpr int NW = BS / kWave;
   __shared__ float s_x[128 * F];
   __shared__ uint64_t s_f[F];
   __shared__ float s_min[F][NW];
@@ -893,7 +901,7 @@ __global__ __launch_bounds__(256, 4) void k_rescore_few(
         x[q] = X + (int64_t)(s_f[f] & kFlagRow) * d;
       }
       __syncthreads();  // the previous run's rows and results are consumed
-      for (int j = t; j < d; j += 256)
+      for (int j = t; j < d; j += BS)
 #pragma unroll
         for (int q = 0; q < F; ++q) s_x[j * F + q] = x[q][j];
       __syncthreads();
@@ -906,18 +914,18 @@ __global__ __launch_bounds__(256, 4) void k_rescore_few(
         k1[q] = -1;
       }
       const bool any = kbeg + t < kend;  // this thread has a centroid
-      for (int64_t c0 = kbeg; c0 < kend; c0 += 256 * U) {
+      for (int64_t c0 = kbeg; c0 < kend; c0 += BS * U) {
         // U centroids a thread, every coordinate of theirs for all F points
         float a[U][F];
         const float* ct[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int64_t c = c0 + u * 256 + t;
+          const int64_t c = c0 + u * BS + t;
           ct[u] = Ct + (c < kend ? c : kend - 1);
 #pragma unroll
           for (int q = 0; q < F; ++q) a[u][q] = 0.f;
         }
-        const int nu = kend - c0 >= 256 * U ? U : (int)((kend - c0 + 255) / 256);  // uniform
+        const int nu = kend - c0 >= BS * U ? U : (int)((kend - c0 + BS - 1) / BS);  // uniform
         auto pass = [&](auto full_u) {
 #pragma unroll 4
           for (int j = 0; j < d; ++j) {
@@ -940,7 +948,7 @@ __global__ __launch_bounds__(256, 4) void k_rescore_few(
         else pass(std::false_type{});
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-          const int64_t c = c0 + u * 256 + t;
+          const int64_t c = c0 + u * BS + t;
           if (c < kend) {
 #pragma unroll
             for (int q = 0; q < F; ++q) {
@@ -984,7 +992,7 @@ __global__ __launch_bounds__(256, 4) void k_rescore_few(
           best[q] = DBL_MAX;
           bk[q] = -1;
         }
-        for (int64_t c = kbeg + t; c < kend; c += 256) {
+        for (int64_t c = kbeg + t; c < kend; c += BS) {
 #pragma unroll
           for (int q = 0; q < F; ++q) {
             const double a = dist2_f64(x[q], C + c * d, d, false);
@@ -2402,20 +2410,20 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
       else go(k_rescore_tiled<0>);
     } else {
       const int gr = grid_for(B.flag_cap, kRfF, 16384);
-      k_rescore_few<kRfF><<<gr, 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, B.flags, 0, labels,
-                                             dists, kg->d_nf, nullptr, 0);
+      k_rescore_few<kRfF, 256><<<gr, 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, B.flags, 0,
+                                                  labels, dists, kg->d_nf, nullptr, 0);
     }
     EAC_LAUNCH_CHECK();
     prof_end(pr2, s);
     k_fit_tally<<<1, 64, 0, s>>>(kg->info, kg->d_nf, nullptr, 0, kg->any);
     EAC_LAUNCH_CHECK();
   } else {
-  // One partition: the re-scoring of up to kFewMax flags needs no sorting and
+  // One partition: the re-scoring of fewer than kFewMax flags needs no sorting and
   // follows without a read-back, straight from the regions.
   if (P == 1) {
     int pr2 = prof_begin(EAC_PROF_KM_RESCORE, 0, s);
-    k_rescore_few<kRfF><<<1024, 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, B.flags_r, 0,
-                                             labels, dists, nullptr, B.nflag, B.region);
+    k_rescore_few<kRfF, 256><<<1024, 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, B.flags_r, 0,
+                                                  labels, dists, nullptr, B.nflag, B.region);
     EAC_LAUNCH_CHECK();
     prof_end(pr2, s);
   }
@@ -2451,13 +2459,14 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
       else if (d <= 64) go(k_rescore_tiled<64>);
       else go(k_rescore_tiled<0>);
     } else {
-      auto go = [&](auto kern, int f) {
-        kern<<<grid_for((int64_t)nf, f, 65536), 256, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, fl,
-                                                             (int64_t)nf, labels, dists, nullptr,
-                                                             nullptr, 0);
+      auto go = [&](auto kern, int f, int bs) {
+        kern<<<grid_for((int64_t)nf, f, 65536), bs, 0, s>>>(X, n, d, C, B.Ct, ktot, B.k_off, fl,
+                                                            (int64_t)nf, labels, dists, nullptr,
+                                                            nullptr, 0);
       };
-      if (sorted_flags) go(k_rescore_few<kRfF>, kRfF);
-      else go(k_rescore_few<1>, 1);
+      if (sorted_flags && ktot <= kRfOneK * P) go(k_rescore_few<kRfF, kWave>, kRfF, kWave);
+      else if (sorted_flags) go(k_rescore_few<kRfF, 256>, kRfF, 256);
+      else go(k_rescore_few<1, 256>, 1, 256);
     }
     EAC_LAUNCH_CHECK();
     prof_end(pr2, s);
