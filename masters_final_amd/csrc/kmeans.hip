@@ -826,6 +826,22 @@ __device__ __forceinline__ void screen_bounds(int d, float& R, float& A) {
   A = (float)d * 4.7e-38f;  // >= d * 2^-124
 }
 
+// The re-scorings' full pass over a subset of the centroids, which includes the
+// partition's first when `first`: strict < in ascending order. A NaN never
+// replaces a distance, and nothing replaces a NaN of the first centroid, which
+// stands here as -infinity (rescored_dist gives it back).
+__device__ __forceinline__ void full_min(double a, bool first, int32_t c, double& best,
+                                         int32_t& bk) {
+  if (first && a != a) a = -(double)INFINITY;
+  if (a < best || (bk < 0 && a == a)) {
+    best = a;
+    bk = c;
+  }
+}
+__device__ __forceinline__ float rescored_dist(double best) {
+  return best == -(double)INFINITY ? __builtin_nanf("") : (float)best;
+}
+
 // Re-scoring of few flagged points (d <= 128): a block takes up to F flags of
 // one partition at a time. Its threads hold U centroids each, read from the
 // transposed copy Ct [d][ktot] (64 consecutive floats per load), and walk the
@@ -914,6 +930,7 @@ __global__ __launch_bounds__(BS, 4) void k_rescore_few(
         k1[q] = -1;
       }
       const bool any = kbeg + t < kend;  // this thread has a centroid
+      bool full = false;
       for (int64_t c0 = kbeg; c0 < kend; c0 += BS * U) {
         // U centroids a thread, every coordinate of theirs for all F points
         float a[U][F];
@@ -946,6 +963,10 @@ __global__ __launch_bounds__(BS, 4) void k_rescore_few(
         };
         if (nu == U) pass(std::true_type{});
         else pass(std::false_type{});
+        if (c0 == kbeg && t == 0) {  // a NaN of the first centroid decides
+#pragma unroll
+          for (int q = 0; q < F; ++q) full = full || a[0][q] != a[0][q];
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
           const int64_t c = c0 + u * BS + t;
@@ -970,7 +991,6 @@ __global__ __launch_bounds__(BS, 4) void k_rescore_few(
       __syncthreads();
       double best[F];
       int32_t bk[F];
-      bool full = false;
 #pragma unroll
       for (int q = 0; q < F; ++q) {
         float m = s_min[q][0];
@@ -995,11 +1015,8 @@ __global__ __launch_bounds__(BS, 4) void k_rescore_few(
         for (int64_t c = kbeg + t; c < kend; c += BS) {
 #pragma unroll
           for (int q = 0; q < F; ++q) {
-            const double a = dist2_f64(x[q], C + c * d, d, false);
-            if (bk[q] < 0 || a < best[q]) {
-              best[q] = a;
-              bk[q] = (int32_t)(c - kbeg);
-            }
+            full_min(dist2_f64(x[q], C + c * d, d, false), c == kbeg, (int32_t)(c - kbeg),
+                     best[q], bk[q]);
           }
         }
       }
@@ -1034,7 +1051,7 @@ __global__ __launch_bounds__(BS, 4) void k_rescore_few(
         const int64_t o =
             (int64_t)p * n + (int64_t)(s_f[done + t] & kFlagRow);
         labels[o] = k;
-        if (dists) dists[o] = (float)b;
+        if (dists) dists[o] = rescored_dist(b);
       }
       __syncthreads();  // the shared results are consumed
       done = end;
@@ -1125,6 +1142,7 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
     };
     constexpr int NX = DX > 0 ? DX : 1;
     float xr[NX];
+    bool full = false;
     __syncthreads();  // the point rows are staged
     if constexpr (DX > 0) {
 #pragma unroll
@@ -1164,6 +1182,10 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
       stage(c0, rows);
       __syncthreads();
       if (!active) continue;
+      if (c0 == kbeg && sub == 0) {  // a NaN of the first centroid decides
+        const float a0 = screen(s_c);
+        full = a0 != a0;
+      }
       int c = sub;
       for (; c + kRtS < rows; c += 2 * kRtS) {
         const float a0 = screen(s_c + c * RC);
@@ -1175,7 +1197,6 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
     }
     s_v1[sub][g] = v1;
     __syncthreads();
-    bool full = false;
     {
       float m = s_v1[0][g];
       for (int q = 1; q < kRtS; ++q) m = fminf(m, s_v1[q][g]);
@@ -1186,14 +1207,14 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
         best = dist2_f64(xa, C + k1 * d, d, false);
         bk = (int32_t)(k1 - kbeg);
       }
-      full = active && (k1 < 0 || !(v2 > T));  // (NaN screens take the full pass)
+      full = full || (active && (k1 < 0 || !(v2 > T)));  // (NaN screens take the full pass)
       s_best[sub][g] = best;
       s_bk[sub][g] = bk;
     }
     // pass 2 (rare): every centroid in FP64 for the whole run
     if (__syncthreads_or(full)) {
       double best = DBL_MAX;
-      int64_t bk = -1;
+      int32_t bk = -1;
       for (int64_t c0 = kbeg; c0 < kend; c0 += kRtT) {
         const int rows = kend - c0 < kRtT ? (int)(kend - c0) : kRtT;
         __syncthreads();
@@ -1204,11 +1225,11 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
           const float* ca = s_c + c * RC;
           double a0 = 0.0;
           for (int j = 0; j < d; ++j) a0 = sq_acc(a0, (double)xa[j] - (double)ca[j]);
-          if (bk < 0 || a0 < best) { best = a0; bk = c0 + c; }
+          full_min(a0, c0 + c == kbeg, (int32_t)(c0 + c - kbeg), best, bk);
         }
       }
       s_best[sub][g] = best;
-      s_bk[sub][g] = bk < 0 ? -1 : (int32_t)(bk - kbeg);
+      s_bk[sub][g] = bk;
       __syncthreads();
     }
     if (active && sub == 0) {
@@ -1221,7 +1242,7 @@ __global__ __launch_bounds__(kRtF * kRtS) void k_rescore_tiled(
       }
       const int64_t o = (int64_t)p * n + (int64_t)(flags[f0 + g] & kRowMask);
       labels[o] = k;
-      if (dists) dists[o] = (float)b;
+      if (dists) dists[o] = rescored_dist(b);
     }
     __syncthreads();
     done = end;
