@@ -417,7 +417,7 @@ def run_kmeans(args):
     b = res["bf16x3"]
     flops = 2.0 * n * k * d
     out = base_line(args, flops / (b["ms"] * 1e-3) / 1e12, "TFLOP/s (2nkd)", b["ms"],
-                    "bf16x3->fp32, fp64 rescore",
+                    "f16 halves x3->fp32, fp64 rescore",
                     {"workload": "kmeans_label_gmm", "n": n, "d": d, "k": k, "seed": 2})
     out["result"] = {"bf16x3_ms": b["ms"], "fp32_ms": res["fp32"]["ms"],
                      "fp64_ms": res["fp64"]["ms"], "speedup_vs_fp32": res["fp32"]["ms"] / b["ms"],

@@ -39,8 +39,9 @@ def labels_from_ensemble(ensemble, n_samples):
 ONE_PASS_MIN_N = 65536  # from here on the estimate pass is cheap against a second visit
 # Below it one visit pays where the pool can hold every pair (4 bytes each and
 # nothing else but 8 bytes a row and window: 0.2 GB at 10,000 points, at most
-# 1 GiB at 23,170, 16,384 with full rows), so that no estimate is needed; 10,000 points and 100 partitions: 355 -> 245 us. Below BOUND_MIN_N the
-# two visits cost no more than the staging (3,000 points: 180 us both ways).
+# 1 GiB at 23,170, 16,384 with full rows), so that no estimate is needed; 10,000
+# points and 100 partitions: 355 -> 245 us. Below BOUND_MIN_N the two visits
+# cost no more than the staging (3,000 points: 180 us both ways).
 BOUND_MIN_N = 4096
 BOUND_MAX_ENTRIES = 1 << 28
 

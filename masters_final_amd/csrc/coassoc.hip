@@ -1082,9 +1082,8 @@ int64_t stage_chunk(const StageLayout& L, int64_t n, int full_rows, size_t stage
 }  // namespace
 }  // namespace eac
 
-// Plan (as eac_coassoc_count) plus the count pass over rows 0, stride,
-// 2 * stride, ...: h_estimate = their nnz sum x (rows / sampled rows),
-// rounded up. Keep ws for eac_coassoc_stage.
+// The plan alone (as eac_coassoc_count builds it); a label of k or more of its
+// partition is an error. Keep ws for eac_coassoc_stage.
 extern "C" int eac_coassoc_plan(const int32_t* labels, int64_t n, const int64_t* h_koff,
                                 int32_t P, void* ws, size_t ws_bytes, void* stream) {
   EAC_TRY(co_check(labels, n, h_koff, P));
@@ -1099,6 +1098,9 @@ extern "C" int eac_coassoc_plan(const int32_t* labels, int64_t n, const int64_t*
   return EAC_OK;
 }
 
+// Plan (as eac_coassoc_count) plus the count pass over rows 0, stride,
+// 2 * stride, ...: h_estimate = their nnz sum x (rows / sampled rows),
+// rounded up. Keep ws for eac_coassoc_stage.
 extern "C" int eac_coassoc_estimate(const int32_t* labels, int64_t n, const int64_t* h_koff,
                                     int32_t P, int32_t full_rows, int64_t sample_stride,
                                     int64_t* h_estimate, void* ws, size_t ws_bytes,

@@ -71,7 +71,9 @@ __device__ __forceinline__ uint32_t label_words(const int32_t* __restrict__ labe
     w[p] = in ? w[p] : 0u;
     any |= w[p];
   }
-  // 32 x 32 bit transposition: bit b of label p becomes bit p of word b
+  // bit b of label p becomes bit p of word b: the 32 x 32 bit-matrix
+  // transposition by halves of Hacker's Delight (Warren, section 7-3), blocks
+  // of 16, 8, 4, 2 and 1 swapped across the diagonal
 #pragma unroll
   for (int j = 16, m = 0xffff; j > 0; j >>= 1, m ^= m << j) {
 #pragma unroll

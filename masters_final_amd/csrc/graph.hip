@@ -2367,9 +2367,13 @@ int mst_forest(MstBuffers& B, int32_t n, int32_t* d_nf, hipStream_t s) {
 // Rounds enqueued before the first read-back: about what a graph of this size
 // needs, and one more for every further weight level (each ends with a round
 // that finds nothing; a graph dense enough for four, a co-association matrix
-// say, needs three more: 15 rounds at 10,000 vertices). One round too few costs the tail once more and two
-// host reads (100 us of 1,200 at a million vertices of degree 40, which need
-// 16), one too many the few microseconds of two launches that return at once.
+// say, needs three more: 15 rounds at 10,000 vertices). One round too few costs
+// the tail once more and two host reads (100 us of 1,200 at a million vertices
+// of degree 40, which need 16), one too many the few microseconds of two
+// launches that return at once. Against three quarters of the bound alone,
+// whole calls of 16,100 to 1,000,000 vertices, degree 5 to 40: 0.70 to 0.80 of
+// the time for most weighted graphs, 1.01 to 1.035 for a few, and 1.04 to 1.14
+// where all weights are equal (one level is enough; the rounds added are idle).
 inline int first_batch(int32_t n, int64_t m, int symmetric) {
   if (tune_value(EAC_TUNE_FIRST_BATCH) > 0) return tune_value(EAC_TUNE_FIRST_BATCH);
   const int vb = vbits_for(n), base = vb * 3 / 4 > 6 ? vb * 3 / 4 : 6;
@@ -3019,10 +3023,10 @@ __global__ __launch_bounds__(kSegT) void k_seg_cut(const uint64_t* __restrict__ 
 // times shorter every round (the first round makes one of a path whose
 // vertices are in order: the whole cut of 48,000 of them into five 0.47 ms, and
 // 8.8 with walks to the root; the union-find below 0.41). Edges that hook the
-// same root in one round overwrite each other, and a walk may pass over a link that is overwritten:
-// whoever made it is still listed and comes again, so the links and the
-// listed edges together always connect what the kept edges do. Parents only
-// fall, so no cycle forms. 64 graphs of 1,000 to 50,000 vertices: the
+// same root in one round overwrite each other, and a walk may pass over a link
+// that is overwritten: whoever made it is still listed and comes again, so the
+// links and the listed edges together always connect what the kept edges do.
+// Parents only fall, so no cycle forms. 64 graphs of 1,000 to 50,000 vertices: the
 // lock-free union-find over the union, its flattening and numbering (the
 // k_batch_* kernels) took 420 us, bound by dependent reads of memory; this 114.
 // They remain for larger graphs (`big`: one with kept edges; without any, as

@@ -31,7 +31,7 @@
 //    the rows it cannot certify (1% on the 64-d workload).
 //    4,194,304 x 64-d points, 2048 centroids: 4.00 -> 1.9 ms a pass (the
 //    single product 1.54, of which the group's FP64 comparison is a third;
-//    bound by vector issue), 300,007 x 37-d, 501 centroids: 239 -> 178 us.
+//    bound by vector issue), 300,007 x 37-d, 501 centroids: 239 -> 155 us.
 #include <algorithm>
 #include <cfloat>
 #include <climits>
@@ -51,14 +51,14 @@ namespace {
 // Layout of the split rows (points in registers, centroids in memory and
 // LDS). Every operand is scaled by a power of two (the centroids of a partition
 // by their largest coordinate, the points of a workgroup by that of most of
-// its rows, see kApart) into f16's normal range and split into two f16 halves, v = h + l + e; halves below
-// f16's smallest normal value are zero, so no product meets a subnormal. Three
-// products h.h + h.l + l.h make the contraction. For d where it saves MFMA
-// steps the three pieces are laid end to end over one K axis of 3 d entries
-// (points: h, l, h; centroids: h, h, l), 32 entries a step: ceil(3 d / 32)
-// steps; otherwise (3 d close to a multiple of 96) h and l are kept as rows
-// of KB = ceil(d / 32) fragments and used twice: 3 KB steps from 2 KB
-// fragments.
+// its rows, see kApart) into f16's normal range and split into two f16 halves,
+// v = h + l + e; halves below f16's smallest normal value are zero, so no
+// product meets a subnormal. Three products h.h + h.l + l.h make the
+// contraction. For d where it saves MFMA steps the three pieces are laid end to
+// end over one K axis of 3 d entries (points: h, l, h; centroids: h, h, l), 32
+// entries a step: ceil(3 d / 32) steps; otherwise (3 d close to a multiple of
+// 96) h and l are kept as rows of KB = ceil(d / 32) fragments and used twice:
+// 3 KB steps from 2 KB fragments.
 struct LabelLayout {
   int KS;      // MFMA steps (32 entries each)
   bool split;  // two rows of KS / 3 fragments
@@ -339,7 +339,7 @@ __device__ __forceinline__ void resolve16(const float* __restrict__ X, int d,
 // Centroid tiles are double buffered in LDS and shared by the block's four
 // waves; each fragment read feeds MB MFMAs.
 // TERMS = 1: only xh.ch (from the h rows of a split layout), a third of the
-// MFMAs with point_bound1, for the first pass of a cascade. LIST: the points
+// MFMAs with point_bound<1>, for the first pass of a cascade. LIST: the points
 // are the rows of a flag list. FUSE (one partition): the group is resolved in
 // the kernel and labels and dists are final.
 //
@@ -2502,7 +2502,7 @@ int kmeans_label(const float* X, int64_t n, int d, const float* C, const int64_t
 }
 
 struct UpdateBufs {
-  int32_t* eflag;  // [ktot + 1]: 1 for an empty cluster (the last entry is 0)
+  int32_t* eflag;  // [ktot + 1]: 1 for an empty cluster (the last entry is scanned, but no result holds it)
   int32_t* erank;  // [ktot + 1]
   uint64_t* dk;
   uint64_t* dks;
